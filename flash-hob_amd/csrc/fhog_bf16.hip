@@ -6,9 +6,11 @@
 //   pass 3  dQ2, ddO    Q-tiled   (fhog/triton_bwdbwd.py:257-313)        d=64: q_sweep_bf16<PASS=3>; d=128: fhog_bf16_pc.hip
 //   pass 4  dK2, dV2    K-tiled   (fhog/triton_bwdbwd.py:467-535)        d=64: k_sweep_bf16;         d=128: fhog_bf16_pc.hip
 //
-// Fused statistics sweep (PASS = 5, opt-in): b_i = sum_j P (E + ddS (dP - d)) - dd_i sum_j P dP
+// Fused statistics sweep (PASS = 5, what the default schedule runs): b_i = sum_j P (E + ddS (dP - d)) - dd_i sum_j P dP
 // needs dd_i only as a factor of a row sum, so dd and b come out of ONE sweep with the five products of pass 2
-// and three running sums per query; the three products of a separate pass 1 are saved.
+// and five running sums per query, all fp32; the three products of a separate pass 1 are saved. The sums are taken
+// over u = dP - d, which the accumulator of dP delivers by starting at -d: 7 VALU instructions and one exponential per
+// element, against 8 when they were taken over dP.
 // PASS = 7 (opt-in schedules whose second sweep already produced ddO, fhog_bf16_ddo.hip): pass 3 for dQ2 alone, d = 64.
 //
 // The kernels of this file are single-role: a workgroup is 256 threads = 4 wave64 owning 128 stationary rows,
@@ -150,7 +152,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
   const float dd = (PASS == 2 || P3) ? (CHAIN ? chain.dd : p.ws_dd[row]) : 0.f;
   const float b = P3 ? (CHAIN ? chain.b : p.ws_b[row]) : 0.f;
   const float kc = __builtin_fmaf(dd, dsum, b);   // per-row constant of dP' = E + (ddS - dd)(dP - d) - kc (passes 2, 3)
-  float red = 0.f, red_dd = 0.f, red_pdp = 0.f;  // the last two: fused sweep only
+  float red = 0.f, red_dd = 0.f, red_vdds = 0.f, red_pu = 0.f, red_p = 0.f;  // all but the first: fused sweep only
   // PASS 3 (d = 64): the second-level products follow in the same wave, with the S-shaped tiles as B operands
   // straight from the registers; lane = query, registers = output columns
   constexpr int NC = D / 32;
@@ -196,21 +198,24 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
         // shadow of the matrix pipe. LDS operands are fetched PF steps ahead.
         //   K  : S += K Q^T, ddS += K ddQ^T
         //   V  : dP += V dO^T            + P = exp2(S c - L)                       (pass 2)
-        //   ddK: ddS += ddK Q^T          + P (pass 1) | u = (dP - d) scale (fused)
+        //   ddK: ddS += ddK Q^T          + P (pass 1) | v = P u, sums of v and of P (fused; u = dP - d as in pass 2)
         //   ddV: E += ddV dO^T           + acc += P (ddS - dd) u   (pass 2: u = dP - d and E' = E - dd d come from
         //                                  accumulators that start at the row constants; with the tail, acc ends as
         //                                  sum P (E' + (ddS - dd) u) = sum P (E + ddS u - dP dd))
-        //                                | acc_dd += P ddS, acc_pdp += P dP, w = ddS u   (fused)
-        //   tail: acc += P ddS (pass 1) | acc += P E (pass 2) | acc += P (w + E) (fused)
+        //                                | acc_dd += P ddS, acc_vdds += v ddS   (fused)
+        //   tail: acc += P ddS (pass 1) | acc += P E (pass 2, fused)
         // Pass 3 (d = 64) runs the same stream with the elementwise work of the producer/consumer kernel (dS = P u behind
         // ddK; w = ddS scale - dd, ddP = P w, z = P (w u - dd d - b) behind ddV; dS' = P E + z in the tail), packs the four
         // tiles to 16 bits and goes on to the second-level products.
         constexpr int kTensorOfPhase[4] = {0, PASS == 1 ? 1 : 2, 1, 3};
         constexpr int NSTEP = NT * KK, PF = 2, NB = PF + 1, EPK = 16 / KK;
         f32x16_t s = {0}, dds = {0}, dp = {0}, e = {0}, pv, us, tt;
-        if (PASS == 2) {   // u = dP - d and E' = E - kc straight from the matrix pipe (in pass 3 this measured slower)
+        if (PASS == 2 || PASS == 5) {   // u = dP - d and E' = E - kc straight from the matrix pipe (in pass 3 this measured slower)
 #pragma unroll
-          for (int r = 0; r < 16; r++) dp[r] = -dsum, e[r] = -kc;
+          for (int r = 0; r < 16; r++) {
+            dp[r] = -dsum;
+            if (PASS == 2) e[r] = -kc;
+          }
         }
         uint32_t pk_ds[8], pk_ds2[8], pk_ddp[8], pk_p[8];   // PASS 3: packed dS, dS', ddP, P (registers 2i, 2i+1)
         bf16x8_t a[NB];
@@ -231,7 +236,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
             for (int r = EPK * kk; r < EPK * (kk + 1); r++) pv[r] = __builtin_amdgcn_exp2f(s[r] * c_scale_log2 - l_log2);
           } else if (ph == 2) {
             dds = mfma<F16>(a[c], Qb[kk], dds);
-            if (P3 && kk == 0 && masked) {
+            if ((P3 || PASS == 5) && kk == 0 && masked) {
               keep_branch();
 #pragma unroll
               for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
@@ -244,12 +249,14 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
                 dp[r] -= dsum;                           // u
                 us[r] = pv[r] * dp[r];                   // dS = P u (scale applied to the accumulator at the end)
               } else if (PASS == 5) {
-                us[r] = (dp[r] - dsum) * p.scale;
+                us[r] = pv[r] * dp[r];                   // v = P u
+                red_pu += us[r];
+                red_p += pv[r];
               }
             }
           } else {
             e = mfma<F16>(a[c], dOb[kk], e);
-            if (!P3 && kk == 0 && masked) {
+            if (PASS == 2 && kk == 0 && masked) {
               keep_branch();
 #pragma unroll
               for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
@@ -271,8 +278,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
                 }
               } else {
                 red_dd = __builtin_fmaf(pv[r], dds[r], red_dd);
-                red_pdp = __builtin_fmaf(pv[r], dp[r], red_pdp);
-                us[r] *= dds[r];
+                red_vdds = __builtin_fmaf(us[r], dds[r], red_vdds);
               }
             }
           }
@@ -286,10 +292,10 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
           }
 #pragma unroll
           for (int r = 0; r < 16; r++) red = __builtin_fmaf(pv[r], dds[r], red);   // scale applied once at the end
-        } else if (PASS == 2) {
+        } else if (!P3) {
 #pragma unroll
           for (int r = 0; r < 16; r++) red = __builtin_fmaf(pv[r], e[r], red);
-        } else if (P3) {
+        } else {
 #pragma unroll
           for (int r = 0; r < 16; r += 2)
             pk_ds2[r / 2] = pack2<F16>(__builtin_fmaf(pv[r], e[r], tt[r]), __builtin_fmaf(pv[r + 1], e[r + 1], tt[r + 1]));
@@ -347,9 +353,6 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
               __builtin_amdgcn_sched_barrier(0);
             }
           }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; r++) red = __builtin_fmaf(pv[r], us[r] + e[r], red);
         }
       }
     }
@@ -389,9 +392,12 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
     return;
   }
   red += __shfl_xor(red, 32);
+  float red_pdp = 0.f;
   if (PASS == 1) red *= p.scale;
   if (PASS == 5) {
+    red = __builtin_fmaf(p.scale, red_vdds + __shfl_xor(red_vdds, 32), red);
     red_dd += __shfl_xor(red_dd, 32);
+    red_pdp = __builtin_fmaf(dsum, red_p, red_pu);   // sum P dP of the keys of this lane's half
     red_pdp += __shfl_xor(red_pdp, 32);
   }
   if (p.n_split > 1) {   // partial sums [split][dd | b | sum P dP][batch * n_q]; combine_stats finishes the pass
