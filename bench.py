@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
 """Headline benchmark: attention double-backward on one MI355X.
 
-One "step" = one call of ``fhog.flash_bwdbwd`` (the reference's four passes dd, b, dQ'+ddO, dK'+dV'; the first also writes d) on
-seeded synthetic tensors that are already resident in HBM.  The workload is the configuration the
+One "step" = one call of ``fhog.flash_bwdbwd`` (its default schedule: the reference's passes dd and b as one sweep, which also
+writes d, then dQ'+ddO, then dK'+dV') on seeded synthetic tensors that are already resident in HBM.  The workload is the configuration the
 metric is quoted on: bf16 causal B=2 H=16 N=4096 d=128.
 
 Prints ONE JSON line.  ``value`` is the whole-path algorithmic throughput
@@ -25,10 +25,10 @@ for p in (ROOT / "flash-hob_amd", ROOT):
 
 PEAK_BF16_TFLOPS = 2516.6   # MI355X dense bf16 MFMA: 256 CU x 4096 FLOP/clk x 2.4 GHz
 PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA
-PASS_NAMES = {0: "rowdot_kernel (not in the 16-bit chain: its pass 1 writes d too)", 1: "q_sweep_bf16<pass 1: d, dd>",
-              2: "q_sweep_bf16<pass 2: b>",
+PASS_NAMES = {0: "rowdot_kernel (not in the 16-bit chain: its first sweep writes d too)",
+              1: "q_sweep_bf16<pass 1: d, dd> (four-pass schedule)", 2: "q_sweep_bf16<pass 2: b> (four-pass schedule)",
               3: "q_sweep3_pc<pass 3: dQ2, ddO>", 4: "k_sweep_pc<pass 4: dK2, dV2>",
-              5: "q_sweep_bf16<fused passes 1+2: d, dd, b> (opt-in schedule)",
+              5: "q_sweep_bf16<fused passes 1+2: d, dd, b> (default schedule)",
               6: "q_sweep_ddo<pass 6: b, ddO from dd> (opt-in schedule)",
               7: "q_sweep3_pc<pass 7: dQ2 alone> (opt-in schedules)",
               8: "q_sweep_ddo<pass 8: d, dd, b, ddO> (opt-in schedule)"}
@@ -232,11 +232,7 @@ def main():
 
     if args.profile_only:
         headline()
-        fused = fhog.BwdBwdPlan(x["Q"], x["K"], x["V"], o, x["dO"], x["ddQ"], x["ddK"], x["ddV"], L, w.scale,
-                                causal=w.causal, fused_stats=True)
-        for _ in range(3):
-            fused.run()   # the opt-in fused statistics sweep, so that it shows in the same trace
-        for name in ("ddo_early", "three_sweep"):   # ... and the schedules that take ddO out of the third sweep
+        for name in ("four_pass", "ddo_early", "three_sweep"):   # the other schedules, so that they show in the same trace
             alt = fhog.BwdBwdPlan(x["Q"], x["K"], x["V"], o, x["dO"], x["ddQ"], x["ddK"], x["ddV"], L, w.scale, causal=w.causal,
                                   schedule=name)
             for _ in range(3):
@@ -266,7 +262,7 @@ def main():
     per_pass = {i: t["mean"] for i, t in t_pass.items()}
     dom = max((i for i in per_pass if i <= 4), key=PASS_CONTRACTIONS.get)   # the kernel of the default schedule with the largest share of the work
     opt_in = {}
-    for name in ("fused_stats", "ddo_early", "three_sweep"):
+    for name in SCHEDULE_PRODUCTS:
         alt = fhog.BwdBwdPlan(x["Q"], x["K"], x["V"], o, x["dO"], x["ddQ"], x["ddK"], x["ddV"], L, w.scale, causal=w.causal,
                               schedule=name)
         alt.run()               # untimed first launch of the schedule's own kernels
@@ -310,9 +306,8 @@ def main():
         "ms_per_step_no_alloc_min": round(t_plan["min"], 4),
         "fused_stats_schedule": {"ms_per_step_no_alloc": round(ms_fused, 4),
                                  "value": round(w.flops_algorithmic / ms_fused / 1e9, 2),
-                                 "note": "opt-in: dd and b from one sweep (22 recomputed products instead of 25)"},
-        # every opt-in schedule on the same tensors (same algorithmic FLOP count, fewer recomputed products); `value`
-        # above is the reference's four-pass schedule (25)
+                                 "note": "the default: dd and b from one sweep (22 recomputed products instead of 25)"},
+        # every schedule on the same tensors (same algorithmic FLOP count, other numbers of recomputed products)
         "opt_in_schedules": opt_in,
         "ms_per_pass": {PASS_NAMES[i]: round(t, 4) for i, t in per_pass.items()},
         "ms_per_pass_median_min": {PASS_NAMES[i]: [round(t["median"], 4), round(t["min"], 4)] for i, t in t_pass.items()},
@@ -331,18 +326,18 @@ def main():
         out["first_order"] = fo
     out["mfma_sustained_tflops"] = mfma_sustained(dev)
     out["roofline"]["frac_of_sustained_random"] = round(dom_tflops / out["mfma_sustained_tflops"]["random"], 4)
-    # What a loop of nothing but MFMAs on random operands would leave of the algorithmic figure under the four-pass
-    # schedule, which issues 25 products for the 12 it is credited with: the ceiling of `value` on this box.
+    # What a loop of nothing but MFMAs on random operands would leave of the algorithmic figure under the default
+    # schedule, which issues 22 products for the 12 it is credited with: the ceiling of `value` on this box.
     sustained = out["mfma_sustained_tflops"]["random"]
     # ... and the same for a loop that also carries one LDS operand read and three VALU instructions per MFMA, the
     # instruction mix of the sweeps (still nothing the matrix pipe waits for: profiles/mfma_rate_instruction_mix.md)
     mix = out["mfma_sustained_tflops"]["random_lds_read_and_3_valu_per_mfma"]
     out["ceiling"] = {"sustained_random_tflops": sustained,
-                      "four_pass_algorithmic_tflops": round(sustained * 12 / 25, 1),
-                      "pct_of_ceiling": round(100 * value / (sustained * 12 / 25), 2),
+                      "algorithmic_tflops": round(sustained * 12 / 22, 1),
+                      "pct_of_ceiling": round(100 * value / (sustained * 12 / 22), 2),
                       "sustained_random_with_sweep_instruction_mix_tflops": mix,
-                      "four_pass_algorithmic_with_mix_tflops": round(mix * 12 / 25, 1),
-                      "pct_of_ceiling_with_mix": round(100 * value / (mix * 12 / 25), 2)}
+                      "algorithmic_with_mix_tflops": round(mix * 12 / 22, 1),
+                      "pct_of_ceiling_with_mix": round(100 * value / (mix * 12 / 22), 2)}
     if args.cpu_heads > 0:
         out["cpu_baseline"] = cpu_baseline(w, x_cpu, min(args.cpu_heads, w.batch), repeats=2)
     print(json.dumps(out))

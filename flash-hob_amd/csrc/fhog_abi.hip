@@ -401,19 +401,20 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   const int impl = select_impl(args);
   // Pass sequences. The first statistics sweep of the 16-bit family writes d_i itself: no separate launch for it there.
   // The schedules that take ddO out of the third sweep exist in the 16-bit family; the fp32-MFMA family runs the
-  // reference's four passes for them.
+  // fused one for them.
   static const int four[] = {FHOG_PASS_D, FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
   static const int fused[] = {FHOG_PASS_D, FHOG_PASS_DD_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
   static const int ddo_early[] = {FHOG_PASS_DD, FHOG_PASS_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   static const int three[] = {FHOG_PASS_DD_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   const int* order = four;
   int first = impl == FHOG_IMPL_BF16 ? 1 : 0, n_pass = 5;
+  const bool fp32 = impl != FHOG_IMPL_BF16;
   // d = 64, launch large enough to fill the GPU: the reference's own arrangement of its four passes, sweeps 1-3 in one launch
   static const int stage1[] = {FHOG_PASS_STAGE1, FHOG_PASS_DK_DV};
   if (args->schedule == FHOG_SCHEDULE_FOUR_PASS && impl == FHOG_IMPL_BF16 && args->d == 64 && fhog::tuning().stage1 != 0 &&
       granted_split(args, impl, FHOG_PASS_DQ_DDO) == 1 && granted_split(args, impl, FHOG_PASS_DD) == 1)
     order = stage1, first = 0, n_pass = 2;
-  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS) order = fused, n_pass = 4;
+  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (fp32 && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 4;
   // Passes 6-8 have no split form: a launch too small to fill the GPU whose workspace lets the reference's passes split
   // their streamed side runs the nearest schedule that can (three sweeps -> fused statistics, ddO early -> four passes).
   const bool small = granted_split(args, impl, FHOG_PASS_DQ_DDO) > 1;

@@ -275,5 +275,5 @@ class FlashAttention(torch.autograd.Function):
 def attention(q, k, v, is_causal=False, window: Optional[int] = None, schedule: Optional[str] = None):
     """Twice-differentiable scaled-dot-product attention (scale = d^-1/2). ``is_causal``: False | True |
     "bottom_right"; ``window``: sliding-window length on top of a causal mask; ``schedule``: pass schedule of the
-    double-backward (see :func:`fhog.flash_bwdbwd`; None = the reference's four passes)."""
+    double-backward (see :func:`fhog.flash_bwdbwd`; None = its default, three sweeps with ``dd`` and ``b`` from the first)."""
     return FlashAttention.apply(q, k, v, is_causal, window, schedule)

@@ -155,8 +155,8 @@ def main():
     P("Commands (from the repository root on one MI355X):\n")
     P(COMMANDS.replace("W=cfg2_bf16_causal_4096_d128", f"W={w.name}"))
     P("""
-`bench.py --profile-only` runs the timed loop of the default four-pass schedule, then three calls each of the opt-in
-schedules (fused statistics: pass 5 replaces passes 1 and 2; ddO early: `q_sweep_ddo<.., true>` = pass 6 and
+`bench.py --profile-only` runs the timed loop of the default schedule (pass 5, then 3 and 4), then three calls each of the
+others (four-pass: passes 1 and 2 instead of pass 5; ddO early: `q_sweep_ddo<.., true>` = pass 6 and
 `q_sweep3_pc<.., true>` = pass 7 replace passes 2 and 3; three sweeps: `q_sweep_ddo<.., false>` = pass 8, then pass 7),
 then three calls of the first-order kernels on the same tensors, then a streaming `torch.add` used to calibrate the byte
 counters. Template arguments of the kernels: `<fp16?, d, [pass,] mask mode[, waves per workgroup | variant]>` (mask mode

@@ -56,7 +56,7 @@ def main():
     ap.add_argument("--dtype", choices=["fp16", "bf16"], default="fp16")
     ap.add_argument("--budget-ms", type=float, default=3000.0, help="timed milliseconds per size (at least 3 calls)")
     ap.add_argument("--fused-stats", action="store_true")
-    ap.add_argument("--schedule", default=None, help="one of the opt-in schedules of flash_bwdbwd (default: the reference's four passes)")
+    ap.add_argument("--schedule", default=None, help="one of the opt-in schedules of flash_bwdbwd (default: that function's own)")
     args = ap.parse_args()
     dtype = {"fp16": torch.float16, "bf16": torch.bfloat16}[args.dtype]
     for n in [s for s in SIZES if s <= args.max_n]:

@@ -89,7 +89,8 @@ extern "C" {
 /* pass schedules of fhog_bwdbwd (fhog_bwdbwd_args.schedule) */
 #define FHOG_SCHEDULE_FOUR_PASS 0   /* the reference's schedule: d, then dd, b, dQ2+ddO, dK2+dV2 as four sweeps
                                        (fhog/triton_bwdbwd.py:185-313, 467-535); 25 recomputed products */
-#define FHOG_SCHEDULE_FUSED_STATS 1 /* opt-in: dd and b from one sweep (FHOG_PASS_DD_B), 22 recomputed products;
+#define FHOG_SCHEDULE_FUSED_STATS 1 /* dd and b from one sweep (FHOG_PASS_DD_B), 22 recomputed products (what the
+                                       Python entry points ask for when nothing is said);
                                        b differs from the four-pass value only by fp32 summation order */
 #define FHOG_SCHEDULE_DDO_EARLY 2   /* opt-in, still four sweeps in the reference's order: dd; b together with ddO
                                        (FHOG_PASS_B_DDO); dQ2 alone (FHOG_PASS_DQ); dK2+dV2. 23 recomputed products.
@@ -97,8 +98,8 @@ extern "C" {
 #define FHOG_SCHEDULE_THREE_SWEEP 3 /* opt-in, three sweeps: dd, b and ddO (FHOG_PASS_DD_B_DDO); dQ2 (FHOG_PASS_DQ);
                                        dK2+dV2. 20 recomputed products. ddP V is formed as (P o ddS) V - dd O with the
                                        caller's 16-bit O: accurate as long as dd_i does not dominate ddS_ij - dd_i.
-                                       Schedules 2 and 3 exist in the 16-bit MFMA family; the fp32-MFMA family runs the
-                                       four-pass schedule for them. Passes 6, 7 and 8 have no split form: a launch too
+                                       Schedules 2 and 3 exist in the 16-bit MFMA family; the fp32-MFMA family runs
+                                       schedule 1 for them. Passes 6, 7 and 8 have no split form: a launch too
                                        small to fill the GPU whose workspace allows a split (ws_bytes) runs the four
                                        passes (schedule 2) or the fused statistics sweep and passes 3, 4 (schedule 3) */
 
