@@ -163,6 +163,10 @@ int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
   return s;
 }
 
+// Family IMPL_FP32: split products on the 16-bit matrix instructions up to d = 64, fp32 MFMA at d = 128 (where the three
+// terms of the stationary operands do not fit the registers).
+bool on_split_kernels(const fhog_bwdbwd_args* a) { return a->d <= 64; }
+
 int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
   fhog::Params p = base;
   p.n_split = granted_split(a, impl, pass);
@@ -182,6 +186,8 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
     e = fhog::launch_rowdot(p, a->dtype, s);
   else if (impl == FHOG_IMPL_BF16)
     e = fhog::launch_bf16_pass(p, pass, s);
+  else if (on_split_kernels(a))
+    e = fhog::launch_split_pass(p, a->dtype, pass, s);
   else if (pass == FHOG_PASS_DD_B) {
     e = fhog::launch_fp32_pass(p, a->dtype, FHOG_PASS_DD, s);
     if (e == hipSuccess) e = fhog::launch_fp32_pass(p, a->dtype, FHOG_PASS_B, s);
@@ -399,7 +405,8 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (rc != FHOG_OK) return rc;
   const fhog::Params p = to_params(args);
   const int impl = select_impl(args);
-  // Pass sequences. The first statistics sweep of the 16-bit family writes d_i itself: no separate launch for it there.
+  // Pass sequences. The first statistics sweep of the 16-bit and the split-product kernels writes d_i itself: no separate
+  // launch for it there.
   // The schedules that take ddO out of the third sweep exist in the 16-bit family; the fp32-MFMA family runs the
   // fused one for them.
   static const int four[] = {FHOG_PASS_D, FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
@@ -407,8 +414,8 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   static const int ddo_early[] = {FHOG_PASS_DD, FHOG_PASS_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   static const int three[] = {FHOG_PASS_DD_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   const int* order = four;
-  int first = impl == FHOG_IMPL_BF16 ? 1 : 0, n_pass = 5;
   const bool fp32 = impl != FHOG_IMPL_BF16;
+  int first = fp32 && !on_split_kernels(args) ? 0 : 1, n_pass = 5;
   // d = 64, launch large enough to fill the GPU: the reference's own arrangement of its four passes, sweeps 1-3 in one launch
   static const int stage1[] = {FHOG_PASS_STAGE1, FHOG_PASS_DK_DV};
   if (args->schedule == FHOG_SCHEDULE_FOUR_PASS && impl == FHOG_IMPL_BF16 && args->d == 64 && fhog::tuning().stage1 != 0 &&

@@ -17,6 +17,7 @@ typedef __attribute__((address_space(3))) bf16x4_t* lds_bf16x4_ptr;
 template <int D>
 __device__ __forceinline__ int swz(int r) {
   if (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
+  if (D == 32) return ((r >> 2) & 3) ^ (r & 2);   // rows of 64 bytes, as in the operand tiles (sop_swz)
   return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
 template <int D>

@@ -1,0 +1,350 @@
+// Split-product kernels of the attention double-backward: products of fp32 accuracy on the 16-bit matrix instructions
+// (fhog_split_util.h). They serve fp32 tensors and d = 32 (and 16-bit tensors for which the fp32 family is asked for) at
+// head dims 32 and 64; fp32-accurate arithmetic throughout, no atomics, nothing of shape (N_Q, N_K) leaves the chip.
+//
+// One kernel template for the sweeps, with the arithmetic of the single-role 16-bit kernels (fhog_bf16.hip): a workgroup of
+// 4 wave64 owns 32 stationary rows per wave (queries in passes 1-3 and 5, keys in pass 4) and keeps their operands in
+// registers as bf16 terms; the other side streams through LDS in 32-row tiles, fetched into registers one step ahead,
+// split into terms once per workgroup and read by all four waves. First-level products have the streamed rows as M and
+// the stationary rows as N, so a lane owns ONE stationary row and its registers run over the streamed rows; split into
+// terms, such a tile is as it stands the B operand of the second-level products, whose A operand is a transposing read of
+// the staged tile in the same row order. Small launches (WS = 2 or 4) put WS waves on the same 32 rows instead: each takes
+// every WS-th streamed tile and the partial results are added through LDS in a fixed order.
+//
+// What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
+// 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (26 MFMAs beside some 450 VALU instructions).
+// Whole chain, us, against the fp32-MFMA kernels that served these shapes before (same box):
+//   bf16 causal 64 x 1024, d = 32: 734 -> 123     fp32 causal 64 x 1024, d = 32: 672 -> 318
+//   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
+// and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
+//
+// Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
+//   S = scale Q K^T, P = exp(S - L), dP = dO V^T, ddS = scale (ddQ K^T + Q ddK^T), E' = dO ddV^T - dd d - b
+//   dS = scale P u, ddP = P w, dS' = scale (P E' + ddP u)
+#include <type_traits>
+
+#include "fhog_split_util.h"
+
+namespace fhog {
+using namespace splitk;
+namespace {
+
+// PASS 1: d, dd; 2: b; 3: dQ2, ddO; 4: dK2, dV2 (K-tiled); 5: d, dd, b.
+template <typename T, int D, int PASS, int MASK, int WS>
+__global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Params p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
+  constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4);      // streamed tensors: K, ddK, V, ddV | Q, ddQ, dO
+  constexpr int NR = PASS == 1 ? 2 : (KSIDE ? 4 : 3);      // stationary tensors: Q, ddQ, dO | K, ddK, V, ddV
+  constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
+  using Stage = Stager<T, D, NT, !STATS>;
+  constexpr int TENSOR = Stage::PLANES * Stage::TILE;
+  constexpr int STAT = KSIDE ? 4 * TS * 4 : 0;             // L log2(e), -d, dd, -(dd d + b) of the 32 staged queries
+  constexpr int STAGE = Stage::BYTES + STAT;
+  constexpr int NBUF = WS == 1 ? 2 : 1;                    // with a wave split the WS tiles of a step take the room of the second buffer
+  constexpr int nw = 4 / WS, ROWS = 32 * nw;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wv / WS, ws = wv % WS;   // row group of the wave, and which of the streamed tiles of a step it takes
+  const int n = lane & 31, h = lane >> 5;
+  const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
+  int bh, tile;
+  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
+  const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
+  const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
+  const int rr = min(ri, n_sta - 1);         // rows past the end compute on a copy of the last row and store nothing
+  const T* src[NT];
+  if constexpr (KSIDE) {
+    src[0] = (const T*)p.q + qoff, src[1] = (const T*)p.ddq + qoff, src[2] = (const T*)p.dO + qoff;
+  } else {
+    src[0] = (const T*)p.k + koff, src[1] = (const T*)p.ddk + koff;
+    if constexpr (NT == 4) src[2] = (const T*)p.v + koff, src[3] = (const T*)p.ddv + koff;
+  }
+
+  typename std::conditional<KSIDE, StreamQueries<MASK>, StreamKeys<MASK>>::type geo(p.mask_off, p.window, n_str);
+  int t_begin, t_end;
+  geo.tile_range(r0, ROWS, t_begin, t_end);
+
+  const int64_t srow = (int64_t)bh * p.n_q;
+  Stage st[WS];
+  float stat_reg[WS] = {}, stat_d[WS] = {}, stat_dd[WS] = {};
+  // pass 4: thread t < 128 carries statistic t / 32 of staged query t % 32
+  const float* stat_src = p.lse;
+  if ((tid >> 5) == 1) stat_src = p.ws_d;
+  if ((tid >> 5) == 2) stat_src = p.ws_dd;
+  if ((tid >> 5) == 3) stat_src = p.ws_b;
+  const auto fetch = [&](int t) {
+#pragma unroll
+    for (int g = 0; g < WS; g++) {
+      const int row0 = (t + g) * TS;
+      st[g].fetch(src, str_ld, min(row0, n_str - 1), n_str, tid);   // a tile past the end is never computed on
+      if (KSIDE && tid < 4 * TS) {
+        const int64_t q = srow + min(row0 + (tid & 31), p.n_q - 1);
+        stat_reg[g] = stat_src[q];
+        if (tid >= 3 * TS) stat_d[g] = p.ws_d[q], stat_dd[g] = p.ws_dd[q];
+      }
+    }
+  };
+  const auto publish = [&](int buf) {
+#pragma unroll
+    for (int g = 0; g < WS; g++) {
+      char* stage = smem + (buf * WS + g) * STAGE;
+      st[g].publish(stage, tid);
+      if (KSIDE && tid < 4 * TS) {
+        const int k = tid / TS;
+        reinterpret_cast<float*>(stage + Stage::BYTES)[tid] =
+            k == 0 ? stat_reg[g] * kLog2e : k == 1 ? -stat_reg[g] : k == 2 ? stat_reg[g] : -__builtin_fmaf(stat_dd[g], stat_d[g], stat_reg[g]);
+      }
+    }
+  };
+  if (t_begin < t_end) fetch(t_begin);
+
+  bf16x8_t res[NR][KK][NF];
+  if constexpr (KSIDE) {
+    load_resident_terms<T, D>(res[0], (const T*)p.k + koff, sta_ld, rr, h);
+    load_resident_terms<T, D>(res[1], (const T*)p.ddk + koff, sta_ld, rr, h);
+    load_resident_terms<T, D>(res[2], (const T*)p.v + koff, sta_ld, rr, h);
+    load_resident_terms<T, D>(res[NR - 1], (const T*)p.ddv + koff, sta_ld, rr, h);
+  } else {
+    load_resident_terms<T, D>(res[0], (const T*)p.q + qoff, sta_ld, rr, h);
+    load_resident_terms<T, D>(res[1], (const T*)p.ddq + qoff, sta_ld, rr, h);
+    if constexpr (PASS != 1) load_resident_terms<T, D>(res[NR - 1], (const T*)p.dO + qoff, sta_ld, rr, h);
+  }
+  const int64_t row = srow + rr;   // Q-tiled passes
+  float l_log2 = 0.f, dsum = 0.f, dd = 0.f, b = 0.f;
+  if constexpr (!KSIDE) {
+    l_log2 = p.lse[row] * kLog2e;
+    if constexpr (PASS == 1 || PASS == 5) {
+      // d_i = sum_c O_ic dO_ic (fhog/triton_bwdbwd.py:580): each lane takes half of its query's row
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++) {
+        const Chunk<T> o = load_chunk<T>((const T*)p.o + qoff + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+        const Chunk<T> g = load_chunk<T>((const T*)p.dO + qoff + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+#pragma unroll
+        for (int e = 0; e < 8; e++) dsum = __builtin_fmaf(chunk_elem(o, e), chunk_elem(g, e), dsum);
+      }
+      dsum += __shfl_xor(dsum, 32);
+      if (h == 0 && ri < p.n_q && ws == 0) p.ws_d[row] = dsum;
+    } else {
+      dsum = p.ws_d[row], dd = p.ws_dd[row];
+      if constexpr (PASS == 3) b = p.ws_b[row];
+    }
+  }
+  const float kc = __builtin_fmaf(dd, dsum, b);
+  const float c_scale_log2 = p.scale * kLog2e;
+
+  int aoff[KK], troff[NC][2];
+#pragma unroll
+  for (int kk = 0; kk < KK; kk++) aoff[kk] = tile_off<D>(n, 2 * kk + h);
+#pragma unroll
+  for (int cb = 0; cb < NC; cb++) troff[cb][0] = tr_lane_off_acc<D>(cb, 0, lane), troff[cb][1] = tr_lane_off_acc<D>(cb, 1, lane);
+
+  f32x16_t acc0[NC], acc1[NC];     // dQ2, ddO | dK2, dV2: lane = stationary row, registers = columns
+#pragma unroll
+  for (int cb = 0; cb < NC; cb++) acc0[cb] = f32x16_t{0}, acc1[cb] = f32x16_t{0};
+  float red[5] = {};               // statistics: b-like sum; fused sweep: dd, sum P u ddS, sum P u, sum P
+
+  const auto block = [&](const char* stage, int s0) {
+    const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
+    f32x16_t s = {0}, dds = {0}, dp = {0}, e = {0};
+    // u = dP - d and E' = E - (dd d + b) come straight from accumulators that start at the row constants
+    if constexpr (KSIDE) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const f32x4_t md4 = *reinterpret_cast<const f32x4_t*>(stat + 1 * TS + 8 * g + 4 * h);
+        const f32x4_t mk4 = *reinterpret_cast<const f32x4_t*>(stat + 3 * TS + 8 * g + 4 * h);
+#pragma unroll
+        for (int i = 0; i < 4; i++) dp[4 * g + i] = md4[i], e[4 * g + i] = mk4[i];
+      }
+    } else if constexpr (PASS != 1) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        dp[r] = -dsum;
+        if (PASS != 5) e[r] = -kc;
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      bf16x8_t a[NT][NF];
+#pragma unroll
+      for (int x = 0; x < NT; x++) read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a[x]);
+      s = mma1<T>(s, a[0], res[0][kk]);                       // K Q^T | Q K^T
+      if constexpr (KSIDE) {
+        dds = mma1<T>(dds, a[1], res[0][kk]);                 // ddQ K^T
+        dp = mma1<T>(dp, a[2], res[2][kk]);                   // dO V^T
+        dds = mma1<T>(dds, a[0], res[1][kk]);                 // + Q ddK^T
+        e = mma1<T>(e, a[2], res[NR - 1][kk]);                // dO ddV^T
+      } else {
+        dds = mma1<T>(dds, a[0], res[1][kk]);                 // K ddQ^T
+        if constexpr (PASS != 1) dp = mma1<T>(dp, a[NT - 2], res[NR - 1][kk]);   // V dO^T
+        dds = mma1<T>(dds, a[1], res[0][kk]);                 // + ddK Q^T
+        if constexpr (PASS != 1) e = mma1<T>(e, a[NT - 1], res[NR - 1][kk]);     // ddV dO^T
+      }
+    }
+    f32x16_t pv;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      f32x4_t l4 = {l_log2, l_log2, l_log2, l_log2};
+      if constexpr (KSIDE) l4 = *reinterpret_cast<const f32x4_t*>(stat + 8 * g + 4 * h);
+#pragma unroll
+      for (int i = 0; i < 4; i++) pv[4 * g + i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * g + i], c_scale_log2, -l4[i]));
+    }
+    if (geo.partial(s0, rw)) {   // wave-uniform: the block holds hidden pairs (mask edge or tensor end)
+      int lo, hi;
+      geo.limits(s0, ri, h, lo, hi);
+      keep_branch();
+#pragma unroll
+      for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
+    }
+    if constexpr (PASS == 1) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) red[1] = __builtin_fmaf(pv[r], dds[r], red[1]);
+    } else if constexpr (PASS == 2) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) red[0] = __builtin_fmaf(pv[r], __builtin_fmaf(__builtin_fmaf(dds[r], p.scale, -dd), dp[r], e[r]), red[0]);
+    } else if constexpr (PASS == 5) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const float v = pv[r] * dp[r];
+        red[0] = __builtin_fmaf(pv[r], e[r], red[0]);
+        red[1] = __builtin_fmaf(pv[r], dds[r], red[1]);
+        red[2] = __builtin_fmaf(v, dds[r], red[2]);
+        red[3] += v;
+        red[4] += pv[r];
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        f32x4_t dd4 = {dd, dd, dd, dd};
+        if constexpr (KSIDE) dd4 = *reinterpret_cast<const f32x4_t*>(stat + 2 * TS + 8 * g + 4 * h);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int r = 4 * g + i;
+          dds[r] = pv[r] * __builtin_fmaf(dds[r], p.scale, -dd4[i]);   // ddP = P w
+          s[r] = pv[r] * dp[r];                                         // dS = P u (scale applied to the accumulators at the end)
+          e[r] = __builtin_fmaf(pv[r], e[r], dds[r] * dp[r]);           // dS' = P E' + ddP u
+        }
+      }
+      second_level<T, D>(acc0, stage + 1 * TENSOR, troff, s);           // dQ2 += dS ddK | dK2 += dS^T ddQ
+      second_level<T, D>(acc1, stage + 2 * TENSOR, troff, dds);         // ddO += ddP V | dV2 += ddP^T dO
+      second_level<T, D>(acc0, stage, troff, e);                        // dQ2 += dS' K | dK2 += dS'^T Q
+      if constexpr (!KSIDE) second_level<T, D>(acc1, stage + (NT - 1) * TENSOR, troff, pv);   // ddO += P ddV
+    }
+  };
+
+  if (t_begin < t_end) publish(0);
+  __syncthreads();
+  for (int t = t_begin; t < t_end; t += WS) {
+    const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
+    const bool more = t + WS < t_end;
+    if (more) fetch(t + WS);
+    const int s0 = (t + ws) * TS;
+    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0);
+    if (NBUF == 1) __syncthreads();   // the tiles are no longer read
+    if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
+    __syncthreads();
+  }
+
+  if constexpr (WS > 1) {
+    // the WS waves of a row group add their partial results in the order of ws; the wave with ws == 0 holds the sum
+    constexpr int VALS = STATS ? 5 : 2 * NC * 16;
+    float* const xch = reinterpret_cast<float*>(smem) + lane;
+    const auto each = [&](auto f) {
+      if constexpr (STATS) {
+#pragma unroll
+        for (int i = 0; i < 5; i++) f(red[i], i);
+      } else {
+#pragma unroll
+        for (int cb = 0; cb < NC; cb++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            float x = acc0[cb][r], y = acc1[cb][r];
+            f(x, cb * 16 + r), f(y, (NC + cb) * 16 + r);
+            acc0[cb][r] = x, acc1[cb][r] = y;
+          }
+      }
+    };
+    if (ws > 0) each([&](float& x, int i) { xch[((group * (WS - 1) + ws - 1) * VALS + i) * 64] = x; });
+    __syncthreads();
+    if (ws > 0) return;
+#pragma unroll
+    for (int o = 1; o < WS; o++) each([&](float& x, int i) { x += xch[((group * (WS - 1) + o - 1) * VALS + i) * 64]; });
+  }
+
+  if constexpr (STATS) {
+#pragma unroll
+    for (int i = 0; i < 5; i++) red[i] += __shfl_xor(red[i], 32);
+    if (h != 0 || ri >= p.n_q) return;
+    if constexpr (PASS == 2) {
+      p.ws_b[row] = red[0];
+    } else {
+      const float dd_i = red[1] * p.scale;
+      p.ws_dd[row] = dd_i;
+      if constexpr (PASS == 5)   // sum P (E + ddS u) - dd sum P dP
+        p.ws_b[row] = __builtin_fmaf(-dd_i, __builtin_fmaf(dsum, red[4], red[3]), __builtin_fmaf(p.scale, red[2], red[0]));
+    }
+  } else {
+    if (ri >= n_sta) return;
+    const int64_t out = (KSIDE ? koff : qoff) + (int64_t)ri * sta_ld;
+    store_rows<T, D>((T*)(KSIDE ? p.dk2 : p.dq2) + out, acc0, p.scale, h);
+    store_rows<T, D>((T*)(KSIDE ? p.dv2 : p.ddo) + out, acc1, 1.f, h);
+  }
+}
+
+template <typename T, int D, int PASS, int MASK, int WS>
+hipError_t launch_ws(const Params& p, hipStream_t s) {
+  constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
+  constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4), nw = 4 / WS;
+  constexpr int stage = Stager<T, D, NT, !STATS>::BYTES + (KSIDE ? 4 * TS * 4 : 0);
+  constexpr int xch = WS > 1 ? nw * (WS - 1) * (STATS ? 5 : 2 * D / 32 * 16) * 64 * 4 : 0;
+  constexpr int smem = (WS == 1 ? 2 : WS) * stage > xch ? (WS == 1 ? 2 : WS) * stage : xch;
+  static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
+  const int n_rows = KSIDE ? p.n_k : p.n_q;
+  const hipError_t e = allow_dynamic_lds<split_sweep<T, D, PASS, MASK, WS>>(smem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((split_sweep<T, D, PASS, MASK, WS>), dim3(grid_blocks((n_rows + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
+  return hipGetLastError();
+}
+
+// Four waves on 128 stationary rows share the streamed tiles and their splitting, the best shape whenever that fills the GPU
+// (256 CUs). With fewer than 128 (64) such workgroups two (four) waves go on the same 32 rows, where the tiles of a step fit
+// the LDS: two fp32 heads of 256 tokens are 4 workgroups otherwise, each running its eight streamed tiles one after the other.
+template <typename T, int D, int PASS, int MASK>
+hipError_t launch_sweep(const Params& p, hipStream_t s) {
+  const int64_t groups = (int64_t)((PASS == 4 ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = PASS == 4 ? p.n_q : p.n_k;
+  if constexpr (D == 32 || std::is_same<T, __bf16>::value) {   // the four tiles of a step fit the LDS
+    if (groups < 64 && n_str > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
+  }
+  if (groups < 128 && n_str > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
+  return launch_ws<T, D, PASS, MASK, 1>(p, s);
+}
+
+template <typename T, int D>
+hipError_t launch_td(const Params& p, int pass, hipStream_t s) {
+#define FHOG_SPLIT_PASS(N) (p.causal ? launch_sweep<T, D, N, MASK_BAND>(p, s) : launch_sweep<T, D, N, MASK_NONE>(p, s))
+  switch (pass) {
+    case FHOG_PASS_DD: return FHOG_SPLIT_PASS(1);
+    case FHOG_PASS_B: return FHOG_SPLIT_PASS(2);
+    case FHOG_PASS_DQ_DDO: return FHOG_SPLIT_PASS(3);
+    case FHOG_PASS_DK_DV: return FHOG_SPLIT_PASS(4);
+    case FHOG_PASS_DD_B: return FHOG_SPLIT_PASS(5);
+    default: return hipErrorInvalidValue;
+  }
+#undef FHOG_SPLIT_PASS
+}
+
+template <typename T>
+hipError_t launch_t(const Params& p, int pass, hipStream_t s) {
+  return p.d == 32 ? launch_td<T, 32>(p, pass, s) : p.d == 64 ? launch_td<T, 64>(p, pass, s) : hipErrorInvalidValue;
+}
+
+}  // namespace
+
+hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s) {
+  if (dtype == FHOG_DTYPE_FP32) return launch_t<float>(p, pass, s);
+  return dtype == FHOG_DTYPE_FP16 ? launch_t<_Float16>(p, pass, s) : launch_t<__bf16>(p, pass, s);
+}
+
+}  // namespace fhog

@@ -1,0 +1,239 @@
+// Device helpers of the split-product kernels (gfx950): contractions of fp32 accuracy on the 16-bit matrix instructions.
+//
+// An fp32 number is the exact sum of three bf16 numbers (8 significant bits each: 24 in all), a fp16 number of two, and a
+// bf16 number is one. A product of two such sums is a sum of bf16 products, each exact in fp32, accumulated in fp32 by
+// v_mfma_f32_32x32x16_bf16, which does 16 times the work of v_mfma_f32_32x32x2_f32 per cycle. Six of the nine terms of
+// an fp32 product are kept; the three left out are below 2^-24 of it, the rounding of one fp32 addition.
+// The S-shaped operands of the second-level products (P, dS, dS', ddP) are split the same way: three terms for fp32
+// tensors; two for 16-bit tensors, whose results are rounded to 11 or 8 bits while two terms carry 16.
+#pragma once
+#include "fhog_bf16_util.h"
+
+namespace fhog {
+namespace splitk {
+using namespace bf16k;
+
+// How a tensor type meets the matrix instructions.
+//   NF   terms of a tensor in the first-level products (tensor x tensor); F16: they are fp16 as they stand
+//   N2   bf16 terms of a tensor in the second-level products (tensor x S-shaped operand); NS: terms of that operand
+//   LDS1, LDS2   planes of a staged tile when only first-level products read it / when both do; OFF2: first plane of the latter
+template <typename T>
+struct Terms;
+template <>
+struct Terms<__bf16> {
+  static constexpr int NF = 1, N2 = 1, NS = 2, LDS1 = 1, LDS2 = 1, OFF2 = 0;
+  static constexpr bool F16 = false;
+};
+template <>
+struct Terms<_Float16> {
+  static constexpr int NF = 1, N2 = 2, NS = 2, LDS1 = 1, LDS2 = 3, OFF2 = 1;
+  static constexpr bool F16 = true;
+};
+template <>
+struct Terms<float> {
+  static constexpr int NF = 3, N2 = 3, NS = 3, LDS1 = 3, LDS2 = 3, OFF2 = 0;
+  static constexpr bool F16 = false;
+};
+
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
+
+// (a, b) -> N packed bf16 terms, each the rounded rest of what the ones before left: x = x0 + x1 (+ x2), exactly for N = 3.
+// The rest x - x0 is exact in fp32; a two-element dot product against (-1, 0) or (0, -1) takes it without unpacking x0.
+template <int N>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&out)[N]) {
+  // The constants are handed over in registers: as the inline operand -1.0, which the compiler uses for the first one, the
+  // instruction did not multiply the low element by -1.
+  uint32_t c0, c1;
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(c0));
+  asm("s_mov_b32 %0, 0xbf800000" : "=s"(c1));
+  const bf16x2_t first = __builtin_bit_cast(bf16x2_t, c0), second = __builtin_bit_cast(bf16x2_t, c1);
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const bf16x2_t t = {(__bf16)a, (__bf16)b};
+    out[i] = __builtin_bit_cast(uint32_t, t);
+    if (i + 1 < N) {
+      a = __builtin_amdgcn_fdot2_f32_bf16(t, first, a, false);
+      b = __builtin_amdgcn_fdot2_f32_bf16(t, second, b, false);
+    }
+  }
+}
+
+// Registers 8t .. 8t+7 of an S-shaped fp32 tile as the B operand of second-level k-step t, in N terms.
+template <int N>
+__device__ __forceinline__ void split_operand(const f32x16_t& x, int t, bf16x8_t (&out)[N]) {
+  u32x4_t u[N];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    uint32_t w[N];
+    split_pair<N>(x[8 * t + 2 * i], x[8 * t + 2 * i + 1], w);
+#pragma unroll
+    for (int s = 0; s < N; s++) u[s][i] = w[s];
+  }
+#pragma unroll
+  for (int s = 0; s < N; s++) out[s] = __builtin_bit_cast(bf16x8_t, u[s]);
+}
+
+// Eight consecutive elements of a row as they lie in memory.
+template <typename T>
+struct Chunk {
+  u32x4_t v[sizeof(T) / 2];
+};
+template <typename T>
+__device__ __forceinline__ Chunk<T> load_chunk(const T* p) {
+  Chunk<T> c;
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(T) / 2; i++) c.v[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(p) + 16 * i);
+  return c;
+}
+template <typename T>
+__device__ __forceinline__ float chunk_elem(const Chunk<T>& c, int e) {
+  if constexpr (sizeof(T) == 4) {
+    const uint32_t bits = c.v[e / 4][e % 4];
+    return __builtin_bit_cast(float, bits);
+  } else {
+    const uint16_t bits = (uint16_t)(c.v[0][e / 2] >> (16 * (e & 1)));
+    return (float)__builtin_bit_cast(T, bits);
+  }
+}
+// ... and its terms: FIRST: those of the first-level products (fp16 stays as it is), else the bf16 terms of the second level
+template <typename T, bool FIRST, int N>
+__device__ __forceinline__ void chunk_terms(const Chunk<T>& c, bf16x8_t (&out)[N]) {
+  if constexpr (sizeof(T) == 2 && (FIRST || N == 1)) {
+    out[0] = __builtin_bit_cast(bf16x8_t, c.v[0]);
+  } else {
+    u32x4_t u[N];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uint32_t w[N];
+      split_pair<N>(chunk_elem(c, 2 * i), chunk_elem(c, 2 * i + 1), w);
+#pragma unroll
+      for (int s = 0; s < N; s++) u[s][i] = w[s];
+    }
+#pragma unroll
+    for (int s = 0; s < N; s++) out[s] = __builtin_bit_cast(bf16x8_t, u[s]);
+  }
+}
+
+// First-level operand of one stationary row: lane (n = lane % 32, h = lane / 32) holds row n, elements 16 kk + 8 h .. + 7.
+template <typename T, int D>
+__device__ __forceinline__ void load_resident_terms(bf16x8_t (&dst)[D / 16][Terms<T>::NF], const T* base, int64_t ld, int row, int h) {
+#pragma unroll
+  for (int kk = 0; kk < D / 16; kk++)
+    chunk_terms<T, true, Terms<T>::NF>(load_chunk<T>(base + (int64_t)row * ld + 16 * kk + 8 * h), dst[kk]);
+}
+
+// acc += a b for operands in NF terms each; the small terms first
+template <typename T>
+__device__ __forceinline__ f32x16_t mma1(f32x16_t acc, const bf16x8_t (&a)[Terms<T>::NF], const bf16x8_t (&b)[Terms<T>::NF]) {
+  constexpr int NF = Terms<T>::NF;
+#pragma unroll
+  for (int order = NF - 1; order >= 0; order--)
+#pragma unroll
+    for (int i = order; i >= 0; i--) acc = mfma<Terms<T>::F16>(a[i], b[order - i], acc);
+  return acc;
+}
+// acc += a b for a tensor operand in N2 terms and an S-shaped one in NS terms
+template <typename T>
+__device__ __forceinline__ f32x16_t mma2(f32x16_t acc, const bf16x8_t (&a)[Terms<T>::N2], const bf16x8_t (&b)[Terms<T>::NS]) {
+  constexpr int N2 = Terms<T>::N2, NS = Terms<T>::NS;
+#pragma unroll
+  for (int order = NS - 1; order >= 0; order--)
+#pragma unroll
+    for (int i = order < N2 ? order : N2 - 1; i >= 0; i--) acc = mfma<false>(a[i], b[order - i], acc);
+  return acc;
+}
+
+// Staging of NX tensors' 32-row tiles by 256 threads through registers: the global loads of the next tile are issued before
+// a step's arithmetic and the split terms written to LDS behind it. Tile planes are 32 rows of D 16-bit elements, swizzled
+// in 16-byte chunks (tile_off); plane q of tensor x starts at (x * PLANES + q) * TILE. Rows past the end of a tensor
+// are copies of its last row, as in the 16-bit kernels.
+template <typename T, int D, int NX, bool SECOND>
+struct Stager {
+  static constexpr int PLANES = SECOND ? Terms<T>::LDS2 : Terms<T>::LDS1;
+  static constexpr int TILE = TS * 2 * D, BYTES = NX * PLANES * TILE;
+  static constexpr int CPR = D / 8;                                // chunks per row
+  static constexpr int PER_TENSOR = TS * CPR;                      // 128 (d = 32) or 256: a wave's chunks are of one tensor
+  static constexpr int XPI = 256 / PER_TENSOR;                     // tensors per round of 256 threads
+  static constexpr int PER = (NX + XPI - 1) / XPI;
+  static_assert(PER_TENSOR == 128 || PER_TENSOR == 256, "d = 32 or 64");
+  Chunk<T> c[PER];
+
+  __device__ __forceinline__ static int tensor_of(int i, int tid) { return XPI * i + (XPI == 2 ? tid >> 7 : 0); }
+  __device__ __forceinline__ void fetch(const T* const (&src)[NX], int64_t ld, int row0, int n_rows, int tid) {
+    const int r = tid / CPR % TS, ch = tid % CPR;
+    const int off = min(r, n_rows - 1 - row0) * (int)ld + 8 * ch;   // row strides are below 2^24 elements
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const T* base = src[XPI * i];
+      if (XPI == 2 && XPI * i + 1 < NX) base = tid >> 7 ? src[XPI * i + 1 < NX ? XPI * i + 1 : 0] : base;
+      if (NX % XPI && tensor_of(i, tid) >= NX) continue;
+      c[i] = load_chunk<T>(base + (int64_t)row0 * ld + off);
+    }
+  }
+  __device__ __forceinline__ void publish(char* stage, int tid) const {
+    const int r = tid / CPR % TS, ch = tid % CPR;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      if (NX % XPI && tensor_of(i, tid) >= NX) continue;
+      char* dst = stage + tensor_of(i, tid) * PLANES * TILE + tile_off<D>(r, ch);
+      bf16x8_t f[Terms<T>::NF];
+      chunk_terms<T, true, Terms<T>::NF>(c[i], f);
+#pragma unroll
+      for (int q = 0; q < Terms<T>::NF; q++) *reinterpret_cast<bf16x8_t*>(dst + q * TILE) = f[q];
+      if constexpr (SECOND && Terms<T>::OFF2 > 0) {
+        bf16x8_t s[Terms<T>::N2];
+        chunk_terms<T, false, Terms<T>::N2>(c[i], s);
+#pragma unroll
+        for (int q = 0; q < Terms<T>::N2; q++) *reinterpret_cast<bf16x8_t*>(dst + (Terms<T>::OFF2 + q) * TILE) = s[q];
+      }
+    }
+  }
+};
+
+// First-level A operand of k-step kk from a staged tensor (row = lane % 32): off = tile_off<D>(n, 2 kk + h)
+template <typename T, int TILE>
+__device__ __forceinline__ void read_terms(const char* tensor, int off, bf16x8_t (&a)[Terms<T>::NF]) {
+#pragma unroll
+  for (int q = 0; q < Terms<T>::NF; q++) a[q] = lds_read128(tensor + q * TILE, off);
+}
+// Second-level A operand of k-step t (transposed): o0 / o1 = tr_lane_off_acc<D>(cb, 0 / 1)
+template <typename T, int D>
+__device__ __forceinline__ void read_terms_tr(const char* tensor, int o0, int o1, int t, bf16x8_t (&a)[Terms<T>::N2]) {
+  constexpr int TILE = TS * 2 * D;
+#pragma unroll
+  for (int q = 0; q < Terms<T>::N2; q++)
+    a[q] = lds_read_tr_pre(tensor + o0, tensor + o1, (Terms<T>::OFF2 + q) * TILE + t * 16 * 2 * D);
+}
+
+// acc += X^T W for a staged tensor X (32 rows) and an S-shaped tile W whose registers run over those rows
+template <typename T, int D>
+__device__ __forceinline__ void second_level(f32x16_t (&acc)[D / 32], const char* tensor, const int (&troff)[D / 32][2], const f32x16_t& w) {
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    bf16x8_t op[Terms<T>::NS];
+    split_operand<Terms<T>::NS>(w, t, op);
+#pragma unroll
+    for (int cb = 0; cb < D / 32; cb++) {
+      bf16x8_t a[Terms<T>::N2];
+      read_terms_tr<T, D>(tensor, troff[cb][0], troff[cb][1], t, a);
+      acc[cb] = mma2<T>(acc[cb], a, op);
+    }
+  }
+}
+
+// acc[cb][r] holds column cb*32 + 8*(r/4) + 4*h + r%4 of the lane's stationary row
+template <typename T, int D>
+__device__ __forceinline__ void store_rows(T* row, const f32x16_t (&acc)[D / 32], float scale, int h) {
+#pragma unroll
+  for (int cb = 0; cb < D / 32; cb++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float x[4] = {acc[cb][4 * g] * scale, acc[cb][4 * g + 1] * scale, acc[cb][4 * g + 2] * scale, acc[cb][4 * g + 3] * scale};
+      T* dst = row + cb * 32 + 8 * g + 4 * h;
+      if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{x[0], x[1], x[2], x[3]};
+      else *reinterpret_cast<u32x2_t*>(dst) = pack4<Terms<T>::F16>(x[0], x[1], x[2], x[3]);
+    }
+}
+
+}  // namespace splitk
+}  // namespace fhog
