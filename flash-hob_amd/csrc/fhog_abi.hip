@@ -198,7 +198,7 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
 }
 
 // bf16 / fp16 tensors with d in {64, 128} run on the 16-bit MFMA kernels, everything else (fp32 tensors, d = 32) on the
-// fp32-MFMA ones
+// split-product ones
 bool attn_on_16bit_kernels(const fhog_attn_args* a) { return a->dtype != FHOG_DTYPE_FP32 && (a->d == 64 || a->d == 128); }
 
 int validate_attn(const fhog_attn_args* a, int backward) {
@@ -337,7 +337,7 @@ int fhog_attn_fwd(const fhog_attn_args* args, void* hip_stream) {
   const int rc = validate_attn(args, 0);
   if (rc != FHOG_OK) return rc;
   const hipError_t e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(to_attn_params(args), 0, (hipStream_t)hip_stream)
-                                                   : fhog::launch_attn_fp32(to_attn_params(args), args->dtype, 0, (hipStream_t)hip_stream);
+                                                   : fhog::launch_attn_split(to_attn_params(args), args->dtype, 0, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention forward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }
@@ -355,10 +355,11 @@ int fhog_attn_bwd(const fhog_attn_args* args, void* hip_stream) {
   rd.batch = p.batch;
   rd.n_q = p.n_q;
   rd.d = p.d;
-  hipError_t e = fhog::launch_rowdot(rd, args->dtype, (hipStream_t)hip_stream);
+  // (the split-product kernel for dQ takes them itself)
+  hipError_t e = attn_on_16bit_kernels(args) ? fhog::launch_rowdot(rd, args->dtype, (hipStream_t)hip_stream) : hipSuccess;
   for (int which = 1; which <= 2 && e == hipSuccess; which++)
     e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(p, which, (hipStream_t)hip_stream)
-                                    : fhog::launch_attn_fp32(p, args->dtype, which, (hipStream_t)hip_stream);
+                                    : fhog::launch_attn_split(p, args->dtype, which, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention backward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }

@@ -1,0 +1,308 @@
+// First-order attention on split products (fhog_split_util.h): contractions of fp32 accuracy on the 16-bit matrix
+// instructions. Forward (O and the fp32 log-sum-exp L, online soft-max; fhog/triton_flash.py:12-133, 252-258) and backward
+// (dQ; dK and dV; the arithmetic of fhog/triton_flash.py:201-220 without the (batch, N_Q, N_K) tensors and without
+// atomics). Serves fp32 tensors and d = 32, the shapes the 16-bit kernels of fhog_attn.hip do not take.
+//
+// Same shape as the double-backward kernels of fhog_split.hip: a workgroup of 4 wave64 owns 32 stationary rows per wave
+// (queries; keys in the K-tiled backward) with their operands in registers as bf16 terms, the other side streams through
+// LDS in 32-row tiles that are split once per workgroup. A lane owns ONE stationary row: in the forward the running maximum,
+// the running sum and the rescaling factor of a query are per-lane scalars. Two terms per fp32 operand less than the
+// double-backward needs leave room for the terms of d = 128 (one wave per SIMD).
+// Small launches (WS = 2 or 4) put WS waves on the same 32 rows: each takes every WS-th streamed tile, and the partial
+// results are merged through LDS in a fixed order.
+#include <type_traits>
+
+#include "fhog_split_util.h"
+
+namespace fhog {
+using namespace splitk;
+namespace {
+
+constexpr int MODE_FWD = 0, MODE_BWD_Q = 1, MODE_BWD_K = 2;
+
+template <typename T, int D, int MODE, int MASK, int WS>
+__global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) attn_split(AttnParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr bool KSIDE = MODE == MODE_BWD_K;
+  constexpr int NR = MODE == MODE_FWD ? 1 : 2;             // stationary tensors: Q | Q, dO | K, V
+  constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
+  using Stage = Stager<T, D, 2, true>;                     // streamed tensors: K, V | Q, dO
+  constexpr int TENSOR = Stage::PLANES * Stage::TILE;
+  constexpr int STAT = KSIDE ? 2 * TS * 4 : 0;             // L log2(e), -d of the 32 staged queries
+  constexpr int STAGE = Stage::BYTES + STAT;
+  constexpr int NBUF = WS == 1 ? 2 : 1;                    // with a wave split the WS tiles of a step take the room of the second buffer
+  constexpr int nw = 4 / WS, ROWS = 32 * nw;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wv / WS, ws = wv % WS;   // row group of the wave, and which of the streamed tiles of a step it takes
+  const int n = lane & 31, h = lane >> 5;
+  const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
+  int bh, tile;
+  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile)) return;
+  const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
+  const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
+  const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
+  const int rr = min(ri, n_sta - 1);         // rows past the end compute on a copy of the last row and store nothing
+  const T* const src[2] = {KSIDE ? (const T*)p.q + qoff : (const T*)p.k + koff, KSIDE ? (const T*)p.dO + qoff : (const T*)p.v + koff};
+
+  typename std::conditional<KSIDE, StreamQueries<MASK>, StreamKeys<MASK>>::type geo(p.mask_off, p.window, n_str);
+  int t_begin, t_end;
+  geo.tile_range(r0, ROWS, t_begin, t_end);
+
+  const int64_t srow = (int64_t)bh * p.n_q;
+  Stage st[WS];
+  float stat_reg[WS] = {};
+  const auto fetch = [&](int t) {
+#pragma unroll
+    for (int g = 0; g < WS; g++) {
+      const int row0 = (t + g) * TS;
+      st[g].fetch(src, str_ld, min(row0, n_str - 1), n_str, tid);   // a tile past the end is never computed on
+      if (KSIDE && tid < 2 * TS) stat_reg[g] = (tid < TS ? p.lse : p.ws_d)[srow + min(row0 + (tid & 31), p.n_q - 1)];
+    }
+  };
+  const auto publish = [&](int buf) {
+#pragma unroll
+    for (int g = 0; g < WS; g++) {
+      char* stage = smem + (buf * WS + g) * STAGE;
+      st[g].publish(stage, tid);
+      if (KSIDE && tid < 2 * TS) reinterpret_cast<float*>(stage + Stage::BYTES)[tid] = tid < TS ? stat_reg[g] * kLog2e : -stat_reg[g];
+    }
+  };
+  if (t_begin < t_end) fetch(t_begin);
+
+  bf16x8_t res[NR][KK][NF];
+  load_resident_terms<T, D>(res[0], KSIDE ? (const T*)p.k + koff : (const T*)p.q + qoff, sta_ld, rr, h);
+  if constexpr (MODE != MODE_FWD)
+    load_resident_terms<T, D>(res[NR - 1], KSIDE ? (const T*)p.v + koff : (const T*)p.dO + qoff, sta_ld, rr, h);
+  const int64_t row = srow + rr;   // Q-tiled kernels
+  float l_log2 = 0.f, dsum = 0.f;
+  if constexpr (MODE == MODE_BWD_Q) {
+    // d_i = sum_c O_ic dO_ic, for this sweep and (through the workspace) for the K-tiled one behind it: each lane takes
+    // half of its query's row
+    l_log2 = p.lse[row] * kLog2e;
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      const Chunk<T> o = load_chunk<T>((const T*)p.o + qoff + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+      const Chunk<T> g = load_chunk<T>((const T*)p.dO + qoff + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+#pragma unroll
+      for (int e = 0; e < 8; e++) dsum = __builtin_fmaf(chunk_elem(o, e), chunk_elem(g, e), dsum);
+    }
+    dsum += __shfl_xor(dsum, 32);
+    if (h == 0 && ri < p.n_q && ws == 0) p.ws_d[row] = dsum;
+  }
+  const float c_scale_log2 = p.scale * kLog2e;
+
+  int aoff[KK], troff[NC][2];
+#pragma unroll
+  for (int kk = 0; kk < KK; kk++) aoff[kk] = tile_off<D>(n, 2 * kk + h);
+#pragma unroll
+  for (int cb = 0; cb < NC; cb++) troff[cb][0] = tr_lane_off_acc<D>(cb, 0, lane), troff[cb][1] = tr_lane_off_acc<D>(cb, 1, lane);
+
+  float m = -INFINITY, l = 0.f;    // forward: running maximum (log2 units) of the row; this lane's half of the row sum
+  f32x16_t acc0[NC], acc1[NC];     // O | dQ | dK, dV: lane = stationary row, registers = columns
+#pragma unroll
+  for (int cb = 0; cb < NC; cb++) acc0[cb] = f32x16_t{0}, acc1[cb] = f32x16_t{0};
+
+  const auto block = [&](const char* stage, int s0) {
+    const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
+    f32x16_t s = {0}, dp = {0};
+    if constexpr (MODE == MODE_BWD_Q) {   // u = dP - d comes straight from an accumulator that starts at -d
+#pragma unroll
+      for (int r = 0; r < 16; r++) dp[r] = -dsum;
+    } else if constexpr (KSIDE) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const f32x4_t md4 = *reinterpret_cast<const f32x4_t*>(stat + TS + 8 * g + 4 * h);
+#pragma unroll
+        for (int i = 0; i < 4; i++) dp[4 * g + i] = md4[i];
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      bf16x8_t a[NF];
+      read_terms<T, Stage::TILE>(stage, aoff[kk], a);
+      s = mma1<T>(s, a, res[0][kk]);                          // K Q^T | Q K^T
+      if constexpr (MODE != MODE_FWD) {
+        bf16x8_t g[NF];
+        read_terms<T, Stage::TILE>(stage + TENSOR, aoff[kk], g);
+        dp = mma1<T>(dp, g, res[NR - 1][kk]);                 // V dO^T | dO V^T
+      }
+    }
+    const bool masked = geo.partial(s0, rw);   // wave-uniform: the block holds hidden pairs (mask edge or tensor end)
+    int lo = 0, hi = 0;
+    if (masked) keep_branch(), geo.limits(s0, ri, h, lo, hi);
+    f32x16_t pv;
+    if constexpr (MODE == MODE_FWD) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[r] *= c_scale_log2;      // before the maximum is taken: any sign of the scale
+      if (masked) {
+        keep_branch();
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = in_limits(r, lo, hi) ? s[r] : -INFINITY;
+      }
+      float tmax = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+      for (int r = 3; r < 15; r += 2) tmax = fmaxf(fmaxf(tmax, s[r]), s[r + 1]);
+      tmax = fmaxf(tmax, s[15]);
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));   // the other half of the wave holds the other 16 keys of the row
+      const float m_new = fmaxf(m, tmax);
+      const float m_ref = m_new == -INFINITY ? 0.f : m_new;   // a row that has seen no key yet keeps its state
+      const float alpha = __builtin_amdgcn_exp2f(m - m_ref);
+      float rs = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        pv[r] = __builtin_amdgcn_exp2f(s[r] - m_ref);
+        rs += pv[r];
+      }
+      l = __builtin_fmaf(l, alpha, rs);
+      if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {   // rescale only when some row's maximum moved
+#pragma unroll
+        for (int cb = 0; cb < NC; cb++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc0[cb][r] *= alpha;
+      }
+      m = m_new;
+      second_level<T, D>(acc0, stage + TENSOR, troff, pv);    // O += P V
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        f32x4_t l4 = {l_log2, l_log2, l_log2, l_log2};
+        if constexpr (KSIDE) l4 = *reinterpret_cast<const f32x4_t*>(stat + 8 * g + 4 * h);
+#pragma unroll
+        for (int i = 0; i < 4; i++) pv[4 * g + i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * g + i], c_scale_log2, -l4[i]));
+      }
+      if (masked) {
+        keep_branch();
+#pragma unroll
+        for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) dp[r] *= pv[r];            // dS = P (dP - d) (scale applied to the accumulators at the end)
+      second_level<T, D>(acc0, stage, troff, dp);             // dQ += dS K | dK += dS^T Q
+      if constexpr (KSIDE) second_level<T, D>(acc1, stage + TENSOR, troff, pv);   // dV += P^T dO
+    }
+  };
+
+  if (t_begin < t_end) publish(0);
+  __syncthreads();
+  for (int t = t_begin; t < t_end; t += WS) {
+    const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
+    const bool more = t + WS < t_end;
+    if (more) fetch(t + WS);
+    const int s0 = (t + ws) * TS;
+    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0);
+    if (NBUF == 1) __syncthreads();   // the tiles are no longer read
+    if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
+    __syncthreads();
+  }
+
+  if constexpr (WS > 1) {
+    // the WS waves of a row group merge their partial results in the order of ws; the wave with ws == 0 holds the outcome
+    constexpr int VALS = (KSIDE ? 2 : 1) * NC * 16 + (MODE == MODE_FWD ? 2 : 0);
+    float* const xch = reinterpret_cast<float*>(smem) + lane;
+    if (ws > 0) {
+      float* dst = xch + (group * (WS - 1) + ws - 1) * VALS * 64;
+#pragma unroll
+      for (int cb = 0; cb < NC; cb++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          dst[(cb * 16 + r) * 64] = acc0[cb][r];
+          if constexpr (KSIDE) dst[((NC + cb) * 16 + r) * 64] = acc1[cb][r];
+        }
+      if constexpr (MODE == MODE_FWD) dst[(VALS - 2) * 64] = m, dst[(VALS - 1) * 64] = l;
+    }
+    __syncthreads();
+    if (ws > 0) return;
+#pragma unroll
+    for (int o = 1; o < WS; o++) {
+      const float* from = xch + (group * (WS - 1) + o - 1) * VALS * 64;
+      float mine = 1.f, theirs = 1.f;
+      if constexpr (MODE == MODE_FWD) {
+        const float mo = from[(VALS - 2) * 64], m_new = fmaxf(m, mo), m_ref = m_new == -INFINITY ? 0.f : m_new;
+        mine = __builtin_amdgcn_exp2f(m - m_ref), theirs = __builtin_amdgcn_exp2f(mo - m_ref);
+        l = __builtin_fmaf(l, mine, from[(VALS - 1) * 64] * theirs);
+        m = m_new;
+      }
+#pragma unroll
+      for (int cb = 0; cb < NC; cb++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          acc0[cb][r] = __builtin_fmaf(from[(cb * 16 + r) * 64], theirs, acc0[cb][r] * mine);
+          if constexpr (KSIDE) acc1[cb][r] += from[((NC + cb) * 16 + r) * 64];
+        }
+    }
+  }
+
+  if constexpr (MODE == MODE_FWD) l += __shfl_xor(l, 32);
+  if (ri >= n_sta) return;
+  const int64_t out = (KSIDE ? koff : qoff) + (int64_t)ri * sta_ld;
+  if constexpr (MODE == MODE_FWD) {
+    store_rows<T, D>((T*)p.o + out, acc0, 1.f / l, h);
+    if (h == 0) p.lse[row] = (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;   // v_log_f32 is log2
+  } else if constexpr (MODE == MODE_BWD_Q) {
+    store_rows<T, D>((T*)p.dq + out, acc0, p.scale, h);
+  } else {
+    store_rows<T, D>((T*)p.dk + out, acc0, p.scale, h);
+    store_rows<T, D>((T*)p.dv + out, acc1, 1.f, h);
+  }
+}
+
+template <typename T, int D, int MODE, int WS>
+constexpr int lds_bytes() {
+  constexpr bool KSIDE = MODE == MODE_BWD_K;
+  constexpr int stages = (WS == 1 ? 2 : WS) * (Stager<T, D, 2, true>::BYTES + (KSIDE ? 2 * TS * 4 : 0));
+  constexpr int xch = WS > 1 ? (4 / WS) * (WS - 1) * ((KSIDE ? 2 : 1) * D / 32 * 16 + 2) * 64 * 4 : 0;
+  return stages > xch ? stages : xch;
+}
+
+template <typename T, int D, int MODE, int MASK, int WS>
+hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
+  constexpr int smem = lds_bytes<T, D, MODE, WS>(), nw = 4 / WS;
+  static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
+  const int n_rows = MODE == MODE_BWD_K ? p.n_k : p.n_q;
+  const hipError_t e = allow_dynamic_lds<attn_split<T, D, MODE, MASK, WS>>(smem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((attn_split<T, D, MODE, MASK, WS>), dim3(grid_blocks((n_rows + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
+  return hipGetLastError();
+}
+
+// As in fhog_split.hip: four waves on 128 rows when that fills the GPU, two or four on the same 32 rows when it does not.
+template <typename T, int D, int MODE, int MASK>
+hipError_t launch_mode(const AttnParams& p, hipStream_t s) {
+  const int64_t groups = (int64_t)((MODE == MODE_BWD_K ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = MODE == MODE_BWD_K ? p.n_q : p.n_k;
+  if constexpr (lds_bytes<T, D, MODE, 4>() <= 160 * 1024) {
+    if (groups < 64 && n_str > 2 * TS) return launch_ws<T, D, MODE, MASK, 4>(p, s);
+  }
+  if (groups < 128 && n_str > TS) return launch_ws<T, D, MODE, MASK, 2>(p, s);
+  return launch_ws<T, D, MODE, MASK, 1>(p, s);
+}
+
+template <typename T, int D>
+hipError_t launch_td(const AttnParams& p, int which, hipStream_t s) {
+  switch (which) {
+    case 0: return p.causal ? launch_mode<T, D, MODE_FWD, MASK_BAND>(p, s) : launch_mode<T, D, MODE_FWD, MASK_NONE>(p, s);
+    case 1: return p.causal ? launch_mode<T, D, MODE_BWD_Q, MASK_BAND>(p, s) : launch_mode<T, D, MODE_BWD_Q, MASK_NONE>(p, s);
+    case 2: return p.causal ? launch_mode<T, D, MODE_BWD_K, MASK_BAND>(p, s) : launch_mode<T, D, MODE_BWD_K, MASK_NONE>(p, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+// which: 0 forward, 1 dQ (and the row sums d), 2 dK and dV; dtype: FHOG_DTYPE_*. fp32 tensors of every head dim, 16-bit
+// tensors of d = 32.
+hipError_t launch_attn_split(const AttnParams& p, int dtype, int which, hipStream_t s) {
+  if (dtype == FHOG_DTYPE_FP32) {
+    switch (p.d) {
+      case 32: return launch_td<float, 32>(p, which, s);
+      case 64: return launch_td<float, 64>(p, which, s);
+      case 128: return launch_td<float, 128>(p, which, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  if (p.d != 32) return hipErrorInvalidValue;
+  return dtype == FHOG_DTYPE_FP16 ? launch_td<_Float16, 32>(p, which, s) : launch_td<__bf16, 32>(p, which, s);
+}
+
+}  // namespace fhog

@@ -152,30 +152,31 @@ struct Stager {
   static constexpr int PLANES = SECOND ? Terms<T>::LDS2 : Terms<T>::LDS1;
   static constexpr int TILE = TS * 2 * D, BYTES = NX * PLANES * TILE;
   static constexpr int CPR = D / 8;                                // chunks per row
-  static constexpr int PER_TENSOR = TS * CPR;                      // 128 (d = 32) or 256: a wave's chunks are of one tensor
-  static constexpr int XPI = 256 / PER_TENSOR;                     // tensors per round of 256 threads
-  static constexpr int PER = (NX + XPI - 1) / XPI;
-  static_assert(PER_TENSOR == 128 || PER_TENSOR == 256, "d = 32 or 64");
+  static constexpr int PER_TENSOR = TS * CPR;                      // 128 (d = 32), 256 or 512 (d = 128)
+  static constexpr int XPI = PER_TENSOR < 256 ? 2 : 1;             // tensors per round of 256 threads (a wave's chunks are of one)
+  static constexpr int RPT = PER_TENSOR > 256 ? 2 : 1;             // rounds per tensor
+  static constexpr int PER = (NX * RPT + XPI - 1) / XPI;
   Chunk<T> c[PER];
 
-  __device__ __forceinline__ static int tensor_of(int i, int tid) { return XPI * i + (XPI == 2 ? tid >> 7 : 0); }
+  __device__ __forceinline__ static int tensor_of(int i, int tid) { return XPI * i / RPT + (XPI == 2 ? tid >> 7 : 0); }
+  __device__ __forceinline__ static int row_of(int i, int tid) { return RPT == 1 ? tid / CPR % TS : tid / CPR + i % RPT * (256 / CPR); }
+  // src[x] + row0 rows is the first row of the tile of tensor x
   __device__ __forceinline__ void fetch(const T* const (&src)[NX], int64_t ld, int row0, int n_rows, int tid) {
-    const int r = tid / CPR % TS, ch = tid % CPR;
-    const int off = min(r, n_rows - 1 - row0) * (int)ld + 8 * ch;   // row strides are below 2^24 elements
 #pragma unroll
     for (int i = 0; i < PER; i++) {
-      const T* base = src[XPI * i];
-      if (XPI == 2 && XPI * i + 1 < NX) base = tid >> 7 ? src[XPI * i + 1 < NX ? XPI * i + 1 : 0] : base;
+      const int x = XPI * i / RPT;
+      const T* base = src[x];
+      if (XPI == 2 && x + 1 < NX) base = tid >> 7 ? src[x + 1 < NX ? x + 1 : 0] : base;
       if (NX % XPI && tensor_of(i, tid) >= NX) continue;
+      const int off = min(row_of(i, tid), n_rows - 1 - row0) * (int)ld + 8 * (tid % CPR);   // row strides are below 2^24 elements
       c[i] = load_chunk<T>(base + (int64_t)row0 * ld + off);
     }
   }
   __device__ __forceinline__ void publish(char* stage, int tid) const {
-    const int r = tid / CPR % TS, ch = tid % CPR;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       if (NX % XPI && tensor_of(i, tid) >= NX) continue;
-      char* dst = stage + tensor_of(i, tid) * PLANES * TILE + tile_off<D>(r, ch);
+      char* dst = stage + tensor_of(i, tid) * PLANES * TILE + tile_off<D>(row_of(i, tid), tid % CPR);
       bf16x8_t f[Terms<T>::NF];
       chunk_terms<T, true, Terms<T>::NF>(c[i], f);
 #pragma unroll

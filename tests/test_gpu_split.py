@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from gpu_util import NAMES, errors, make_case, normalised_max_error, reference_fp64_cpu, require_gpu, run_fhog, with_caches
+from oracle.bwdbwd_oracle import first_backward, forward_o_lse
 
 pytestmark = pytest.mark.gpu
 # fp32: the gate of the fp32 family. 16-bit tensors: products and sums are as accurate, but O is rounded before
@@ -40,3 +41,28 @@ def test_double_backward_on_split_products(shape, d, dtype):
     torch.cuda.synchronize()
     for got, fused, name in zip(plan.ws.view(3, -1), outs[4], ("d", "dd", "b")):
         assert normalised_max_error(got, fused.reshape(-1)) < 1e-4, name
+
+
+@pytest.mark.parametrize("case", [(t, d) for t in TOL for d in (32, 64, 128) if t == torch.float32 or d == 32])
+@pytest.mark.parametrize("shape", [(1, 1, 1, False, None), (1, 33, 65, False, None), (3, 64, 300, "bottom_right", 40),
+                                   (1, 97, 97, True, 1), (70, 128, 95, False, None), (130, 161, 161, True, 33),
+                                   (130, 128, 130, "bottom_right", None)])
+def test_first_order_on_split_products(shape, case):
+    """Forward and first backward in every wave split, ragged on both sides, rows whose window starts in a later tile."""
+    import fhog
+    dtype, d = case
+    batch, n_q, n_k, causal, window = shape
+    x = make_case(batch, n_q, n_k, d, dtype, seed=64)
+    scale = d ** -0.5
+    o, L = fhog.attention_forward(x["Q"], x["K"], x["V"], scale, causal, window=window, use_hip=True)
+    got = fhog.attention_backward(x["Q"], x["K"], x["V"], o, x["dO"], L, scale, causal, window=window, use_hip=True)
+    sel = slice(None) if batch < 4 else slice(0, batch, 43)
+    c = {n: t[sel].double().cpu().numpy() for n, t in x.items()}
+    o_ref, l_ref = forward_o_lse(c["Q"], c["K"], c["V"], scale, causal, window)
+    assert normalised_max_error(o[sel], o_ref) < (1e-4 if dtype == torch.float32 else TOL[dtype] / 2)   # rounded once
+    assert (L[sel].double().cpu() - torch.from_numpy(l_ref)).abs().max() < 1e-4
+    want = first_backward(c["Q"], c["K"], c["V"], c["dO"], scale, causal, window)
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        # one visible key per query (n_k = 1 or a window of 1): dS vanishes identically and the rounding of O is what is left
+        floor = 1e-4 if dtype == torch.float32 else 1e-2
+        assert (g[sel].double().cpu() - torch.from_numpy(w)).abs().max() < TOL[dtype] * abs(w).max() + floor, name
