@@ -25,7 +25,7 @@ for p in (ROOT / "flash-hob_amd", ROOT):
 
 PEAK_BF16_TFLOPS = 2516.6   # MI355X dense bf16 MFMA: 256 CU x 4096 FLOP/clk x 2.4 GHz
 PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA
-PASS_NAMES = {0: "rowdot_kernel (not in the 16-bit chain: its first sweep writes d too)",
+PASS_NAMES = {0: "rowdot_kernel (not in the chain: its first sweep writes d too)",
               1: "q_sweep_bf16<pass 1: d, dd> (four-pass schedule)", 2: "q_sweep_bf16<pass 2: b> (four-pass schedule)",
               3: "q_sweep3_pc<pass 3: dQ2, ddO>", 4: "k_sweep_pc<pass 4: dK2, dV2>",
               5: "q_sweep_bf16<fused passes 1+2: d, dd, b> (default schedule)",
@@ -106,8 +106,8 @@ def other_workloads(dev, skip):
         tflops = w.flops_algorithmic / ms / 1e9
         fp32 = plan.impl == 1
         res[name] = {"ms_per_step_no_alloc": round(ms, 4), "value": round(tflops, 2),
-                     "kernel_family": "fp32-mfma" if fp32 else "bf16-mfma",
-                     # against the peak of the matrix instructions the workload runs on
+                     "kernel_family": "split-product" if fp32 else "bf16-mfma",
+                     # against the peak of the matrix instructions of the tensors' type
                      ("pct_fp32_mfma_peak" if fp32 else "pct_bf16_mfma_peak"):
                          round(100 * tflops / (PEAK_FP32_TFLOPS if fp32 else PEAK_BF16_TFLOPS), 2)}
         del x, o, L, plan
@@ -128,7 +128,7 @@ def first_order(w, x, iters):
     res = {"forward_ms": round(fwd, 4), "forward_tflops": round(2 * unit / fwd / 1e9, 1),
            "backward_ms": round(bwd, 4), "backward_tflops": round(5 * unit / bwd / 1e9, 1),
            "note": "fhog_attn_fwd / fhog_attn_bwd including output allocation; not part of `value`"}
-    # the fp32-MFMA first-order kernels at their largest head dim (fp32 tensors, causal, 32 slices of 2048 tokens)
+    # the split-product first-order kernels at their largest head dim (fp32 tensors, causal, 32 slices of 2048 tokens)
     import torch
     g = torch.Generator().manual_seed(0)
     q, k, v, do = (torch.randn(32, 2048, 128, generator=g).to(x["Q"].device) for _ in range(4))
@@ -296,7 +296,7 @@ def main():
         "dtype": "bf16" if w.dtype == torch.bfloat16 else "f32",
         "data": "synthetic",
         "config": {"workload": w.name, "B": w.B, "H": w.H, "n_q": w.n_q, "n_k": w.n_k, "d": w.d, "causal": w.causal,
-                   "seed": 0, "kernel_family": {1: "fp32-mfma", 2: "bf16-mfma"}[plan.impl]},
+                   "seed": 0, "kernel_family": {1: "split-product", 2: "bf16-mfma"}[plan.impl]},
         "pct_bf16_mfma_peak": round(100 * value / PEAK_BF16_TFLOPS, 2),
         "executed_tflops": round(w.flops_executed / ms / 1e9, 2),
         "peak_mem_gb": round(peak_total / 1e9, 4),

@@ -163,10 +163,6 @@ int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
   return s;
 }
 
-// Family IMPL_FP32: split products on the 16-bit matrix instructions up to d = 64, fp32 MFMA at d = 128 (where the three
-// terms of the stationary operands do not fit the registers).
-bool on_split_kernels(const fhog_bwdbwd_args* a) { return a->d <= 64; }
-
 int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
   fhog::Params p = base;
   p.n_split = granted_split(a, impl, pass);
@@ -186,13 +182,8 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
     e = fhog::launch_rowdot(p, a->dtype, s);
   else if (impl == FHOG_IMPL_BF16)
     e = fhog::launch_bf16_pass(p, pass, s);
-  else if (on_split_kernels(a))
+  else
     e = fhog::launch_split_pass(p, a->dtype, pass, s);
-  else if (pass == FHOG_PASS_DD_B) {
-    e = fhog::launch_fp32_pass(p, a->dtype, FHOG_PASS_DD, s);
-    if (e == hipSuccess) e = fhog::launch_fp32_pass(p, a->dtype, FHOG_PASS_B, s);
-  } else
-    e = fhog::launch_fp32_pass(p, a->dtype, pass, s);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "pass %d: HIP error %d (%s)", pass, (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }
@@ -406,30 +397,29 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (rc != FHOG_OK) return rc;
   const fhog::Params p = to_params(args);
   const int impl = select_impl(args);
-  // Pass sequences. The first statistics sweep of the 16-bit and the split-product kernels writes d_i itself: no separate
-  // launch for it there.
-  // The schedules that take ddO out of the third sweep exist in the 16-bit family; the fp32-MFMA family runs the
+  // Pass sequences. The first statistics sweep writes d_i itself: no separate launch for it.
+  // The schedules that take ddO out of the third sweep exist in the 16-bit family; the split-product family runs the
   // fused one for them.
-  static const int four[] = {FHOG_PASS_D, FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
-  static const int fused[] = {FHOG_PASS_D, FHOG_PASS_DD_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
+  static const int four[] = {FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
+  static const int fused[] = {FHOG_PASS_DD_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
   static const int ddo_early[] = {FHOG_PASS_DD, FHOG_PASS_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   static const int three[] = {FHOG_PASS_DD_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
   const int* order = four;
-  const bool fp32 = impl != FHOG_IMPL_BF16;
-  int first = fp32 && !on_split_kernels(args) ? 0 : 1, n_pass = 5;
+  const bool split_products = impl != FHOG_IMPL_BF16;
+  int n_pass = 4;
   // d = 64, launch large enough to fill the GPU: the reference's own arrangement of its four passes, sweeps 1-3 in one launch
   static const int stage1[] = {FHOG_PASS_STAGE1, FHOG_PASS_DK_DV};
   if (args->schedule == FHOG_SCHEDULE_FOUR_PASS && impl == FHOG_IMPL_BF16 && args->d == 64 && fhog::tuning().stage1 != 0 &&
       granted_split(args, impl, FHOG_PASS_DQ_DDO) == 1 && granted_split(args, impl, FHOG_PASS_DD) == 1)
-    order = stage1, first = 0, n_pass = 2;
-  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (fp32 && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 4;
+    order = stage1, n_pass = 2;
+  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (split_products && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 3;
   // Passes 6-8 have no split form: a launch too small to fill the GPU whose workspace lets the reference's passes split
   // their streamed side runs the nearest schedule that can (three sweeps -> fused statistics, ddO early -> four passes).
   const bool small = granted_split(args, impl, FHOG_PASS_DQ_DDO) > 1;
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && small) order = fused, n_pass = 4;
-  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !small) order = ddo_early, first = 0, n_pass = 4;
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !small) order = three, first = 0, n_pass = 3;
-  for (int i = first; i < n_pass; i++) {
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && small) order = fused, n_pass = 3;
+  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !small) order = ddo_early, n_pass = 4;
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !small) order = three, n_pass = 3;
+  for (int i = 0; i < n_pass; i++) {
     const int r = run_pass(args, p, impl, order[i], (hipStream_t)hip_stream);
     if (r != FHOG_OK) return r;
   }

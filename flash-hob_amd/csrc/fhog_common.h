@@ -111,8 +111,7 @@ inline hipError_t allow_dynamic_lds(int bytes) {
 
 // Launchers implemented in the kernel translation units. Each returns hipGetLastError().
 hipError_t launch_rowdot(const Params& p, int dtype, hipStream_t s);                 // pass 0
-hipError_t launch_fp32_pass(const Params& p, int dtype, int pass, hipStream_t s);   // passes 1..4, fp32 MFMA (d = 128)
-hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products (d = 32, 64)
+hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products
 hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);              // passes 1..4, bf16 MFMA
 hipError_t launch_attn_bf16(const AttnParams& p, int which, hipStream_t s);         // 0 forward, 1 dQ, 2 dK and dV
 hipError_t launch_attn_split(const AttnParams& p, int dtype, int which, hipStream_t s); // same, split products (fp32 tensors, d = 32)

@@ -1,6 +1,6 @@
 // Split-product kernels of the attention double-backward: products of fp32 accuracy on the 16-bit matrix instructions
-// (fhog_split_util.h). They serve fp32 tensors and d = 32 (and 16-bit tensors for which the fp32 family is asked for) at
-// head dims 32 and 64; fp32-accurate arithmetic throughout, no atomics, nothing of shape (N_Q, N_K) leaves the chip.
+// (fhog_split_util.h). They serve fp32 tensors and d = 32, and 16-bit tensors for which this family is asked for;
+// fp32-accurate arithmetic throughout, no atomics, nothing of shape (N_Q, N_K) leaves the chip.
 //
 // One kernel template for the sweeps, with the arithmetic of the single-role 16-bit kernels (fhog_bf16.hip): a workgroup of
 // 4 wave64 owns 32 stationary rows per wave (queries in passes 1-3 and 5, keys in pass 4) and keeps their operands in
@@ -13,9 +13,10 @@
 //
 // What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
 // 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (26 MFMAs beside some 450 VALU instructions).
-// Whole chain, us, against the fp32-MFMA kernels that served these shapes before (same box):
+// Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same box):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 123     fp32 causal 64 x 1024, d = 32: 672 -> 318
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2422
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
@@ -29,9 +30,43 @@ namespace fhog {
 using namespace splitk;
 namespace {
 
+// Stationary fp32 operands too many for their terms to stay in registers.
+template <typename T, int D>
+constexpr bool is_raw = sizeof(T) == 4 && D == 128;
+
+// Stationary operand of a lane: its row's elements 16 kk + 8 h .. + 7 of every k-step, as terms or as they lie in memory.
+template <typename T, int D>
+struct Resident {
+  static constexpr int KK = D / 16, NF = Terms<T>::NF;
+  typename std::conditional<is_raw<T, D>, Chunk<T>, bf16x8_t[NF]>::type r[KK];
+  __device__ __forceinline__ void load(const T* row, int h) {
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      const Chunk<T> c = load_chunk<T>(row + 16 * kk + 8 * h);
+      if constexpr (is_raw<T, D>) r[kk] = c;
+      else chunk_terms<T, true, NF>(c, r[kk]);
+    }
+  }
+  __device__ __forceinline__ void terms(int kk, bf16x8_t (&out)[NF]) const {
+    if constexpr (is_raw<T, D>) {
+      Chunk<T> c = r[kk];
+      // splitting is to happen here, tile after tile: hoisted out of the sweep, the terms would be spilled
+      asm volatile("" : "+v"(c.v[0]), "+v"(c.v[1]));
+      chunk_terms<T, true, NF>(c, out);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NF; q++) out[q] = r[kk][q];
+    }
+  }
+};
+
+// Stages of the ring: two where they fit (a wave split stages WS tiles at a time instead).
+template <typename T, int D, int WS>
+constexpr int n_buffers(int stage) { return WS == 1 && !is_raw<T, D> && 2 * stage <= 160 * 1024 ? 2 : 1; }
+
 // PASS 1: d, dd; 2: b; 3: dQ2, ddO; 4: dK2, dV2 (K-tiled); 5: d, dd, b.
 template <typename T, int D, int PASS, int MASK, int WS>
-__global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Params p) {
+__global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4);      // streamed tensors: K, ddK, V, ddV | Q, ddQ, dO
@@ -41,7 +76,13 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   constexpr int TENSOR = Stage::PLANES * Stage::TILE;
   constexpr int STAT = KSIDE ? 4 * TS * 4 : 0;             // L log2(e), -d, dd, -(dd d + b) of the 32 staged queries
   constexpr int STAGE = Stage::BYTES + STAT;
-  constexpr int NBUF = WS == 1 ? 2 : 1;                    // with a wave split the WS tiles of a step take the room of the second buffer
+  // fp32, d = 128: the terms of three or four stationary tensors are 288 or 384 registers, so the wave keeps the fp32 numbers
+  // (the last tensor of passes 3 and 4, dO or ddV, in LDS) and splits them again for every tile, one k-step at a time behind the MFMAs of
+  // the one before: 28 VALU instructions per tensor and k-step beside 30 MFMAs.
+  constexpr bool RAW = is_raw<T, D>;
+  constexpr bool LAST_IN_LDS = RAW && !STATS;
+  constexpr int NREG = LAST_IN_LDS ? NR - 1 : NR;
+  constexpr int NBUF = n_buffers<T, D, WS>(STAGE);
   constexpr int nw = 4 / WS, ROWS = 32 * nw;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -101,16 +142,20 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   };
   if (t_begin < t_end) fetch(t_begin);
 
-  bf16x8_t res[NR][KK][NF];
-  if constexpr (KSIDE) {
-    load_resident_terms<T, D>(res[0], (const T*)p.k + koff, sta_ld, rr, h);
-    load_resident_terms<T, D>(res[1], (const T*)p.ddk + koff, sta_ld, rr, h);
-    load_resident_terms<T, D>(res[2], (const T*)p.v + koff, sta_ld, rr, h);
-    load_resident_terms<T, D>(res[NR - 1], (const T*)p.ddv + koff, sta_ld, rr, h);
-  } else {
-    load_resident_terms<T, D>(res[0], (const T*)p.q + qoff, sta_ld, rr, h);
-    load_resident_terms<T, D>(res[1], (const T*)p.ddq + qoff, sta_ld, rr, h);
-    if constexpr (PASS != 1) load_resident_terms<T, D>(res[NR - 1], (const T*)p.dO + qoff, sta_ld, rr, h);
+  const T* const sta[4] = {KSIDE ? (const T*)p.k + koff : (const T*)p.q + qoff, KSIDE ? (const T*)p.ddk + koff : (const T*)p.ddq + qoff,
+                           KSIDE ? (const T*)p.v + koff : (const T*)p.dO + qoff, (const T*)p.ddv + koff};
+  Resident<T, D> res[NREG];
+#pragma unroll
+  for (int x = 0; x < NREG; x++) res[x].load(sta[x] + (int64_t)rr * sta_ld, h);
+  // the last tensor of the wave's rows, 16 bytes of a lane beside those of the next one
+  f32x4_t* const last = reinterpret_cast<f32x4_t*>(smem + NBUF * WS * STAGE) + wv * (KK * 2 * 64) + lane;
+  if constexpr (LAST_IN_LDS) {
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      const Chunk<T> c = load_chunk<T>(sta[NR - 1] + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+      last[(2 * kk) * 64] = __builtin_bit_cast(f32x4_t, c.v[0]);
+      last[(2 * kk + 1) * 64] = __builtin_bit_cast(f32x4_t, c.v[sizeof(T) / 2 - 1]);
+    }
   }
   const int64_t row = srow + rr;   // Q-tiled passes
   float l_log2 = 0.f, dsum = 0.f, dd = 0.f, b = 0.f;
@@ -146,7 +191,8 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   for (int cb = 0; cb < NC; cb++) acc0[cb] = f32x16_t{0}, acc1[cb] = f32x16_t{0};
   float red[5] = {};               // statistics: b-like sum; fused sweep: dd, sum P u ddS, sum P u, sum P
 
-  const auto block = [&](const char* stage, int s0) {
+  // prefetch: what requests the next tile; called where the registers it lands in are free
+  const auto block = [&](const char* stage, int s0, auto prefetch) {
     const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
     f32x16_t s = {0}, dds = {0}, dp = {0}, e = {0};
     // u = dP - d and E' = E - (dd d + b) come straight from accumulators that start at the row constants
@@ -167,21 +213,34 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
     }
 #pragma unroll
     for (int kk = 0; kk < KK; kk++) {
-      bf16x8_t a[NT][NF];
-#pragma unroll
-      for (int x = 0; x < NT; x++) read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a[x]);
-      s = mma1<T>(s, a[0], res[0][kk]);                       // K Q^T | Q K^T
-      if constexpr (KSIDE) {
-        dds = mma1<T>(dds, a[1], res[0][kk]);                 // ddQ K^T
-        dp = mma1<T>(dp, a[2], res[2][kk]);                   // dO V^T
-        dds = mma1<T>(dds, a[0], res[1][kk]);                 // + Q ddK^T
-        e = mma1<T>(e, a[2], res[NR - 1][kk]);                // dO ddV^T
-      } else {
-        dds = mma1<T>(dds, a[0], res[1][kk]);                 // K ddQ^T
-        if constexpr (PASS != 1) dp = mma1<T>(dp, a[NT - 2], res[NR - 1][kk]);   // V dO^T
-        dds = mma1<T>(dds, a[1], res[0][kk]);                 // + ddK Q^T
-        if constexpr (PASS != 1) e = mma1<T>(e, a[NT - 1], res[NR - 1][kk]);     // ddV dO^T
+      bf16x8_t r0[NF], r1[NF], r2[NF], r3[NF], a[NF];
+      res[0].terms(kk, r0), res[1].terms(kk, r1);
+      const auto last_terms = [&](bf16x8_t (&out)[NF]) {
+        if constexpr (LAST_IN_LDS) {
+          Chunk<T> c;
+          c.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]), c.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
+          chunk_terms<T, true, NF>(c, out);
+        } else {
+          res[NREG - 1].terms(kk, out);
+        }
+      };
+      if constexpr (KSIDE) res[2].terms(kk, r2), last_terms(r3);
+      else if constexpr (PASS != 1) last_terms(r2);
+      read_terms<T, Stage::TILE>(stage, aoff[kk], a);
+      s = mma1<T>(s, a, r0);                                  // K Q^T | Q K^T
+      dds = mma1<T>(dds, a, r1);                              // K ddQ^T | Q ddK^T
+      if constexpr (PASS != 1) {
+        read_terms<T, Stage::TILE>(stage + 2 * TENSOR, aoff[kk], a);
+        dp = mma1<T>(dp, a, r2);                              // V dO^T | dO V^T
+        if constexpr (KSIDE) e = mma1<T>(e, a, r3);           // dO ddV^T
       }
+      read_terms<T, Stage::TILE>(stage + 1 * TENSOR, aoff[kk], a);
+      dds = mma1<T>(dds, a, r0);                              // + ddK Q^T | ddQ K^T
+      if constexpr (PASS != 1 && !KSIDE) {
+        read_terms<T, Stage::TILE>(stage + (NT - 1) * TENSOR, aoff[kk], a);
+        e = mma1<T>(e, a, r2);                                // ddV dO^T
+      }
+      if constexpr (RAW) __builtin_amdgcn_sched_barrier(0);
     }
     f32x16_t pv;
 #pragma unroll
@@ -191,7 +250,12 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
 #pragma unroll
       for (int i = 0; i < 4; i++) pv[4 * g + i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * g + i], c_scale_log2, -l4[i]));
     }
-    if (geo.partial(s0, rw)) {   // wave-uniform: the block holds hidden pairs (mask edge or tensor end)
+    if (RAW && MASK != MASK_NONE) {
+      int lo, hi;
+      geo.limits(s0, ri, h, lo, hi);
+#pragma unroll
+      for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
+    } else if (geo.partial(s0, rw)) {   // wave-uniform: the block holds hidden pairs (mask edge or tensor end)
       int lo, hi;
       geo.limits(s0, ri, h, lo, hi);
       keep_branch();
@@ -227,21 +291,36 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
           e[r] = __builtin_fmaf(pv[r], e[r], dds[r] * dp[r]);           // dS' = P E' + ddP u
         }
       }
-      second_level<T, D>(acc0, stage + 1 * TENSOR, troff, s);           // dQ2 += dS ddK | dK2 += dS^T ddQ
-      second_level<T, D>(acc1, stage + 2 * TENSOR, troff, dds);         // ddO += ddP V | dV2 += ddP^T dO
-      second_level<T, D>(acc0, stage, troff, e);                        // dQ2 += dS' K | dK2 += dS'^T Q
-      if constexpr (!KSIDE) second_level<T, D>(acc1, stage + (NT - 1) * TENSOR, troff, pv);   // ddO += P ddV
+      if constexpr (!KSIDE) second_level<T, D, RAW>(acc1, stage + (NT - 1) * TENSOR, troff, pv);   // ddO += P ddV
+      second_level<T, D, RAW>(acc0, stage + 1 * TENSOR, troff, s);           // dQ2 += dS ddK | dK2 += dS^T ddQ
+      second_level<T, D, RAW>(acc1, stage + 2 * TENSOR, troff, dds);         // ddO += ddP V | dV2 += ddP^T dO
+      prefetch();
+      second_level<T, D, RAW>(acc0, stage, troff, e);                        // dQ2 += dS' K | dK2 += dS'^T Q
     }
   };
 
+  constexpr bool LATE = RAW && !STATS;   // the next tile is requested towards the end of a step: no registers for it before
   if (t_begin < t_end) publish(0);
   __syncthreads();
   for (int t = t_begin; t < t_end; t += WS) {
     const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
     const bool more = t + WS < t_end;
-    if (more) fetch(t + WS);
+    const auto next = [&]() {
+      if (more) fetch(t + WS);
+    };
+    if (!LATE) next();
     const int s0 = (t + ws) * TS;
-    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0);
+    if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, rw))) {
+      block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
+        if (LATE) {
+          __builtin_amdgcn_sched_barrier(0);
+          next();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      });
+    } else if (LATE) {
+      next();
+    }
     if (NBUF == 1) __syncthreads();   // the tiles are no longer read
     if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
     __syncthreads();
@@ -293,15 +372,21 @@ __global__ void __launch_bounds__(256, D == 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   }
 }
 
-template <typename T, int D, int PASS, int MASK, int WS>
-hipError_t launch_ws(const Params& p, hipStream_t s) {
+template <typename T, int D, int PASS, int WS>
+constexpr int lds_bytes() {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4), nw = 4 / WS;
   constexpr int stage = Stager<T, D, NT, !STATS>::BYTES + (KSIDE ? 4 * TS * 4 : 0);
+  constexpr int stages = n_buffers<T, D, WS>(stage) * WS * stage + (is_raw<T, D> && !STATS ? 4 * TS * D * 4 : 0);
   constexpr int xch = WS > 1 ? nw * (WS - 1) * (STATS ? 5 : 2 * D / 32 * 16) * 64 * 4 : 0;
-  constexpr int smem = (WS == 1 ? 2 : WS) * stage > xch ? (WS == 1 ? 2 : WS) * stage : xch;
+  return stages > xch ? stages : xch;
+}
+
+template <typename T, int D, int PASS, int MASK, int WS>
+hipError_t launch_ws(const Params& p, hipStream_t s) {
+  constexpr int smem = lds_bytes<T, D, PASS, WS>(), nw = 4 / WS;
   static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
-  const int n_rows = KSIDE ? p.n_k : p.n_q;
+  const int n_rows = PASS == 4 ? p.n_k : p.n_q;
   const hipError_t e = allow_dynamic_lds<split_sweep<T, D, PASS, MASK, WS>>(smem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((split_sweep<T, D, PASS, MASK, WS>), dim3(grid_blocks((n_rows + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
@@ -314,10 +399,12 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 template <typename T, int D, int PASS, int MASK>
 hipError_t launch_sweep(const Params& p, hipStream_t s) {
   const int64_t groups = (int64_t)((PASS == 4 ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = PASS == 4 ? p.n_q : p.n_k;
-  if constexpr (D == 32 || std::is_same<T, __bf16>::value) {   // the four tiles of a step fit the LDS
+  if constexpr (lds_bytes<T, D, PASS, 4>() <= 160 * 1024) {
     if (groups < 64 && n_str > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
   }
-  if (groups < 128 && n_str > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
+  if constexpr (lds_bytes<T, D, PASS, 2>() <= 160 * 1024) {
+    if (groups < 128 && n_str > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
+  }
   return launch_ws<T, D, PASS, MASK, 1>(p, s);
 }
 
@@ -337,7 +424,12 @@ hipError_t launch_td(const Params& p, int pass, hipStream_t s) {
 
 template <typename T>
 hipError_t launch_t(const Params& p, int pass, hipStream_t s) {
-  return p.d == 32 ? launch_td<T, 32>(p, pass, s) : p.d == 64 ? launch_td<T, 64>(p, pass, s) : hipErrorInvalidValue;
+  switch (p.d) {
+    case 32: return launch_td<T, 32>(p, pass, s);
+    case 64: return launch_td<T, 64>(p, pass, s);
+    case 128: return launch_td<T, 128>(p, pass, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace

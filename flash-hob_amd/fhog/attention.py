@@ -12,7 +12,7 @@ commented stub (``fhog/triton_bwdbwd.py:538-554``).  Here it is wired:
 
 The forward and the first-order backward are the callers on either side of the hot path.  They run as HIP
 kernels of the same library (``fhog_attn_fwd`` / ``fhog_attn_bwd``): 16-bit MFMA kernels for bf16 and fp16 tensors
-with d in {64, 128}, fp32-MFMA kernels for fp32 tensors and d = 32.  A linear-memory torch composition on the GPU
+with d in {64, 128}, split-product kernels for fp32 tensors and d = 32.  A linear-memory torch composition on the GPU
 (blocked over heads and query rows, fp32 accumulation) remains for arguments the kernels reject (a non-positive
 scale on 16-bit tensors) and as the second implementation the tests compare with (``use_hip=False``).
 The double-backward is always the HIP library.

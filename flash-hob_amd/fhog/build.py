@@ -16,7 +16,7 @@ PKG_DIR = Path(__file__).resolve().parent            # .../flash-hob_amd/fhog
 CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libfhog_hip.so"
-SOURCES = ["fhog_abi.hip", "fhog_fp32.hip", "fhog_split.hip", "fhog_bf16.hip", "fhog_bf16_pc.hip", "fhog_bf16_ddo.hip", "fhog_attn.hip", "fhog_attn_split.hip", "fhog_probe.hip"]
+SOURCES = ["fhog_abi.hip", "fhog_rowdot.hip", "fhog_split.hip", "fhog_bf16.hip", "fhog_bf16_pc.hip", "fhog_bf16_ddo.hip", "fhog_attn.hip", "fhog_attn_split.hip", "fhog_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -26,6 +26,9 @@ HIPCC_FLAGS = [
     "-fno-gpu-rdc",
     # packed-fp32 VALU forms are kept out of every kernel of this library
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # registers spill to scratch memory only: a kernel whose accumulators take every AGPR and that spilled VGPRs to AGPRs as
+    # well was compiled wrongly (fp16 operands of the K-tiled split-product sweep at d = 128: NaN in dK2)
+    "-mllvm", "-amdgpu-spill-vgpr-to-agpr=0",
     "-Wno-unused-command-line-argument",
 ] + os.environ.get("FHOG_EXTRA", "").split()   # extra hipcc flags for experiments
 

@@ -144,7 +144,7 @@ def flash_bwdbwd(Q, K, V, O, dO, ddQ, ddK, ddV, L, scale, *, causal=False, windo
             only the ``window`` most recent visible keys stay visible. Both kernel families take every mask and
             skip the tiles outside the band.
         impl: None/"auto" | "fp32" | "bf16" - kernel family; "auto" takes the 16-bit MFMA kernels ("bf16": products
-            in the tensor type, bf16 or fp16) for 16-bit tensors whose shape they support, the fp32-MFMA kernels
+            in the tensor type, bf16 or fp16) for 16-bit tensors whose shape they support, the split-product kernels
             otherwise.
         fused_stats: the same as ``schedule="fused_stats"``.
         schedule: None / "fused_stats" (``dd`` and ``b`` from one sweep instead of the reference's two,

@@ -53,8 +53,7 @@ extern "C" {
 /* pass ids for fhog_bwdbwd_pass */
 #define FHOG_PASS_D 0      /* d_i  = sum_c O_ic dO_ic                         (fhog/triton_bwdbwd.py:580)     */
 #define FHOG_PASS_DD 1     /* dd_i = sum_j ddS_ij P_ij                        (fhog/triton_bwdbwd.py:185-211);
-                              the 16-bit kernels of passes 1 and 5 also write d_i, so fhog_bwdbwd launches pass 0
-                              only for the fp32-MFMA family */
+                              the kernels of passes 1 and 5 also write d_i: fhog_bwdbwd never launches pass 0 */
 #define FHOG_PASS_B 2      /* b_i  = sum_j dP'_ij P_ij                        (fhog/triton_bwdbwd.py:217-251) */
 #define FHOG_PASS_DQ_DDO 3 /* dQ2 = dS ddK + dS' K ; ddO = P ddV + ddP V      (fhog/triton_bwdbwd.py:257-313) */
 #define FHOG_PASS_DK_DV 4  /* dK2 = dS^T ddQ + dS'^T Q ; dV2 = ddP^T dO       (fhog/triton_bwdbwd.py:467-535) */
@@ -74,8 +73,9 @@ extern "C" {
                                 streamed side not split; writes d, dd, b, dQ2, ddO */
 
 /* kernel families (fhog_bwdbwd_args.impl) */
-#define FHOG_IMPL_AUTO 0   /* 16-bit MFMA kernels for bf16/fp16 tensors when the shape allows, else the fp32-MFMA kernels */
-#define FHOG_IMPL_FP32 1   /* force the fp32-MFMA kernels (any dtype; every intermediate in fp32) */
+#define FHOG_IMPL_AUTO 0   /* 16-bit MFMA kernels for bf16/fp16 tensors when the shape allows, else the split-product kernels */
+#define FHOG_IMPL_FP32 1   /* force the split-product kernels (any dtype): contractions of fp32 accuracy, put together from 16-bit
+                               MFMA products of bf16 terms (three of an fp32 number, exactly); everything else in fp32 */
 #define FHOG_IMPL_BF16 2   /* force the 16-bit MFMA kernels (bf16 or fp16 tensors, products in the tensor type);
                               error if the shape/dtype does not fit */
 
@@ -98,7 +98,7 @@ extern "C" {
 #define FHOG_SCHEDULE_THREE_SWEEP 3 /* opt-in, three sweeps: dd, b and ddO (FHOG_PASS_DD_B_DDO); dQ2 (FHOG_PASS_DQ);
                                        dK2+dV2. 20 recomputed products. ddP V is formed as (P o ddS) V - dd O with the
                                        caller's 16-bit O: accurate as long as dd_i does not dominate ddS_ij - dd_i.
-                                       Schedules 2 and 3 exist in the 16-bit MFMA family; the fp32-MFMA family runs
+                                       Schedules 2 and 3 exist in the 16-bit MFMA family; the split-product family runs
                                        schedule 1 for them. Passes 6, 7 and 8 have no split form: a launch too
                                        small to fill the GPU whose workspace allows a split (ws_bytes) runs the four
                                        passes (schedule 2) or the fused statistics sweep and passes 3, 4 (schedule 3) */
@@ -208,7 +208,7 @@ int fhog_bwdbwd_pass(const fhog_bwdbwd_args* args, int pass, void* hip_stream);
 /* ---- first-order attention: the callers on either side of the double-backward ---------------------------
  * bf16, fp16 or fp32 tensors, d in {32, 64, 128}, any n_q and n_k (fhog_attn_validate tells); the layout rules
  * above apply. bf16 / fp16 tensors with d in {64, 128} run on 16-bit MFMA kernels (they need scale > 0), fp32
- * tensors and d = 32 on fp32-MFMA kernels. O and dO/dQ share the q strides, dK/dV the k strides. */
+ * tensors and d = 32 on split-product kernels. O and dO/dQ share the q strides, dK/dV the k strides. */
 typedef struct fhog_attn_args {
   const void* q;   /* (batch, n_q, d) */
   const void* k;   /* (batch, n_k, d) */

@@ -1,4 +1,4 @@
-"""GPU tier: the split-product kernels (fp32-accurate contractions on the 16-bit matrix instructions) at d = 32 and 64."""
+"""GPU tier: the split-product kernels (fp32-accurate contractions on the 16-bit matrix instructions)."""
 import pytest
 import torch
 
@@ -17,7 +17,7 @@ def _dev():
 
 
 @pytest.mark.parametrize("dtype", list(TOL))
-@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("shape", [(1, 1, 1, False, None), (1, 33, 65, False, None), (3, 64, 300, "bottom_right", 40),
                                    (1, 97, 97, True, 1), (70, 128, 95, False, None), (130, 161, 161, True, 33),
                                    (130, 128, 130, "bottom_right", None)])
