@@ -112,6 +112,22 @@ def lib() -> ctypes.CDLL:
     return L
 
 
+_TORCH_EXT = None
+
+
+def torch_ext():
+    """Load (once) and return the native host side of the PyTorch entry points; raise if it is not there."""
+    global _TORCH_EXT
+    if _TORCH_EXT is None:
+        lib()
+        try:
+            from . import _fhog_torch
+        except ImportError as why:
+            raise RuntimeError("_fhog_torch.so is missing or does not load: build it with `python flash-hob_amd/fhog/build.py`") from why
+        _TORCH_EXT = _fhog_torch
+    return _TORCH_EXT
+
+
 def check(rc: int) -> None:
     if rc != 0:
         raise FhogError(rc, lib().fhog_last_error().decode())

@@ -10,6 +10,8 @@ commented stub (``fhog/triton_bwdbwd.py:538-554``).  Here it is wired:
     AttnBwd.forward          -> dQ, dK, dV   (first-order backward)
     AttnBwd.backward         -> flash_bwdbwd(...) -> dQ', dK', dV', ddO
 
+:func:`attention` builds the same chain out of native nodes (``csrc/fhog_torch.cpp``).
+
 The forward and the first-order backward are the callers on either side of the hot path.  They run as HIP
 kernels of the same library (``fhog_attn_fwd`` / ``fhog_attn_bwd``): 16-bit MFMA kernels for bf16 and fp16 tensors
 with d in {64, 128}, split-product kernels for fp32 tensors and d = 32.  A linear-memory torch composition on the GPU
@@ -28,7 +30,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .bwdbwd import flash_bwdbwd, mask_code
+from .bwdbwd import _SCHEDULES, flash_bwdbwd, mask_code, native_mask
 
 _HIP_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16, torch.float32: _lib.DTYPE_FP32}
 _BLOCK_ELEMS = 1 << 26  # fp32 elements of one materialised (heads, rows, N_K) block (256 MiB)
@@ -153,6 +155,10 @@ def attention_forward(q, k, v, scale: Optional[float] = None, causal=False, *, w
     that are not multiples of 16 bytes, CPU tensors), a ``TorchCompositionWarning`` names the reason and the blocked
     torch composition runs instead. True = the HIP kernel or a ``ValueError``; False = the torch composition.
     """
+    if use_hip is not False and q.is_cuda:
+        res = _lib.torch_ext().forward(q, k, v, float(q.shape[-1] ** -0.5 if scale is None else scale), *native_mask(causal, window))
+        if res is not None:
+            return res
     if q.dim() == 4:
         B, H = q.shape[:2]
         o, L = attention_forward(q.flatten(0, 1), k.flatten(0, 1), v.flatten(0, 1), scale, causal, window=window,
@@ -188,6 +194,10 @@ def attention_backward(q, k, v, o, do, L, scale: float, causal, *, window: Optio
                        use_hip: Optional[bool] = None):
     """First-order backward (dQ, dK, dV); the arithmetic of ``fhog/triton_flash.py:201-220`` without the
     (batch, N_Q, N_K) tensors. ``use_hip`` as in :func:`attention_forward`."""
+    if use_hip is not False and q.is_cuda:
+        res = _lib.torch_ext().backward(q, k, v, o, do, L, float(scale), *native_mask(causal, window))
+        if res is not None:
+            return res
     batch, n_q, d = q.shape
     n_k = k.shape[1]
     if use_hip is not False:
@@ -276,4 +286,9 @@ def attention(q, k, v, is_causal=False, window: Optional[int] = None, schedule: 
     """Twice-differentiable scaled-dot-product attention (scale = d^-1/2). ``is_causal``: False | True |
     "bottom_right"; ``window``: sliding-window length on top of a causal mask; ``schedule``: pass schedule of the
     double-backward (see :func:`fhog.flash_bwdbwd`; None = its default, three sweeps with ``dd`` and ``b`` from the first)."""
+    if q.is_cuda:
+        # the same chain as native autograd nodes; declines what the kernels do not cover
+        out = _lib.torch_ext().attention(q, k, v, *native_mask(is_causal, window), _SCHEDULES.get(schedule, -1))
+        if out is not None:
+            return out
     return FlashAttention.apply(q, k, v, is_causal, window, schedule)

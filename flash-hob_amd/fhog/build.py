@@ -1,7 +1,7 @@
-"""Build libfhog_hip.so (gfx950) in-tree with hipcc.
+"""Build libfhog_hip.so (gfx950) and _fhog_torch.so in-tree.
 
-The shared library is the only native artefact of the package: HIP kernels plus the C ABI
-declared in ``include/fhog_hip.h``.  It is compiled ahead of time (hipcc cross-compiles
+The shared library holds the HIP kernels and the C ABI declared in ``include/fhog_hip.h``; the extension module is the
+native host side of the PyTorch entry points on top of that ABI.  Both are compiled ahead of time (hipcc cross-compiles
 without a GPU); nothing is JIT-compiled at run time.
 """
 from __future__ import annotations
@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent            # .../flash-hob_amd/fhog
@@ -40,8 +41,20 @@ def hipcc() -> str:
     return exe
 
 
+def _torch_ext_commands(obj: Path):
+    """g++ command lines that compile csrc/fhog_torch.cpp and link it against torch and libfhog_hip.so next to it."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    inc = [f"-I{p}" for p in (*include_paths("cuda"), sysconfig.get_paths()["include"], INCLUDE)]
+    compile_ = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_fhog_torch",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, "-c", str(CSRC / "fhog_torch.cpp"), "-o", str(obj)]
+    link = ["g++", "-shared", "-o", str(PKG_DIR / "_fhog_torch.so"), str(obj), *(f"-L{p}" for p in library_paths("cuda")), f"-L{PKG_DIR}",
+            "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lfhog_hip", "-Wl,-rpath,$ORIGIN"]
+    return compile_, link
+
+
 def build(verbose: bool = True, jobs: int = 9) -> Path:
-    """Compile every source and link ``libfhog_hip.so`` next to this file. Always recompiles."""
+    """Compile every source and link ``libfhog_hip.so`` and ``_fhog_torch.so`` next to this file. Always recompiles."""
     objdir = PKG_DIR.parent / "build"
     objdir.mkdir(exist_ok=True)
     procs = []
@@ -55,11 +68,19 @@ def build(verbose: bool = True, jobs: int = 9) -> Path:
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         if len(procs) >= jobs:
             _drain(procs, verbose)
+    ext_obj = objdir / "fhog_torch.o"
+    ext_compile, ext_link = _torch_ext_commands(ext_obj)
+    if verbose:
+        print(" ".join(ext_compile), flush=True)
+    procs.append(("fhog_torch.cpp", subprocess.Popen(ext_compile, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     _drain(procs, verbose)
     cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB_PATH), *objs]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
+    if verbose:
+        print(" ".join(ext_link), flush=True)
+    subprocess.run(ext_link, check=True)
     return LIB_PATH
 
 
@@ -68,7 +89,7 @@ def _drain(procs, verbose):
         out, _ = pr.communicate()
         lines = [l for l in out.splitlines() if "packed-fp32-ops" not in l]
         if pr.returncode != 0:
-            raise RuntimeError(f"hipcc failed on {src}:\n" + "\n".join(lines))
+            raise RuntimeError(f"compiling {src} failed:\n" + "\n".join(lines))
         if verbose and lines:
             print("\n".join(lines), flush=True)
     procs.clear()

@@ -86,6 +86,15 @@ def mask_code(causal, window, n_q: int, n_k: int):
     return code, int(window)
 
 
+_MASK_CODES = {None: _lib.MASK_NONE, False: _lib.MASK_NONE, True: _lib.MASK_TOP_LEFT, "bottom_right": _lib.MASK_BOTTOM_RIGHT}
+
+
+def native_mask(causal, window):
+    """The mask arguments for the native host side, which declines what it does not know (-1)."""
+    code = _MASK_CODES.get(causal, -1) if causal is None or isinstance(causal, (bool, int, str)) else -1
+    return code, 0 if window is None else int(window) if int(window) >= 1 else -1
+
+
 def _workspace(args: "_lib.BwdBwdArgs", device, split: bool) -> torch.Tensor:
     """Allocate the workspace of a call and enter it into ``args``: the three row statistics ``d | dd | b`` and, with
     ``split``, room for the partial results of launches that split their streamed side (``fhog_bwdbwd_workspace_hint``)."""
@@ -164,6 +173,16 @@ def flash_bwdbwd(Q, K, V, O, dO, ddQ, ddK, ddV, L, scale, *, causal=False, windo
     Returns:
         dQ2, dK2, dV2, ddO shaped and typed like Q, K, V, O (+ ``(d, dd, b)`` if ``return_stats``).
     """
+    if only_pass is None and not return_stats and isinstance(Q, torch.Tensor) and Q.is_cuda:
+        sched = -1 if fused_stats and schedule not in (None, "fused_stats") else _SCHEDULES.get("fused_stats" if fused_stats else schedule, -1)
+        try:
+            res = _lib.torch_ext().double_backward(Q, K, V, O, dO, ddQ, ddK, ddV, L, float(scale), *native_mask(causal, window),
+                                                   _IMPLS.get(impl, -1), sched, bool(split))
+        except TypeError:   # not tensors: named below
+            res = None
+        if res is not None:
+            return res
+    # what the native call does not do (statistics, single passes) or declined: checked argument by argument
     tensors = dict(Q=Q, K=K, V=V, O=O, dO=dO, ddQ=ddQ, ddK=ddK, ddV=ddV)
     for n, t in tensors.items():
         if not isinstance(t, torch.Tensor):

@@ -1,0 +1,87 @@
+"""GPU tier: the native host side of the entry points against the Python wrappers around the same kernels."""
+import pytest
+import torch
+
+from gpu_util import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _dev():
+    return require_gpu()
+
+
+def _make(layout, n, d, dtype, g):
+    """A (2, 3, n, d) or (6, n, d) tensor lying in memory as named."""
+    x = torch.randn(2, 3, n, d, generator=g).to(dtype).cuda()
+    if layout == "heads_last":      # (B, N, H, d) seen as (B, H, N, d)
+        return x.transpose(1, 2).contiguous().transpose(1, 2)
+    if layout == "padded":          # rows 16 elements longer than d
+        y = torch.zeros(2, 3, n, d + 16, dtype=dtype, device="cuda")
+        y[..., :d] = x
+        return y[..., :d]
+    return x.flatten(0, 1) if layout == "3d" else x
+
+
+@pytest.mark.parametrize("layouts", [("3d", "3d"), ("4d", "4d"), ("heads_last", "heads_last"), ("padded", "padded"), ("4d", "heads_last"),
+                                     ("padded", "4d")])
+@pytest.mark.parametrize("case", [(torch.bfloat16, 128, True), (torch.float32, 64, False), (torch.float16, 32, "bottom_right")])
+def test_native_and_python_chains_agree_bit_for_bit(layouts, case):
+    """attention() through native nodes against FlashAttention.apply, and flash_bwdbwd against its own slow path (which
+    return_stats takes): same kernels on the same tensors, so the same bits, and results laid out like the inputs."""
+    import fhog
+    dtype, d, causal = case
+    g = torch.Generator().manual_seed(65)
+    q, do, ddq = (_make(layouts[0], 70, d, dtype, g) for _ in range(3))
+    k, v, ddk, ddv = (_make(layouts[1], 70 if causal is True else 90, d, dtype, g) for _ in range(4))
+
+    def chain(attn):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v, do)]
+        out = attn(*leaves[:3], causal)
+        first = torch.autograd.grad(out, leaves[:3], leaves[3], create_graph=True)
+        second = torch.autograd.grad(first, leaves, (ddq, ddk, ddv))
+        return (out, *first, *second)
+
+    for a, b in zip(chain(fhog.attention), chain(fhog.FlashAttention.apply)):
+        assert a.shape == b.shape and torch.equal(a, b)
+    o, L = fhog.attention_forward(q, k, v, None, causal)
+    args = (q, k, v, o, do, ddq, ddk, ddv, L, d ** -0.5)
+    native, python = fhog.flash_bwdbwd(*args, causal=causal), fhog.flash_bwdbwd(*args, causal=causal, return_stats=True)[:4]
+    for a, b, like in zip(native, python, (q, k, v, o)):
+        assert a.shape == like.shape and a.dtype == dtype and torch.equal(a, b)
+
+
+def test_third_derivatives_are_refused():
+    import fhog
+    q, k, v, w = (torch.randn(1, 40, 64, device="cuda").requires_grad_(True) for _ in range(4))
+    first = torch.autograd.grad(fhog.attention(q, k, v), (q, k, v), w, create_graph=True)
+    second = torch.autograd.grad(first[0].square().sum(), q, create_graph=True)[0]
+    with pytest.raises(RuntimeError, match="differentiate twice"):
+        second.sum().backward()
+
+
+def test_use_on_another_stream_and_thread():
+    """The native call launches on the calling thread's current stream, backward included."""
+    import threading
+    import fhog
+    q, k, v = (torch.randn(2, 300, 64, device="cuda") for _ in range(3))
+
+    def grads():
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        return torch.autograd.grad(fhog.attention(*leaves, True).sum(), leaves)
+
+    want, got = grads(), []
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+            got.extend(grads())
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
