@@ -429,7 +429,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_bf16(Params 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // with a split, n_split consecutive "slices" share one (batch*head) slice and take its streamed tiles in turn
   int bh, tile, split = 0;
-  if (!decode_block((p.n_q + 32 * NW - 1) / (32 * NW), p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  if (!decode_block((p.n_q + 32 * NW - 1) / (32 * NW), p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && NW == 4)) return;
   if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   RowChain unused;
   q_sweep_run<F16, D, PASS, MASK, NW, SUB, false>(p, smem, bh, tile, split, unused);
@@ -611,7 +611,7 @@ __global__ void __launch_bounds__(256, 2) k_sweep_bf16(Params p) {
   constexpr int STAGE = 3 * TILE + STAT;   // Q, ddQ, dO tiles, statistics
 
   int bh, tile, split = 0;
-  if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major, bh, tile)) return;
+  if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major, bh, tile, MASK != MASK_NONE)) return;
   if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -1,0 +1,37 @@
+"""GPU tier: the order in which workgroups take the tiles of a masked launch (decode_block), around the 32nd, 64th and 65th
+workgroup of an XCD: every tile of every slice is computed, exactly as when the slice is launched alone."""
+import pytest
+import torch
+
+from gpu_util import make_case, require_gpu, run_fhog
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _dev():
+    return require_gpu()
+
+
+# slices per XCD (a multiple of 8 slices, slices / 8 each) x tiles of 128 rows: 32, 33, 63, 64 and 65 workgroups of an XCD
+@pytest.mark.parametrize("slices,tiles", [(64, 4), (24, 11), (168, 3), (128, 4), (40, 13)])
+@pytest.mark.parametrize("d,causal", [(32, True), (64, True), (64, "bottom_right"), (128, True)])
+def test_batched_launch_equals_its_slices(slices, tiles, d, causal):
+    import fhog
+    n = 128 * tiles - 5
+    scale = d ** -0.5
+    x = make_case(slices, n, n if causal is True else n + 70, d, torch.bfloat16, seed=71, grad_std=0.1)
+
+    def outputs(x):
+        o, L = fhog.attention_forward(x["Q"], x["K"], x["V"], scale, causal, use_hip=True)
+        first = fhog.attention_backward(x["Q"], x["K"], x["V"], o, x["dO"], L, scale, causal, use_hip=True)
+        second = [t for s in ("fused_stats", "three_sweep") for t in run_fhog(dict(x, O=o, L=L), scale, causal, schedule=s, split=False)]
+        return (o, L, *first, *second)
+
+    got = outputs(x)
+    for s in (0, slices // 2, slices - 1):
+        # as many copies of one slice as put four waves on its rows in the small launch too
+        alone = outputs({name: t[s:s + 1].expand(43, -1, -1).contiguous() for name, t in x.items()})
+        for a, b in zip(got, alone):
+            assert torch.equal(a[s], b[0]) and torch.equal(a[s], b[42])
+    assert all(torch.isfinite(t.float()).all() for t in got)
