@@ -163,9 +163,45 @@ int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
   return s;
 }
 
+// Splits a pass runs with. Passes 3 and 4 at d = 128 keep one workgroup on a CU: what matters there is rounds of 256
+// workgroups times the tiles of one, under the mask, and what the partial results cost. In steps of one tile (1.9 us): a
+// workgroup needs about 4 to start and to store, combining 2 plus its bytes at 5 TB/s (14.5 us for 66 MB, 8 for 33).
+// Where the work of the workgroups differs (causal) the longest one and the average load bound the launch.
+// bf16 16 x 1000 x 3001, window 700, us, as many splits as give 512 workgroups -> this rule: pass 3 with 4 -> 2 splits 49.2 + 14.5
+// (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
+int launch_split_of(const fhog_bwdbwd_args* a, const fhog::Params& p, int impl, int pass) {
+  const int most = granted_split(a, impl, pass);
+  if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
+  const bool kside = pass == FHOG_PASS_DK_DV;
+  const int64_t n_sta = kside ? a->n_k : a->n_q, n_str = kside ? a->n_q : a->n_k;
+  int64_t live = 0, longest = 0, sum = 0;   // workgroups of a slice with a visible pair, and the tiles they visit
+  for (int64_t r0 = 0; r0 < n_sta; r0 += 128) {   // fewer than 512 workgroups, or nothing would split
+    int64_t lo = 0, hi = n_str;   // streamed rows visible to [r0, r0 + 128)
+    if (p.causal) {
+      const int64_t first = kside ? r0 - p.mask_off : r0 + p.mask_off - p.window + 1;
+      const int64_t last = kside ? r0 + 127 - p.mask_off + p.window - 1 : r0 + 127 + p.mask_off;
+      lo = first > 0 ? first : 0, hi = last + 1 < n_str ? last + 1 : n_str;
+    }
+    if (lo >= hi) continue;
+    const int64_t tiles = (hi - 1) / 32 - lo / 32 + 1;
+    live++, sum += tiles, longest = tiles > longest ? tiles : longest;
+  }
+  if (live == 0) return 1;
+  int best = 1;
+  double best_cost = 0;
+  for (int s = 1; s <= most; s *= 2) {
+    const double rounds = (double)((live * a->batch * s + 255) / 256), mean = (double)sum / (double)live;
+    const double alone = (double)longest / s + 4, load = rounds * (mean / s + 4);
+    double cost = alone > load ? alone : load;
+    if (s > 1) cost += 2 + (double)s * split_bytes(a, pass) / (5e6 * 1.9);
+    if (s == 1 || cost < best_cost) best = s, best_cost = cost;
+  }
+  return best;
+}
+
 int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
   fhog::Params p = base;
-  p.n_split = granted_split(a, impl, pass);
+  p.n_split = launch_split_of(a, p, impl, pass);
   // Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all
   // of them first) balances the end of a launch; from 16384 stationary rows on a slice alone has tiles enough for that
   // and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x

@@ -1,0 +1,28 @@
+"""GPU tier: how many splits passes 3 and 4 run with at d = 128 (rounds of workgroups under the mask against the cost of
+combining): whatever the rule picks, results are those of the launch that does not split."""
+import pytest
+import torch
+
+from gpu_util import NAMES, make_case, normalised_max_error, require_gpu, run_fhog, with_caches
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _dev():
+    return require_gpu()
+
+
+# keys without a query at the front of the K side, one split of several, uneven work of a causal mask, 2 rounds that become 1
+@pytest.mark.parametrize("shape", [(16, 1000, 3001, "bottom_right", 700), (1, 300, 5000, "bottom_right", 64), (2, 2048, 2048, True, None),
+                                   (24, 1536, 1536, True, 100), (3, 4095, 513, False, None), (40, 1025, 1024, False, None)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_by_rounds(shape, dtype):
+    batch, n_q, n_k, causal, window = shape
+    scale = 128 ** -0.5
+    x = with_caches(make_case(batch, n_q, n_k, 128, dtype, seed=72, grad_std=0.1), scale, causal, window)
+    split, whole = [run_fhog(x, scale, causal, window=window, split=s) for s in (True, False)]
+    # sums in another order, rounded once: one unit of the type at the largest element (2^-8 for bf16, 2^-11 for fp16)
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for name, a, b in zip(NAMES, split, whole):
+        assert normalised_max_error(a, b.float()) <= unit, name
