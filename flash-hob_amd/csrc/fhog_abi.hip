@@ -373,17 +373,7 @@ int fhog_attn_bwd(const fhog_attn_args* args, void* hip_stream) {
   const int rc = validate_attn(args, 1);
   if (rc != FHOG_OK) return rc;
   const fhog::AttnParams p = to_attn_params(args);
-  fhog::Params rd = {};  // row sums d_i = sum_c o_ic dO_ic with the kernel of pass 0
-  rd.o = args->o;
-  rd.dO = args->dO;
-  rd.ws_d = args->ws;
-  rd.stride_qb = p.stride_qb;
-  rd.stride_qn = p.stride_qn;
-  rd.batch = p.batch;
-  rd.n_q = p.n_q;
-  rd.d = p.d;
-  // (the split-product kernel for dQ takes them itself)
-  hipError_t e = attn_on_16bit_kernels(args) ? fhog::launch_rowdot(rd, args->dtype, (hipStream_t)hip_stream) : hipSuccess;
+  hipError_t e = hipSuccess;   // the dQ kernel also writes the row sums d that the one for dK and dV reads
   for (int which = 1; which <= 2 && e == hipSuccess; which++)
     e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(p, which, (hipStream_t)hip_stream)
                                     : fhog::launch_attn_split(p, args->dtype, which, (hipStream_t)hip_stream);

@@ -13,6 +13,11 @@
 // second-level MFMA whose contraction runs over the streamed rows: slot e of k-step t stands for streamed row
 // 16t + 8(e/4) + 4h + e%4, and the A operand (the transposed value tile) is fetched from LDS with transposing
 // reads that use the same row order. Second-level operands therefore never pass through LDS.
+//
+// What bounds them: vector and matrix instructions of a SIMD. Forward, 32 x 4096, d = 128, no mask: the matrix pipe is busy 43 %
+// of the cycles and the VALU 48 %, and taking out the exponentials, the LDS reads or half of the staging moves the time by less
+// than 5 %. Issuing the first level of a tile beside the second level of the tile before, each behind the other's
+// elementwise work, measured equal (d = 64: +-3 %, d = 128: 2 % slower); fewer VALU instructions per block is what paid.
 #include "fhog_bf16_util.h"
 
 namespace fhog {
@@ -102,13 +107,15 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
   Dma<D> dma;
   dma.init(p.stride_kn, wave, lane);
   const uint32_t ring_lds = lds_addr(smem);
-  dma.template issue_all<2>(ring_lds + (j_begin & 1) * STAGE, TILE, src, (int64_t)j_begin * TS * p.stride_kn, wave, p.n_k - j_begin * TS);
+  dma.template issue_all<2>(ring_lds, TILE, src, (int64_t)j_begin * TS * p.stride_kn, wave, p.n_k - j_begin * TS);
   dma_wait();
   __syncthreads();
 
-  for (int j = j_begin; j < j_end; j++) {
+  // Tile j in ring slot u. The slot is a constant: it goes into the offsets of the LDS reads.
+  const auto step = [&](auto slot, int j) {
+    constexpr int u = decltype(slot)::value;
     if (j + 1 < j_end) {
-      const uint32_t dst = ring_lds + ((j + 1) & 1) * STAGE;
+      const uint32_t dst = ring_lds + (u ^ 1) * STAGE;
       const int64_t adv = (int64_t)(j + 1) * TS * p.stride_kn;
       dma.template issue_all<2>(dst, TILE, src, adv, wave, p.n_k - (j + 1) * TS);
     }
@@ -117,7 +124,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
     if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
-      const char* stage = smem + (j & 1) * STAGE;
+      const char* stage = smem + u * STAGE;
       f32x16_t s[1] = {f32x16_t{0}};
       const bf16x8_t* const res[1] = {Qb};
       first_level<F16, D, 1>(stage, aoff, res, s);  // S^T: s[r] = (key k0 + 8(r/4) + 4h + r%4, query qi)
@@ -160,7 +167,10 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
     }
     dma_wait();
     __syncthreads();
-  }
+  };
+  int j = j_begin;
+  for (; j + 1 < j_end; j += 2) step(Slot<0>{}, j), step(Slot<1>{}, j + 1);
+  if (j < j_end) step(Slot<0>{}, j);
   l += __shfl_xor(l, 32);
   const float inv = 1.f / l;
   if (qi >= p.n_q) return;
@@ -176,7 +186,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
   if (h == 0) p.lse[(int64_t)bh * p.n_q + qi] = (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;  // v_log_f32 is log2
 }
 
-// ---- backward, Q-tiled: dQ -----------------------------------------------------------------------------
+// ---- backward, Q-tiled: dQ, and d for the K-tiled kernel behind it ---------------------------------------
 template <bool F16, int D, int MASK>
 __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -196,7 +206,18 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
   load_resident<D>(Qb, (const __bf16*)p.q + qoff, p.stride_qn, qr, h);
   load_resident<D>(dOb, (const __bf16*)p.dO + qoff, p.stride_qn, qr, h);
   const int64_t row = (int64_t)bh * p.n_q + qr;
-  const float l_log2 = p.lse[row] * kLog2e, dsum = p.ws_d[row];
+  const float l_log2 = p.lse[row] * kLog2e;
+  float dsum = 0.f;   // d_i = sum_c O_ic dO_ic: each lane takes half of its query's row
+  {
+    bf16x8_t Ob[KK];
+    load_resident<D>(Ob, (const __bf16*)p.o + qoff, p.stride_qn, qr, h);
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) dsum = __builtin_fmaf(to_f32<F16>(Ob[kk][e]), to_f32<F16>(dOb[kk][e]), dsum);
+    dsum += __shfl_xor(dsum, 32);
+    if (h == 0 && qi < p.n_q) p.ws_d[row] = dsum;
+  }
   wait_vm0();
   const float c_scale_log2 = p.scale * kLog2e;
 
@@ -218,13 +239,15 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
   Dma<D> dma;
   dma.init(p.stride_kn, wave, lane);
   const uint32_t ring_lds = lds_addr(smem);
-  dma.template issue_all<2>(ring_lds + (j_begin & 1) * STAGE, TILE, src, (int64_t)j_begin * TS * p.stride_kn, wave, p.n_k - j_begin * TS);
+  dma.template issue_all<2>(ring_lds, TILE, src, (int64_t)j_begin * TS * p.stride_kn, wave, p.n_k - j_begin * TS);
   dma_wait();
   __syncthreads();
 
-  for (int j = j_begin; j < j_end; j++) {
+  // Tile j in ring slot u. The slot is a constant: it goes into the offsets of the LDS reads.
+  const auto step = [&](auto slot, int j) {
+    constexpr int u = decltype(slot)::value;
     if (j + 1 < j_end) {
-      const uint32_t dst = ring_lds + ((j + 1) & 1) * STAGE;
+      const uint32_t dst = ring_lds + (u ^ 1) * STAGE;
       const int64_t adv = (int64_t)(j + 1) * TS * p.stride_kn;
       dma.template issue_all<2>(dst, TILE, src, adv, wave, p.n_k - (j + 1) * TS);
     }
@@ -233,7 +256,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
     if (!geo.dead(k0, qw)) {
-      const char* stage = smem + (j & 1) * STAGE;
+      const char* stage = smem + u * STAGE;
       f32x16_t s[1] = {f32x16_t{0}}, dp[1];
 #pragma unroll
       for (int r = 0; r < 16; r++) dp[0][r] = -dsum;        // the accumulator ends as dP - d
@@ -255,7 +278,10 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
     }
     dma_wait();
     __syncthreads();
-  }
+  };
+  int j = j_begin;
+  for (; j + 1 < j_end; j += 2) step(Slot<0>{}, j), step(Slot<1>{}, j + 1);
+  if (j < j_end) step(Slot<0>{}, j);
   if (qi >= p.n_q) return;
   __bf16* o = (__bf16*)p.dq + qoff + (int64_t)qi * p.stride_qn;
 #pragma unroll
