@@ -179,7 +179,9 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
   dma_wait();
   __syncthreads();
 
-  for (int jj = j_begin; jj < j_end; jj += SUB) {
+  // one group of SUB tiles, in the first or the second half of the ring
+  const auto group = [&](auto half_of_ring, int jj) {
+    constexpr int GRP = decltype(half_of_ring)::value * SUB;
 #pragma unroll
     for (int u = 0; u < SUB; u++)
       if (jj + SUB + u < j_end) stage_tile(jj + SUB + u);
@@ -192,7 +194,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
       int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
       if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
       if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
-        const char* stage = smem + (((jj - j_begin) & SUB) + u) * STAGE;
+        const char* stage = smem + (GRP + u) * STAGE;
         // The products are issued as a stream of NT*KK k-steps (K, then V, ddK, ddV); the elementwise work
         // is cut into small pieces placed right behind the MFMAs of the same wave, where it runs in the
         // shadow of the matrix pipe. LDS operands are fetched PF steps ahead.
@@ -356,9 +358,14 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
         }
       }
     }
+    // sums stay in their step: carried over to the next one, as the compiler would, their summands take its registers
+    if (!P3) asm volatile("" : "+v"(red), "+v"(red_dd), "+v"(red_vdds), "+v"(red_pu), "+v"(red_p));
     dma_wait();
     __syncthreads();
-  }
+  };
+  int jj = j_begin;
+  for (; jj + SUB < j_end; jj += 2 * SUB) group(Slot<0>{}, jj), group(Slot<1>{}, jj + SUB);
+  if (jj < j_end) group(Slot<0>{}, jj);
   if (WITH_DDO && p.n_split > 1) {   // fp32 partial rows [split][dQ2 | ddO][batch * n_q][D]
     if (qi >= p.n_q) return;
     const int64_t rows = (int64_t)p.batch * p.n_q;
@@ -695,8 +702,8 @@ __global__ void __launch_bounds__(256, 2) k_sweep_bf16(Params p) {
   dma_wait();
   __syncthreads();
 
-  for (int jj = t_begin; jj < t_end; jj += SUB) {
-    const int grp = (jj - t_begin) & SUB;   // first ring slot of this group; the other group starts at grp ^ SUB
+  const auto group = [&](auto half_of_ring, int jj) {
+    constexpr int grp = decltype(half_of_ring)::value * SUB;   // first ring slot of this group; the other group starts at grp ^ SUB
 #pragma unroll
     for (int u = 0; u < SUB; u++)
       if (jj + SUB + u < t_end) {
@@ -801,7 +808,10 @@ __global__ void __launch_bounds__(256, 2) k_sweep_bf16(Params p) {
     }
     dma_wait();
     __syncthreads();
-  }
+  };
+  int jj = t_begin;
+  for (; jj + SUB < t_end; jj += 2 * SUB) group(Slot<0>{}, jj), group(Slot<1>{}, jj + SUB);
+  if (jj < t_end) group(Slot<0>{}, jj);
   if (kj >= p.n_k) return;
   if (p.n_split > 1) {   // fp32 partial rows [split][dK2 | dV2][batch * n_k][D]
     const int64_t rows = (int64_t)p.batch * p.n_k;

@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_ddo(Params p
   dma.init(p.stride_kn, wave & 3, lane);
   const uint32_t ring_lds = lds_addr(smem) + half * NLD * TILE;
   const auto stage_tile = [&](int j) {
-    dma.template issue_all<NLD>(ring_lds + (j & 1) * STAGE, TILE, srcl, (int64_t)j * TS * p.stride_kn, wave & 3, p.n_k - j * TS);
+    dma.template issue_all<NLD>(ring_lds + ((j - j_begin) & 1) * STAGE, TILE, srcl, (int64_t)j * TS * p.stride_kn, wave & 3, p.n_k - j * TS);
   };
   if (j_begin < j_end) stage_tile(j_begin);
 
@@ -91,14 +91,14 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_ddo(Params p
   __syncthreads();
 
   float red = 0.f;   // KNOWN_DD = false: this lane's share of sum_j P_ij ddS_ij scale
-  for (int j = j_begin; j < j_end; j++) {
+  const auto step = [&](auto slot, int j) {   // tile j in ring slot `slot`
     if (j + 1 < j_end) stage_tile(j + 1);
     const int k0 = j * TS;
     const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
     if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
-      const char* stage = smem + (j & 1) * STAGE;
+      const char* stage = smem + decltype(slot)::value * STAGE;
       // first level, a stream of 2 KK k-steps with the LDS operands fetched PF steps ahead (stage order K, ddK, V, ddV):
       //   K  : S += K Q^T, ddS += K ddQ^T
       //   ddK: ddS += ddK Q^T          + P = exp2(S c - L) behind the MFMAs (in place of S)
@@ -173,7 +173,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_ddo(Params p
     }
     dma_wait();
     __syncthreads();
-  }
+  };
+  int j = j_begin;
+  for (; j + 1 < j_end; j += 2) step(Slot<0>{}, j), step(Slot<1>{}, j + 1);
+  if (j < j_end) step(Slot<0>{}, j);
 
   // end of the row: dd, d, ddO and b = dO . ddO - d dd. Each lane holds half of its query's columns.
   float dd = dd_in, dsum = d_in;
