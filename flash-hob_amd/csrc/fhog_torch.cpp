@@ -94,6 +94,13 @@ struct Group {
   Tensor like() const { return at::empty_strided(t[0].sizes(), t[0].strides(), t[0].options()); }
 };
 
+// What autograd hands over, packed. contiguous() passes over the stride of a dimension of one (a single query that came back
+// through (B, 1, H, d)) and over the address, both of which the kernels look at.
+Tensor packed(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return layout_of(c).direct ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
 Tensor as_lse(const Tensor& L) { return L.scalar_type() == at::kFloat && L.is_contiguous() ? L : L.to(at::kFloat).contiguous(); }
 Tensor workspace(int64_t bytes, const Tensor& like) { return at::empty({(bytes + 3) / 4}, like.options().dtype(at::kFloat)); }
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -214,7 +221,7 @@ struct FirstBackward : torch::autograd::Function<FirstBackward> {
                                                                (g[2].defined() && g[2].requires_grad()));
     {
       const at::NoGradGuard no_grad;
-      const auto dir = [&](size_t i) { return g[i].defined() ? g[i].contiguous() : at::zeros_like(s[i]); };
+      const auto dir = [&](size_t i) { return g[i].defined() ? packed(g[i]) : at::zeros_like(s[i]); };
       const auto r = double_backward(s[0], s[1], s[2], s[3], s[4], dir(0), dir(1), dir(2), s[5], scale_of(s[0]), Mask{(int32_t)arg[0], arg[1]},
                                      FHOG_IMPL_AUTO, (int)arg[2], true);
       TORCH_CHECK(r, "fhog: double-backward: ", fhog_last_error());
@@ -247,7 +254,7 @@ struct Attention : torch::autograd::Function<Attention> {
     if (!g[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto arg = ctx->saved_data["arg"].toIntVector();
-    const auto r = FirstBackward::apply(s[0], s[1], s[2], s[3], g[0].contiguous(), s[4], arg[0], arg[1], arg[2]);
+    const auto r = FirstBackward::apply(s[0], s[1], s[2], s[3], packed(g[0]), s[4], arg[0], arg[1], arg[2]);
     out[0] = r[0], out[1] = r[1], out[2] = r[2];
     return out;
   }

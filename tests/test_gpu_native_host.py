@@ -52,6 +52,31 @@ def test_native_and_python_chains_agree_bit_for_bit(layouts, case):
         assert a.shape == like.shape and a.dtype == dtype and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n", [1, 2, 33])
+@pytest.mark.parametrize("lie", ["heads_last", "unaligned"])
+def test_gradients_that_only_look_contiguous(n, lie):
+    """Gradients of both orders in layouts that is_contiguous() accepts and the kernels do not: one query that comes back through
+    (B, 1, H, d), and addresses off a multiple of 16 bytes. The same bits as packed ones."""
+    import fhog
+    g = torch.Generator().manual_seed(66)
+
+    def laid_out(x):
+        if lie == "heads_last":
+            return x.transpose(1, 2).contiguous().transpose(1, 2)
+        y = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+        return y.copy_(x)
+
+    q, k, v, do, ddq, ddk, ddv = (torch.randn(2, 3, n, 64, generator=g).bfloat16().cuda() for _ in range(7))
+
+    def chain(f):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v, f(do))]
+        first = torch.autograd.grad(fhog.attention(*leaves[:3]), leaves[:3], leaves[3], create_graph=True)
+        return (*first, *torch.autograd.grad(first, leaves, (f(ddq), f(ddk), f(ddv))))
+
+    for a, b in zip(chain(laid_out), chain(lambda t: t)):
+        assert torch.equal(a, b)
+
+
 def test_third_derivatives_are_refused():
     import fhog
     q, k, v, w = (torch.randn(1, 40, 64, device="cuda").requires_grad_(True) for _ in range(4))
