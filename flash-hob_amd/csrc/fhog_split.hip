@@ -64,6 +64,14 @@ struct Resident {
 template <typename T, int D, int WS>
 constexpr int n_buffers(int stage) { return WS == 1 && !is_raw<T, D> && 2 * stage <= 160 * 1024 ? 2 : 1; }
 
+// A statistics sweep whose four waves share their rows: each streamed tile has one reader, and its rows as they lie in memory
+// are the A operand of the first level, which is all these sweeps have. The wave loads them two k-steps ahead straight into
+// registers: no staging through LDS, no barriers, and no LDS limit on the split (fp32: two tiles of four tensors at d = 64, one
+// at 128). Pass 5, us, staged -> direct: fp32 2 x 256, d = 64 20.8 -> 14.1; fp32 causal 1 x 4096, d = 128 977 -> 240;
+// fp32 causal 1 x 6000, d = 64 365 -> 169; bf16 1 x 8000, d = 32 66 -> 38; bf16 causal 2 x 512, d = 32 7.3 -> 6.0.
+template <int PASS, int WS>
+constexpr bool is_direct = WS == 4 && (PASS == 1 || PASS == 2 || PASS == 5);
+
 // PASS 1: d, dd; 2: b; 3: dQ2, ddO; 4: dK2, dV2 (K-tiled); 5: d, dd, b.
 template <typename T, int D, int PASS, int MASK, int WS>
 __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Params p) {
@@ -82,6 +90,7 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   constexpr bool RAW = is_raw<T, D>;
   constexpr bool LAST_IN_LDS = RAW && !STATS;
   constexpr int NREG = LAST_IN_LDS ? NR - 1 : NR;
+  constexpr bool DIRECT = is_direct<PASS, WS>;
   constexpr int NBUF = n_buffers<T, D, WS>(STAGE);
   constexpr int nw = 4 / WS, ROWS = 32 * nw;
 
@@ -140,7 +149,7 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
       }
     }
   };
-  if (t_begin < t_end) fetch(t_begin);
+  if (!DIRECT && t_begin < t_end) fetch(t_begin);
 
   const T* const sta[4] = {KSIDE ? (const T*)p.k + koff : (const T*)p.q + qoff, KSIDE ? (const T*)p.ddk + koff : (const T*)p.ddq + qoff,
                            KSIDE ? (const T*)p.v + koff : (const T*)p.dO + qoff, (const T*)p.ddv + koff};
@@ -191,6 +200,13 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   for (int cb = 0; cb < NC; cb++) acc0[cb] = f32x16_t{0}, acc1[cb] = f32x16_t{0};
   float red[5] = {};               // statistics: b-like sum; fused sweep: dd, sum P u ddS, sum P u, sum P
 
+  Chunk<T> ahead[2][NT];           // DIRECT: the next two k-steps of the lane's streamed row
+  const auto load_step = [&](int t, int kk) {
+    const int64_t off = (int64_t)min(t * TS + n, n_str - 1) * str_ld + 16 * kk + 8 * h;
+#pragma unroll
+    for (int x = 0; x < NT; x++) ahead[kk & 1][x] = load_chunk<T>(src[x] + off);
+  };
+
   // prefetch: what requests the next tile; called where the registers it lands in are free
   const auto block = [&](const char* stage, int s0, auto prefetch) {
     const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
@@ -226,21 +242,26 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
       };
       if constexpr (KSIDE) res[2].terms(kk, r2), last_terms(r3);
       else if constexpr (PASS != 1) last_terms(r2);
-      read_terms<T, Stage::TILE>(stage, aoff[kk], a);
+      const auto streamed = [&](int x) {
+        if constexpr (DIRECT) chunk_terms<T, true, NF>(ahead[kk & 1][x], a);
+        else read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a);
+      };
+      streamed(0);
       s = mma1<T>(s, a, r0);                                  // K Q^T | Q K^T
       dds = mma1<T>(dds, a, r1);                              // K ddQ^T | Q ddK^T
       if constexpr (PASS != 1) {
-        read_terms<T, Stage::TILE>(stage + 2 * TENSOR, aoff[kk], a);
+        streamed(2);
         dp = mma1<T>(dp, a, r2);                              // V dO^T | dO V^T
         if constexpr (KSIDE) e = mma1<T>(e, a, r3);           // dO ddV^T
       }
-      read_terms<T, Stage::TILE>(stage + 1 * TENSOR, aoff[kk], a);
+      streamed(1);
       dds = mma1<T>(dds, a, r0);                              // + ddK Q^T | ddQ K^T
       if constexpr (PASS != 1 && !KSIDE) {
-        read_terms<T, Stage::TILE>(stage + (NT - 1) * TENSOR, aoff[kk], a);
+        streamed(NT - 1);
         e = mma1<T>(e, a, r2);                                // ddV dO^T
       }
-      if constexpr (RAW) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (DIRECT) load_step(s0 / TS + (kk + 2 < KK ? 0 : WS), (kk + 2) % KK);   // past the last tile: its last row again
+      if constexpr (RAW || DIRECT) __builtin_amdgcn_sched_barrier(0);
     }
     f32x16_t pv;
 #pragma unroll
@@ -300,9 +321,14 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   };
 
   constexpr bool LATE = RAW && !STATS;   // the next tile is requested towards the end of a step: no registers for it before
-  if (t_begin < t_end) publish(0);
-  __syncthreads();
-  for (int t = t_begin; t < t_end; t += WS) {
+  if constexpr (DIRECT) {
+    // the range of 32 rows holds no tile that is dead to the wave
+    if (t_begin + ws < t_end) load_step(t_begin + ws, 0), load_step(t_begin + ws, 1);
+    for (int t = t_begin + ws; t < t_end; t += WS) block(smem, t * TS, [] {});
+  }
+  if (!DIRECT && t_begin < t_end) publish(0);
+  if (!DIRECT) __syncthreads();
+  for (int t = t_begin; !DIRECT && t < t_end; t += WS) {
     const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
     const bool more = t + WS < t_end;
     const auto next = [&]() {
@@ -377,7 +403,7 @@ constexpr int lds_bytes() {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4), nw = 4 / WS;
   constexpr int stage = Stager<T, D, NT, !STATS>::BYTES + (KSIDE ? 4 * TS * 4 : 0);
-  constexpr int stages = n_buffers<T, D, WS>(stage) * WS * stage + (is_raw<T, D> && !STATS ? 4 * TS * D * 4 : 0);
+  constexpr int stages = is_direct<PASS, WS> ? 0 : n_buffers<T, D, WS>(stage) * WS * stage + (is_raw<T, D> && !STATS ? 4 * TS * D * 4 : 0);
   constexpr int xch = WS > 1 ? nw * (WS - 1) * (STATS ? 5 : 2 * D / 32 * 16) * 64 * 4 : 0;
   return stages > xch ? stages : xch;
 }
@@ -395,7 +421,7 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 
 // Four waves on 128 stationary rows share the streamed tiles and their splitting, the best shape whenever that fills the GPU
 // (256 CUs). With fewer than 128 (64) such workgroups two (four) waves go on the same 32 rows, where the tiles of a step fit
-// the LDS: two fp32 heads of 256 tokens are 4 workgroups otherwise, each running its eight streamed tiles one after the other.
+// the LDS (four waves of a statistics sweep stage nothing): two fp32 heads of 256 tokens are 4 workgroups otherwise, each running its eight streamed tiles one after the other.
 template <typename T, int D, int PASS, int MASK>
 hipError_t launch_sweep(const Params& p, hipStream_t s) {
   const int64_t groups = (int64_t)((PASS == 4 ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = PASS == 4 ? p.n_q : p.n_k;

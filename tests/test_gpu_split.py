@@ -66,3 +66,34 @@ def test_first_order_on_split_products(shape, case):
         # one visible key per query (n_k = 1 or a window of 1): dS vanishes identically and the rounding of O is what is left
         floor = 1e-4 if dtype == torch.float32 else 1e-2
         assert (g[sel].double().cpu() - torch.from_numpy(w)).abs().max() < TOL[dtype] * abs(w).max() + floor, name
+
+
+@pytest.mark.parametrize("dtype", list(TOL))
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape", [(1, 33, 66, False, None), (2, 40, 333, False, None), (1, 290, 290, True, None), (1, 31, 400, "bottom_right", 200)])
+def test_statistics_sweep_that_stages_nothing(shape, d, dtype):
+    """Four waves on the same rows reading their own tiles: three tiles for four waves, eleven (a remainder in the last round and
+    in the last tile), a causal range that grows, a band whose first tile is not the first one. Padded rows on the streamed side. With 16-bit tensors O is rounded before
+    d = rowsum(O * dO): an absolute error up to 2^-9 sum |O dO|, which the largest |d| of some 30 rows is well above; the d of a
+    single row need not be."""
+    from fhog import BwdBwdPlan
+    batch, n_q, n_k, causal, window = shape
+    x = with_caches(make_case(batch, n_q, n_k, d, dtype, seed=67), d ** -0.5, causal, window)
+    ref = reference_fp64_cpu(x, d ** -0.5, causal, window)
+
+    def padded(t):
+        y = torch.full((*t.shape[:-1], d + 8), float("nan"), dtype=t.dtype, device=t.device)
+        y[..., :d] = t
+        return y[..., :d]
+
+    for lay in (lambda t: t, padded):
+        plan = BwdBwdPlan(x["Q"], lay(x["K"]), lay(x["V"]), x["O"], x["dO"], x["ddQ"], lay(x["ddK"]), lay(x["ddV"]), x["L"], d ** -0.5,
+                          causal=causal, window=window, impl="fp32")
+        for passes in ((5,), (1, 2)):
+            plan.ws.fill_(float("nan"))
+            for i in passes:
+                plan.run(only_pass=i)
+            torch.cuda.synchronize()
+            for got, name in zip(plan.ws[:3 * batch * n_q].view(3, -1), ("d", "dd", "b")):
+                want = torch.as_tensor(ref[name]).reshape(-1)
+                assert normalised_max_error(got, want) < (1e-4 if dtype == torch.float32 else 5e-3), (name, passes)
