@@ -422,11 +422,23 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 // Four waves on 128 stationary rows share the streamed tiles and their splitting, the best shape whenever that fills the GPU
 // (256 CUs). With fewer than 128 (64) such workgroups two (four) waves go on the same 32 rows, where the tiles of a step fit
 // the LDS (four waves of a statistics sweep stage nothing): two fp32 heads of 256 tokens are 4 workgroups otherwise, each running its eight streamed tiles one after the other.
+// A statistics sweep that stages nothing splits every tile into terms once per 32 rows instead of once per 128, but its workgroups
+// are a quarter of the size: worth it beyond 64 workgroups where the staged form leaves CUs to the heaviest tiles of a causal
+// triangle, or has one wave per row block. Pass 5, us, staged -> direct, at so many 128-row workgroups:
+//   triangle: fp32 d = 128 497 -> 130 (64), 502 -> 302 (240); bf16 d = 32 43.7 -> 24.7 (240), 60 x 500 14.0 -> 11.5 (240);
+//             fp32 d = 64 184 -> 82 (128), but 60 x 500 52.2 -> 60.4 (240)
+//   no mask:  fp32 d = 128 553 -> 435 (126); bf16 d = 32 43.0 -> 32.5 (126); fp32 d = 64 129 -> 137 (96)
 template <typename T, int D, int PASS, int MASK>
 hipError_t launch_sweep(const Params& p, hipStream_t s) {
   const int64_t groups = (int64_t)((PASS == 4 ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = PASS == 4 ? p.n_q : p.n_k;
   if constexpr (lds_bytes<T, D, PASS, 4>() <= 160 * 1024) {
-    if (groups < 64 && n_str > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
+    int64_t line = 64;
+    if constexpr (is_direct<PASS, 4>) {
+      const bool triangle = MASK != MASK_NONE && p.mask_off == 0 && p.window >= p.n_k;
+      constexpr bool splits_dear = sizeof(T) == 4 && D < 128;
+      line = triangle ? (splits_dear ? 160 : 256) : splits_dear ? 64 : 128;
+    }
+    if (groups < line && n_str > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
   }
   if constexpr (lds_bytes<T, D, PASS, 2>() <= 160 * 1024) {
     if (groups < 128 && n_str > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
