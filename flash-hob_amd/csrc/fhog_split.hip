@@ -12,11 +12,12 @@
 // every WS-th streamed tile and the partial results are added through LDS in a fixed order.
 //
 // What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
-// 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (26 MFMAs beside some 450 VALU instructions).
+// 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (34 MFMAs beside some 400
+// VALU instructions, half of them the split of P, dS, dS' and ddP).
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same box):
-//   bf16 causal 64 x 1024, d = 32: 734 -> 123     fp32 causal 64 x 1024, d = 32: 672 -> 318
+//   bf16 causal 64 x 1024, d = 32: 734 -> 136     fp32 causal 64 x 1024, d = 32: 672 -> 296
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
-//   fp32 causal 32 x 2048, d = 128: 3833 -> 2422
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2340
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:

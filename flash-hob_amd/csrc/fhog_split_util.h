@@ -4,8 +4,8 @@
 // bf16 number is one. A product of two such sums is a sum of bf16 products, each exact in fp32, accumulated in fp32 by
 // v_mfma_f32_32x32x16_bf16, which does 16 times the work of v_mfma_f32_32x32x2_f32 per cycle. Six of the nine terms of
 // an fp32 product are kept; the three left out are below 2^-24 of it, the rounding of one fp32 addition.
-// The S-shaped operands of the second-level products (P, dS, dS', ddP) are split the same way: three terms for fp32
-// tensors; two for 16-bit tensors, whose results are rounded to 11 or 8 bits while two terms carry 16.
+// The S-shaped operands of the second-level products (P, dS, dS', ddP) are fp32 numbers whatever the tensors are, and three
+// terms for every tensor type: two carry 16 bits, which shows in sums that cancel.
 #pragma once
 #include "fhog_bf16_util.h"
 
@@ -21,12 +21,12 @@ template <typename T>
 struct Terms;
 template <>
 struct Terms<__bf16> {
-  static constexpr int NF = 1, N2 = 1, NS = 2, LDS1 = 1, LDS2 = 1, OFF2 = 0;
+  static constexpr int NF = 1, N2 = 1, NS = 3, LDS1 = 1, LDS2 = 1, OFF2 = 0;
   static constexpr bool F16 = false;
 };
 template <>
 struct Terms<_Float16> {
-  static constexpr int NF = 1, N2 = 2, NS = 2, LDS1 = 1, LDS2 = 3, OFF2 = 1;
+  static constexpr int NF = 1, N2 = 2, NS = 3, LDS1 = 1, LDS2 = 3, OFF2 = 1;
   static constexpr bool F16 = true;
 };
 template <>

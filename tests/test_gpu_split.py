@@ -97,3 +97,33 @@ def test_statistics_sweep_that_stages_nothing(shape, d, dtype):
             for got, name in zip(plan.ws[:3 * batch * n_q].view(3, -1), ("d", "dd", "b")):
                 want = torch.as_tensor(ref[name]).reshape(-1)
                 assert normalised_max_error(got, want) < (1e-4 if dtype == torch.float32 else 5e-3), (name, passes)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("batch", [2, 70, 140])
+def test_weights_beside_16_bit_tensors_are_fp32(batch, d, dtype):
+    """Sums of the weights against +-pairs cancel down to their spread, 2^-13 of a weight here: what is left of them shows how many
+    bits the weights carried. With fp32 ones the roundings of the exponent and of L remain, 2^-22 of a weight each at fewer than 256
+    keys: 2^-8 of the result, besides its own rounding to the type (16 bits of a weight leave 2^-6). Four, two and one wave on the
+    same rows."""
+    import fhog
+    n, s = 190, 2.0 ** -6.5
+    g = torch.Generator().manual_seed(73)
+    q, k = ((torch.randn(batch, n, d, generator=g) * s).to(dtype).cuda() for _ in range(2))
+    pairs = torch.randn(batch, n, d, generator=g).to(dtype).cuda()
+    pairs[:, 1::2] = -pairs[:, ::2]
+    zero = torch.zeros_like(q)
+    scale = d ** -0.5
+    sel = slice(0, batch, 43)
+    p = torch.softmax(q[sel].double().cpu() @ k[sel].double().cpu().transpose(1, 2).contiguous() * scale, -1)
+    x = pairs[sel].double().cpu()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    o, L = fhog.attention_forward(q, k, pairs, scale)
+    got = {"ddo": (fhog.flash_bwdbwd(q, k, zero, o, zero, zero, zero, pairs, L, scale, impl="fp32")[3], p @ x)}
+    if d == 32:   # the first-order kernels of the other head dims are 16-bit ones
+        got["o"] = (o, p @ x)
+        got["dv"] = (fhog.attention_backward(q, k, zero, zero, pairs, L, scale, False)[2], p.transpose(1, 2).contiguous() @ x)
+    for name, (a, want) in got.items():
+        e = normalised_max_error(a[sel], want)
+        assert e < unit + 2.0 ** -8, (name, e)
