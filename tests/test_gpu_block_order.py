@@ -1,5 +1,5 @@
 """GPU tier: the order in which workgroups take the tiles of a masked launch (decode_block), around the 32nd, 64th and 65th
-workgroup of an XCD: every tile of every slice is computed, exactly as when the slice is launched alone."""
+workgroup of an XCD: every tile of every slice is computed, exactly as in a launch of another number of slices."""
 import pytest
 import torch
 
@@ -29,9 +29,12 @@ def test_batched_launch_equals_its_slices(slices, tiles, d, causal):
         return (o, L, *first, *second)
 
     got = outputs(x)
+    # Copies of one slice, enough that both launches lie on the same side of every line at which the number of workgroups changes the
+    # order of sums: the highest is 256, up to which the statistics sweep of the split products puts four waves on the same rows.
+    copies = 256 // tiles + 8
+    assert min(copies, slices) * tiles >= 256
     for s in (0, slices // 2, slices - 1):
-        # as many copies of one slice as put four waves on its rows in the small launch too
-        alone = outputs({name: t[s:s + 1].expand(43, -1, -1).contiguous() for name, t in x.items()})
-        for a, b in zip(got, alone):
-            assert torch.equal(a[s], b[0]) and torch.equal(a[s], b[42])
+        other = outputs({name: t[s:s + 1].expand(copies, -1, -1).contiguous() for name, t in x.items()})
+        for a, b in zip(got, other):
+            assert torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1])
     assert all(torch.isfinite(t.float()).all() for t in got)
