@@ -8,6 +8,7 @@
 // torch's own two calls of autograd.grad. On fresh tensors, where the Python nodes also hand the interpreter lock back and forth
 // between the caller's and autograd's threads, that program went from 393 to 149 us on 2 x 256 bf16 rows.
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -262,6 +263,8 @@ struct Attention : torch::autograd::Function<Attention> {
 
 // What attention() takes here: what ::forward takes, checked before a node of the graph exists
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, int64_t causal, int64_t window, int64_t schedule) {
+  // torch.jit.trace records a Python node as a call of it; of a native one it would record the allocations and miss the launches
+  if (at::tracer::impl::is_dispatch_enabled()) return std::nullopt;
   for (const Tensor* t : {&q, &k, &v}) {
     const int64_t dim = t->dim();
     if (!t->is_cuda() || t->device() != q.device() || t->scalar_type() != q.scalar_type() || (dim != 3 && dim != 4) || dim != q.dim()) return std::nullopt;

@@ -110,3 +110,19 @@ def test_use_on_another_stream_and_thread():
     t.join()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("requires_grad", [False, True])
+def test_traced_module_computes_on_new_inputs(requires_grad):
+    """torch.jit.trace: the traced module computes, and differentiates where its inputs ask for it, like the function itself."""
+    import fhog
+    g = torch.Generator().manual_seed(74)
+    q, k, v = (torch.randn(2, 70, 64, generator=g).cuda().requires_grad_(requires_grad) for _ in range(3))
+    traced = torch.jit.trace(lambda a, b, c: fhog.attention(a, b, c, True), (q, k, v), check_trace=False)
+    new = [torch.randn(2, 70, 64, generator=g).cuda().requires_grad_(requires_grad) for _ in range(3)]
+    got, want = traced(*new), fhog.attention(*new, True)
+    assert torch.equal(got, want) and got.requires_grad == requires_grad
+    if requires_grad:
+        w = torch.randn(2, 70, 64, generator=g).cuda()
+        for a, b in zip(torch.autograd.grad(got, new, w), torch.autograd.grad(want, new, w)):
+            assert torch.equal(a, b)
