@@ -267,6 +267,8 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   if (at::tracer::impl::is_dispatch_enabled()) return std::nullopt;
   for (const Tensor* t : {&q, &k, &v}) {
     const int64_t dim = t->dim();
+    // tensors that dispatch to Python (fake ones among them) have no memory to launch on
+    if (t->unsafeGetTensorImpl()->is_python_dispatch()) return std::nullopt;
     if (!t->is_cuda() || t->device() != q.device() || t->scalar_type() != q.scalar_type() || (dim != 3 && dim != 4) || dim != q.dim()) return std::nullopt;
     for (int64_t i = 0; i < dim; i++)
       if (i != dim - 2 && t->size(i) != q.size(i)) return std::nullopt;

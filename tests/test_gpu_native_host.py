@@ -126,3 +126,18 @@ def test_traced_module_computes_on_new_inputs(requires_grad):
         w = torch.randn(2, 70, 64, generator=g).cuda()
         for a, b in zip(torch.autograd.grad(got, new, w), torch.autograd.grad(want, new, w)):
             assert torch.equal(a, b)
+
+
+def test_fake_tensors_propagate_shapes():
+    """Under FakeTensorMode there is no memory to launch on: the torch composition stands in, with the right shapes and types, first
+    derivatives included."""
+    import fhog
+    from fhog.attention import TorchCompositionWarning
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    q, k, v = (torch.randn(2, n, 64, device="cuda", dtype=torch.bfloat16) for n in (70, 90, 90))
+    with FakeTensorMode() as mode, pytest.warns(TorchCompositionWarning):
+        leaves = [mode.from_tensor(t).requires_grad_(True) for t in (q, k, v)]
+        out = fhog.attention(*leaves)
+        grads = torch.autograd.grad(out.float().sum(), leaves)
+    for a, b in zip((out, *grads), (q, q, k, v)):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.device == b.device
