@@ -102,6 +102,12 @@ Tensor packed(const Tensor& t) {
   return layout_of(c).direct ? c : c.clone(at::MemoryFormat::Contiguous);
 }
 
+// What a saved-tensor hook gave back may lie anywhere; where it lies as it was saved nothing is copied.
+Tensor unpacked(const Tensor& t) { return layout_of(t).direct ? t : packed(t); }
+Tensor unpacked_lse(const Tensor& L) {
+  return reinterpret_cast<uintptr_t>(L.data_ptr()) % 16 == 0 ? L : L.clone(at::MemoryFormat::Contiguous);
+}
+
 Tensor as_lse(const Tensor& L) { return L.scalar_type() == at::kFloat && L.is_contiguous() ? L : L.to(at::kFloat).contiguous(); }
 Tensor workspace(int64_t bytes, const Tensor& like) { return at::empty({(bytes + 3) / 4}, like.options().dtype(at::kFloat)); }
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -209,7 +215,7 @@ struct FirstBackward : torch::autograd::Function<FirstBackward> {
   }
   static std::tuple<Tensor, Tensor, Tensor> backward_(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& grad,
                                                       const Tensor& L, int64_t causal, int64_t window) {
-    const auto r = ::backward(q, k, v, o, grad, L, scale_of(q), Mask{(int32_t)causal, window}, false);
+    const auto r = ::backward(unpacked(q), unpacked(k), unpacked(v), unpacked(o), grad, unpacked_lse(L), scale_of(q), Mask{(int32_t)causal, window}, false);
     TORCH_CHECK(r, "fhog: first-order backward: ", fhog_last_error());
     return *r;
   }
@@ -223,8 +229,8 @@ struct FirstBackward : torch::autograd::Function<FirstBackward> {
     {
       const at::NoGradGuard no_grad;
       const auto dir = [&](size_t i) { return g[i].defined() ? packed(g[i]) : at::zeros_like(s[i]); };
-      const auto r = double_backward(s[0], s[1], s[2], s[3], s[4], dir(0), dir(1), dir(2), s[5], scale_of(s[0]), Mask{(int32_t)arg[0], arg[1]},
-                                     FHOG_IMPL_AUTO, (int)arg[2], true);
+      const auto r = double_backward(unpacked(s[0]), unpacked(s[1]), unpacked(s[2]), unpacked(s[3]), unpacked(s[4]), dir(0), dir(1), dir(2),
+                                     unpacked_lse(s[5]), scale_of(s[0]), Mask{(int32_t)arg[0], arg[1]}, FHOG_IMPL_AUTO, (int)arg[2], true);
       TORCH_CHECK(r, "fhog: double-backward: ", fhog_last_error());
       // O and L are caches of (q, k, v): the four results are already total derivatives
       out[0] = std::get<0>(*r), out[1] = std::get<1>(*r), out[2] = std::get<2>(*r), out[4] = std::get<3>(*r);
