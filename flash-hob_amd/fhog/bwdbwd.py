@@ -59,6 +59,9 @@ def workspace_floats(batch: int, n_q: int) -> int:
     return _lib.lib().fhog_bwdbwd_workspace_bytes(batch, n_q) // 4
 
 
+_MAX_WINDOW = 2 ** 31 - 1   # the C ABI's first-order window; rows number at most 2^24, so a longer one hides nothing
+
+
 def mask_code(causal, window, n_q: int, n_k: int):
     """(FHOG_MASK_* code, window) of the C ABI for the Python-level mask arguments.
 
@@ -83,7 +86,7 @@ def mask_code(causal, window, n_q: int, n_k: int):
         return code, 0
     if int(window) < 1:
         raise ValueError(f"window must be >= 1, got {window}")
-    return code, int(window)
+    return code, min(int(window), _MAX_WINDOW)
 
 
 _MASK_CODES = {None: _lib.MASK_NONE, False: _lib.MASK_NONE, True: _lib.MASK_TOP_LEFT, "bottom_right": _lib.MASK_BOTTOM_RIGHT}
@@ -92,7 +95,7 @@ _MASK_CODES = {None: _lib.MASK_NONE, False: _lib.MASK_NONE, True: _lib.MASK_TOP_
 def native_mask(causal, window):
     """The mask arguments for the native host side, which declines what it does not know (-1)."""
     code = _MASK_CODES.get(causal, -1) if causal is None or isinstance(causal, (bool, int, str)) else -1
-    return code, 0 if window is None else int(window) if int(window) >= 1 else -1
+    return code, 0 if window is None else min(int(window), _MAX_WINDOW) if int(window) >= 1 else -1
 
 
 def _workspace(args: "_lib.BwdBwdArgs", device, split: bool) -> torch.Tensor:

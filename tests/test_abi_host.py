@@ -261,6 +261,16 @@ def test_python_wrapper_errors():
         fhog.produce_L(q, t(2, 128, 64), is_causal=True)
 
 
+@pytest.mark.parametrize("window", [2 ** 31, 2 ** 32 + 5, 2 ** 63, 2 ** 70])
+def test_windows_beyond_32_bits_hide_nothing(window):
+    """Such a window is longer than any tensor: it is handed on as the longest one that fits the arguments, to the native host side
+    and to the Python wrappers alike."""
+    from fhog.bwdbwd import mask_code, native_mask
+    for n_k, causal in ((8, True), (9, "bottom_right")):
+        code, w = mask_code(causal, window, 8, n_k)
+        assert w == 2 ** 31 - 1 and (code, w) == native_mask(causal, window)
+
+
 def test_product_does_not_import_oracle():
     """The shipped package must not reach into oracle/ (it is the checker, not the product)."""
     for f in (ROOT / "flash-hob_amd").rglob("*.py"):
