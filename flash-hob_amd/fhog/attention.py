@@ -194,7 +194,7 @@ def attention_backward(q, k, v, o, do, L, scale: float, causal, *, window: Optio
                        use_hip: Optional[bool] = None):
     """First-order backward (dQ, dK, dV); the arithmetic of ``fhog/triton_flash.py:201-220`` without the
     (batch, N_Q, N_K) tensors. ``use_hip`` as in :func:`attention_forward`."""
-    if use_hip is not False and q.is_cuda:
+    if use_hip is not False and q.is_cuda and q.dim() == 3:
         res = _lib.torch_ext().backward(q, k, v, o, do, L, float(scale), *native_mask(causal, window))
         if res is not None:
             return res

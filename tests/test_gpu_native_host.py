@@ -165,3 +165,10 @@ def test_saved_tensors_that_come_back_elsewhere(layout):
         got = chain()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_attention_backward_takes_three_dimensions_only():
+    import fhog
+    x, L = torch.zeros(1, 2, 40, 64, device="cuda"), torch.zeros(1, 2, 40, device="cuda")
+    with pytest.raises(ValueError):
+        fhog.attention_backward(x, x, x, x, x, L, 0.125, False)
