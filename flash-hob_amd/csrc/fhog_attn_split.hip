@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
   constexpr bool KSIDE = MODE == MODE_BWD_K;
   constexpr int NR = MODE == MODE_FWD ? 1 : 2;             // stationary tensors: Q | Q, dO | K, V
   constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
-  using Stage = Stager<T, D, 2, true>;                     // streamed tensors: K, V | Q, dO
+  using Stage = Stager<T, D, 2, true, 0>;                     // streamed tensors: K, V | Q, dO
   constexpr int TENSOR = Stage::PLANES * Stage::TILE;
   constexpr int STAT = KSIDE ? 2 * TS * 4 : 0;             // L log2(e), -d of the 32 staged queries
   constexpr int STAGE = Stage::BYTES + STAT;
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
 template <typename T, int D, int MODE, int WS>
 constexpr int lds_bytes() {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
-  constexpr int stages = (WS == 1 ? 2 : WS) * (Stager<T, D, 2, true>::BYTES + (KSIDE ? 2 * TS * 4 : 0));
+  constexpr int stages = (WS == 1 ? 2 : WS) * (Stager<T, D, 2, true, 0>::BYTES + (KSIDE ? 2 * TS * 4 : 0));
   constexpr int xch = WS > 1 ? (4 / WS) * (WS - 1) * ((KSIDE ? 2 : 1) * D / 32 * 16 + 2) * 64 * 4 : 0;
   return stages > xch ? stages : xch;
 }

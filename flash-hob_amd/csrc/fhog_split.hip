@@ -35,7 +35,8 @@ namespace {
 template <typename T, int D>
 constexpr bool is_raw = sizeof(T) == 4 && D == 128;
 
-// Stationary operand of a lane: its row's elements 16 kk + 8 h .. + 7 of every k-step, as terms or as they lie in memory.
+// Stationary operand of a lane: its row's elements 16 kk + 8 h .. + 7 of every k-step, as terms or as they lie in memory. Split
+// without ANY: where one of them is not finite, the outputs of its row are not either.
 template <typename T, int D>
 struct Resident {
   static constexpr int KK = D / 16, NF = Terms<T>::NF;
@@ -45,7 +46,7 @@ struct Resident {
     for (int kk = 0; kk < KK; kk++) {
       const Chunk<T> c = load_chunk<T>(row + 16 * kk + 8 * h);
       if constexpr (is_raw<T, D>) r[kk] = c;
-      else chunk_terms<T, true, NF>(c, r[kk]);
+      else chunk_terms<T, true, false>(c, r[kk]);
     }
   }
   __device__ __forceinline__ void terms(int kk, bf16x8_t (&out)[NF]) const {
@@ -53,7 +54,7 @@ struct Resident {
       Chunk<T> c = r[kk];
       // splitting is to happen here, tile after tile: hoisted out of the sweep, the terms would be spilled
       asm volatile("" : "+v"(c.v[0]), "+v"(c.v[1]));
-      chunk_terms<T, true, NF>(c, out);
+      chunk_terms<T, true, false>(c, out);
     } else {
 #pragma unroll
       for (int q = 0; q < NF; q++) out[q] = r[kk][q];
@@ -81,7 +82,9 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4);      // streamed tensors: K, ddK, V, ddV | Q, ddQ, dO
   constexpr int NR = PASS == 1 ? 2 : (KSIDE ? 4 : 3);      // stationary tensors: Q, ddQ, dO | K, ddK, V, ddV
   constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
-  using Stage = Stager<T, D, NT, !STATS>;
+  // An infinity in K, ddK, Q or ddQ makes a NaN of dd and, with it, of whole rows; one in V, ddV or dO leaves other columns of
+  // ddO or dV2 as they are. The statistics sweeps have sums over rows only.
+  using Stage = Stager<T, D, NT, !STATS, STATS ? NT : 2>;
   constexpr int TENSOR = Stage::PLANES * Stage::TILE;
   constexpr int STAT = KSIDE ? 4 * TS * 4 : 0;             // L log2(e), -d, dd, -(dd d + b) of the 32 staged queries
   constexpr int STAGE = Stage::BYTES + STAT;
@@ -236,7 +239,7 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
         if constexpr (LAST_IN_LDS) {
           Chunk<T> c;
           c.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]), c.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
-          chunk_terms<T, true, NF>(c, out);
+          chunk_terms<T, true, false>(c, out);
         } else {
           res[NREG - 1].terms(kk, out);
         }
@@ -244,7 +247,7 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
       if constexpr (KSIDE) res[2].terms(kk, r2), last_terms(r3);
       else if constexpr (PASS != 1) last_terms(r2);
       const auto streamed = [&](int x) {
-        if constexpr (DIRECT) chunk_terms<T, true, NF>(ahead[kk & 1][x], a);
+        if constexpr (DIRECT) chunk_terms<T, true, false>(ahead[kk & 1][x], a);
         else read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a);
       };
       streamed(0);
@@ -403,7 +406,7 @@ template <typename T, int D, int PASS, int WS>
 constexpr int lds_bytes() {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4), nw = 4 / WS;
-  constexpr int stage = Stager<T, D, NT, !STATS>::BYTES + (KSIDE ? 4 * TS * 4 : 0);
+  constexpr int stage = Stager<T, D, NT, !STATS, 0>::BYTES + (KSIDE ? 4 * TS * 4 : 0);
   constexpr int stages = is_direct<PASS, WS> ? 0 : n_buffers<T, D, WS>(stage) * WS * stage + (is_raw<T, D> && !STATS ? 4 * TS * D * 4 : 0);
   constexpr int xch = WS > 1 ? nw * (WS - 1) * (STATS ? 5 : 2 * D / 32 * 16) * 64 * 4 : 0;
   return stages > xch ? stages : xch;

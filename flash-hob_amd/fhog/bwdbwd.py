@@ -157,7 +157,7 @@ def flash_bwdbwd(Q, K, V, O, dO, ddQ, ddK, ddV, L, scale, *, causal=False, windo
             skip the tiles outside the band.
         impl: None/"auto" | "fp32" | "bf16" - kernel family; "auto" takes the 16-bit MFMA kernels ("bf16": products
             in the tensor type, bf16 or fp16) for 16-bit tensors whose shape they support, the split-product kernels
-            otherwise.
+            otherwise (accurate to fp32 for inputs below 3.396e38; an output that should be infinite may be NaN there).
         fused_stats: the same as ``schedule="fused_stats"``.
         schedule: None / "fused_stats" (``dd`` and ``b`` from one sweep instead of the reference's two,
             ``fhog/triton_bwdbwd.py:185-251``: 22 recomputed products; ``b`` differs from the four sweeps' value only by

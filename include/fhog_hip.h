@@ -75,7 +75,9 @@ extern "C" {
 /* kernel families (fhog_bwdbwd_args.impl) */
 #define FHOG_IMPL_AUTO 0   /* 16-bit MFMA kernels for bf16/fp16 tensors when the shape allows, else the split-product kernels */
 #define FHOG_IMPL_FP32 1   /* force the split-product kernels (any dtype): contractions of fp32 accuracy, put together from 16-bit
-                               MFMA products of bf16 terms (three of an fp32 number, exactly); everything else in fp32 */
+                               MFMA products of bf16 terms (three of an fp32 number, exactly); everything else in fp32.
+                               Finite results need finite inputs below 3.396e38 (bf16's largest number). An infinity or NaN in V,
+                               ddV or dO stays in its column of ddO or dV2; an output that should be infinite may be NaN */
 #define FHOG_IMPL_BF16 2   /* force the 16-bit MFMA kernels (bf16 or fp16 tensors, products in the tensor type);
                               error if the shape/dtype does not fit */
 

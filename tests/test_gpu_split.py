@@ -127,3 +127,55 @@ def test_weights_beside_16_bit_tensors_are_fp32(batch, d, dtype):
     for name, (a, want) in got.items():
         e = normalised_max_error(a[sel], want)
         assert e < unit + 2.0 ** -8, (name, e)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 32)])
+@pytest.mark.parametrize("batch", [2, 70, 140])
+def test_numbers_that_bf16_cannot_hold(batch, dtype, d, value):
+    """One infinity, NaN or number beyond bf16's largest in V, dO or ddV changes its own column of O, dV and ddO alone: infinite with
+    its sign, the weighted sum where the number is finite (fp32 tensors; beside 16-bit ones the three terms of a weight may meet an
+    infinity with both signs, so not finite is all that is said). One in a row of K, where an infinite score hides the key or takes
+    the row, stays in the rows that it takes."""
+    import fhog
+    n, row, col = 190, 67, 5
+    if dtype != torch.float32 and value == 3.4e38:
+        pytest.skip("no such number in 16 bits")
+    g = torch.Generator().manual_seed(76)
+    q, k, v, do, ddv = (torch.randn(batch, n, d, generator=g).to(dtype).cuda() for _ in range(5))
+    zero = torch.zeros_like(q)
+    scale = d ** -0.5
+
+    def marked(t):
+        t = t.clone()
+        t[:, row, col] = value
+        return t
+
+    def others(t):
+        return torch.cat([t[..., :col], t[..., col + 1:]], -1)
+
+    o, L = fhog.attention_forward(q, k, v, scale, use_hip=True)
+    o1, L1 = fhog.attention_forward(q, k, marked(v), scale, use_hip=True)
+    p = torch.softmax(q.double().cpu() @ k.double().cpu().transpose(1, 2).contiguous() * scale, -1)
+    second = lambda x: fhog.flash_bwdbwd(q, k, zero, zero, zero, zero, zero, x, L, scale)[3]
+    dv = lambda x: fhog.attention_backward(q, k, zero, zero, x, L, scale, False, use_hip=True)[2]
+    assert torch.equal(L, L1)
+    for got, plain, weight in ((o1, o, p[:, :, row]), (second(marked(ddv)), second(ddv), p[:, :, row]),
+                               (dv(marked(do)), dv(do), p[:, row, :])):
+        assert torch.equal(others(got), others(plain))
+        x = got[..., col].double().cpu()
+        if dtype != torch.float32:
+            assert not torch.isfinite(x).any()
+        elif value == 3.4e38:   # the marked element decides the sum; fp32 roundings of the exponent and of L, 2^-22 of a weight each at scores below 16
+            assert (x / (weight * 3.4e38) - 1).abs().max() < 1e-5
+        elif value != value:
+            assert torch.isnan(x).all()
+        else:
+            assert (x == value).all()
+    # a score of -Inf hides its key, one of +Inf or NaN takes the row
+    if dtype == torch.float32 and abs(value) == float("inf"):
+        o2 = fhog.attention_forward(q, marked(k), v, scale, use_hip=True)[0]
+        hidden = q[..., col] * value < 0
+        keys = [j for j in range(n) if j != row]
+        want = fhog.attention_forward(q, k[:, keys].contiguous(), v[:, keys].contiguous(), scale, use_hip=True)[0]
+        assert normalised_max_error(o2[hidden], want[hidden]) < 1e-5 and torch.isnan(o2[~hidden]).all()
