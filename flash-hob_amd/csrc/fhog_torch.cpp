@@ -10,6 +10,7 @@
 #include <ATen/ATen.h>
 #include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -271,6 +272,8 @@ struct Attention : torch::autograd::Function<Attention> {
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, int64_t causal, int64_t window, int64_t schedule) {
   // torch.jit.trace records a Python node as a call of it; of a native one it would record the allocations and miss the launches
   if (at::tracer::impl::is_dispatch_enabled()) return std::nullopt;
+  // torch.func transforms: the Python nodes say that they have no rule for them
+  if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return std::nullopt;
   for (const Tensor* t : {&q, &k, &v}) {
     const int64_t dim = t->dim();
     // tensors that dispatch to Python (fake ones among them) have no memory to launch on

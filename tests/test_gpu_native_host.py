@@ -172,3 +172,18 @@ def test_attention_backward_takes_three_dimensions_only():
     x, L = torch.zeros(1, 2, 40, 64, device="cuda"), torch.zeros(1, 2, 40, device="cuda")
     with pytest.raises(ValueError):
         fhog.attention_backward(x, x, x, x, x, L, 0.125, False)
+
+
+def test_transforms_and_forward_mode_are_refused_by_name():
+    """torch.func transforms, around wrapped or plain tensors, and dual tensors: refused with the reason, not computed and not failing
+    on an address."""
+    import fhog
+    q, k, v = (torch.randn(2, 40, 64, device="cuda") for _ in range(3))
+    for f in (lambda: torch.func.grad(lambda a: fhog.attention(a, k, v).sum())(q),
+              lambda: torch.func.vmap(lambda a: fhog.attention(a, k, v))(q[None]),
+              lambda: torch.func.grad(lambda a: (fhog.attention(q, k, v) * a).sum())(q)):
+        with pytest.raises(RuntimeError, match="setup_context"):
+            f()
+    import torch.autograd.forward_ad as fwAD
+    with fwAD.dual_level(), pytest.raises(RuntimeError, match="(?i)forward AD|jvp"):
+        fhog.attention(fwAD.make_dual(q, torch.ones_like(q)), k, v)
