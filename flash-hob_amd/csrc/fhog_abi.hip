@@ -163,14 +163,13 @@ int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
   return s;
 }
 
-// Splits a pass runs with. Passes 3 and 4 at d = 128 keep one workgroup on a CU: what matters there is rounds of 256
+// Splits a pass runs with, of `most`. Passes 3 and 4 at d = 128 keep one workgroup on a CU: what matters there is rounds of 256
 // workgroups times the tiles of one, under the mask, and what the partial results cost. In steps of one tile (1.9 us): a
 // workgroup needs about 4 to start and to store, combining 2 plus its bytes at 5 TB/s (14.5 us for 66 MB, 8 for 33).
 // Where the work of the workgroups differs (causal) the longest one and the average load bound the launch.
 // bf16 16 x 1000 x 3001, window 700, us, as many splits as give 512 workgroups -> this rule: pass 3 with 4 -> 2 splits 49.2 + 14.5
 // (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
-int launch_split_of(const fhog_bwdbwd_args* a, const fhog::Params& p, int impl, int pass) {
-  const int most = granted_split(a, impl, pass);
+int split_up_to(int most, const fhog_bwdbwd_args* a, const fhog::Params& p, int pass) {
   if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
   const bool kside = pass == FHOG_PASS_DK_DV;
   const int64_t n_sta = kside ? a->n_k : a->n_q, n_str = kside ? a->n_q : a->n_k;
@@ -197,6 +196,10 @@ int launch_split_of(const fhog_bwdbwd_args* a, const fhog::Params& p, int impl, 
     if (s == 1 || cost < best_cost) best = s, best_cost = cost;
   }
   return best;
+}
+
+int launch_split_of(const fhog_bwdbwd_args* a, const fhog::Params& p, int impl, int pass) {
+  return split_up_to(granted_split(a, impl, pass), a, p, pass);
 }
 
 int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
@@ -394,9 +397,10 @@ size_t fhog_bwdbwd_workspace_bytes(int64_t batch, int64_t n_q) {
 size_t fhog_bwdbwd_workspace_hint(const fhog_bwdbwd_args* args) {
   if (validate(args) != FHOG_OK) return 0;
   const int impl = select_impl(args);
+  const fhog::Params p = to_params(args);
   size_t extra = 0;
   for (int pass = FHOG_PASS_DD; pass <= FHOG_PASS_DD_B; pass++) {
-    const int s = wanted_split(args, impl, pass);
+    const int s = split_up_to(wanted_split(args, impl, pass), args, p, pass);
     if (s > 1 && (size_t)s * split_bytes(args, pass) > extra) extra = (size_t)s * split_bytes(args, pass);
   }
   return extra ? stats_bytes(args) + extra : fhog_bwdbwd_workspace_bytes(args->batch, args->n_q);
@@ -441,7 +445,10 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (split_products && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 3;
   // Passes 6-8 have no split form: a launch too small to fill the GPU whose workspace lets the reference's passes split
   // their streamed side runs the nearest schedule that can (three sweeps -> fused statistics, ddO early -> four passes).
-  const bool small = granted_split(args, impl, FHOG_PASS_DQ_DDO) > 1;
+  // Asked of pass 3, by the splits that it runs with: under a window it may fill the GPU unsplit although the workspace has room.
+  // us, substitute -> schedule asked for, d = 128, three sweeps | ddO early: bf16 causal 2 x 16000, window 300 112 -> 92 | 141 -> 125;
+  // 32 x 1024, window 128 73.0 -> 64.5 | 91.8 -> 83.8; bottom-right 16 x 1000 x 3001, window 40 65.6 -> 59.5 | 81.2 -> 76.4.
+  const bool small = launch_split_of(args, p, impl, FHOG_PASS_DQ_DDO) > 1;
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && small) order = fused, n_pass = 3;
   if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !small) order = ddo_early, n_pass = 4;
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !small) order = three, n_pass = 3;

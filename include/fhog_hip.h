@@ -102,7 +102,7 @@ extern "C" {
                                        caller's 16-bit O: accurate as long as dd_i does not dominate ddS_ij - dd_i.
                                        Schedules 2 and 3 exist in the 16-bit MFMA family; the split-product family runs
                                        schedule 1 for them. Passes 6, 7 and 8 have no split form: a launch too
-                                       small to fill the GPU whose workspace allows a split (ws_bytes) runs the four
+                                       small to fill the GPU, whose pass 3 would run split (ws_bytes allowing), runs the four
                                        passes (schedule 2) or the fused statistics sweep and passes 3, 4 (schedule 3) */
 
 /* Launch choices (the counterpart of the reference's autotune list, fhog/triton_bwdbwd.py:12-36) are fixed functions of

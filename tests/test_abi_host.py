@@ -174,6 +174,19 @@ def test_workspace_hint(L):
     assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == 0   # invalid arguments
 
 
+def test_workspace_hint_counts_the_splits_that_run(L):
+    """d = 128, 4 x 4096 rows under a window of 128 keys: 128 workgroups, of which the statistics sweeps run four each; passes 3 and 4
+    run one, of nine tiles at most, and need no room."""
+    a = good_args()
+    a.batch, a.n_q, a.n_k, a.d, a.causal, a.window = 4, 4096, 4096, 128, 1, 128
+    a.stride_qn = a.stride_kn = 128
+    a.stride_qb = a.stride_kb = 4096 * 128
+    row = 4 * 4096 * 4
+    assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == 3 * row + 4 * 3 * row
+    a.causal = a.window = 0                   # all keys visible: passes 3 and 4 split as far as there are CUs
+    assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == 3 * row + 2 * 2 * 128 * row
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_workspace_hint_stays_below_its_stated_bound(L, d):
     """Whatever batch and N: the partial results of split launches take fewer than 2 * 131072 * d floats (a pass stops

@@ -26,3 +26,21 @@ def test_split_by_rounds(shape, dtype):
     unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     for name, a, b in zip(NAMES, split, whole):
         assert normalised_max_error(a, b.float()) <= unit, name
+
+
+@pytest.mark.parametrize("schedule", ["three_sweep", "ddo_early"])
+@pytest.mark.parametrize("shape", [(4, 4096, 4096, True, 128), (16, 1000, 3001, "bottom_right", 40)])
+def test_schedules_run_as_asked_where_pass_3_does_not_split(shape, schedule):
+    """Few enough workgroups that passes may split, and a mask under which pass 3 keeps one workgroup per tile: the schedule asked for
+    runs, with the bits of the call that has no workspace for splits."""
+    batch, n_q, n_k, causal, window = shape
+    scale = 128 ** -0.5
+    x = with_caches(make_case(batch, n_q, n_k, 128, torch.bfloat16, seed=77, grad_std=0.1), scale, causal, window)
+    got, want = (run_fhog(x, scale, causal, window=window, schedule=schedule, split=s) for s in (True, False))
+    other = run_fhog(x, scale, causal, window=window, schedule="fused_stats" if schedule == "three_sweep" else "four_pass")
+    assert any(not torch.equal(a, b) for a, b in zip(got, other))
+    if schedule == "three_sweep":   # its sweeps have no split form
+        assert bool(torch.equal(got[0], want[0])) and bool(torch.equal(got[3], want[3]))
+    # the sweep for dd of the other one, and pass 4, may have split: sums in another order, one unit of the type
+    for name, a, b in zip(NAMES, got, want):
+        assert normalised_max_error(a, b.float()) <= 2.0 ** -8, name
