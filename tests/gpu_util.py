@@ -6,7 +6,7 @@ import torch
 from oracle.bwdbwd_oracle import autograd_double_backward, closed_form, normalised_max_error  # noqa: F401
 
 NAMES = ("dq2", "dk2", "dv2", "ddo")
-TOL = {torch.float32: 1e-4, torch.bfloat16: 2e-2}   # north-star gates: normalised max error
+TOL = {torch.float32: 1e-4, torch.bfloat16: 2e-2}   # gates: normalised max error
 
 
 def require_gpu():

@@ -78,7 +78,7 @@ def good_attn_args():
     (lambda a: setattr(a, "dO", 0), 0, 0, ""),            # forward does not look at the backward-only pointers
     (lambda a: setattr(a, "dO", 0), 1, -1, "dO"),
     (lambda a: setattr(a, "lse", 0), 0, -1, "lse"),
-    (lambda a: setattr(a, "dtype", 1), 0, 0, ""),             # fp32 tensors: the fp32-MFMA first-order kernels
+    (lambda a: setattr(a, "dtype", 1), 0, 0, ""),             # fp32 tensors: the split-product first-order kernels
     (lambda a: setattr(a, "dtype", 5), 0, -3, "dtype"),
     (lambda a: (setattr(a, "dtype", 1), setattr(a, "stride_kn", 68), setattr(a, "stride_kb", 512 * 68)), 1, 0, ""),   # 16 bytes = 4 floats
     (lambda a: (setattr(a, "dtype", 1), setattr(a, "scale", -0.125)), 0, 0, ""),   # any sign of the scale there
@@ -118,7 +118,7 @@ def test_validate_accepts_good(L):
     assert L.fhog_select_impl(ctypes.byref(a)) in (1, 2)
     a.dtype = 1
     a.stride_qn = a.stride_kn = 64
-    assert L.fhog_select_impl(ctypes.byref(a)) == 1  # fp32 tensors always take the fp32-MFMA family
+    assert L.fhog_select_impl(ctypes.byref(a)) == 1  # fp32 tensors always take the split-product family
 
 
 @pytest.mark.parametrize("mutate, code, word", [
@@ -168,7 +168,7 @@ def test_workspace_hint(L):
     a.stride_qb, a.stride_kb = 256 * 64, 512 * 64
     assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == L.fhog_bwdbwd_workspace_bytes(4096, 256)
     a = good_args()
-    a.dtype = 1                               # fp32 tensors: the fp32-MFMA family does not split
+    a.dtype = 1                               # fp32 tensors: the split-product family does not split
     assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == minimum
     a.d = 96
     assert L.fhog_bwdbwd_workspace_hint(ctypes.byref(a)) == 0   # invalid arguments

@@ -131,7 +131,7 @@ def test_strided_rows_and_4d_input():
 @pytest.mark.parametrize("case", [(torch.float32, 2, 256, 256, 64), (torch.float32, 3, 100, 177, 128), (torch.float32, 2, 33, 129, 32),
                                   (torch.bfloat16, 2, 200, 200, 32), (torch.float16, 1, 300, 300, 32), (torch.float32, 1, 1, 1, 64)])
 def test_fp32_mfma_first_order_kernels(case, causal):
-    """fp32 tensors (the producer of O and L for the first benchmark configuration) and d = 32 run on the fp32-MFMA
+    """fp32 tensors (the producer of O and L for the first benchmark configuration) and d = 32 run on the split-product
     first-order kernels: O, L, dQ, dK, dV against the fp64 oracle, at the fp32 gate for fp32 tensors."""
     import fhog
     from fhog.attention import attention_backward
@@ -157,7 +157,7 @@ def test_fp32_mfma_first_order_kernels(case, causal):
 
 
 def test_fp32_kernels_take_a_negative_scale_and_16_bit_ones_fall_back():
-    """The fp32-MFMA forward scales the scores before it takes their maximum: any sign of the scale. The 16-bit forward
+    """The split-product forward scales the scores before it takes their maximum: any sign of the scale. The 16-bit forward
     needs a positive one: use_hip=True raises, the default warns and takes the torch composition."""
     import fhog
     y = make_case(2, 128, 160, 64, torch.float32, seed=24)

@@ -47,7 +47,7 @@ def test_reference_fixture_bf16(golden, impl):
 
 
 def test_reference_fixture_fp32_tensors(golden):
-    """Same tensors kept in fp32 through the fp32-MFMA family, against the fp64 closed form."""
+    """Same tensors kept in fp32 through the split-product family, against the fp64 closed form."""
     g = {k: torch.tensor(v) for k, v in golden.items()}
     x = {n: g[k][None].cuda() for n, k in (("Q", "q"), ("K", "k"), ("V", "v"), ("dO", "do"), ("ddQ", "ddq"),
                                             ("ddK", "ddk"), ("ddV", "ddv"))}
@@ -62,7 +62,7 @@ def test_reference_fixture_fp32_tensors(golden):
 # ---------------------------------------------------------------- fp32 family, small and ragged
 @pytest.mark.parametrize("seed", [0, 1, 2])
 def test_cfg0_fp32_noncausal(seed):
-    """configs[0]: fp32 non-causal B=1 H=2 N=256 d=64, all seven tensors N(0,1)."""
+    """fp32 non-causal B=1 H=2 N=256 d=64, all seven tensors N(0,1)."""
     x = make_case(2, 256, 256, 64, torch.float32, seed)
     scale = 64 ** -0.5
     x = with_caches(x, scale, False)
@@ -99,7 +99,7 @@ def test_fp32_family_ragged(shape, causal, dtype):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("shape", [(2, 256, 256, 64), (70, 128, 200, 32), (130, 128, 96, 64), (40, 300, 300, 64), (3, 100, 40, 64)])
 def test_fp32_family_launch_sizes(shape, causal):
-    """The fp32-MFMA kernels put one, two or four waves on the same 32 stationary rows depending on how many workgroups
+    """The split-product kernels put one, two or four waves on the same 32 stationary rows depending on how many workgroups
     the launch has (four, each taking every fourth streamed tile, for a problem as small as the first benchmark
     configuration): every regime against the fp64 closed form at the fp32 gate, row statistics included."""
     batch, n_q, n_k, d = shape
@@ -121,7 +121,7 @@ def test_fp32_family_launch_sizes(shape, causal):
                                   ("bottom_right", 1, 64, 96), ("bottom_right", 500, 31, 31), (True, 7, 256, 256)])
 def test_bottom_right_and_sliding_window_masks(mask, dtype):
     """The masks of the reference's specification (fhog/jax_refs/jax_impl.py:110-115), which its Triton path lacks:
-    bottom-right alignment for N_Q != N_K and a sliding window; fp32 tensors take the fp32-MFMA kernels, bf16 tensors
+    bottom-right alignment for N_Q != N_K and a sliding window; fp32 tensors take the split-product kernels, bf16 tensors
     the 16-bit ones."""
     causal, window, n_q, n_k = mask
     d = 64
@@ -147,7 +147,7 @@ def test_band_masks_agree_between_the_kernel_families(mask):
     x = make_case(3, n_q, n_k, d, torch.bfloat16, seed=19, grad_std=0.1)
     scale = d ** -0.5
     x = with_caches(x, scale, causal, window)
-    fast = run_fhog(x, scale, causal, window=window, impl="bf16", return_stats=True)
+    fast = run_fhog(x, scale, causal, window=window, impl="bf16", schedule="four_pass", return_stats=True)
     slow = run_fhog(x, scale, causal, window=window, impl="fp32", return_stats=True)
     fused = run_fhog(x, scale, causal, window=window, impl="bf16", fused_stats=True)
     # first against the oracle (fp64 closed form): outputs at the 2e-2 gate, row statistics of every family
@@ -206,17 +206,17 @@ def test_strided_and_4d_inputs():
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("shape", [(2, 128, 128, 64), (3, 256, 256, 128), (2, 128, 384, 64), (9, 384, 128, 128),
                                    (1, 512, 512, 128)])
-@pytest.mark.parametrize("fused_stats", [False, True])
-def test_bf16_family_small(shape, causal, fused_stats):
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
+def test_bf16_family_small(shape, causal, schedule):
     """bf16 MFMA kernels against the fp64 closed form, including the row vectors of passes 0..2, under the
-    four-pass schedule and the opt-in fused statistics sweep."""
+    four-pass schedule and the default one (fused statistics sweep)."""
     batch, n_q, n_k, d = shape
     if causal:
         n_k = n_q
     x = make_case(batch, n_q, n_k, d, torch.bfloat16, seed=5, grad_std=0.1)
     scale = d ** -0.5
     x = with_caches(x, scale, causal)
-    outs = run_fhog(x, scale, causal, impl="bf16", return_stats=True, fused_stats=fused_stats)
+    outs = run_fhog(x, scale, causal, impl="bf16", return_stats=True, schedule=schedule)
     ref = reference_fp64_cpu(x, scale, causal)
     e = errors(outs[:4], [ref[n] for n in NAMES])
     assert max(e.values()) < 2e-2, e
@@ -252,17 +252,17 @@ def test_bf16_fused_statistics_match_separate_passes(d, causal):
     assert normalised_max_error(fused[2], separate[2]) < 1e-3      # dd_i * sum_j P dP taken out of the sum
 
 
-@pytest.mark.parametrize("fused_stats", [False, True])
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(3, 333, 333, 128), (2, 100, 77, 64)])
-def test_bf16_chain_writes_row_sums_d_itself(shape, dtype, fused_stats):
+def test_bf16_chain_writes_row_sums_d_itself(shape, dtype, schedule):
     """The 16-bit chain launches no separate kernel for d = rowsum(O * dO) (fhog/triton_bwdbwd.py:580): its first
     statistics sweep writes it. Checked on a NaN-filled workspace against fp64 and against the stand-alone pass 0."""
     from fhog import BwdBwdPlan
     batch, n_q, n_k, d = shape
     x = with_caches(make_case(batch, n_q, n_k, d, dtype, seed=21, grad_std=0.1), d ** -0.5, False)
     plan = BwdBwdPlan(x["Q"], x["K"], x["V"], x["O"], x["dO"], x["ddQ"], x["ddK"], x["ddV"], x["L"], d ** -0.5,
-                      impl="bf16", fused_stats=fused_stats)
+                      impl="bf16", schedule=schedule)
     plan.ws.fill_(float("nan"))
     plan.run()
     torch.cuda.synchronize()
@@ -275,13 +275,13 @@ def test_bf16_chain_writes_row_sums_d_itself(shape, dtype, fused_stats):
     assert normalised_max_error(plan.ws.view(3, -1)[0], got) < 1e-5
 
 
-@pytest.mark.parametrize("fused_stats", [False, True])
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
 @pytest.mark.parametrize("case", [((1, 2048, 2048, 64), False, None, torch.bfloat16), ((1, 2048, 2048, 64), True, None, torch.float16),
                                   ((2, 1000, 1500, 64), "bottom_right", None, torch.bfloat16),
                                   ((1, 1536, 1536, 64), True, 300, torch.bfloat16), ((1, 130, 4100, 64), False, None, torch.bfloat16),
                                   ((1, 2048, 2048, 128), True, None, torch.bfloat16), ((2, 1000, 1500, 128), False, None, torch.float16),
                                   ((1, 1536, 1536, 128), "bottom_right", 700, torch.bfloat16)])
-def test_split_streamed_side_matches_the_unsplit_launch(case, fused_stats):
+def test_split_streamed_side_matches_the_unsplit_launch(case, schedule):
     """Few (batch*head) slices: with the workspace of fhog_bwdbwd_workspace_hint every pass splits its
     streamed side over several workgroups (fp32 partial results, added by a second kernel). Same gate against the
     fp64 oracle as the unsplit launch, row statistics equal up to summation order, outputs within a 16-bit rounding."""
@@ -293,7 +293,7 @@ def test_split_streamed_side_matches_the_unsplit_launch(case, fused_stats):
     scale = d ** -0.5
     x = with_caches(make_case(batch, n_q, n_k, d, dtype, seed=23, grad_std=0.1), scale, causal, window)
     plans = [BwdBwdPlan(x["Q"], x["K"], x["V"], x["O"], x["dO"], x["ddQ"], x["ddK"], x["ddV"], x["L"], scale, causal=causal,
-                        window=window, impl="bf16", fused_stats=fused_stats, split=sp) for sp in (True, False)]
+                        window=window, impl="bf16", schedule=schedule, split=sp) for sp in (True, False)]
     assert plans[0].args.ws_bytes > plans[1].args.ws_bytes == _lib.lib().fhog_bwdbwd_workspace_bytes(batch, n_q)
     res = []
     for plan in plans:
@@ -316,7 +316,7 @@ def test_split_streamed_side_matches_the_unsplit_launch(case, fused_stats):
 @pytest.mark.parametrize("seed", range(12))
 def test_split_launches_on_random_shapes_against_the_fp32_family(seed):
     """Random ragged lengths, masks, head dims and row strides in the range where launches split (few slices, at least
-    16 streamed tiles): the 16-bit kernels with partial results and the fp32-MFMA kernels against the oracle (fp32
+    16 streamed tiles): the 16-bit kernels with partial results and the split-product kernels against the oracle (fp32
     autograd for the outputs, fp64 closed form for the row statistics), then against each other."""
     import random
     rnd = random.Random(1000 + seed)
@@ -365,19 +365,19 @@ def test_split_launches_on_random_shapes_against_the_fp32_family(seed):
         assert normalised_max_error(a, b) < 1e-2, name
 
 
-@pytest.mark.parametrize("fused_stats", [False, True])
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
 @pytest.mark.parametrize("case", [(130, 1000, 1000, "causal", None, torch.bfloat16), (128, 1025, 700, "none", None, torch.float16),
                                   (171, 770, 1100, "bottom_right", 300, torch.bfloat16), (64, 2050, 520, "none", None, torch.bfloat16)])
-def test_many_slices_d128_statistics_in_256_row_workgroups(case, fused_stats):
+def test_many_slices_d128_statistics_in_256_row_workgroups(case, schedule):
     """At d = 128, launches of the b and dd+b sweeps with at least 512 workgroups of 256 query rows use those (8 waves)
     instead of 128-row workgroups: ragged lengths (last workgroup partly or, for its upper waves, wholly past the end),
-    masks and dtypes against the oracle on sampled slices and against the fp32-MFMA kernels, statistics included."""
+    masks and dtypes against the oracle on sampled slices and against the split-product kernels, statistics included."""
     batch, n_q, n_k, kind, window, dtype = case
     causal = {"none": False, "causal": True, "bottom_right": "bottom_right"}[kind]
     x = make_case(batch, n_q, n_k, 128, dtype, seed=77, grad_std=0.1)
     scale = 128 ** -0.5
     x = with_caches(x, scale, causal, window)
-    fast = run_fhog(x, scale, causal, window=window, impl="bf16", fused_stats=fused_stats, return_stats=True)
+    fast = run_fhog(x, scale, causal, window=window, impl="bf16", schedule=schedule, return_stats=True)
     slow = run_fhog(x, scale, causal, window=window, impl="fp32", return_stats=True)
     # the oracle on four sampled slices, the last one included (its last workgroup is the ragged one): fp32 autograd
     # for the outputs, fp64 closed form for the row statistics
@@ -400,7 +400,7 @@ def test_many_slices_d128_statistics_in_256_row_workgroups(case, fused_stats):
 def test_many_rows_d128_dd_sweep_with_64_queries_per_wave(case):
     """At d = 128 a dd sweep of at least 2048 workgroups of 256 query rows runs 64 queries per wave (two 32-query blocks,
     either of which a mask can leave out of a step): ragged ends, masks and dtypes; d and dd against the fp64 closed form
-    on sampled slices and against the fp32-MFMA kernels on all of them, outputs against fp32 autograd on sampled slices."""
+    on sampled slices and against the split-product kernels on all of them, outputs against fp32 autograd on sampled slices."""
     batch, n_q, n_k, kind, window, dtype = case
     causal = {"none": False, "causal": True, "bottom_right": "bottom_right"}[kind]
     x = make_case(batch, n_q, n_k, 128, dtype, seed=78, grad_std=0.1)
@@ -424,7 +424,7 @@ def test_many_rows_d128_dd_sweep_with_64_queries_per_wave(case):
 @pytest.mark.parametrize("shape", [(2, 256, 128, 64), (3, 384, 384, 128)])
 def test_fp16_tensors_both_families(shape, impl, causal):
     """fp16 tensors (the dtype of the reference's benchmark sweep, fhog/benchhhh.py:15-26) through the 16-bit MFMA
-    kernels (products in fp16) and through the fp32-MFMA kernels."""
+    kernels (products in fp16) and through the split-product kernels."""
     batch, n_q, n_k, d = shape
     if causal:
         n_k = n_q
@@ -470,11 +470,11 @@ def test_single_head_spreads_over_the_chip():
     assert max(e.values()) < 2e-2, e
 
 
-@pytest.mark.parametrize("fused_stats", [False, True])
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("shape", [(3, 100, 77, 64), (2, 33, 129, 128), (2, 333, 333, 128), (1, 1, 1, 64), (2, 31, 31, 128),
                                    (2, 129, 257, 64), (1, 1000, 1000, 128), (5, 160, 96, 64)])
-def test_bf16_family_ragged_lengths(shape, causal, fused_stats):
+def test_bf16_family_ragged_lengths(shape, causal, schedule):
     """Sequence lengths that are no multiple of the 128-row workgroup tile or of the 32-row stage: rows past the end
     are computed on copies of the last row and masked / not stored."""
     batch, n_q, n_k, d = shape
@@ -484,7 +484,7 @@ def test_bf16_family_ragged_lengths(shape, causal, fused_stats):
     scale = d ** -0.5
     x = with_caches(x, scale, causal)
     canary = 7.0
-    outs = run_fhog(x, scale, causal, impl="bf16", return_stats=True, fused_stats=fused_stats)
+    outs = run_fhog(x, scale, causal, impl="bf16", return_stats=True, schedule=schedule)
     ref = reference_fp64_cpu(x, scale, causal)
     e = errors(outs[:4], [ref[n] for n in NAMES])
     assert max(e.values()) < 2e-2, e
@@ -493,7 +493,7 @@ def test_bf16_family_ragged_lengths(shape, causal, fused_stats):
     # nothing is written past the end of a tensor: outputs are views into larger canary-filled buffers
     from fhog import BwdBwdPlan
     plan = BwdBwdPlan(x["Q"], x["K"], x["V"], x["O"], x["dO"], x["ddQ"], x["ddK"], x["ddV"], x["L"], scale, causal=causal,
-                      impl="bf16", fused_stats=fused_stats)
+                      impl="bf16", schedule=schedule)
     big = [torch.full((t.numel() + 4096,), canary, dtype=t.dtype, device=t.device) for t in plan.outs]
     ws_floats = (plan.args.ws_bytes + 3) // 4   # d | dd | b and, for a split launch, the partial results
     assert ws_floats <= plan.ws_all.numel()
@@ -519,16 +519,16 @@ def test_bf16_auto_dispatch():
     assert plan.impl == 2          # ragged lengths stay on the 16-bit kernels
     z = with_caches(make_case(2, 128, 128, 32, torch.bfloat16, seed=6), 32 ** -0.5, False)
     plan = BwdBwdPlan(z["Q"], z["K"], z["V"], z["O"], z["dO"], z["ddQ"], z["ddK"], z["ddV"], z["L"], 32 ** -0.5)
-    assert plan.impl == 1          # d = 32 is served by the fp32-MFMA kernels
+    assert plan.impl == 1          # d = 32 is served by the split-product kernels
 
 
-def _full_config(name, seed, heads=None, fused_stats=False):
+def _full_config(name, seed, heads=None, schedule=None):
     from fhog.workloads import WORKLOADS, make_inputs
     w = WORKLOADS[name]
     x = make_inputs(w, seed, device="cuda:0")
     x = {n: t.flatten(0, 1) for n, t in x.items()}
     x = with_caches(x, w.scale, w.causal)
-    outs = run_fhog(x, w.scale, w.causal, fused_stats=fused_stats)
+    outs = run_fhog(x, w.scale, w.causal, schedule=schedule)
     hs = list(range(w.batch)) if heads is None else heads
     worst = {}
     for h0 in range(0, len(hs), 4):
@@ -555,14 +555,15 @@ def test_cfg2_bf16_causal_4096_d128_headline(seed):
 
 @pytest.mark.parametrize("name,heads", [("cfg1_bf16_nc_2048_d64", None), ("cfg2_bf16_causal_4096_d128", None),
                                         ("cfg3_bf16_causal_16384_d128", [3, 30]), ("cfg4_bf16_cross_1024x8192_d64", None)])
-def test_full_size_configs_fused_statistics_schedule(name, heads):
-    """The opt-in schedule (dd and b from one sweep) on every 16-bit benchmark configuration at full size."""
-    w, e = _full_config(name, 2, heads=heads, fused_stats=True)
+@pytest.mark.parametrize("schedule", ["four_pass", "fused_stats"])
+def test_full_size_configs_schedules(name, heads, schedule):
+    """The four passes, and dd and b from one sweep (the default), on every 16-bit benchmark configuration at full size."""
+    w, e = _full_config(name, 2, heads=heads, schedule=schedule)
     assert max(e.values()) < 2e-2, e
 
 
 def test_cfg3_bf16_causal_16384_d128_sampled_heads():
-    """all 32 heads run through the HIP path; 4 sampled heads are compared with the fp32 reference."""
+    """All 32 heads run through the HIP path; 4 sampled heads are compared with the fp32 reference."""
     w, e = _full_config("cfg3_bf16_causal_16384_d128", 0, heads=[0, 9, 18, 27])
     assert max(e.values()) < 2e-2, e
 

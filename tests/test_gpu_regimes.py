@@ -3,7 +3,7 @@
 * the reference's own benchmark sweep far beyond its first point (fhog/benchhhh.py:15-27,93-108: one head, d = 64,
   fp16, non-causal, N up to 2097152), pinned at N = 131072 by quantities that stay affordable there: sampled query rows
   against the fp64 closed form (non-causal rows are independent), the zero column sums of the key-side outputs, and the
-  fp32-MFMA kernels on the same tensors;
+  split-product kernels on the same tensors;
 * `fhog.produce_L` (fhog/triton_flash.py:252-258) against the oracle's log-sum-exp;
 * the launch choices behind FHOG_TUNE, each forced in a child process (the variable is read once per process), on a shape
   the defaults would never give them.
@@ -67,10 +67,10 @@ def test_reference_sweep_regime_long_n_131072(dtype):
         print(f"long-N {dtype}: |sum_j {name}_j| = {col:.3e}, bound {bound:.3e}")
         assert col < bound, (name, col, bound)
 
-    # (3) the key-side outputs against the fp32-MFMA kernels on the same tensors (every product and intermediate in fp32)
+    # (3) the key-side outputs against the split-product kernels on the same tensors (every product and intermediate in fp32)
     _, dk2_32, dv2_32, _ = run_fhog(x, scale, False, impl="fp32")
     e_k = {"dk2": normalised_max_error(dk2, dk2_32.float()), "dv2": normalised_max_error(dv2, dv2_32.float())}
-    print(f"long-N {dtype}: against the fp32-MFMA family {e_k}")
+    print(f"long-N {dtype}: against the split-product family {e_k}")
     assert max(e_k.values()) < 2e-2, e_k
 
 

@@ -80,7 +80,7 @@ def test_schedules_on_a_launch_too_small_to_fill_the_gpu(schedule, split):
 
 @pytest.mark.parametrize("schedule", SCHEDULES)
 def test_schedules_against_the_default_one(schedule):
-    """Same tensors through the reference schedule and an opt-in one: dK2, dV2 and dQ2 depend on the row statistics
+    """Same tensors through the default schedule and an opt-in one: dK2, dV2 and dQ2 depend on the row statistics
     (dd, b) only, so they move by no more than the statistics' own rounding; ddO is rounded once in both."""
     x = with_caches(make_case(5, 640, 640, 128, torch.bfloat16, seed=54, grad_std=0.1), 128 ** -0.5, True)
     base = run_fhog(x, 128 ** -0.5, True, return_stats=True)
@@ -92,7 +92,7 @@ def test_schedules_against_the_default_one(schedule):
 
 
 @pytest.mark.parametrize("schedule", SCHEDULES)
-def test_schedules_fp32_tensors_run_the_reference_schedule(schedule):
+def test_schedules_fp32_tensors_run_the_default_schedule(schedule):
     x = with_caches(make_case(2, 96, 160, 64, torch.float32, seed=55), 0.125, False)
     base = run_fhog(x, 0.125, False)
     alt = run_fhog(x, 0.125, False, schedule=schedule)
