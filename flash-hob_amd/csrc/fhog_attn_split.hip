@@ -7,7 +7,8 @@
 // (queries; keys in the K-tiled backward) with their operands in registers as bf16 terms, the other side streams through
 // LDS in 32-row tiles that are split once per workgroup. A lane owns ONE stationary row: in the forward the running maximum,
 // the running sum and the rescaling factor of a query are per-lane scalars. Two terms per fp32 operand less than the
-// double-backward needs leave room for the terms of d = 128 (one wave per SIMD).
+// double-backward needs leave room for the terms of d = 128 (one wave per SIMD); only dK, dV on fp32 tensors there does not quite
+// fit and keeps 44 VGPRs of a lane in scratch memory under a mask, 76 with two waves on the same rows.
 // Small launches (WS = 2 or 4) put WS waves on the same 32 rows: each takes every WS-th streamed tile, and the partial
 // results are merged through LDS in a fixed order.
 #include <type_traits>

@@ -13,7 +13,9 @@
 //
 // What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
 // 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (34 MFMAs beside some 400
-// VALU instructions, half of them the split of P, dS, dS' and ddP).
+// VALU instructions, half of them the split of P, dS, dS' and ddP). Some do not quite fit the register file and keep VGPRs of a
+// lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 54 to 60, in pass 4 at d = 64 with
+// four waves on the same rows 18 to 21, at d = 32 under a mask in pass 3 6 and without one in pass 4 15; 16-bit tensors at d = 128 up to 89.
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same box):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 136     fp32 causal 64 x 1024, d = 32: 672 -> 296
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
@@ -429,6 +431,9 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 // A statistics sweep that stages nothing splits every tile into terms once per 32 rows instead of once per 128, but its workgroups
 // are a quarter of the size: worth it beyond 64 workgroups where the staged form leaves CUs to the heaviest tiles of a causal
 // triangle, or has one wave per row block. Pass 5, us, staged -> direct, at so many 128-row workgroups:
+// Left as it is: triangles of 160 to 255 workgroups on fp32 tensors at d <= 64, where 15 x 2048 would gain (d = 64: 185 -> 151) what
+// 60 x 500 would lose (the number of streamed tiles tells them apart), and windows and bottom-right masks beyond 128 (fp32
+// d <= 64: 64), which were not measured.
 //   triangle: fp32 d = 128 497 -> 130 (64), 502 -> 302 (240); bf16 d = 32 43.7 -> 24.7 (240), 60 x 500 14.0 -> 11.5 (240);
 //             fp32 d = 64 184 -> 82 (128), but 60 x 500 52.2 -> 60.4 (240)
 //   no mask:  fp32 d = 128 553 -> 435 (126); bf16 d = 32 43.0 -> 32.5 (126); fp32 d = 64 129 -> 137 (96)

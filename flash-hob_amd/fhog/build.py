@@ -27,8 +27,11 @@ HIPCC_FLAGS = [
     "-fno-gpu-rdc",
     # packed-fp32 VALU forms are kept out of every kernel of this library
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # registers spill to scratch memory only: a kernel whose accumulators take every AGPR and that spilled VGPRs to AGPRs as
-    # well was compiled wrongly (fp16 operands of the K-tiled split-product sweep at d = 128: NaN in dK2)
+    # registers spill to scratch memory only: this compiler (clang 22.0.0git, roc-7.2.0) loses registers that it spills to AGPRs
+    # out of a tuple that it reloads into AGPRs. In the sweep for dK2 and dV2 of fp16 tensors at d = 128 (split products, two waves
+    # on the same rows, band mask) v[8:11] goes to scratch (v8 to v10) and a189 (v11); a[64:67], an operand of the next MFMAs,
+    # comes back as three registers from scratch, a189 is never read and a67 still holds an accumulator: NaN in dK2.
+    # Of the other files only fhog_attn_split.hip has code that differs with the flag.
     "-mllvm", "-amdgpu-spill-vgpr-to-agpr=0",
     "-Wno-unused-command-line-argument",
 ] + os.environ.get("FHOG_EXTRA", "").split()   # extra hipcc flags for experiments
