@@ -16,7 +16,7 @@
 // VALU instructions, half of them the split of P, dS, dS' and ddP). Some do not quite fit the register file and keep VGPRs of a
 // lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 54 to 60, in pass 4 at d = 64 with
 // four waves on the same rows 18 to 21, at d = 32 under a mask in pass 3 6 and without one in pass 4 15; 16-bit tensors at d = 128 up to 89.
-// Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same box):
+// Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 136     fp32 causal 64 x 1024, d = 32: 672 -> 296
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
 //   fp32 causal 32 x 2048, d = 128: 3833 -> 2340

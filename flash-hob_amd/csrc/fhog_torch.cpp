@@ -4,7 +4,7 @@
 // the workspace afterwards (row statistics, single passes).
 //
 // Why native: on short sequences the GPU finishes before Python has prepared the next launch. Host time per call, the Python
-// wrappers -> here (same box): flash_bwdbwd 56 -> 14 us; attention() differentiated twice 208 -> 154 us, of which some 100 are
+// wrappers -> here (same machine): flash_bwdbwd 56 -> 14 us; attention() differentiated twice 208 -> 154 us, of which some 100 are
 // torch's own two calls of autograd.grad. On fresh tensors, where the Python nodes also hand the interpreter lock back and forth
 // between the caller's and autograd's threads, that program went from 393 to 149 us on 2 x 256 bf16 rows.
 #include <ATen/ATen.h>

@@ -69,6 +69,11 @@ def _hip_args(q, k, v, scale, causal, window=None) -> _lib.AttnArgs:
     """Arguments for the HIP first-order kernels; raises _NotCovered when they do not cover these tensors."""
     if not q.is_cuda:
         raise _NotCovered("the tensors are not on a ROCm device")
+    # the library sees addresses only: what it would read beyond a tensor, or in host memory, is refused here
+    if k.device != q.device or v.device != q.device:
+        raise _NotCovered(f"k and v are on {k.device} and {v.device}, expected {q.device} like q")
+    if k.shape[0] < q.shape[0] or k.shape[2] != q.shape[2] or v.shape != k.shape:
+        raise _NotCovered(f"k and v have shapes {tuple(k.shape)} and {tuple(v.shape)}: expected ({q.shape[0]}, N_K, {q.shape[2]}) for both")
     if q.dtype not in _HIP_DTYPES or not (k.dtype == v.dtype == q.dtype):
         raise _NotCovered(f"dtypes {q.dtype}, {k.dtype}, {v.dtype}: need one of bf16, fp16, fp32 for all tensors")
     a = _lib.AttnArgs()
@@ -112,6 +117,11 @@ def _attention_backward_hip(q, k, v, o, do, L, scale, causal, window=None):
         ts_k = [t.contiguous() for t in ts_k]
     (q, o, do), (k, v) = ts_q, ts_k
     a = _hip_args(q, k, v, scale, causal, window)
+    for name, t in (("o", o), ("do", do), ("L", L)):
+        if t.device != q.device:
+            raise _NotCovered(f"{name} is on {t.device}, expected {q.device} like q")
+    if o.shape != q.shape or do.shape != q.shape:
+        raise _NotCovered(f"o and do have shapes {tuple(o.shape)} and {tuple(do.shape)}, expected {tuple(q.shape)} like q")
     if o.dtype != q.dtype or do.dtype != q.dtype:
         raise _NotCovered(f"O and dO have dtypes {o.dtype}, {do.dtype}: need {q.dtype} like Q")
     L_ = _lib.lib()

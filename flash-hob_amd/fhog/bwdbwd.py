@@ -114,6 +114,16 @@ def _workspace(args: "_lib.BwdBwdArgs", device, split: bool) -> torch.Tensor:
 def _build_args(Q, K, V, O, dO, ddQ, ddK, ddV, L, scale, causal, impl, outs, ws, schedule=0,
                 window=None) -> _lib.BwdBwdArgs:
     """``ws``: a workspace tensor of the minimum size, or None when :func:`_workspace` fills it in afterwards."""
+    # the library sees addresses only: what it would read beyond a tensor, or in host memory, is refused here
+    for n, t, like in (("K", K, K), ("V", V, K), ("O", O, Q), ("dO", dO, Q), ("ddQ", ddQ, Q), ("ddK", ddK, K), ("ddV", ddV, K), ("L", L, L)):
+        if t.device != Q.device or not t.is_cuda:
+            raise ValueError(f"{n} is on {t.device}, expected {Q.device} like Q, on a ROCm device")
+        if n != "L" and t.dtype != Q.dtype:
+            raise TypeError(f"{n} has dtype {t.dtype}, expected {Q.dtype} like Q")
+        if t.shape != like.shape:
+            raise ValueError(f"{n} has shape {tuple(t.shape)}, expected {tuple(like.shape)}")
+    if K.shape[0] != Q.shape[0] or K.shape[2] != Q.shape[2]:
+        raise ValueError(f"K has shape {tuple(K.shape)}, expected ({Q.shape[0]}, N_K, {Q.shape[2]})")
     a = _lib.BwdBwdArgs()
     a.q, a.k, a.v, a.o, a.dO = Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dO.data_ptr()
     a.ddq, a.ddk, a.ddv = ddQ.data_ptr(), ddK.data_ptr(), ddV.data_ptr()

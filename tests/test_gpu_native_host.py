@@ -1,4 +1,6 @@
 """GPU tier: the native host side of the entry points against the Python wrappers around the same kernels."""
+import warnings
+
 import pytest
 import torch
 
@@ -187,3 +189,23 @@ def test_transforms_and_forward_mode_are_refused_by_name():
     import torch.autograd.forward_ad as fwAD
     with fwAD.dual_level(), pytest.raises(RuntimeError, match="(?i)forward AD|jvp"):
         fhog.attention(fwAD.make_dual(q, torch.ones_like(q)), k, v)
+
+
+def test_tensors_elsewhere_or_of_other_shapes_are_refused():
+    """Host memory beside device tensors, and tensors shorter than the others: errors of the wrappers (or of the torch composition that
+    the first-order ones hand such calls to), before any launch."""
+    import fhog
+    x, short, L = torch.zeros(2, 40, 64, device="cuda"), torch.zeros(2, 33, 64, device="cuda"), torch.zeros(2, 40, device="cuda")
+    host = x.cpu()
+    for f in (lambda: fhog.attention(x, host, x), lambda: fhog.attention(x, x, short), lambda: fhog.attention_forward(x, x, host),
+              lambda: fhog.attention_forward(x, x, short), lambda: fhog.attention_forward(x, x[:1], x[:1], use_hip=True),
+              lambda: fhog.attention_backward(x, x, x, host, x, L, 0.125, False), lambda: fhog.attention_backward(x, x, x, x, short, L, 0.125, False),
+              lambda: fhog.attention_backward(x, x, x, x, x, L.cpu(), 0.125, False),
+              lambda: fhog.flash_bwdbwd(x, x, x, x, x, x, x, x, L.cpu(), 0.125),
+              lambda: fhog.BwdBwdPlan(x, x, x, x, x, x, x, x, L.cpu(), 0.125), lambda: fhog.BwdBwdPlan(x, x, x, x, short, x, x, x, L, 0.125),
+              lambda: fhog.BwdBwdPlan(x, x, short, x, x, x, x, x, L, 0.125)):
+        with pytest.raises((ValueError, RuntimeError)), warnings.catch_warnings():
+            warnings.simplefilter("ignore")
+            f()
+    with pytest.raises(TypeError):
+        fhog.BwdBwdPlan(x, x, x, x, x, x.half(), x, x, L, 0.125)
