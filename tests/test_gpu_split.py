@@ -129,8 +129,9 @@ def test_weights_beside_16_bit_tensors_are_fp32(batch, d, dtype):
         assert e < unit + 2.0 ** -8, (name, e)
 
 
-@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38])
-@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 32)])
+@pytest.mark.parametrize("dtype,d,value", [(t, d, x) for x in (float("inf"), float("-inf"), float("nan"), 3.4e38)
+                                           for t, d in ((torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32),
+                                                        (torch.float16, 32)) if t == torch.float32 or x != 3.4e38])
 @pytest.mark.parametrize("batch", [2, 70, 140])
 def test_numbers_that_bf16_cannot_hold(batch, dtype, d, value):
     """One infinity, NaN or number beyond bf16's largest in V, dO or ddV changes its own column of O, dV and ddO alone: infinite with
@@ -139,8 +140,6 @@ def test_numbers_that_bf16_cannot_hold(batch, dtype, d, value):
     the row, stays in the rows that it takes."""
     import fhog
     n, row, col = 190, 67, 5
-    if dtype != torch.float32 and value == 3.4e38:
-        pytest.skip("no such number in 16 bits")
     g = torch.Generator().manual_seed(76)
     q, k, v, do, ddv = (torch.randn(batch, n, d, generator=g).to(dtype).cuda() for _ in range(5))
     zero = torch.zeros_like(q)
