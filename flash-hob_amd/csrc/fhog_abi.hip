@@ -227,6 +227,50 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
   return FHOG_OK;
 }
 
+// ---- small launches of the 16-bit kernels (fhog_small.hip) ------------------------------------------------------
+// Waves that a launch puts on the same 32 stationary rows: 4 or 2, or 0 for the kernels with four waves on 128 rows.
+// One workgroup fits a CU: 4 waves as long as that is one round of the 256 CUs, 2 as long as they give one or, where the other
+// kernels would leave CUs idle, two rounds. `groups` counts 128-row groups of all sides that share a launch, `tiles` the streamed
+// tiles of one. A triangle (or a window) is in favour of small workgroups, whose work evens out; the double-backward's other
+// kernels split long streams over workgroups (workspace) and win them back there.
+// us, other kernels -> 4 waves | 2 waves, square shapes, bf16:
+//   forward           d = 64: 64 x 256 9.2 -> 6.5 | 7.4; 8 x 2048 36.7 -> 19.5 | 25.2; causal 32 x 1000 23 -> 16.5 | 17.6
+//                     d = 128: 16 x 512 15.7 -> 9.5 | 13.2; 64 x 256 11.0 -> 13.5 | 10.4; 1 x 8192 163 -> 64 | 118
+//   first backward    d = 64: 8 x 256 19.0 -> 7.3 | 9.7; 32 x 256 19.4 -> 12.5 | 10.5; 16 x 1024 48 -> 42 | 37; 1 x 8192 303 -> 114 | 152
+//                     d = 128: 8 x 256 25 -> 12 | 18; causal 32 x 512 39 -> 41 | 35, no mask 38 -> 51 | 43
+//   double-backward   d = 64: 8 x 256 37.7 -> 15.0 | 19.1; 64 x 256 40 -> 42 | 31; 8 x 2048 134 -> 135 | 126; 1 x 8192 216 -> 240 | 288
+//                     d = 128: 8 x 256 52 -> 23 | 31; 16 x 512 71 -> 50 | 51; causal 32 x 512 81 -> 74 | 60; 16 x 1024 125 -> 146 | 131
+enum class Small { forward, backward, double_backward };
+int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int64_t d, int32_t causal, int64_t window) {
+  if (fhog::tuning().small >= 0) return fhog::tuning().small;
+  const int64_t g_q = (n_q + 127) / 128 * batch, g_k = (n_k + 127) / 128 * batch;
+  // from 256 groups of a side on the kernels with 128 rows fill the GPU
+  if (g_q >= 256 || (what != Small::forward && g_k >= 256)) return 0;
+  const int64_t off = causal == FHOG_MASK_BOTTOM_RIGHT ? n_k - n_q : 0;
+  const bool windowed = causal != FHOG_MASK_NONE && window > 0 && window < n_k;
+  const bool uneven = causal != FHOG_MASK_NONE && (windowed || 2 * off <= n_k);
+  const int64_t streamed = what == Small::forward || n_k > n_q ? n_k : n_q;
+  const int64_t tiles = ((windowed && window + 63 < streamed ? window + 63 : streamed) + 31) / 32;
+  if (what == Small::forward) {
+    if (g_q <= 64) return 4;
+    if (g_q <= 128) return d == 64 || (uneven && tiles >= 32) ? 4 : 2;
+    if (tiles < 32) return 0;
+    return d == 64 ? (uneven ? 4 : 2) : (uneven ? 2 : 0);
+  }
+  const int64_t groups = g_q + g_k;
+  if (what == Small::backward) {
+    if (groups <= 64) return 4;
+    if (groups <= 128) return tiles <= 8 ? 2 : 4;
+    if (groups <= 256) return d == 64 || uneven ? 2 : 0;
+    return d == 64 && uneven && tiles >= 32 ? 2 : 0;
+  }
+  if (groups <= 64) return tiles <= (d == 64 ? 128 : 64) ? 4 : 0;
+  if (groups <= 128) return tiles <= 8 ? 2 : tiles <= (d == 64 ? 128 : uneven ? 64 : 32) ? 4 : 0;
+  if (groups <= 256) return tiles <= (d == 64 || uneven ? 64 : 16) ? 2 : 0;
+  return d == 64 && uneven && tiles >= 16 && tiles <= 64 ? 2 : 0;
+}
+int small_waves(Small what, const fhog_attn_args* a) { return small_waves(what, a->batch, a->n_q, a->n_k, a->d, a->causal, a->window); }
+
 // bf16 / fp16 tensors with d in {64, 128} run on the 16-bit MFMA kernels, everything else (fp32 tensors, d = 32) on the
 // split-product ones
 bool attn_on_16bit_kernels(const fhog_attn_args* a) { return a->dtype != FHOG_DTYPE_FP32 && (a->d == 64 || a->d == 128); }
@@ -343,6 +387,10 @@ const Tuning& tuning() {
       else if (!strcmp(tok, "dd64")) flag(tok, val, &r.dd64);
       else if (!strcmp(tok, "stage64")) flag(tok, val, &r.stage64);
       else if (!strcmp(tok, "stage1")) flag(tok, val, &r.stage1);
+      else if (!strcmp(tok, "small")) {
+        if (!strcmp(val, "0") || !strcmp(val, "2") || !strcmp(val, "4")) r.small = val[0] - '0';
+        else fprintf(stderr, "libfhog_hip: FHOG_TUNE: small is '0', '2' or '4', not '%s'; ignored\n", val);
+      }
       else if (!strcmp(tok, "order")) {
         if (!strcmp(val, "tile")) r.order = 1;
         else if (!strcmp(val, "slice")) r.order = 0;
@@ -366,7 +414,9 @@ int fhog_attn_validate(const fhog_attn_args* args, int backward) { return valida
 int fhog_attn_fwd(const fhog_attn_args* args, void* hip_stream) {
   const int rc = validate_attn(args, 0);
   if (rc != FHOG_OK) return rc;
-  const hipError_t e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(to_attn_params(args), 0, (hipStream_t)hip_stream)
+  const int small = attn_on_16bit_kernels(args) ? small_waves(Small::forward, args) : 0;
+  const hipError_t e = small ? fhog::launch_small_attn(to_attn_params(args), false, small, (hipStream_t)hip_stream)
+                       : attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(to_attn_params(args), 0, (hipStream_t)hip_stream)
                                                    : fhog::launch_attn_split(to_attn_params(args), args->dtype, 0, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention forward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
   return FHOG_OK;
@@ -376,6 +426,11 @@ int fhog_attn_bwd(const fhog_attn_args* args, void* hip_stream) {
   const int rc = validate_attn(args, 1);
   if (rc != FHOG_OK) return rc;
   const fhog::AttnParams p = to_attn_params(args);
+  if (const int small = attn_on_16bit_kernels(args) ? small_waves(Small::backward, args) : 0) {
+    const hipError_t e = fhog::launch_small_attn(p, true, small, (hipStream_t)hip_stream);
+    if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention backward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
+    return FHOG_OK;
+  }
   hipError_t e = hipSuccess;   // the dQ kernel also writes the row sums d that the one for dK and dV reads
   for (int which = 1; which <= 2 && e == hipSuccess; which++)
     e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(p, which, (hipStream_t)hip_stream)
@@ -427,6 +482,17 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (rc != FHOG_OK) return rc;
   const fhog::Params p = to_params(args);
   const int impl = select_impl(args);
+  // Small launches: the default schedule in two launches. The schedules that take ddO out of the third sweep do the same as long as
+  // that is one round of the CUs (us, 2 x 86, d = 64: 41 -> 13), their own sweeps beyond.
+  int small = 0;
+  if (impl == FHOG_IMPL_BF16 && (args->schedule == FHOG_SCHEDULE_FUSED_STATS ||
+                                 (args->schedule != FHOG_SCHEDULE_FOUR_PASS && ((args->n_q + 127) / 128 + (args->n_k + 127) / 128) * args->batch <= 128)))
+    small = small_waves(Small::double_backward, args->batch, args->n_q, args->n_k, args->d, args->causal, args->window);
+  if (small) {
+    const hipError_t e = fhog::launch_small_bwdbwd(p, small, (hipStream_t)hip_stream);
+    if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "HIP error %d (%s)", (int)e, hipGetErrorString(e));
+    return FHOG_OK;
+  }
   // Pass sequences. The first statistics sweep writes d_i itself: no separate launch for it.
   // The schedules that take ddO out of the third sweep exist in the 16-bit family; the split-product family runs the
   // fused one for them.
@@ -448,10 +514,10 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   // Asked of pass 3, by the splits that it runs with: under a window it may fill the GPU unsplit although the workspace has room.
   // us, substitute -> schedule asked for, d = 128, three sweeps | ddO early: bf16 causal 2 x 16000, window 300 112 -> 92 | 141 -> 125;
   // 32 x 1024, window 128 73.0 -> 64.5 | 91.8 -> 83.8; bottom-right 16 x 1000 x 3001, window 40 65.6 -> 59.5 | 81.2 -> 76.4.
-  const bool small = launch_split_of(args, p, impl, FHOG_PASS_DQ_DDO) > 1;
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && small) order = fused, n_pass = 3;
-  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !small) order = ddo_early, n_pass = 4;
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !small) order = three, n_pass = 3;
+  const bool splits = launch_split_of(args, p, impl, FHOG_PASS_DQ_DDO) > 1;
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && splits) order = fused, n_pass = 3;
+  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early, n_pass = 4;
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three, n_pass = 3;
   for (int i = 0; i < n_pass; i++) {
     const int r = run_pass(args, p, impl, order[i], (hipStream_t)hip_stream);
     if (r != FHOG_OK) return r;

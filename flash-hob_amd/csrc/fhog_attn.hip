@@ -18,53 +18,11 @@
 // of the cycles and the VALU 48 %, and taking out the exponentials, the LDS reads or half of the staging moves the time by less
 // than 5 %. Issuing the first level of a tile beside the second level of the tile before, each behind the other's
 // elementwise work, measured equal (d = 64: +-3 %, d = 128: 2 % slower); fewer VALU instructions per block is what paid.
-#include "fhog_bf16_util.h"
+#include "fhog_bf16_blocks.h"
 
 namespace fhog {
 using namespace bf16k;
 namespace {
-
-// acc[cb] += tile^T (columns 32cb..32cb+31) x operand, for both k-steps and all column blocks of the tile
-template <bool F16, int D, int NOP>
-__device__ __forceinline__ void second_level(const char* const (&tile)[NOP], const int (&troff)[D / 32][2],
-                                             const bf16x8_t (&op)[NOP][2], f32x16_t (&acc)[NOP][D / 32]) {
-  constexpr int NC = D / 32, NIT = 2 * NC;
-  bf16x8_t a[2][NOP];
-#pragma unroll
-  for (int x = 0; x < NOP; x++) a[0][x] = lds_read_tr_pre(tile[x] + troff[0][0], tile[x] + troff[0][1], 0);
-#pragma unroll
-  for (int it = 0; it < NIT; it++) {
-    const int t = it / NC, cb = it % NC, c = it & 1;
-    if (it + 1 < NIT) {
-      const int t1 = (it + 1) / NC, cb1 = (it + 1) % NC;
-#pragma unroll
-      for (int x = 0; x < NOP; x++)
-        a[c ^ 1][x] = lds_read_tr_pre(tile[x] + troff[cb1][0], tile[x] + troff[cb1][1], t1 * 16 * 2 * D);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int x = 0; x < NOP; x++) acc[x][cb] = mfma<F16>(a[c][x], op[x][t], acc[x][cb]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// first-level product of one streamed tile with resident rows: out += tile x res^T (streamed rows = M)
-template <bool F16, int D, int NRES>
-__device__ __forceinline__ void first_level(const char* tile, const int (&aoff)[D / 16], const bf16x8_t* const (&res)[NRES],
-                                            f32x16_t (&out)[NRES]) {
-  constexpr int KK = D / 16, PF = 2, NB = PF + 1;
-  bf16x8_t a[NB];
-#pragma unroll
-  for (int i = 0; i < PF; i++) a[i] = lds_read128(tile, aoff[i]);
-#pragma unroll
-  for (int kk = 0; kk < KK; kk++) {
-    if (kk + PF < KK) a[(kk + PF) % NB] = lds_read128(tile, aoff[kk + PF]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int x = 0; x < NRES; x++) out[x] = mfma<F16>(a[kk % NB], res[x][kk], out[x]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
 
 // ---- forward -----------------------------------------------------------------------------------------
 template <bool F16, int D, int MASK>
@@ -125,45 +83,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
     if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
       const char* stage = smem + u * STAGE;
-      f32x16_t s[1] = {f32x16_t{0}};
-      const bf16x8_t* const res[1] = {Qb};
-      first_level<F16, D, 1>(stage, aoff, res, s);  // S^T: s[r] = (key k0 + 8(r/4) + 4h + r%4, query qi)
-      f32x16_t x = s[0];   // raw scores; the scale (positive) goes into the exponent's FMA, maxima commute with it
-      if (masked) {
-        keep_branch();
-#pragma unroll
-        for (int r = 0; r < 16; r++) x[r] = in_limits(r, lo, hi) ? x[r] : -INFINITY;
-      }
-      float tmax = fmaxf(fmaxf(x[0], x[1]), x[2]);
-#pragma unroll
-      for (int r = 3; r < 15; r += 2) tmax = fmaxf(fmaxf(tmax, x[r]), x[r + 1]);
-      tmax = fmaxf(tmax, x[15]) * c_scale_log2;
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-      // The running maximum follows the row maximum only in jumps of more than kMaxSlack (in log2 units): P may then
-      // reach 2^kMaxSlack instead of 1, which costs no precision in a 16-bit float or in the fp32 sums, and the output
-      // accumulators are rescaled only in the rare steps where some row jumps (else on about every second tile).
-      constexpr float kMaxSlack = 8.f;
-      const float m_new = tmax > m + kMaxSlack ? tmax : m;
-      // a row whose window starts in a later tile has seen no key yet: keep exp2(-inf - (-inf)) out of it
-      const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m - m_ref);
-      float rs = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[r], c_scale_log2, -m_ref));
-        rs += x[r];
-      }
-      l = __builtin_fmaf(l, alpha, rs);
-      if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {  // rescale only when some row's maximum moved
-#pragma unroll
-        for (int cb = 0; cb < NC; cb++)
-#pragma unroll
-          for (int r = 0; r < 16; r++) acc[0][cb][r] *= alpha;
-      }
-      m = m_new;
-      const bf16x8_t op[1][2] = {{pack_operand<F16>(x, 0), pack_operand<F16>(x, 1)}};
-      const char* const vt[1] = {stage + TILE};
-      second_level<F16, D, 1>(vt, troff, op, acc);  // O^T += V^T P^T
+      fwd_block<F16, D>(stage, aoff, troff, Qb, masked, lo, hi, c_scale_log2, m, l, acc);
     }
     dma_wait();
     __syncthreads();
@@ -257,24 +177,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
     if (!geo.dead(k0, qw)) {
       const char* stage = smem + u * STAGE;
-      f32x16_t s[1] = {f32x16_t{0}}, dp[1];
-#pragma unroll
-      for (int r = 0; r < 16; r++) dp[0][r] = -dsum;        // the accumulator ends as dP - d
-      const bf16x8_t* const rq[1] = {Qb};
-      const bf16x8_t* const rdo[1] = {dOb};
-      first_level<F16, D, 1>(stage, aoff, rq, s);           // S^T  = K Q^T
-      first_level<F16, D, 1>(stage + TILE, aoff, rdo, dp);  // dP^T = V dO^T - d
-      f32x16_t ds;
-#pragma unroll
-      for (int r = 0; r < 16; r++) ds[r] = __builtin_amdgcn_exp2f(s[0][r] * c_scale_log2 - l_log2) * dp[0][r];
-      if (masked) {
-        keep_branch();
-#pragma unroll
-        for (int r = 0; r < 16; r++) ds[r] = in_limits(r, lo, hi) ? ds[r] : 0.f;
-      }
-      const bf16x8_t op[1][2] = {{pack_operand<F16>(ds, 0), pack_operand<F16>(ds, 1)}};
-      const char* const kt[1] = {stage};
-      second_level<F16, D, 1>(kt, troff, op, acc);  // dQ^T += K^T dS^T
+      bwd_q_block<F16, D>(stage, aoff, troff, Qb, dOb, masked, lo, hi, c_scale_log2, l_log2, dsum, acc);
     }
     dma_wait();
     __syncthreads();
@@ -367,36 +270,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_k_bf16(AttnParams p) {
     const int qb = j * TS;
     if (!geo.dead(qb, kw)) {  // else no query of the tile sees a key of this wave
       const char* stage = smem + st * STAGE;
-      const float* stat = reinterpret_cast<const float*>(stage + 2 * TILE);
-      f32x16_t s[1] = {f32x16_t{0}}, dp[1] = {f32x16_t{0}};
-      const bf16x8_t* const rk[1] = {Kb};
-      const bf16x8_t* const rv[1] = {Vb};
-      first_level<F16, D, 1>(stage, aoff, rk, s);           // S  = Q K^T : s[r] = (query qb + 8(r/4) + 4h + r%4, key kj)
-      first_level<F16, D, 1>(stage + TILE, aoff, rv, dp);   // dP = dO V^T
-      f32x16_t pv, ds;
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(stat + 8 * g + 4 * h);
-        const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(stat + TS + 8 * g + 4 * h);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int r = 4 * g + e;
-          pv[r] = __builtin_amdgcn_exp2f(s[0][r] * c_scale_log2 - l4[e]);
-          ds[r] = dp[0][r] - d4[e];
-        }
-      }
-      if (geo.partial(qb, kw)) {  // wave-uniform: the block holds hidden (query, key) pairs
-        int lo, hi;                // query row 8g + 4h + e of the tile counts iff lo <= 8g + e <= hi: it exists and sees key kj
-        geo.limits(qb, kj, h, lo, hi);
-        keep_branch();
-#pragma unroll
-        for (int r = 0; r < 16; r++) pv[r] = in_limits(r, lo, hi) ? pv[r] : 0.f;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r++) ds[r] *= pv[r];
-      const bf16x8_t op[2][2] = {{pack_operand<F16>(ds, 0), pack_operand<F16>(ds, 1)}, {pack_operand<F16>(pv, 0), pack_operand<F16>(pv, 1)}};
-      const char* const tl[2] = {stage, stage + TILE};
-      second_level<F16, D, 2>(tl, troff, op, acc);  // dK^T += Q^T dS ; dV^T += dO^T P
+      bwd_k_block<F16, D>(geo, stage, aoff, troff, Kb, Vb, qb, kw, kj, h, c_scale_log2, acc);
     }
     if (j + 1 < t_end) {
       wait_vm0();

@@ -129,18 +129,19 @@ __device__ __forceinline__ f32x16_t mfma(bf16x8_t a, bf16x8_t b, f32x16_t c) {
 // that lands on chunk position pc of row r fetches chunk pc ^ swz(r) of that row.
 // The load is issued from inline asm, so the compiler does not track it: the caller must execute
 // dma_wait() before the barrier that publishes the tile.
-template <int D>
+// LOADERS: waves that share the rows of a tile.
+template <int D, int LOADERS = 4>
 struct Dma {
   static constexpr int CPR = D / 8;             // 16-byte chunks per row
   static constexpr int RPI = 64 / CPR;          // rows per instruction (4 at d=128, 8 at d=64)
   static constexpr int IPT = TS / RPI;          // instructions per 32-row tile (8 or 4)
-  static constexpr int PER_WAVE = IPT / 4;      // instructions per tile for each of 4 loader waves (2 or 1)
+  static constexpr int PER_WAVE = IPT / LOADERS;   // instructions per tile for each loader wave (2 or 1 of 4 waves)
   uint32_t voff[PER_WAVE];                      // per-lane byte offset from the tile's first row
   int64_t ld_;
   int lw_, lane_;
 
   __device__ __forceinline__ uint32_t lane_offset(int u, int rows_valid) const {
-    const int q = lw_ + 4 * u;
+    const int q = lw_ + LOADERS * u;
     const int r = q * RPI + lane_ / CPR, pc = lane_ % CPR;
     const int rs = r < rows_valid ? r : rows_valid - 1;  // rows past the end of the tensor re-read its last row
     return (uint32_t)((rs * ld_ + ((pc ^ swz<D>(r)) << 3)) * 2);
@@ -166,7 +167,7 @@ struct Dma {
 #pragma unroll
       for (int x = 0; x < N; x++)
 #pragma unroll
-        for (int u = 0; u < PER_WAVE; u++) issue_one(tile_lds + x * tile_stride + (lw + 4 * u) * 1024, voff[u], src[x] + adv);
+        for (int u = 0; u < PER_WAVE; u++) issue_one(tile_lds + x * tile_stride + (lw + LOADERS * u) * 1024, voff[u], src[x] + adv);
     } else {
       uint32_t off[PER_WAVE];
 #pragma unroll
@@ -174,7 +175,7 @@ struct Dma {
 #pragma unroll
       for (int x = 0; x < N; x++)
 #pragma unroll
-        for (int u = 0; u < PER_WAVE; u++) issue_one(tile_lds + x * tile_stride + (lw + 4 * u) * 1024, off[u], src[x] + adv);
+        for (int u = 0; u < PER_WAVE; u++) issue_one(tile_lds + x * tile_stride + (lw + LOADERS * u) * 1024, off[u], src[x] + adv);
     }
   }
   // M0 is on the clobber list: the compiler never allocates it, but it does write it ahead of instructions of its own
@@ -331,8 +332,7 @@ __host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) {
 // without -> with: bf16 causal 64 x 1024, d = 32: dQ 25.8 -> 21.9, passes 3 and 4 89.5 -> 83.1; Hessian-vector product 199.4 -> 195.9,
 // fp16 48 x 1537, d = 64 347 -> 342, training step bf16 32 x 4096, d = 128 622 -> 615. With one workgroup per CU
 // (producer/consumer kernels) the ids 32.. start as CUs fall free and heaviest-first is the right order for them too.
-__device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs = false) {
-  const int id = blockIdx.x;
+__device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs = false, int id = blockIdx.x) {
   const int xcd = id & 7;
   int slot = id >> 3;
   const int xs = xcds_per_slice(batch), per_round = 8 / xs, tiles_per_xcd = (n_tiles + xs - 1) / xs;

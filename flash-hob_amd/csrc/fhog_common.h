@@ -62,10 +62,12 @@ struct Params {
 //   split=0|1          let launches too small to fill the GPU split their streamed side over several workgroups (default 1)
 //   dd64=0|1           dd sweep at d = 128: 32 | 64 queries per wave (default: 64 when that still gives 2048 workgroups)
 //   stage64=0|1        single-role sweeps at d = 64: one | two 32-row tiles staged and consumed per barrier (default 0: measured equal within 1 %)
+//   small=0|2|4        first-order passes and the double-backward (all schedules but the reference's) on 16-bit tensors: four waves on
+//                      128 stationary rows | that many on the same 32 (fhog_small.hip; default: by the size of the launch)
 //   stage1=0|1         d = 64, reference schedule: sweeps 1-3 as three launches | as one launch whose workgroups run them one
 //                      after the other for their tile (FHOG_PASS_STAGE1)
 struct Tuning {
-  int b8 = -1, order = -1, split = 1, dd64 = -1, stage64 = 0, stage1 = 0;
+  int b8 = -1, order = -1, split = 1, dd64 = -1, stage64 = 0, stage1 = 0, small = -1;
 };
 const Tuning& tuning();
 
@@ -116,6 +118,8 @@ hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);          
 hipError_t launch_attn_bf16(const AttnParams& p, int which, hipStream_t s);         // 0 forward, 1 dQ, 2 dK and dV
 hipError_t launch_attn_split(const AttnParams& p, int dtype, int which, hipStream_t s); // same, split products (fp32 tensors, d = 32)
 hipError_t launch_attn_bwd_k_pc(const AttnParams& p, hipStream_t s);                // dK and dV at d = 128 (producer/consumer)
+hipError_t launch_small_bwdbwd(const Params& p, int waves, hipStream_t s);  // default schedule, 16-bit tensors: 4 or 2 waves on 32 rows
+hipError_t launch_small_attn(const AttnParams& p, bool backward, int waves, hipStream_t s);   // first-order passes, likewise
 hipError_t launch_mfma_rate(float* out, int blocks, int trips, int data_mode, int waves, hipStream_t s);  // measurement aid
 bool bf16_shape_supported(int64_t n_q, int64_t n_k, int64_t d, int causal);
 
