@@ -223,7 +223,7 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
     e = fhog::launch_bf16_pass(p, pass, s);
   else
     e = fhog::launch_split_pass(p, a->dtype, pass, s);
-  if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "pass %d: HIP error %d (%s)", pass, (int)e, hipGetErrorString(e));
+  if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "pass %d: HIP error %d (%s)", pass == fhog::kPassGrads ? FHOG_PASS_DQ_DDO : pass, (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }
 
@@ -519,8 +519,11 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early, n_pass = 4;
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three, n_pass = 3;
   for (int i = 0; i < n_pass; i++) {
-    const int r = run_pass(args, p, impl, order[i], (hipStream_t)hip_stream);
+    // split products: passes 3 and 4, the last two, share a launch
+    const bool both = split_products && order[i] == FHOG_PASS_DQ_DDO;
+    const int r = run_pass(args, p, impl, both ? fhog::kPassGrads : order[i], (hipStream_t)hip_stream);
     if (r != FHOG_OK) return r;
+    if (both) break;
   }
   return FHOG_OK;
 }

@@ -111,6 +111,8 @@ inline hipError_t allow_dynamic_lds(int bytes) {
   return e;
 }
 
+constexpr int kPassGrads = -1;   // launch_split_pass: passes 3 and 4 in one launch
+
 // Launchers implemented in the kernel translation units. Each returns hipGetLastError().
 hipError_t launch_rowdot(const Params& p, int dtype, hipStream_t s);                 // pass 0
 hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products

@@ -9,7 +9,7 @@
 // the stationary rows as N, so a lane owns ONE stationary row and its registers run over the streamed rows; split into
 // terms, such a tile is as it stands the B operand of the second-level products, whose A operand is a transposing read of
 // the staged tile in the same row order. Small launches (WS = 2 or 4) put WS waves on the same 32 rows instead: each takes
-// every WS-th streamed tile and the partial results are added through LDS in a fixed order.
+// every WS-th streamed tile and the partial results are added through LDS in a fixed order. Passes 3 and 4 share a launch (launch_grads).
 //
 // What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
 // 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (34 MFMAs beside some 400
@@ -17,9 +17,9 @@
 // lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 54 to 60, in pass 4 at d = 64 with
 // four waves on the same rows 18 to 21, at d = 32 under a mask in pass 3 6 and without one in pass 4 15; 16-bit tensors at d = 128 up to 89.
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
-//   bf16 causal 64 x 1024, d = 32: 734 -> 136     fp32 causal 64 x 1024, d = 32: 672 -> 296
-//   fp32 causal 32 x 2048, d = 64: 2101 -> 984    fp32 64 x 2048, d = 64: 7521 -> 3667
-//   fp32 causal 32 x 2048, d = 128: 3833 -> 2340
+//   bf16 causal 64 x 1024, d = 32: 734 -> 121     fp32 causal 64 x 1024, d = 32: 672 -> 279
+//   fp32 causal 32 x 2048, d = 64: 2101 -> 950    fp32 64 x 2048, d = 64: 7521 -> 3590
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2381
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
@@ -78,8 +78,7 @@ constexpr bool is_direct = WS == 4 && (PASS == 1 || PASS == 2 || PASS == 5);
 
 // PASS 1: d, dd; 2: b; 3: dQ2, ddO; 4: dK2, dV2 (K-tiled); 5: d, dd, b.
 template <typename T, int D, int PASS, int MASK, int WS>
-__global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Params p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+__device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4);      // streamed tensors: K, ddK, V, ddV | Q, ddQ, dO
   constexpr int NR = PASS == 1 ? 2 : (KSIDE ? 4 : 3);      // stationary tensors: Q, ddQ, dO | K, ddK, V, ddV
@@ -106,7 +105,7 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && D < 64 && WS == 1)) return;
+  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && D < 64 && WS == 1, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
@@ -404,6 +403,23 @@ __global__ void __launch_bounds__(256, D >= 64 || WS > 1 ? 1 : 2) split_sweep(Pa
   }
 }
 
+template <int D, int WS>
+constexpr int min_workgroups = D >= 64 || WS > 1 ? 1 : 2;
+
+template <typename T, int D, int PASS, int MASK, int WS>
+__global__ void __launch_bounds__(256, (min_workgroups<D, WS>)) split_sweep(Params p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  split_run<T, D, PASS, MASK, WS>(p, smem, blockIdx.x);
+}
+
+// Passes 3 (workgroups [0, q_blocks)) and 4 (the others) in one launch: given the row statistics neither needs the other.
+template <typename T, int D, int MASK, int WS3, int WS4>
+__global__ void __launch_bounds__(256, (min_workgroups<D, (WS3 > WS4 ? WS3 : WS4)>)) split_grads(Params p, int q_blocks) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < q_blocks) split_run<T, D, 3, MASK, WS3>(p, smem, blockIdx.x);
+  else split_run<T, D, 4, MASK, WS4>(p, smem, (int)blockIdx.x - q_blocks);
+}
+
 template <typename T, int D, int PASS, int WS>
 constexpr int lds_bytes() {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
@@ -418,10 +434,9 @@ template <typename T, int D, int PASS, int MASK, int WS>
 hipError_t launch_ws(const Params& p, hipStream_t s) {
   constexpr int smem = lds_bytes<T, D, PASS, WS>(), nw = 4 / WS;
   static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
-  const int n_rows = PASS == 4 ? p.n_k : p.n_q;
   const hipError_t e = allow_dynamic_lds<split_sweep<T, D, PASS, MASK, WS>>(smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((split_sweep<T, D, PASS, MASK, WS>), dim3(grid_blocks((n_rows + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
+  hipLaunchKernelGGL((split_sweep<T, D, PASS, MASK, WS>), dim3(grid_blocks((p.n_q + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
   return hipGetLastError();
 }
 
@@ -430,7 +445,7 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 // the LDS (four waves of a statistics sweep stage nothing): two fp32 heads of 256 tokens are 4 workgroups otherwise, each running its eight streamed tiles one after the other.
 // A statistics sweep that stages nothing splits every tile into terms once per 32 rows instead of once per 128, but its workgroups
 // are a quarter of the size: worth it beyond 64 workgroups where the staged form leaves CUs to the heaviest tiles of a causal
-// triangle, or has one wave per row block. Pass 5, us, staged -> direct, at so many 128-row workgroups:
+// triangle, or has one wave per row block. Statistics sweeps only; passes 3 and 4 are launch_grads' below. Pass 5, us, staged -> direct, at so many 128-row workgroups:
 // Left as it is: triangles of 160 to 255 workgroups on fp32 tensors at d <= 64, where 15 x 2048 would gain (d = 64: 185 -> 151) what
 // 60 x 500 would lose (the number of streamed tiles tells them apart), and windows and bottom-right masks beyond 128 (fp32
 // d <= 64: 64), which were not measured.
@@ -439,20 +454,49 @@ hipError_t launch_ws(const Params& p, hipStream_t s) {
 //   no mask:  fp32 d = 128 553 -> 435 (126); bf16 d = 32 43.0 -> 32.5 (126); fp32 d = 64 129 -> 137 (96)
 template <typename T, int D, int PASS, int MASK>
 hipError_t launch_sweep(const Params& p, hipStream_t s) {
-  const int64_t groups = (int64_t)((PASS == 4 ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = PASS == 4 ? p.n_q : p.n_k;
-  if constexpr (lds_bytes<T, D, PASS, 4>() <= 160 * 1024) {
-    int64_t line = 64;
-    if constexpr (is_direct<PASS, 4>) {
-      const bool triangle = MASK != MASK_NONE && p.mask_off == 0 && p.window >= p.n_k;
-      constexpr bool splits_dear = sizeof(T) == 4 && D < 128;
-      line = triangle ? (splits_dear ? 160 : 256) : splits_dear ? 64 : 128;
-    }
-    if (groups < line && n_str > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
-  }
+  const int64_t groups = (int64_t)(p.n_q + 127) / 128 * p.batch;
+  const bool triangle = MASK != MASK_NONE && p.mask_off == 0 && p.window >= p.n_k;
+  constexpr bool splits_dear = sizeof(T) == 4 && D < 128;
+  const int64_t line = triangle ? (splits_dear ? 160 : 256) : splits_dear ? 64 : 128;
+  if (groups < line && p.n_k > 2 * TS) return launch_ws<T, D, PASS, MASK, 4>(p, s);
   if constexpr (lds_bytes<T, D, PASS, 2>() <= 160 * 1024) {
-    if (groups < 128 && n_str > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
+    if (groups < 128 && p.n_k > TS) return launch_ws<T, D, PASS, MASK, 2>(p, s);
   }
   return launch_ws<T, D, PASS, MASK, 1>(p, s);
+}
+
+template <int WS>
+unsigned blocks(int rows, int batch) { return grid_blocks((rows + 128 / WS - 1) / (128 / WS), batch); }
+
+// At most MOST waves on the same rows, as many as let either pass fit the LDS. sides: 1 pass 3, 2 pass 4, 3 both
+template <typename T, int D, int MASK, int MOST>
+hipError_t launch_grads_most(const Params& p, int sides, hipStream_t s) {
+  constexpr int ws3 = MOST >= 4 && lds_bytes<T, D, 3, 4>() <= 160 * 1024 ? 4 : MOST >= 2 && lds_bytes<T, D, 3, 2>() <= 160 * 1024 ? 2 : 1;
+  constexpr int ws4 = MOST >= 4 && lds_bytes<T, D, 4, 4>() <= 160 * 1024 ? 4 : MOST >= 2 && lds_bytes<T, D, 4, 2>() <= 160 * 1024 ? 2 : 1;
+  constexpr int l3 = lds_bytes<T, D, 3, ws3>(), l4 = lds_bytes<T, D, 4, ws4>(), smem = l3 > l4 ? l3 : l4;
+  static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
+  const hipError_t e = allow_dynamic_lds<split_grads<T, D, MASK, ws3, ws4>>(smem);
+  if (e != hipSuccess) return e;
+  const unsigned gq = sides & 1 ? blocks<ws3>(p.n_q, p.batch) : 0, gk = sides & 2 ? blocks<ws4>(p.n_k, p.batch) : 0;
+  hipLaunchKernelGGL((split_grads<T, D, MASK, ws3, ws4>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq);
+  return hipGetLastError();
+}
+
+// Passes 3 and 4 side by side are faster than one after the other whatever the size: their workgroups fill CUs for each other where
+// one pass has too few, and the light end of a triangle goes under the other pass. Four waves on the same rows while that gives one
+// workgroup per CU, two as long as the workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. Double-backward, us,
+// two launches (the rule before) -> one launch with four | two | one waves on the same rows:
+//   fp32 d = 64   2 x 256 67 -> 45 | - | -; 32 x 256 83 -> 66 | 54 | 70; 64 x 256 124 -> 108 | 92 | 83; causal 16 x 1024 382 -> 195 | 166 | 213,
+//                 32 x 1024 435 -> 375 | 318 | 296, 32 x 2048 980 -> 1190 | 1034 | 950; no mask 32 x 2048 1808 -> 2186 | 1937 | 1793
+//   fp32 d = 128  (one wave at all sizes, LDS) 2 x 256 234 -> 133; causal 16 x 2048 2104 -> 1440; 32 x 2048 2383 -> 2381
+//   bf16 d = 32   2 x 256 20 -> 13 | - | -; causal 16 x 1024 99 -> 59 | 47 | 56, 32 x 1024 114 -> 119 | 90 | 96, 64 x 1024 127 -> 218 | 160 | 121
+template <typename T, int D, int MASK>
+hipError_t launch_grads(const Params& p, int sides, hipStream_t s) {
+  const int64_t groups = (int64_t)((p.n_q + 127) / 128 + (p.n_k + 127) / 128) * p.batch;
+  const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  if (groups <= 64 || (D == 32 && triangle && groups <= 128 && p.n_k >= 1024)) return launch_grads_most<T, D, MASK, 4>(p, sides, s);
+  if (groups < (triangle ? (D == 32 ? 512 : 257) : 160)) return launch_grads_most<T, D, MASK, 2>(p, sides, s);
+  return launch_grads_most<T, D, MASK, 1>(p, sides, s);
 }
 
 template <typename T, int D>
@@ -461,9 +505,10 @@ hipError_t launch_td(const Params& p, int pass, hipStream_t s) {
   switch (pass) {
     case FHOG_PASS_DD: return FHOG_SPLIT_PASS(1);
     case FHOG_PASS_B: return FHOG_SPLIT_PASS(2);
-    case FHOG_PASS_DQ_DDO: return FHOG_SPLIT_PASS(3);
-    case FHOG_PASS_DK_DV: return FHOG_SPLIT_PASS(4);
+    case FHOG_PASS_DQ_DDO: return p.causal ? launch_grads<T, D, MASK_BAND>(p, 1, s) : launch_grads<T, D, MASK_NONE>(p, 1, s);
+    case FHOG_PASS_DK_DV: return p.causal ? launch_grads<T, D, MASK_BAND>(p, 2, s) : launch_grads<T, D, MASK_NONE>(p, 2, s);
     case FHOG_PASS_DD_B: return FHOG_SPLIT_PASS(5);
+    case kPassGrads: return p.causal ? launch_grads<T, D, MASK_BAND>(p, 3, s) : launch_grads<T, D, MASK_NONE>(p, 3, s);
     default: return hipErrorInvalidValue;
   }
 #undef FHOG_SPLIT_PASS

@@ -88,3 +88,42 @@ def test_rule_for_small_launches(tmp_path):
     for i, (shape, picks) in enumerate(PICKS):
         for part, pick in zip((slice(0, 2), slice(2, 5), slice(5, None)), picks):
             assert all(torch.equal(x, y) for x, y in zip(default[i][part], forced[pick][i][part])), (shape, part)
+
+
+# batch, n_q, n_k, mask, window: both sides of the lines at which the number of waves on the same rows changes, 63 to 65 groups of 128
+# rows on the two sides together, 159 and 161 without a mask, 256 to 258 and 511 under a triangle
+@pytest.mark.parametrize("shape", [(31, 100, 130, False, None), (32, 130, 100, True, 30), (53, 200, 128, False, None), (23, 385, 385, False, None),
+                                   (64, 256, 256, True, None), (43, 300, 300, True, None), (73, 500, 300, False, None), (2, 90, 4000, "bottom_right", 100)])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 64)])
+def test_passes_3_and_4_in_one_launch(shape, dtype, d):
+    """The split-product sweeps for dQ2, ddO and dK2, dV2 side by side: bit for bit as from the passes launched one by one, and against
+    the fp64 closed form at the gates of those sweeps."""
+    from fhog import BwdBwdPlan
+    from gpu_util import NAMES, errors, make_case, reference_fp64_cpu, with_caches
+    batch, n_q, n_k, causal, window = shape
+    if causal is True:
+        n_k = n_q
+    x = with_caches(make_case(batch, n_q, n_k, d, dtype, seed=81, grad_std=0.1), d ** -0.5, causal, window)
+    plans = [BwdBwdPlan(x["Q"], x["K"], x["V"], x["O"], x["dO"], x["ddQ"], x["ddK"], x["ddV"], x["L"], d ** -0.5, causal=causal, window=window,
+                        impl="fp32", schedule="fused_stats") for _ in range(2)]
+    for p in plans:
+        for t in p.outs:
+            t.fill_(float("nan"))
+    plans[0].run()
+    for i in (5, 3, 4):
+        plans[1].run(only_pass=i)
+    torch.cuda.synchronize()
+    for a, b in zip(plans[0].outs, plans[1].outs):
+        assert torch.equal(a, b) and torch.isfinite(a.float()).all()
+    sel = [0, batch // 2, batch - 1]
+    ref = reference_fp64_cpu(x, d ** -0.5, causal, window, heads=sel)
+    outs = dict(zip(("dq2", "dk2", "dv2", "ddo"), plans[0].outs))
+    e = errors([outs[n].view(batch, -1, d)[sel] for n in NAMES], [ref[n] for n in NAMES])
+    assert max(e.values()) < {torch.float32: 1e-4, torch.bfloat16: 2e-2, torch.float16: 2.5e-3}[dtype], e
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_weights_are_fp32_with_two_waves_on_the_same_rows(d, dtype):
+    from test_gpu_split import test_weights_beside_16_bit_tensors_are_fp32 as check
+    check(35, d, dtype)   # 70 groups of 128 rows a side
