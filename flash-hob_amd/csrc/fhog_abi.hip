@@ -417,7 +417,7 @@ int fhog_attn_fwd(const fhog_attn_args* args, void* hip_stream) {
   const int small = attn_on_16bit_kernels(args) ? small_waves(Small::forward, args) : 0;
   const hipError_t e = small ? fhog::launch_small_attn(to_attn_params(args), false, small, (hipStream_t)hip_stream)
                        : attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(to_attn_params(args), 0, (hipStream_t)hip_stream)
-                                                   : fhog::launch_attn_split(to_attn_params(args), args->dtype, 0, (hipStream_t)hip_stream);
+                                                   : fhog::launch_attn_split(to_attn_params(args), args->dtype, false, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention forward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }
@@ -426,15 +426,15 @@ int fhog_attn_bwd(const fhog_attn_args* args, void* hip_stream) {
   const int rc = validate_attn(args, 1);
   if (rc != FHOG_OK) return rc;
   const fhog::AttnParams p = to_attn_params(args);
-  if (const int small = attn_on_16bit_kernels(args) ? small_waves(Small::backward, args) : 0) {
-    const hipError_t e = fhog::launch_small_attn(p, true, small, (hipStream_t)hip_stream);
-    if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention backward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
-    return FHOG_OK;
+  hipError_t e;
+  if (!attn_on_16bit_kernels(args)) {
+    e = fhog::launch_attn_split(p, args->dtype, true, (hipStream_t)hip_stream);
+  } else if (const int small = small_waves(Small::backward, args)) {
+    e = fhog::launch_small_attn(p, true, small, (hipStream_t)hip_stream);
+  } else {
+    e = fhog::launch_attn_bf16(p, 1, (hipStream_t)hip_stream);   // dQ, and the row sums d that the kernel for dK and dV reads
+    if (e == hipSuccess) e = fhog::launch_attn_bf16(p, 2, (hipStream_t)hip_stream);
   }
-  hipError_t e = hipSuccess;   // the dQ kernel also writes the row sums d that the one for dK and dV reads
-  for (int which = 1; which <= 2 && e == hipSuccess; which++)
-    e = attn_on_16bit_kernels(args) ? fhog::launch_attn_bf16(p, which, (hipStream_t)hip_stream)
-                                    : fhog::launch_attn_split(p, args->dtype, which, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "attention backward: HIP error %d (%s)", (int)e, hipGetErrorString(e));
   return FHOG_OK;
 }

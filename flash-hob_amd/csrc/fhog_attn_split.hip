@@ -10,7 +10,7 @@
 // double-backward needs leave room for the terms of d = 128 (one wave per SIMD); only dK, dV on fp32 tensors there does not quite
 // fit and keeps 44 VGPRs of a lane in scratch memory under a mask, 76 with two waves on the same rows.
 // Small launches (WS = 2 or 4) put WS waves on the same 32 rows: each takes every WS-th streamed tile, and the partial
-// results are merged through LDS in a fixed order.
+// results are merged through LDS in a fixed order. dQ and dK, dV share a launch unless each fills the GPU (launch_bwd).
 #include <type_traits>
 
 #include "fhog_split_util.h"
@@ -21,9 +21,9 @@ namespace {
 
 constexpr int MODE_FWD = 0, MODE_BWD_Q = 1, MODE_BWD_K = 2;
 
-template <typename T, int D, int MODE, int MASK, int WS>
-__global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) attn_split(AttnParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+// OWN_D: dK, dV without the sweep for dQ before it
+template <typename T, int D, int MODE, int MASK, int WS, bool OWN_D>
+__device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id) {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
   constexpr int NR = MODE == MODE_FWD ? 1 : 2;             // stationary tensors: Q | Q, dO | K, V
   constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, MASK != MASK_NONE && sizeof(T) * D < 256 && WS == 1)) return;
+  if (!decode_block((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, MASK != MASK_NONE && sizeof(T) * D < 256 && WS == 1, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
@@ -53,13 +53,21 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
 
   const int64_t srow = (int64_t)bh * p.n_q;
   Stage st[WS];
+  // dK, dV: L and d of the staged queries. OWN_D: d_i = sum_c O_ic dO_ic is taken here, by the threads that stage the row of dO.
+  constexpr int DO0 = Stage::RPT / Stage::XPI;                     // first chunk of dO among the chunks that a thread stages
   float stat_reg[WS] = {};
+  Chunk<T> o_reg[WS][KSIDE && OWN_D ? Stage::RPT : 1];
   const auto fetch = [&](int t) {
 #pragma unroll
     for (int g = 0; g < WS; g++) {
-      const int row0 = (t + g) * TS;
-      st[g].fetch(src, str_ld, min(row0, n_str - 1), n_str, tid);   // a tile past the end is never computed on
-      if (KSIDE && tid < 2 * TS) stat_reg[g] = (tid < TS ? p.lse : p.ws_d)[srow + min(row0 + (tid & 31), p.n_q - 1)];
+      const int row0 = min((t + g) * TS, n_str - 1);                // a tile past the end is never computed on
+      st[g].fetch(src, str_ld, row0, n_str, tid);
+      if (KSIDE && tid < (OWN_D ? 1 : 2) * TS) stat_reg[g] = (tid < TS ? p.lse : p.ws_d)[srow + min(row0 + (tid & 31), p.n_q - 1)];
+      if constexpr (KSIDE && OWN_D) {
+#pragma unroll
+        for (int i = 0; i < Stage::RPT; i++)
+          o_reg[g][i] = load_chunk<T>((const T*)p.o + qoff + (int64_t)min(row0 + Stage::row_of(DO0 + i, tid), p.n_q - 1) * str_ld + 8 * (tid % Stage::CPR));
+      }
     }
   };
   const auto publish = [&](int buf) {
@@ -67,7 +75,20 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
     for (int g = 0; g < WS; g++) {
       char* stage = smem + (buf * WS + g) * STAGE;
       st[g].publish(stage, tid);
-      if (KSIDE && tid < 2 * TS) reinterpret_cast<float*>(stage + Stage::BYTES)[tid] = tid < TS ? stat_reg[g] * kLog2e : -stat_reg[g];
+      float* const stat = reinterpret_cast<float*>(stage + Stage::BYTES);
+      if (KSIDE && tid < (OWN_D ? 1 : 2) * TS) stat[tid] = tid < TS ? stat_reg[g] * kLog2e : -stat_reg[g];
+      if constexpr (KSIDE && OWN_D) {
+#pragma unroll
+        for (int i = 0; i < Stage::RPT; i++) {
+          float d = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; e++) d = __builtin_fmaf(chunk_elem(o_reg[g][i], e), chunk_elem(st[g].c[DO0 + i], e), d);
+#pragma unroll
+          for (int m = 1; m < Stage::CPR; m *= 2) d += __shfl_xor(d, m);
+          // two tensors in a round of threads: the second half of them holds dO
+          if (tid % Stage::CPR == 0 && (Stage::XPI == 1 || tid >= 128)) stat[TS + Stage::row_of(DO0 + i, tid)] = -d;
+        }
+      }
     }
   };
   if (t_begin < t_end) fetch(t_begin);
@@ -249,6 +270,23 @@ __global__ void __launch_bounds__(256, sizeof(T) * D >= 256 || WS > 1 ? 1 : 2) a
   }
 }
 
+template <typename T, int D, int WS>
+constexpr int min_workgroups = sizeof(T) * D >= 256 || WS > 1 ? 1 : 2;
+
+template <typename T, int D, int MODE, int MASK, int WS>
+__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS>)) attn_split(AttnParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  attn_run<T, D, MODE, MASK, WS, false>(p, smem, blockIdx.x);
+}
+
+// dQ (workgroups [0, q_blocks)) and dK, dV (the others) in one launch
+template <typename T, int D, int MASK, int WS>
+__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS>)) attn_split_bwd(AttnParams p, int q_blocks) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < q_blocks) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, blockIdx.x);
+  else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, (int)blockIdx.x - q_blocks);
+}
+
 template <typename T, int D, int MODE, int WS>
 constexpr int lds_bytes() {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
@@ -257,53 +295,87 @@ constexpr int lds_bytes() {
   return stages > xch ? stages : xch;
 }
 
+template <int WS>
+unsigned blocks(int rows, int batch) { return grid_blocks((rows + 128 / WS - 1) / (128 / WS), batch); }
+
 template <typename T, int D, int MODE, int MASK, int WS>
 hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
-  constexpr int smem = lds_bytes<T, D, MODE, WS>(), nw = 4 / WS;
+  constexpr int smem = lds_bytes<T, D, MODE, WS>();
   static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
-  const int n_rows = MODE == MODE_BWD_K ? p.n_k : p.n_q;
   const hipError_t e = allow_dynamic_lds<attn_split<T, D, MODE, MASK, WS>>(smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((attn_split<T, D, MODE, MASK, WS>), dim3(grid_blocks((n_rows + 32 * nw - 1) / (32 * nw), p.batch)), dim3(256), smem, s, p);
+  hipLaunchKernelGGL((attn_split<T, D, MODE, MASK, WS>), dim3(blocks<WS>(MODE == MODE_BWD_K ? p.n_k : p.n_q, p.batch)), dim3(256), smem, s, p);
+  return hipGetLastError();
+}
+
+template <typename T, int D, int MASK, int WS>
+hipError_t launch_bwd_ws(const AttnParams& p, hipStream_t s) {
+  constexpr int lq = lds_bytes<T, D, MODE_BWD_Q, WS>(), lk = lds_bytes<T, D, MODE_BWD_K, WS>(), smem = lq > lk ? lq : lk;
+  static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
+  const hipError_t e = allow_dynamic_lds<attn_split_bwd<T, D, MASK, WS>>(smem);
+  if (e != hipSuccess) return e;
+  const unsigned gq = blocks<WS>(p.n_q, p.batch), gk = blocks<WS>(p.n_k, p.batch);
+  hipLaunchKernelGGL((attn_split_bwd<T, D, MASK, WS>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq);
   return hipGetLastError();
 }
 
 // As in fhog_split.hip: four waves on 128 rows when that fills the GPU, two or four on the same 32 rows when it does not.
-template <typename T, int D, int MODE, int MASK>
-hipError_t launch_mode(const AttnParams& p, hipStream_t s) {
-  const int64_t groups = (int64_t)((MODE == MODE_BWD_K ? p.n_k : p.n_q) + 127) / 128 * p.batch, n_str = MODE == MODE_BWD_K ? p.n_q : p.n_k;
-  if constexpr (lds_bytes<T, D, MODE, 4>() <= 160 * 1024) {
-    if (groups < 64 && n_str > 2 * TS) return launch_ws<T, D, MODE, MASK, 4>(p, s);
+template <typename T, int D, int MASK>
+hipError_t launch_fwd(const AttnParams& p, hipStream_t s) {
+  const int64_t groups = (int64_t)(p.n_q + 127) / 128 * p.batch;
+  if constexpr (lds_bytes<T, D, MODE_FWD, 4>() <= 160 * 1024) {
+    if (groups < 64 && p.n_k > 2 * TS) return launch_ws<T, D, MODE_FWD, MASK, 4>(p, s);
   }
-  if (groups < 128 && n_str > TS) return launch_ws<T, D, MODE, MASK, 2>(p, s);
-  return launch_ws<T, D, MODE, MASK, 1>(p, s);
+  if (groups < 128 && p.n_k > TS) return launch_ws<T, D, MODE_FWD, MASK, 2>(p, s);
+  return launch_ws<T, D, MODE_FWD, MASK, 1>(p, s);
+}
+
+// dQ and dK, dV side by side fill CUs for each other, as passes 3 and 4 do in fhog_split.hip, and the rule for waves on the same rows is of
+// the same kind. The price is the row sums d, which the sweep for dK, dV then takes once per key block: nothing at d = 32, 3 to 9 % on
+// fp32 tensors of d = 64 and 128, whose launches of full rounds (256 workgroups each) go one after the other. First backward, us, two
+// launches (the rule before) -> one launch with four | two | one waves on the same rows:
+//   bf16 d = 32   2 x 256 11.7 -> 7.9 | 9.8 | 12; causal 16 x 1024 56 -> 28 | 34 | 38, 64 x 1024 59 -> 81 | 57 | 49; no mask 16 x 1024 53 -> 37 | 35 | 37
+//   fp32 d = 64   2 x 256 27 -> 16 | 21 | 31; causal 16 x 1024 181 -> 99 | 83 | 106, 32 x 1024 182 -> 192 | 135 | 122; no mask 48 x 1024
+//                 309 -> - | 345 | 283, 64 x 1024 338 -> - | 459 | 362
+//   fp32 d = 128  2 x 256 66 -> - | 46 | 59; causal 16 x 1024 325 -> - | 188 | 217, 64 x 1024 408 -> - | 620 | 428; no mask 64 x 1024 609 -> - | 989 | 631
+template <typename T, int D, int MASK>
+hipError_t launch_bwd(const AttnParams& p, hipStream_t s) {
+  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
+  const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  if constexpr (lds_bytes<T, D, MODE_BWD_K, 4>() <= 160 * 1024) {
+    if (groups <= (triangle && p.n_k >= 1024 ? (D == 32 ? 256 : 128) : D == 32 ? 128 : 64)) return launch_bwd_ws<T, D, MASK, 4>(p, s);
+  }
+  if (groups < (triangle ? (D == 32 ? 512 : 257) : D == 32 ? 320 : 129)) return launch_bwd_ws<T, D, MASK, 2>(p, s);
+  if constexpr (D > 32) {
+    const int64_t rounds = (groups + 255) / 256, apart = (g_q + 255) / 256 + (g_k + 255) / 256;
+    if (triangle ? groups >= (p.n_k >= 1024 ? 1024 : 512) : 12 * apart < 13 * rounds) {
+      const hipError_t e = launch_ws<T, D, MODE_BWD_Q, MASK, 1>(p, s);
+      return e != hipSuccess ? e : launch_ws<T, D, MODE_BWD_K, MASK, 1>(p, s);
+    }
+  }
+  return launch_bwd_ws<T, D, MASK, 1>(p, s);
 }
 
 template <typename T, int D>
-hipError_t launch_td(const AttnParams& p, int which, hipStream_t s) {
-  switch (which) {
-    case 0: return p.causal ? launch_mode<T, D, MODE_FWD, MASK_BAND>(p, s) : launch_mode<T, D, MODE_FWD, MASK_NONE>(p, s);
-    case 1: return p.causal ? launch_mode<T, D, MODE_BWD_Q, MASK_BAND>(p, s) : launch_mode<T, D, MODE_BWD_Q, MASK_NONE>(p, s);
-    case 2: return p.causal ? launch_mode<T, D, MODE_BWD_K, MASK_BAND>(p, s) : launch_mode<T, D, MODE_BWD_K, MASK_NONE>(p, s);
-    default: return hipErrorInvalidValue;
-  }
+hipError_t launch_td(const AttnParams& p, bool backward, hipStream_t s) {
+  if (backward) return p.causal ? launch_bwd<T, D, MASK_BAND>(p, s) : launch_bwd<T, D, MASK_NONE>(p, s);
+  return p.causal ? launch_fwd<T, D, MASK_BAND>(p, s) : launch_fwd<T, D, MASK_NONE>(p, s);
 }
 
 }  // namespace
 
-// which: 0 forward, 1 dQ (and the row sums d), 2 dK and dV; dtype: FHOG_DTYPE_*. fp32 tensors of every head dim, 16-bit
-// tensors of d = 32.
-hipError_t launch_attn_split(const AttnParams& p, int dtype, int which, hipStream_t s) {
+// dtype: FHOG_DTYPE_*. fp32 tensors of every head dim, 16-bit tensors of d = 32.
+hipError_t launch_attn_split(const AttnParams& p, int dtype, bool backward, hipStream_t s) {
   if (dtype == FHOG_DTYPE_FP32) {
     switch (p.d) {
-      case 32: return launch_td<float, 32>(p, which, s);
-      case 64: return launch_td<float, 64>(p, which, s);
-      case 128: return launch_td<float, 128>(p, which, s);
+      case 32: return launch_td<float, 32>(p, backward, s);
+      case 64: return launch_td<float, 64>(p, backward, s);
+      case 128: return launch_td<float, 128>(p, backward, s);
       default: return hipErrorInvalidValue;
     }
   }
   if (p.d != 32) return hipErrorInvalidValue;
-  return dtype == FHOG_DTYPE_FP16 ? launch_td<_Float16, 32>(p, which, s) : launch_td<__bf16, 32>(p, which, s);
+  return dtype == FHOG_DTYPE_FP16 ? launch_td<_Float16, 32>(p, backward, s) : launch_td<__bf16, 32>(p, backward, s);
 }
 
 }  // namespace fhog

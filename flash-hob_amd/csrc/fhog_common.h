@@ -118,7 +118,7 @@ hipError_t launch_rowdot(const Params& p, int dtype, hipStream_t s);            
 hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products
 hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);              // passes 1..4, bf16 MFMA
 hipError_t launch_attn_bf16(const AttnParams& p, int which, hipStream_t s);         // 0 forward, 1 dQ, 2 dK and dV
-hipError_t launch_attn_split(const AttnParams& p, int dtype, int which, hipStream_t s); // same, split products (fp32 tensors, d = 32)
+hipError_t launch_attn_split(const AttnParams& p, int dtype, bool backward, hipStream_t s); // split products (fp32 tensors, d = 32)
 hipError_t launch_attn_bwd_k_pc(const AttnParams& p, hipStream_t s);                // dK and dV at d = 128 (producer/consumer)
 hipError_t launch_small_bwdbwd(const Params& p, int waves, hipStream_t s);  // default schedule, 16-bit tensors: 4 or 2 waves on 32 rows
 hipError_t launch_small_attn(const AttnParams& p, bool backward, int waves, hipStream_t s);   // first-order passes, likewise

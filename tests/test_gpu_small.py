@@ -127,3 +127,34 @@ def test_passes_3_and_4_in_one_launch(shape, dtype, d):
 def test_weights_are_fp32_with_two_waves_on_the_same_rows(d, dtype):
     from test_gpu_split import test_weights_beside_16_bit_tensors_are_fp32 as check
     check(35, d, dtype)   # 70 groups of 128 rows a side
+
+
+# both sides of the lines at which waves share rows and the two sweeps share a launch: 127 to 130 groups of 128 rows on both sides together,
+# 159 and 161, 256 to 258 and 511 under a triangle, full rounds of 256 workgroups (whose sweeps run one after the other at d = 64 and 128)
+@pytest.mark.parametrize("shape", [(64, 100, 127, False, None), (65, 33, 128, False, None), (43, 130, 200, False, None), (23, 385, 385, False, None),
+                                   (128, 65, 40, True, None), (73, 300, 300, True, 70), (256, 33, 97, False, None), (8, 1030, 1030, True, None)])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 32)])
+def test_first_backward_on_split_products(shape, dtype, d):
+    """dQ beside dK and dV, whose sweep takes d = rowsum(O dO) itself, on padded rows, against fp64: the gates of the split products."""
+    import fhog
+    from gpu_util import make_case
+    from oracle.bwdbwd_oracle import first_backward
+    batch, n_q, n_k, causal, window = shape
+    if causal is True:
+        n_k = n_q
+    x = make_case(batch, n_q, n_k, d, dtype, seed=82, grad_std=0.1)
+    scale = d ** -0.5
+
+    def padded(t):
+        y = torch.full((*t.shape[:-1], d + 8), float("nan"), dtype=t.dtype, device=t.device)
+        y[..., :d] = t
+        return y[..., :d]
+
+    o, L = fhog.attention_forward(x["Q"], x["K"], x["V"], scale, causal, window=window, use_hip=True)
+    got = fhog.attention_backward(*map(padded, (x["Q"], x["K"], x["V"], o, x["dO"])), L, scale, causal, window=window, use_hip=True)
+    sel = [0, batch // 2, batch - 1]
+    c = {n: t[sel].double().cpu().numpy() for n, t in x.items()}
+    want = first_backward(c["Q"], c["K"], c["V"], c["dO"], scale, causal, window)
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        assert torch.isfinite(g.float()).all()
+        assert normalised_max_error(g[sel], w) < {torch.float32: 1e-4, torch.bfloat16: 2e-2, torch.float16: 2.5e-3}[dtype], name
