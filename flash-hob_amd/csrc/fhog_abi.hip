@@ -132,6 +132,7 @@ fhog::Params to_params(const fhog_bwdbwd_args* a) {
   p.part = nullptr;
   const int order = fhog::tuning().order;
   p.tile_major = order < 0 ? p.causal : order;
+  p.n_split_k = 1, p.tile_major_k = p.tile_major, p.part_k = nullptr;
   return p;
 }
 
@@ -163,18 +164,14 @@ int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
   return s;
 }
 
-// Splits a pass runs with, of `most`. Passes 3 and 4 at d = 128 keep one workgroup on a CU: what matters there is rounds of 256
-// workgroups times the tiles of one, under the mask, and what the partial results cost. In steps of one tile (1.9 us): a
-// workgroup needs about 4 to start and to store, combining 2 plus its bytes at 5 TB/s (14.5 us for 66 MB, 8 for 33).
-// Where the work of the workgroups differs (causal) the longest one and the average load bound the launch.
-// bf16 16 x 1000 x 3001, window 700, us, as many splits as give 512 workgroups -> this rule: pass 3 with 4 -> 2 splits 49.2 + 14.5
-// (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
-int split_up_to(int most, const fhog_bwdbwd_args* a, const fhog::Params& p, int pass) {
-  if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
-  const bool kside = pass == FHOG_PASS_DK_DV;
+// Workgroups (128 stationary rows) of a slice with a visible pair, and the tiles they visit
+struct Work {
+  int64_t live = 0, longest = 0, sum = 0;
+};
+Work work_of(const fhog_bwdbwd_args* a, const fhog::Params& p, bool kside) {
+  Work w;
   const int64_t n_sta = kside ? a->n_k : a->n_q, n_str = kside ? a->n_q : a->n_k;
-  int64_t live = 0, longest = 0, sum = 0;   // workgroups of a slice with a visible pair, and the tiles they visit
-  for (int64_t r0 = 0; r0 < n_sta; r0 += 128) {   // fewer than 512 workgroups, or nothing would split
+  for (int64_t r0 = 0; r0 < n_sta; r0 += 128) {   // fewer than 512 workgroups on the side that would split
     int64_t lo = 0, hi = n_str;   // streamed rows visible to [r0, r0 + 128)
     if (p.causal) {
       const int64_t first = kside ? r0 - p.mask_off : r0 + p.mask_off - p.window + 1;
@@ -183,14 +180,26 @@ int split_up_to(int most, const fhog_bwdbwd_args* a, const fhog::Params& p, int 
     }
     if (lo >= hi) continue;
     const int64_t tiles = (hi - 1) / 32 - lo / 32 + 1;
-    live++, sum += tiles, longest = tiles > longest ? tiles : longest;
+    w.live++, w.sum += tiles, w.longest = tiles > w.longest ? tiles : w.longest;
   }
-  if (live == 0) return 1;
+  return w;
+}
+
+// Splits that pass 3 or 4 runs with on its own, of `most`. At d = 128 they keep one workgroup on a CU: what matters there is rounds of 256
+// workgroups times the tiles of one, under the mask, and what the partial results cost. In steps of one tile (1.9 us): a
+// workgroup needs about 4 to start and to store, combining 2 plus its bytes at 5 TB/s (14.5 us for 66 MB, 8 for 33).
+// Where the work of the workgroups differs (causal) the longest one and the average load bound the launch.
+// bf16 16 x 1000 x 3001, window 700, us, as many splits as give 512 workgroups -> this rule: pass 3 with 4 -> 2 splits 49.2 + 14.5
+// (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
+int split_up_to(int most, const fhog_bwdbwd_args* a, const fhog::Params& p, int pass) {
+  if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
+  const Work w = work_of(a, p, pass == FHOG_PASS_DK_DV);
+  if (w.live == 0) return 1;
   int best = 1;
   double best_cost = 0;
   for (int s = 1; s <= most; s *= 2) {
-    const double rounds = (double)((live * a->batch * s + 255) / 256), mean = (double)sum / (double)live;
-    const double alone = (double)longest / s + 4, load = rounds * (mean / s + 4);
+    const double rounds = (double)((w.live * a->batch * s + 255) / 256), mean = (double)w.sum / (double)w.live;
+    const double alone = (double)w.longest / s + 4, load = rounds * (mean / s + 4);
     double cost = alone > load ? alone : load;
     if (s > 1) cost += 2 + (double)s * split_bytes(a, pass) / (5e6 * 1.9);
     if (s == 1 || cost < best_cost) best = s, best_cost = cost;
@@ -202,21 +211,93 @@ int launch_split_of(const fhog_bwdbwd_args* a, const fhog::Params& p, int impl, 
   return split_up_to(granted_split(a, impl, pass), a, p, pass);
 }
 
-int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
+// When the last of n_a jobs of length a and then n_b jobs of length b ends on 256 CUs, each taken by the CU that is free first
+double makespan(int64_t n_a, double a, int64_t n_b, double b) {
+  struct { int64_t cus; double load; } g[32] = {{256, 0}};   // CUs with the same load
+  int groups = 1;
+  double end = 0;
+  for (int side = 0; side < 2; side++) {
+    const double length = side ? b : a;
+    for (int64_t n = side ? n_b : n_a; n > 0;) {
+      int m = 0;
+      for (int i = 1; i < groups; i++)
+        if (g[i].load < g[m].load) m = i;
+      if (groups == 1 && n >= 512) {   // whole rounds
+        g[0].load += length * (double)(n / 256), n %= 256;
+      } else if (n >= g[m].cus || groups == 32) {
+        n -= g[m].cus, g[m].load += length;
+      } else {
+        g[groups++] = {n, g[m].load + length};
+        g[m].cus -= n, n = 0;
+      }
+    }
+  }
+  for (int i = 0; i < groups; i++) end = g[i].load > end ? g[i].load : end;
+  return end;
+}
+
+// Splits of the two sides where they share a launch, out of those that either would like alone and the workspace has room for. The same
+// reckoning in steps of a tile (d = 128 1.9 us, 64: 1.1), over the workgroups of both.
+void joint_splits(const fhog_bwdbwd_args* a, const fhog::Params& p, int* s_q, int* s_k) {
+  const int most_q = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DQ_DDO), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
+  *s_q = *s_k = 1;
+  const int64_t have = a->ws_bytes - (int64_t)stats_bytes(a);
+  if ((most_q == 1 && most_k == 1) || have <= 0) return;
+  const Work q = work_of(a, p, false), k = work_of(a, p, true);
+  if (q.live == 0 || k.live == 0) return;
+  const double fixed = a->d == 128 ? 4 : 2, tile_us = a->d == 128 ? 1.9 : 1.1;
+  const int64_t bytes_q = (int64_t)split_bytes(a, FHOG_PASS_DQ_DDO), bytes_k = (int64_t)split_bytes(a, FHOG_PASS_DK_DV);
+  double best = 0;
+  for (int x = 1; x <= most_q; x *= 2)
+    for (int y = 1; y <= most_k; y *= 2) {
+      const int64_t part = (x > 1 ? x * bytes_q : 0) + (y > 1 ? y * bytes_k : 0);
+      if (part > have) continue;
+      const double lq = (double)q.sum / (double)q.live / x + fixed, lk = (double)k.sum / (double)k.live / y + fixed;
+      const int64_t nq = q.live * a->batch * x, nk = k.live * a->batch * y;
+      const double longest = (double)(q.longest / x > k.longest / y ? q.longest / x : k.longest / y) + fixed;
+      double cost = makespan(nq, lq, nk, lk);   // pass 3 comes first
+      if (longest > cost) cost = longest;
+      if (part > 0) cost += (4 + (double)part / 2.5e6) / tile_us;   // a launch, and the partial results written and read
+      if ((x == 1 && y == 1) || cost < best) best = cost, *s_q = x, *s_k = y;
+    }
+}
+
+// Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all
+// of them first) balances the end of a launch; from 16384 stationary rows on a slice alone has tiles enough for that
+// and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x
+// instead of 4-10x, sweeps b, 3 and 4 0.1-3 % faster, the dd sweep with its three workgroups per CU 4 % slower).
+bool slice_order(const fhog_bwdbwd_args* a, const fhog::Params& p, int64_t rows) { return fhog::tuning().order < 0 && p.causal && rows >= 16384; }
+
+// Pass 3 or 7 (q_pass, 0: none) and pass 4 (k_side) of the 16-bit kernels, in one launch
+int run_grads(const fhog_bwdbwd_args* a, const fhog::Params& base, int q_pass, bool k_side, hipStream_t s) {
   fhog::Params p = base;
-  p.n_split = launch_split_of(a, p, impl, pass);
-  // Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all
-  // of them first) balances the end of a launch; from 16384 stationary rows on a slice alone has tiles enough for that
-  // and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x
-  // instead of 4-10x, sweeps b, 3 and 4 0.1-3 % faster, the dd sweep with its three workgroups per CU 4 % slower).
-  if (fhog::tuning().order < 0 && p.causal && pass != FHOG_PASS_DD && (pass == FHOG_PASS_DK_DV ? a->n_k : a->n_q) >= 16384)
-    p.tile_major = 0;
+  if (q_pass == FHOG_PASS_DQ_DDO && k_side) {
+    joint_splits(a, p, &p.n_split, &p.n_split_k);
+  } else {
+    p.n_split = q_pass ? launch_split_of(a, p, FHOG_IMPL_BF16, q_pass) : 1;
+    p.n_split_k = k_side ? launch_split_of(a, p, FHOG_IMPL_BF16, FHOG_PASS_DK_DV) : 1;
+  }
+  if (slice_order(a, p, a->n_q)) p.tile_major = 0;
+  if (slice_order(a, p, a->n_k)) p.tile_major_k = 0;
   p.part = reinterpret_cast<float*>(reinterpret_cast<char*>(a->ws) + stats_bytes(a));
-  hipError_t e;
+  p.part_k = p.part + (p.n_split > 1 ? p.n_split * (split_bytes(a, FHOG_PASS_DQ_DDO) / sizeof(float)) : 0);
+  const hipError_t e = fhog::launch_bf16_grads(p, q_pass, k_side, s);
+  if (e != hipSuccess) return fail(FHOG_E_LAUNCH, "passes %d and %d: HIP error %d (%s)", q_pass, k_side ? FHOG_PASS_DK_DV : 0, (int)e, hipGetErrorString(e));
+  return FHOG_OK;
+}
+
+int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int pass, hipStream_t s) {
   if (pass > FHOG_PASS_DD_B && impl != FHOG_IMPL_BF16)
     return fail(FHOG_E_PASS, "pass %d exists in the 16-bit MFMA family only (bf16 / fp16 tensors, d in {64, 128})", pass);
   if (pass == FHOG_PASS_STAGE1 && a->d != 64)
     return fail(FHOG_E_PASS, "pass %d (three sweeps in one launch) exists for d = 64 only", pass);
+  if (impl == FHOG_IMPL_BF16 && (pass == FHOG_PASS_DQ_DDO || pass == FHOG_PASS_DQ)) return run_grads(a, base, pass, false, s);
+  if (impl == FHOG_IMPL_BF16 && pass == FHOG_PASS_DK_DV) return run_grads(a, base, 0, true, s);
+  fhog::Params p = base;
+  p.n_split = launch_split_of(a, p, impl, pass);
+  if (pass != FHOG_PASS_DD && slice_order(a, p, pass == FHOG_PASS_DK_DV ? a->n_k : a->n_q)) p.tile_major = 0;
+  p.part = reinterpret_cast<float*>(reinterpret_cast<char*>(a->ws) + stats_bytes(a));
+  hipError_t e;
   if (pass == FHOG_PASS_D)
     e = fhog::launch_rowdot(p, a->dtype, s);
   else if (impl == FHOG_IMPL_BF16)
@@ -229,8 +310,8 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
 
 // ---- small launches of the 16-bit kernels (fhog_small.hip) ------------------------------------------------------
 // Waves that a launch puts on the same 32 stationary rows: 4 or 2, or 0 for the kernels with four waves on 128 rows.
-// One workgroup fits a CU: 4 waves as long as that is one round of the 256 CUs, 2 as long as they give one or, where the other
-// kernels would leave CUs idle, two rounds. `groups` counts 128-row groups of all sides that share a launch, `tiles` the streamed
+// One workgroup fits a CU: 4 waves as long as that is one round of the 256 CUs (first order, and short streams: 2 waves up to one or two
+// rounds where the other kernels would leave CUs idle). `groups` counts 128-row groups of all sides that share a launch, `tiles` the streamed
 // tiles of one. A triangle (or a window) is in favour of small workgroups, whose work evens out; the double-backward's other
 // kernels split long streams over workgroups (workspace) and win them back there.
 // us, other kernels -> 4 waves | 2 waves, square shapes, bf16:
@@ -238,8 +319,8 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
 //                     d = 128: 16 x 512 15.7 -> 9.5 | 13.2; 64 x 256 11.0 -> 13.5 | 10.4; 1 x 8192 163 -> 64 | 118
 //   first backward    d = 64: 8 x 256 19.0 -> 7.3 | 9.7; 32 x 256 19.4 -> 12.5 | 10.5; 16 x 1024 48 -> 42 | 37; 1 x 8192 303 -> 114 | 152
 //                     d = 128: 8 x 256 25 -> 12 | 18; causal 32 x 512 39 -> 41 | 35, no mask 38 -> 51 | 43
-//   double-backward   d = 64: 8 x 256 37.7 -> 15.0 | 19.1; 64 x 256 40 -> 42 | 31; 8 x 2048 134 -> 135 | 126; 1 x 8192 216 -> 240 | 288
-//                     d = 128: 8 x 256 52 -> 23 | 31; 16 x 512 71 -> 50 | 51; causal 32 x 512 81 -> 74 | 60; 16 x 1024 125 -> 146 | 131
+//   double-backward   d = 64: 4 x 256 24.1 -> 14.7 | 18.9; 64 x 256 27.2 -> 41 | 30; causal 8 x 1024 46.6 -> 33.8 | 45; 1 x 4096 59 -> 78 | 142
+//                     d = 128: 8 x 256 33.3 -> 22.8 | 30.5; 16 x 512 49.7 -> 49.2 | 49.7; causal 3 x 1536 69 -> 62 | 101; 1 x 2048 55 -> 72 | 127
 enum class Small { forward, backward, double_backward };
 int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int64_t d, int32_t causal, int64_t window) {
   if (fhog::tuning().small >= 0) return fhog::tuning().small;
@@ -264,10 +345,9 @@ int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int64_t d, 
     if (groups <= 256) return d == 64 || uneven ? 2 : 0;
     return d == 64 && uneven && tiles >= 32 ? 2 : 0;
   }
-  if (groups <= 64) return tiles <= (d == 64 ? 128 : 64) ? 4 : 0;
-  if (groups <= 128) return tiles <= 8 ? 2 : tiles <= (d == 64 ? 128 : uneven ? 64 : 32) ? 4 : 0;
-  if (groups <= 256) return tiles <= (d == 64 || uneven ? 64 : 16) ? 2 : 0;
-  return d == 64 && uneven && tiles >= 16 && tiles <= 64 ? 2 : 0;
+  if (groups <= 64) return tiles <= (d == 64 ? 64 : 48) ? 4 : 0;
+  if (groups <= 128) return tiles <= 8 ? 2 : tiles <= (uneven ? (d == 64 ? 64 : groups <= 96 ? 48 : 32) : d == 64 ? 32 : 16) ? 4 : 0;
+  return groups <= 256 && d == 64 && uneven && tiles <= 32 ? 2 : 0;
 }
 int small_waves(Small what, const fhog_attn_args* a) { return small_waves(what, a->batch, a->n_q, a->n_k, a->d, a->causal, a->window); }
 
@@ -519,11 +599,11 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early, n_pass = 4;
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three, n_pass = 3;
   for (int i = 0; i < n_pass; i++) {
-    // split products: passes 3 and 4, the last two, share a launch
-    const bool both = split_products && order[i] == FHOG_PASS_DQ_DDO;
-    const int r = run_pass(args, p, impl, both ? fhog::kPassGrads : order[i], (hipStream_t)hip_stream);
-    if (r != FHOG_OK) return r;
-    if (both) break;
+    const bool last_two = order[i] == FHOG_PASS_DQ_DDO || order[i] == FHOG_PASS_DQ;   // they share a launch
+    const int r = !last_two ? run_pass(args, p, impl, order[i], (hipStream_t)hip_stream)
+                  : split_products ? run_pass(args, p, impl, fhog::kPassGrads, (hipStream_t)hip_stream)
+                                   : run_grads(args, p, order[i], true, (hipStream_t)hip_stream);
+    if (r != FHOG_OK || last_two) return r;
   }
   return FHOG_OK;
 }

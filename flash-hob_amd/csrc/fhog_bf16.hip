@@ -48,24 +48,31 @@ __global__ void __launch_bounds__(256) combine_stats(Params p) {
   if (PASS == 5) p.ws_b[row] = __builtin_fmaf(-a, c, b);
 }
 
-// Finishes pass 3 or 4 that ran split: out0 = scale * sum of the first partial tensor, out1 = sum of the second,
-// rounded to the tensor type. One thread per four columns of a row.
+// Finishes passes 3 and 4 (either or both) that ran split: out0 = scale * sum of the first partial tensor, out1 = sum of the
+// second, rounded to the tensor type. One thread per four columns of a row; the first `first_blocks` workgroups do side a.
+struct Combine {
+  const float* part;
+  int n_split, n;
+  int64_t rows, stride_b, stride_n;
+  uint16_t *out0, *out1;
+};
 template <bool F16, int D>
-__global__ void __launch_bounds__(256) combine_out(const float* part, int n_split, int batch, int n, int64_t stride_b,
-                                                   int64_t stride_n, uint16_t* out0, uint16_t* out1, float scale) {
-  const int64_t rows = (int64_t)batch * n, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) combine_out(Combine a, Combine b, unsigned first_blocks, float scale) {
+  const bool first = blockIdx.x < first_blocks;
+  const Combine c = first ? a : b;
+  const int64_t idx = (int64_t)(blockIdx.x - (first ? 0 : first_blocks)) * 256 + threadIdx.x;
   const int64_t row = idx / (D / 4);
   const int col = (int)(idx % (D / 4)) * 4;
-  if (row >= rows) return;
-  f32x4_t a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < n_split; s++) {
-    const float* ps = part + ((int64_t)s * 2 * rows + row) * D + col;
-    a += *reinterpret_cast<const f32x4_t*>(ps);
-    b += *reinterpret_cast<const f32x4_t*>(ps + rows * D);
+  if (row >= c.rows) return;
+  f32x4_t x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < c.n_split; s++) {
+    const float* ps = c.part + ((int64_t)s * 2 * c.rows + row) * D + col;
+    x += *reinterpret_cast<const f32x4_t*>(ps);
+    y += *reinterpret_cast<const f32x4_t*>(ps + c.rows * D);
   }
-  const int64_t o = (row / n) * stride_b + (row % n) * stride_n + col;
-  *reinterpret_cast<u32x2_t*>(out0 + o) = pack4<F16>(a[0] * scale, a[1] * scale, a[2] * scale, a[3] * scale);
-  *reinterpret_cast<u32x2_t*>(out1 + o) = pack4<F16>(b[0], b[1], b[2], b[3]);
+  const int64_t o = (row / c.n) * c.stride_b + (row % c.n) * c.stride_n + col;
+  *reinterpret_cast<u32x2_t*>(c.out0 + o) = pack4<F16>(x[0] * scale, x[1] * scale, x[2] * scale, x[3] * scale);
+  *reinterpret_cast<u32x2_t*>(c.out1 + o) = pack4<F16>(y[0], y[1], y[2], y[3]);
 }
 
 // Row statistics of the wave's queries handed from one sweep to the next inside a launch that runs several of them for
@@ -451,16 +458,12 @@ __global__ void __launch_bounds__(256, 2) dd_sweep64_bf16(Params p) {
 // products (contraction over the queries), whose A operands are transposing reads of the staged Q-side tiles.
 // At d = 64 everything fits 256 registers, so no S-shaped tile passes through LDS.
 // SUB: 32-query tiles staged and consumed per barrier (see q_sweep_bf16).
-template <bool F16, int D, int MASK, int SUB = 1>
-__global__ void __launch_bounds__(256, 2) k_sweep_bf16(Params p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+template <bool F16, int D, int MASK, int SUB>
+__device__ __forceinline__ void k_sweep_run(const Params& p, char* smem, int bh, int tile, int split) {
   constexpr int KK = D / 16, NC = D / 32, TILE = TS * 2 * D;
   constexpr int STAT = 4 * TS * 4;         // L log2(e), -d, dd, -(dd d + b) of the 32 staged queries
   constexpr int STAGE = 3 * TILE + STAT;   // Q, ddQ, dO tiles, statistics
 
-  int bh, tile, split = 0;
-  if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major, bh, tile, MASK != MASK_NONE)) return;
-  if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -603,6 +606,26 @@ __global__ void __launch_bounds__(256, 2) k_sweep_bf16(Params p) {
     }
 }
 
+// Passes 3 or 7 (workgroups [0, q_blocks)) and 4 (the others) in one launch at d = 64: given the row statistics neither needs the
+// other. Either side may be empty.
+template <bool F16, int D, int QPASS, int MASK, int SUB>
+__global__ void __launch_bounds__(256, 2) grads_bf16(Params p, int q_blocks, bool mixed) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  int bh, tile, split = 0, id = blockIdx.x;
+  const bool pairs = MASK != MASK_NONE && !mixed;   // workgroups that join others of their own sweep on a CU
+  if (first_of_two(q_blocks, mixed, MASK != MASK_NONE, id)) {
+    if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, pairs, id)) return;
+    if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
+    RowChain unused;
+    q_sweep_run<F16, D, QPASS, MASK, 4, SUB, false>(p, smem, bh, tile, split, unused);
+  } else {
+    p.n_split = p.n_split_k, p.part = p.part_k;
+    if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, pairs && q_blocks == 0, id)) return;
+    if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
+    k_sweep_run<F16, D, MASK, SUB>(p, smem, bh, tile, split);
+  }
+}
+
 template <auto Kernel>
 hipError_t launch_sweep(unsigned grid, int smem, hipStream_t s, const Params& p, unsigned threads = 256) {
   const hipError_t e = allow_dynamic_lds<Kernel>(smem);
@@ -615,9 +638,8 @@ template <bool F16, int D, int MASK>
 hipError_t launch_single_d(const Params& p, int pass, hipStream_t s) {
   const int tile = TS * 2 * D, slices = p.batch * p.n_split;
   const unsigned gq = grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, slices);
-  const unsigned gk = grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, slices);
   const bool split = p.n_split > 1;
-  const int64_t rows_q = (int64_t)p.batch * p.n_q, rows_k = (int64_t)p.batch * p.n_k;
+  const int64_t rows_q = (int64_t)p.batch * p.n_q;
   hipError_t e;
   // Passes 2 and 5 with plenty of workgroups run 256 rows per workgroup (8 waves, one workgroup per CU): each staged
   // tile then serves twice the rows, i.e. half the staging loads per row (cfg2: pass 2 -7 %). Pass 1 (two tensors,
@@ -660,40 +682,10 @@ hipError_t launch_single_d(const Params& p, int pass, hipStream_t s) {
               : launch_sweep<q_sweep_bf16<F16, D, 5, MASK>>(gq, 2 * 4 * tile, s, p);
       if (e == hipSuccess && split) hipLaunchKernelGGL(combine_stats<5>, dim3((unsigned)((rows_q + 255) / 256)), dim3(256), 0, s, p);
       break;
-    case FHOG_PASS_DQ_DDO:
-      if constexpr (D == 64) {
-        e = two ? launch_sweep<q_sweep_bf16<F16, D, 3, MASK, 4, S2>>(gq, 2 * S2 * 4 * tile, s, p)
-                : launch_sweep<q_sweep_bf16<F16, D, 3, MASK>>(gq, 2 * 4 * tile, s, p);
-        if (e == hipSuccess && split)
-          hipLaunchKernelGGL((combine_out<F16, D>), dim3((unsigned)((rows_q * (D / 4) + 255) / 256)), dim3(256), 0, s, p.part, p.n_split,
-                             p.batch, p.n_q, p.stride_qb, p.stride_qn, (uint16_t*)p.dq2, (uint16_t*)p.ddo, p.scale);
-      } else {
-        return hipErrorInvalidValue;
-      }
-      break;
     case FHOG_PASS_STAGE1:
       if constexpr (D == 64) {
         if (split) return hipErrorInvalidValue;
         e = launch_sweep<q_stage1_bf16<F16, D, MASK>>(gq, 2 * 4 * tile, s, p);
-      } else {
-        return hipErrorInvalidValue;
-      }
-      break;
-    case FHOG_PASS_DQ:
-      if constexpr (D == 64) {
-        e = two ? launch_sweep<q_sweep_bf16<F16, D, 7, MASK, 4, S2>>(gq, 2 * S2 * 4 * tile, s, p)
-                : launch_sweep<q_sweep_bf16<F16, D, 7, MASK>>(gq, 2 * 4 * tile, s, p);
-      } else {
-        return hipErrorInvalidValue;
-      }
-      break;
-    case FHOG_PASS_DK_DV:
-      if constexpr (D == 64) {
-        e = two ? launch_sweep<k_sweep_bf16<F16, D, MASK, S2>>(gk, 2 * S2 * (3 * tile + 4 * TS * 4), s, p)
-                : launch_sweep<k_sweep_bf16<F16, D, MASK>>(gk, 2 * (3 * tile + 4 * TS * 4), s, p);
-        if (e == hipSuccess && split)
-          hipLaunchKernelGGL((combine_out<F16, D>), dim3((unsigned)((rows_k * (D / 4) + 255) / 256)), dim3(256), 0, s, p.part, p.n_split,
-                             p.batch, p.n_k, p.stride_kb, p.stride_kn, (uint16_t*)p.dk2, (uint16_t*)p.dv2, p.scale);
       } else {
         return hipErrorInvalidValue;
       }
@@ -703,9 +695,35 @@ hipError_t launch_single_d(const Params& p, int pass, hipStream_t s) {
   return e != hipSuccess ? e : hipGetLastError();
 }
 
+template <bool F16, int QPASS, int MASK, int SUB>
+hipError_t launch_grads64(const Params& p, bool q_side, bool k_side, hipStream_t s) {
+  const int tile = TS * 2 * 64, q_lds = 2 * SUB * 4 * tile, k_lds = 2 * SUB * (3 * tile + 4 * TS * 4);
+  const unsigned gq = q_side ? grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split) : 0;
+  const unsigned gk = k_side ? grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split_k) : 0;
+  const hipError_t e = allow_dynamic_lds<grads_bf16<F16, 64, QPASS, MASK, SUB>>(q_lds > k_lds ? q_lds : k_lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((grads_bf16<F16, 64, QPASS, MASK, SUB>), dim3(gq + gk), dim3(256), q_lds > k_lds ? q_lds : k_lds, s, p, (int)gq, mixed_order(gq, gk, p.tile_major && p.tile_major_k));
+  return hipGetLastError();
+}
+
+template <bool F16, int MASK>
+hipError_t launch_grads64_f(const Params& p, int q_pass, bool k_side, hipStream_t s) {
+  const bool two = tuning().stage64 != 0;
+  if (q_pass == FHOG_PASS_DQ) return two ? launch_grads64<F16, 7, MASK, 2>(p, true, k_side, s) : launch_grads64<F16, 7, MASK, 1>(p, true, k_side, s);
+  return two ? launch_grads64<F16, 3, MASK, 2>(p, q_pass != 0, k_side, s) : launch_grads64<F16, 3, MASK, 1>(p, q_pass != 0, k_side, s);
+}
+
+template <bool F16, int D>
+hipError_t launch_combine(const Params& p, bool q_side, bool k_side, hipStream_t s) {
+  const Combine q = {p.part, p.n_split, p.n_q, (int64_t)p.batch * p.n_q, p.stride_qb, p.stride_qn, (uint16_t*)p.dq2, (uint16_t*)p.ddo};
+  const Combine k = {p.part_k, p.n_split_k, p.n_k, (int64_t)p.batch * p.n_k, p.stride_kb, p.stride_kn, (uint16_t*)p.dk2, (uint16_t*)p.dv2};
+  const unsigned bq = q_side ? (unsigned)((q.rows * (D / 4) + 255) / 256) : 0, bk = k_side ? (unsigned)((k.rows * (D / 4) + 255) / 256) : 0;
+  hipLaunchKernelGGL((combine_out<F16, D>), dim3(bq + bk), dim3(256), 0, s, q, k, bq, p.scale);
+  return hipGetLastError();
+}
+
 }  // namespace
 
-hipError_t launch_bf16_pc_pass(const Params& p, int pass, hipStream_t s);
 hipError_t launch_bf16_ddo_pass(const Params& p, int pass, hipStream_t s);
 
 bool bf16_shape_supported(int64_t n_q, int64_t n_k, int64_t d, int causal) {
@@ -716,22 +734,7 @@ bool bf16_shape_supported(int64_t n_q, int64_t n_k, int64_t d, int causal) {
 hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s) {
   if (!bf16_shape_supported(p.n_q, p.n_k, p.d, p.causal)) return hipErrorInvalidValue;
   if (pass == FHOG_PASS_B_DDO || pass == FHOG_PASS_DD_B_DDO) return launch_bf16_ddo_pass(p, pass, s);
-  if (pass == FHOG_PASS_DQ && p.d == 128) return launch_bf16_pc_pass(p, pass, s);
-  // d = 128: passes 3 and 4 need the producer/consumer split to fit the registers; d = 64: single-role kernels throughout
-  if (p.d == 128 && (pass == FHOG_PASS_DQ_DDO || pass == FHOG_PASS_DK_DV)) {
-    const hipError_t e = launch_bf16_pc_pass(p, pass, s);
-    if (e != hipSuccess || p.n_split == 1) return e;
-    const bool kside = pass == FHOG_PASS_DK_DV;
-    const int n = kside ? p.n_k : p.n_q;
-    const dim3 grid((unsigned)(((int64_t)p.batch * n * (128 / 4) + 255) / 256));
-    uint16_t* out0 = (uint16_t*)(kside ? p.dk2 : p.dq2);
-    uint16_t* out1 = (uint16_t*)(kside ? p.dv2 : p.ddo);
-    const int64_t sb = kside ? p.stride_kb : p.stride_qb, sn = kside ? p.stride_kn : p.stride_qn;
-    if (p.f16) hipLaunchKernelGGL((combine_out<true, 128>), grid, dim3(256), 0, s, p.part, p.n_split, p.batch, n, sb, sn, out0, out1, p.scale);
-    else hipLaunchKernelGGL((combine_out<false, 128>), grid, dim3(256), 0, s, p.part, p.n_split, p.batch, n, sb, sn, out0, out1, p.scale);
-    return hipGetLastError();
-  }
-  if (pass != FHOG_PASS_STAGE1 && (pass < FHOG_PASS_DD || pass > FHOG_PASS_DQ || pass == FHOG_PASS_B_DDO)) return hipErrorInvalidValue;
+  if (pass != FHOG_PASS_STAGE1 && pass != FHOG_PASS_DD && pass != FHOG_PASS_B && pass != FHOG_PASS_DD_B) return hipErrorInvalidValue;
   const int mask = mask_mode(p);
 #define FHOG_SINGLE(F, DD)                                                             \
   (mask == MASK_NONE ? launch_single_d<F, DD, MASK_NONE>(p, pass, s)                   \
@@ -739,6 +742,26 @@ hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s) {
   if (p.f16) return p.d == 128 ? FHOG_SINGLE(true, 128) : FHOG_SINGLE(true, 64);
   return p.d == 128 ? FHOG_SINGLE(false, 128) : FHOG_SINGLE(false, 64);
 #undef FHOG_SINGLE
+}
+
+// d = 128: passes 3 and 4 need the producer/consumer split to fit the registers; d = 64: single-role kernels throughout
+hipError_t launch_bf16_grads(const Params& p, int q_pass, bool k_side, hipStream_t s) {
+  if (!bf16_shape_supported(p.n_q, p.n_k, p.d, p.causal)) return hipErrorInvalidValue;
+  hipError_t e;
+  if (p.d == 128) {
+    e = launch_grads_pc(p, q_pass, k_side, s);
+  } else {
+    const int mask = mask_mode(p);
+#define FHOG_GRADS(F)                                                             \
+  (mask == MASK_NONE ? launch_grads64_f<F, MASK_NONE>(p, q_pass, k_side, s)       \
+                     : mask == MASK_CAUSAL ? launch_grads64_f<F, MASK_CAUSAL>(p, q_pass, k_side, s) : launch_grads64_f<F, MASK_BAND>(p, q_pass, k_side, s))
+    e = p.f16 ? FHOG_GRADS(true) : FHOG_GRADS(false);
+#undef FHOG_GRADS
+  }
+  const bool q_parts = q_pass != 0 && p.n_split > 1, k_parts = k_side && p.n_split_k > 1;
+  if (e != hipSuccess || !(q_parts || k_parts)) return e;
+  if (p.f16) return p.d == 128 ? launch_combine<true, 128>(p, q_parts, k_parts, s) : launch_combine<true, 64>(p, q_parts, k_parts, s);
+  return p.d == 128 ? launch_combine<false, 128>(p, q_parts, k_parts, s) : launch_combine<false, 64>(p, q_parts, k_parts, s);
 }
 
 }  // namespace fhog

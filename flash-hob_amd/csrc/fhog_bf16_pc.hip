@@ -339,16 +339,9 @@ __device__ __forceinline__ void consume_dq(const Params& p, char* smem, const St
     }
 }
 
-template <bool F16, int D, int MASK, bool DQ_ONLY = false>
-__global__ void __launch_bounds__(PC_THREADS) q_sweep3_pc(Params p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+template <bool F16, int D, int MASK, bool DQ_ONLY>
+__device__ __forceinline__ void q_run_pc(const Params& p, char* smem, int bh, int tile, int split) {
   using SM = PCSmem<D, false>;
-  constexpr int NC = D / 32;
-
-  // with a split, n_split consecutive "slices" share one (batch*head) slice and take its streamed tiles in turn
-  int bh, tile, split = 0;
-  if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
-  if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: lets the compiler branch on scalars
   const bool producer = wave < 4;
@@ -411,14 +404,10 @@ __device__ __forceinline__ int sop_tr_lane_off(int s, int lane) {
 }
 
 template <bool F16, int D, int MASK>
-__global__ void __launch_bounds__(PC_THREADS) k_sweep_pc(Params p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+__device__ __forceinline__ void k_run_pc(const Params& p, char* smem, int bh, int tile, int split) {
   using SM = PCSmem<D, true>;
   constexpr int NC = D / 32;
 
-  int bh, tile, split = 0;
-  if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major, bh, tile)) return;
-  if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: lets the compiler branch on scalars
   const bool producer = wave < 4;
@@ -609,6 +598,24 @@ __global__ void __launch_bounds__(PC_THREADS) k_sweep_pc(Params p) {
             odv[o] = to_elem<F16>(acc_dv[kb][cl][r]);
           }
         }
+  }
+}
+
+// Passes 3 or 7 (workgroups [0, q_blocks)) and 4 (the others) in one launch: given the row statistics neither needs the other. Either
+// side may be empty. With a split, n_split consecutive "slices" share one (batch*head) slice and take its streamed tiles in turn.
+template <bool F16, int D, int MASK, bool DQ_ONLY>
+__global__ void __launch_bounds__(PC_THREADS) grads_pc(Params p, int q_blocks, bool mixed) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  int bh, tile, split = 0, id = blockIdx.x;
+  if (first_of_two(q_blocks, mixed, false, id)) {
+    if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, false, id)) return;
+    if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
+    q_run_pc<F16, D, MASK, DQ_ONLY>(p, smem, bh, tile, split);
+  } else {
+    p.n_split = p.n_split_k, p.part = p.part_k;
+    if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, false, id)) return;
+    if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
+    k_run_pc<F16, D, MASK>(p, smem, bh, tile, split);
   }
 }
 
@@ -829,26 +836,14 @@ hipError_t launch_attn_bwd_k_pc_d(const AttnParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <bool F16, int D, int MASK>
-hipError_t launch_pc_d(const Params& p, int pass, hipStream_t s) {
-  const dim3 block(PC_THREADS);
-  hipError_t e;
-  if (pass == FHOG_PASS_DQ) {
-    const int smem = PCSmem<D, false>::TOTAL;
-    e = allow_dynamic_lds<q_sweep3_pc<F16, D, MASK, true>>(smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((q_sweep3_pc<F16, D, MASK, true>), dim3(grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch)), block, smem, s, p);
-  } else if (pass == FHOG_PASS_DQ_DDO) {
-    const int smem = PCSmem<D, false>::TOTAL;
-    e = allow_dynamic_lds<q_sweep3_pc<F16, D, MASK>>(smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((q_sweep3_pc<F16, D, MASK>), dim3(grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split)), block, smem, s, p);
-  } else {
-    const int smem = PCSmem<D, true>::TOTAL;
-    e = allow_dynamic_lds<k_sweep_pc<F16, D, MASK>>(smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_sweep_pc<F16, D, MASK>), dim3(grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split)), block, smem, s, p);
-  }
+template <bool F16, int D, int MASK, bool DQ_ONLY>
+hipError_t launch_grads_pc_d(const Params& p, bool q_side, bool k_side, hipStream_t s) {
+  constexpr int smem = PCSmem<D, false>::TOTAL > PCSmem<D, true>::TOTAL ? PCSmem<D, false>::TOTAL : PCSmem<D, true>::TOTAL;
+  const hipError_t e = allow_dynamic_lds<grads_pc<F16, D, MASK, DQ_ONLY>>(smem);
+  if (e != hipSuccess) return e;
+  const unsigned gq = q_side ? grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split) : 0;
+  const unsigned gk = k_side ? grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split_k) : 0;
+  hipLaunchKernelGGL((grads_pc<F16, D, MASK, DQ_ONLY>), dim3(gq + gk), dim3(PC_THREADS), smem, s, p, (int)gq, mixed_order(gq, gk, p.tile_major && p.tile_major_k));
   return hipGetLastError();
 }
 
@@ -865,14 +860,14 @@ hipError_t launch_attn_bwd_k_pc(const AttnParams& p, hipStream_t s) {
 #undef FHOG_BWDK
 }
 
-hipError_t launch_bf16_pc_pass(const Params& p, int pass, hipStream_t s) {
+hipError_t launch_grads_pc(const Params& p, int q_pass, bool k_side, hipStream_t s) {
   const int mask = mask_mode(p);
-#define FHOG_PC(F, DD)                                                          \
-  (mask == MASK_NONE ? launch_pc_d<F, DD, MASK_NONE>(p, pass, s)                \
-                     : mask == MASK_CAUSAL ? launch_pc_d<F, DD, MASK_CAUSAL>(p, pass, s) : launch_pc_d<F, DD, MASK_BAND>(p, pass, s))
+#define FHOG_PC_Q(F, M) (q_pass == FHOG_PASS_DQ ? launch_grads_pc_d<F, 128, M, true>(p, true, k_side, s) : launch_grads_pc_d<F, 128, M, false>(p, q_pass != 0, k_side, s))
+#define FHOG_PC(F) (mask == MASK_NONE ? FHOG_PC_Q(F, MASK_NONE) : mask == MASK_CAUSAL ? FHOG_PC_Q(F, MASK_CAUSAL) : FHOG_PC_Q(F, MASK_BAND))
   if (p.d != 128) return hipErrorInvalidValue;   // d = 64 runs on the single-role kernels
-  return p.f16 ? FHOG_PC(true, 128) : FHOG_PC(false, 128);
+  return p.f16 ? FHOG_PC(true) : FHOG_PC(false);
 #undef FHOG_PC
+#undef FHOG_PC_Q
 }
 
 }  // namespace fhog

@@ -52,6 +52,9 @@ struct Params {
   // Workgroup ids of one XCD enumerate its tiles (decode_block). tile_major: the slices that share the XCD advance
   // through their tiles together instead of one slice after the other (the default with a mask).
   int32_t tile_major;
+  // The same three of the K-tiled side where both share a launch (launch_bf16_grads)
+  int32_t n_split_k, tile_major_k;
+  float* part_k;
 };
 
 // Launch choices that can be overridden for experiments through the environment variable FHOG_TUNE, a comma-separated
@@ -116,7 +119,9 @@ constexpr int kPassGrads = -1;   // launch_split_pass: passes 3 and 4 in one lau
 // Launchers implemented in the kernel translation units. Each returns hipGetLastError().
 hipError_t launch_rowdot(const Params& p, int dtype, hipStream_t s);                 // pass 0
 hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products
-hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);              // passes 1..4, bf16 MFMA
+hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);              // statistics sweeps (1, 2, 5, 6, 8) and the one-launch stage 1, 16-bit MFMA
+hipError_t launch_bf16_grads(const Params& p, int q_pass, bool k_side, hipStream_t s);   // pass 3 or 7 (0: none) beside pass 4
+hipError_t launch_grads_pc(const Params& p, int q_pass, bool k_side, hipStream_t s);     // the sweeps of that at d = 128
 hipError_t launch_attn_bf16(const AttnParams& p, int which, hipStream_t s);         // 0 forward, 1 dQ, 2 dK and dV
 hipError_t launch_attn_split(const AttnParams& p, int dtype, bool backward, hipStream_t s); // split products (fp32 tensors, d = 32)
 hipError_t launch_attn_bwd_k_pc(const AttnParams& p, hipStream_t s);                // dK and dV at d = 128 (producer/consumer)

@@ -23,8 +23,9 @@ FORMS = [(b, n_q, n_k, d, dtype, causal, window, pad)
              (2, 97, 640, "float16", "bottom_right", None, 0), (2, 300, 400, "bfloat16", "bottom_right", 200, 8),
              (1, 33, 1000, "bfloat16", "bottom_right", 17, 0), (1, 1030, 1030, "float16", True, None, 0), (4, 1000, 63, "bfloat16", False, None, 0)]]
 # shapes whose default lies on either side of the lines of the rule, and what it picks for (forward, first backward, double-backward)
-PICKS = [((16, 256, 64, True), (4, 4, 4)), ((33, 256, 64, False), (4, 2, 2)), ((64, 200, 128, False), (2, 0, 2)), ((2, 1024, 128, False), (4, 4, 4)),
-         ((64, 128, 64, False), (4, 2, 2)), ((8, 1024, 128, False), (4, 4, 4)), ((1, 4224, 128, False), (4, 4, 0)), ((256, 100, 64, True), (0, 0, 0))]
+PICKS = [((16, 256, 64, True), (4, 4, 4)), ((33, 256, 64, False), (4, 2, 0)), ((33, 256, 64, True), (4, 2, 2)), ((64, 200, 128, False), (2, 0, 0)),
+         ((2, 1024, 128, False), (4, 4, 4)), ((64, 128, 64, False), (4, 2, 2)), ((8, 1024, 128, True), (4, 4, 4)), ((8, 1024, 128, False), (4, 4, 0)),
+         ((1, 4224, 128, False), (4, 4, 0)), ((256, 100, 64, True), (0, 0, 0))]
 
 _CHILD = r"""
 import sys, torch
