@@ -307,19 +307,17 @@ __device__ __forceinline__ bool in_limits(int r, int lo, int hi) {  // r: regist
   return x >= lo && x <= hi;
 }
 
-// XCD-aware 1-D grid. Workgroup ids go round-robin over the 8 XCDs (id % 8 = XCD), each with its own L2.
-// With 8 or more (batch*head) slices every slice is pinned to one XCD, so that all its tiles stream the slice's
-// other side through ONE L2. With fewer slices a slice is spread over 8/batch (rounded down to a power of two)
-// XCDs, tiles interleaved, so that a single long head still fills the chip.
-//   xcds_per_slice XS = 8, 4, 2, 2, 1, ... for batch = 1, 2, 3, 4, >= 5;  slices per round = 8 / XS
-__host__ __device__ __forceinline__ int xcds_per_slice(int batch) { return batch >= 5 ? 1 : batch >= 3 ? 2 : batch == 2 ? 4 : 8; }
+// XCD-aware 1-D grid. Workgroup ids go round-robin over the 8 XCDs (id % 8 = XCD), each with its own L2. Whole (batch*head) slices go
+// to one XCD each, so that all tiles of a slice stream its other side through ONE L2; the tiles of the batch % 8 slices that are left
+// are dealt out over all eight, each XCD a stretch of them or, tile-major, every eighth tile (one, two or four slices: to 8, 4 or 2 XCDs
+// each). They used to go to one XCD each when there were 5 or more in all: 5 slices left three XCDs idle, 9 gave one XCD twice the work.
+// Forward | first backward | double-backward, us, so -> dealt out: bf16 d = 64 causal 6 x 4096 38 | 131 | 196 -> 29 | 107 | 167, no mask
+// 12 x 4096 89 | 240 | 635 -> 85 | 217 | 527; d = 128 no mask 9 x 4096 125 | 354 | 905 -> 125 | 352 | 760; fp32 d = 64 no mask 9 x 4096
+// 371 | 1358 | 3380 -> 360 | 1070 | 2734. With 25 slices or more the difference is small: bf16 d = 64 causal 36 x 2048 44 | 103 | 245 ->
+// 43 | 100 | 227.
 // number of workgroups to launch for n_tiles tiles per slice
-__host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) {
-  const int xs = xcds_per_slice(batch), per_round = 8 / xs;
-  const int rounds = (batch + per_round - 1) / per_round, tiles_per_xcd = (n_tiles + xs - 1) / xs;
-  return (unsigned)(rounds * 8 * tiles_per_xcd);
-}
-// Returns false when the id falls beyond the last slice or tile.
+__host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) { return (unsigned)(((int64_t)n_tiles * batch + 7) / 8 * 8); }
+// Returns false when the id falls beyond the last tile.
 // tile_major: the slices that share an XCD advance through their tiles together (ids enumerate tile 0 of every
 // slice, then tile 1 of every slice, ...) instead of one slice after the other. With a mask the work of a tile grows
 // with its index; heaviest-first over ALL workgroups of the XCD is what lets the light tiles at the end fill the
@@ -332,22 +330,42 @@ __host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) {
 // without -> with: bf16 causal 64 x 1024, d = 32: dQ 25.8 -> 21.9, passes 3 and 4 89.5 -> 83.1; Hessian-vector product 199.4 -> 195.9,
 // fp16 48 x 1537, d = 64 347 -> 342, training step bf16 32 x 4096, d = 128 622 -> 615. With one workgroup per CU
 // (producer/consumer kernels) the ids 32.. start as CUs fall free and heaviest-first is the right order for them too.
-__device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs = false, int id = blockIdx.x) {
-  const int xcd = id & 7;
+__host__ __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs, int id) {
+  const int xcd = id & 7, whole = batch >> 3, left = batch & 7;   // slices of this XCD alone, and those that are dealt out
   int slot = id >> 3;
-  const int xs = xcds_per_slice(batch), per_round = 8 / xs, tiles_per_xcd = (n_tiles + xs - 1) / xs;
-  const int rounds = (batch + per_round - 1) / per_round;   // slices this XCD (group) serves
   if (pairs && tile_major && slot >= 32) {
-    const int last = min(64, rounds * tiles_per_xcd) - 1;
+    const int last = min(64, (int)(((uint32_t)n_tiles * (uint32_t)batch + 7) / 8)) - 1;
     if (slot <= last) slot = 32 + last - slot;
   }
-  const int r = tile_major ? slot % rounds : slot / tiles_per_xcd;
-  const int t = tile_major ? slot / rounds : slot % tiles_per_xcd;
-  bh = xcd / xs + per_round * r;
-  tile = t * xs + xcd % xs;
-  if (bh >= batch || tile >= n_tiles) return false;
+  if (tile_major) {
+    // ceil(t batch / 8) slots come before tile t of the XCD's slices: t `whole` of them and ceil(t left / 8) dealt ones, so that none
+    // of the latter comes after lighter tiles
+    const uint32_t t = 8u * slot / (uint32_t)batch, o = slot - ((t * (uint32_t)batch + 7) >> 3);
+    bh = xcd + 8 * (int)o, tile = (int)t;
+    if ((int)o >= whole) {
+      const int dealt = (int)((t * left + 7) >> 3), u = 8 * dealt + xcd;
+      if (left == 1 || left == 2 || left == 4) bh = xcd * left >> 3, tile = dealt * (8 / left) + (xcd & (8 / left - 1));
+      else tile = u / left, bh = u % left;
+      bh += 8 * whole;
+    }
+    if (tile >= n_tiles) return false;
+  } else {
+    const int s = slot / n_tiles;
+    bh = xcd + 8 * s, tile = slot - s * n_tiles;
+    if (s >= whole) {
+      const int from = (int)((uint32_t)(xcd * left) * (uint32_t)n_tiles >> 3), to = (int)((uint32_t)(xcd * left + left) * (uint32_t)n_tiles >> 3);
+      const int u = from + slot - whole * n_tiles;
+      if (u >= to) return false;
+      bh = u / n_tiles, tile = u - bh * n_tiles;
+      bh += 8 * whole;
+    }
+  }
   if (heavy_first) tile = n_tiles - 1 - tile;
   return true;
+}
+
+__device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs = false) {
+  return decode_block(n_tiles, batch, heavy_first, tile_major, bh, tile, pairs, blockIdx.x);
 }
 
 // Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of

@@ -1,0 +1,50 @@
+"""The order in which workgroups take the tiles of a launch (decode_block, first_of_two), compiled for the host: every tile of every slice
+is handed out exactly once, whatever the numbers of tiles and slices, and the tiles of an XCD come heaviest first where that is asked for."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+_PROGRAM = r"""
+#include <cstdio>
+#include <set>
+#include <utility>
+#include "fhog_bf16_util.h"
+using namespace fhog::bf16k;
+int main() {
+  const int tiles[] = {1, 2, 3, 4, 5, 7, 8, 13, 16, 31, 32, 33, 63, 64, 65, 130}, slices[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 25, 36, 63, 64, 100};
+  for (int T : tiles) for (int B : slices) for (int mode = 0; mode < 8; mode++) {
+    const bool major = mode & 1, pairs = mode & 2, two = mode & 4;
+    const unsigned grid = grid_blocks(T, B);
+    std::set<std::pair<int, int>> seen[2];
+    int last_tile[8] = {};
+    for (unsigned i = 0; i < (two ? 2 * grid : grid); i++) {
+      int id = (int)i, bh, tile;
+      const int side = two && !first_of_two((int)grid, mode & 1, pairs, id);
+      if (!decode_block(T, B, false, major, bh, tile, pairs && !two, id)) continue;
+      if (bh < 0 || bh >= B || tile < 0 || tile >= T || !seen[side].insert({bh, tile}).second) return printf("%d tiles, %d slices, mode %d, id %u\n", T, B, mode, i), 1;
+      // tile by tile: nothing follows lighter tiles of the XCD's own slices
+      if (major && !pairs && !two && tile < last_tile[i % 8]) return printf("order: %d tiles, %d slices, id %u\n", T, B, i), 1;
+      if (bh < B / 8 * 8) last_tile[i % 8] = tile;
+    }
+    for (int side = 0; side <= (two ? 1 : 0); side++)
+      if ((int)seen[side].size() != T * B) return printf("%d tiles, %d slices, mode %d: %zu\n", T, B, mode, seen[side].size()), 1;
+  }
+  return 0;
+}
+"""
+
+
+@pytest.mark.skipif(not shutil.which("hipcc") and not Path("/opt/rocm/bin/hipcc").exists(), reason="needs hipcc")
+def test_every_tile_once(tmp_path):
+    src = tmp_path / "order.hip"
+    src.write_text(_PROGRAM)
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    exe = tmp_path / "order"
+    r = subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{ROOT}/include", f"-I{ROOT}/flash-hob_amd/csrc", str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout
