@@ -27,23 +27,53 @@ COMMANDS = __doc__.split("cd <repo>\n")[1].split("\n\n``bench.py``")[0]
 
 
 def short(name):
-    k = name.replace("void fhog::(anonymous namespace)::", "").replace("(fhog::Params)", "").replace("(fhog::AttnParams)", "")
+    k = re.sub(r"\(fhog::\w*Params[^)]*\)$", "", name.replace("void fhog::(anonymous namespace)::", ""))
     if "rowdot" in k:
         k = "rowdot_kernel"
     return k
 
 
+def labelled(rows):
+    """[(label, row)] of the library's kernels in a trace. The gradient sweeps over queries and keys share a launch (`grads_*`): the
+    launches with the most workgroups are passes 3 + 4 (7 + 4 without ddO), smaller ones are pass 3 alone, which
+    `bench.py --profile-only` runs too."""
+    rows = [r for r in rows if "fhog" in r["Kernel_Name"]]
+    size = lambda r: int(r.get("Grid_Size") or r["Grid_Size_X"])
+    most = {}
+    for r in rows:
+        most[r["Kernel_Name"]] = max(size(r), most.get(r["Kernel_Name"], 0))
+    out = []
+    for r in rows:
+        k = short(r["Kernel_Name"])
+        if k.startswith("grads_"):
+            dq_only = re.match(r"grads_pc<\w+, \d+, \d, true>", k) or re.match(r"grads_bf16<\w+, \d+, 7,", k)
+            k += " 7+4" if dq_only else " 3+4" if size(r) == most[r["Kernel_Name"]] else " 3"
+        out.append((k, r))
+    return out
+
+
+def durations(path):
+    """{kernel: row of figures} of a kernel trace, from the launches themselves."""
+    t = collections.defaultdict(list)
+    for k, r in labelled(csv.DictReader(open(path))):
+        t[k].append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
+    total = sum(map(sum, t.values()))
+    return {k: {"Calls": len(v), "AverageNs": sum(v) / len(v), "MinNs": min(v), "MaxNs": max(v), "TotalDurationNs": sum(v),
+                "Percentage": 100 * sum(v) / total} for k, v in t.items()}
+
+
 def pass_of(kernel):
-    """Pass id of a double-backward kernel (fhog_hip.h), 'fwd' / 'bwd_q' / 'bwd_k' for the first-order ones, else None."""
+    """Pass id of a double-backward kernel (fhog_hip.h), '3+4' / '7+4' where two share a launch, 'fwd' / 'bwd_q' / 'bwd_k' for the first-order ones, else None."""
     m = re.match(r"q_sweep_bf16<\w+, \d+, (\d)", kernel)
     if m:
         return int(m.group(1))
     m = re.match(r"q_sweep_ddo<\w+, \d+, \d, (\w+)[,>]", kernel)
     if m:
         return 6 if m.group(1) == "true" else 8
-    if re.match(r"q_sweep3_pc<\w+, \d+, \d, true>", kernel):
-        return 7
-    for prefix, p in (("dd_sweep64_bf16", 1), ("q_stage1_bf16", 9), ("q_sweep3_pc", 3), ("k_sweep_pc", 4), ("k_sweep_bf16", 4), ("rowdot", 0), ("attn_fwd", "fwd"),
+    if kernel.startswith("grads_"):
+        p = kernel.rsplit(" ", 1)[1]
+        return 3 if p == "3" else p
+    for prefix, p in (("dd_sweep64_bf16", 1), ("q_stage1_bf16", 9), ("rowdot", 0), ("attn_fwd", "fwd"),
                       ("attn_bwd_q", "bwd_q"), ("attn_bwd_k", "bwd_k")):
         if kernel.startswith(prefix):
             return p
@@ -57,6 +87,7 @@ def algorithmic_mib(w, p):
     table = {0: (2 * qt, rv), 1: (4 * qt + 2 * kt + rv, 2 * rv), 2: (3 * qt + 4 * kt + 3 * rv, rv),
              5: (4 * qt + 4 * kt + rv, 3 * rv), 6: (3 * qt + 4 * kt + 3 * rv, qt + rv), 7: (3 * qt + 4 * kt + 4 * rv, qt),
              8: (4 * qt + 4 * kt + rv, qt + 3 * rv), 9: (4 * qt + 4 * kt + rv, 2 * qt + 3 * rv), 3: (3 * qt + 4 * kt + 4 * rv, 2 * qt), 4: (3 * qt + 4 * kt + 4 * rv, 2 * kt),
+             "3+4": (3 * qt + 4 * kt + 4 * rv, 2 * qt + 2 * kt), "7+4": (3 * qt + 4 * kt + 4 * rv, qt + 2 * kt),
              "fwd": (qt + 2 * kt, qt + rv), "bwd_q": (2 * qt + 2 * kt + 2 * rv, qt), "bwd_k": (2 * qt + 2 * kt + 2 * rv, 2 * kt)}
     return table.get(p)
 
@@ -64,11 +95,11 @@ def algorithmic_mib(w, p):
 def counters(path):
     """{kernel: {counter: mean value per dispatch}}; 'calib' = the last three dispatches of the streaming torch.add."""
     a = collections.defaultdict(lambda: collections.defaultdict(list))
-    for r in csv.DictReader(open(path)):
-        k = r["Kernel_Name"]
-        if "fhog" in k:
-            a[short(k)][r["Counter_Name"]].append(float(r["Counter_Value"]))
-        elif "elementwise" in k:
+    rows = list(csv.DictReader(open(path)))
+    for k, r in labelled(rows):
+        a[k][r["Counter_Name"]].append(float(r["Counter_Value"]))
+    for r in rows:
+        if "elementwise" in r["Kernel_Name"]:
             a["calib"][r["Counter_Name"]].append(float(r["Counter_Value"]))
     for c in a.get("calib", {}):
         a["calib"][c] = a["calib"][c][-3:]
@@ -83,13 +114,13 @@ def compare(w, variants):
     P("|---|---|---|---|---|---|---|---|---|")
     for label, root in variants:
         root = Path(root)
-        kt = {short(r["Name"]): r for r in csv.DictReader(open(root / "prof_kt" / "kt_kernel_stats.csv")) if "fhog" in r["Name"]}
+        kt = durations(root / "prof_kt" / "kt_kernel_trace.csv")
         fe = counters(root / "prof_fetch" / "f_counter_collection.csv")
         sq = counters(root / "prof_sq" / "s_counter_collection.csv")
         sf = 262144 / fe["calib"]["FETCH_SIZE"]
         for k in sorted(kt, key=lambda k: str(pass_of(k))):
             p = pass_of(k)
-            if not isinstance(p, int) or p == 0 or k not in sq or int(kt[k]["Calls"]) < 4:
+            if p in (None, 0, "fwd", "bwd_q", "bwd_k") or k not in sq or int(kt[k]["Calls"]) < 4:
                 continue
             d = sq[k]
             cyc, ns = d["SQ_BUSY_CYCLES"] / 32, float(kt[k]["AverageNs"])
@@ -144,27 +175,27 @@ def main():
     if args.compare:
         return compare(w, [tuple(c.rsplit("@", 1)) for c in args.compare])
     root = Path(args.root)
-    kt = {short(r["Name"]): r for r in csv.DictReader(open(root / "prof_kt" / "kt_kernel_stats.csv")) if "fhog" in r["Name"]}
+    kt = durations(root / "prof_kt" / "kt_kernel_trace.csv")
     fe = counters(root / "prof_fetch" / "f_counter_collection.csv")
     wr = counters(root / "prof_write" / "w_counter_collection.csv")
     sq = counters(root / "prof_sq" / "s_counter_collection.csv")
-    order = sorted(kt, key=lambda k: -float(kt[k]["TotalDurationNs"]) if "TotalDurationNs" in kt[k] else -float(kt[k]["Percentage"]))
+    order = sorted(kt, key=lambda k: -kt[k]["TotalDurationNs"])
     P = print
     P(f"# rocprofv3 summary: double-backward kernels, workload {w.name} (B={w.B} H={w.H} N_Q={w.n_q} N_K={w.n_k} d={w.d} "
       f"{'causal' if w.causal else 'non-causal'} {str(w.dtype).replace('torch.', '')})\n")
     P("Commands (from the repository root on one MI355X):\n")
     P(COMMANDS.replace("W=cfg2_bf16_causal_4096_d128", f"W={w.name}"))
     P("""
-`bench.py --profile-only` runs the timed loop of the default schedule (pass 5, then 3 and 4), then three calls each of the
-others (four-pass: passes 1 and 2 instead of pass 5; ddO early: `q_sweep_ddo<.., true>` = pass 6 and
-`q_sweep3_pc<.., true>` = pass 7 replace passes 2 and 3; three sweeps: `q_sweep_ddo<.., false>` = pass 8, then pass 7),
+`bench.py --profile-only` runs the timed loop of the default schedule (pass 5, then 3 and 4 in one launch), three launches of pass 3 alone, then
+three calls each of the others (four-pass: passes 1 and 2 instead of pass 5; ddO early: `q_sweep_ddo<.., true>` = pass 6, then
+passes 7 and 4 in one launch; three sweeps: `q_sweep_ddo<.., false>` = pass 8, then 7 and 4),
 then three calls of the first-order kernels on the same tensors, then a streaming `torch.add` used to calibrate the byte
 counters. Template arguments of the kernels: `<fp16?, d, [pass,] mask mode[, waves per workgroup | variant]>` (mask mode
 1 = square causal mask).
 
-## kernel-trace --stats (kt_kernel_stats.csv), library kernels only
+## kernel trace (kt_kernel_trace.csv), library kernels only
 
-| kernel | calls | avg ns | min ns | max ns | % of GPU time in the run |
+| kernel | calls | avg ns | min ns | max ns | % of the library's GPU time in the run |
 |---|---|---|---|---|---|""")
     for k in order:
         r = kt[k]
@@ -188,7 +219,7 @@ the counters read FETCH_SIZE={cf:.1f}, WRITE_SIZE={cw:.1f} -> scale factors {sf:
         ratio = f"{(f + wv) / sum(alg):.2f}" if alg else ""
         alg_s = f"{alg[0]:.1f} + {alg[1]:.1f}" if alg else ""
         P(f"| {k} | {fe[k]['FETCH_SIZE']:.1f} | {wr[k]['WRITE_SIZE']:.1f} | {f:.1f} | {wv:.1f} | {alg_s} | {ratio} |")
-        if isinstance(pass_of(k), int) and str(pass_of(k)) not in traffic:
+        if pass_of(k) not in (None, "fwd", "bwd_q", "bwd_k") and str(pass_of(k)) not in traffic:
             traffic[str(pass_of(k))] = int((f + wv) * 2 ** 20)
     P(f"\n<!-- traffic_bytes: {json.dumps(traffic, sort_keys=True)} -->")
     P("""
