@@ -330,6 +330,14 @@ hipError_t launch_fwd(const AttnParams& p, hipStream_t s) {
   return launch_ws<T, D, MODE_FWD, MASK, 1>(p, s);
 }
 
+template <typename T, int D, int MODE, int MASK>
+hipError_t launch_side(const AttnParams& p, int waves, hipStream_t s) {
+  if constexpr (lds_bytes<T, D, MODE, 4>() <= 160 * 1024) {
+    if (waves == 4) return launch_ws<T, D, MODE, MASK, 4>(p, s);
+  }
+  return waves >= 2 ? launch_ws<T, D, MODE, MASK, 2>(p, s) : launch_ws<T, D, MODE, MASK, 1>(p, s);
+}
+
 // dQ and dK, dV side by side fill CUs for each other, as passes 3 and 4 do in fhog_split.hip, and the rule for waves on the same rows is of
 // the same kind. The price is the row sums d, which the sweep for dK, dV then takes once per key block: nothing at d = 32, 3 to 9 % on
 // fp32 tensors of d = 64 and 128, whose launches of full rounds (256 workgroups each) go one after the other. First backward, us, two
@@ -342,6 +350,10 @@ template <typename T, int D, int MASK>
 hipError_t launch_bwd(const AttnParams& p, hipStream_t s) {
   const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
   const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  if (sizeof(T) * D < 512 && lopsided(p.n_q, p.n_k, MASK != MASK_NONE ? (int64_t)p.window : (int64_t)p.n_q + p.n_k) && groups > 64) {   // as in fhog_split.hip
+    const hipError_t e = launch_side<T, D, MODE_BWD_Q, MASK>(p, waves_of_side(g_q, p.n_k), s);
+    return e != hipSuccess ? e : launch_side<T, D, MODE_BWD_K, MASK>(p, waves_of_side(g_k, p.n_q), s);
+  }
   if constexpr (lds_bytes<T, D, MODE_BWD_K, 4>() <= 160 * 1024) {
     if (groups <= (triangle && p.n_k >= 1024 ? (D == 32 ? 256 : 128) : D == 32 ? 128 : 64)) return launch_bwd_ws<T, D, MASK, 4>(p, s);
   }

@@ -3,8 +3,8 @@
 // leaves the chip:
 //   pass 1  d_i, dd_i   Q-tiled   (fhog/triton_bwdbwd.py:580, 185-211)   q_sweep_bf16<PASS=1>
 //   pass 2  b_i         Q-tiled   (fhog/triton_bwdbwd.py:217-251)        q_sweep_bf16<PASS=2>
-//   pass 3  dQ2, ddO    Q-tiled   (fhog/triton_bwdbwd.py:257-313)        d=64: q_sweep_bf16<PASS=3>; d=128: fhog_bf16_pc.hip
-//   pass 4  dK2, dV2    K-tiled   (fhog/triton_bwdbwd.py:467-535)        d=64: k_sweep_bf16;         d=128: fhog_bf16_pc.hip
+//   pass 3  dQ2, ddO    Q-tiled   (fhog/triton_bwdbwd.py:257-313)        d=64: grads_bf16; d=128: grads_pc (fhog_bf16_pc.hip)
+//   pass 4  dK2, dV2    K-tiled   (fhog/triton_bwdbwd.py:467-535)        in the same launch
 //
 // Fused statistics sweep (PASS = 5, what the default schedule runs): b_i = sum_j P (E + ddS (dP - d)) - dd_i sum_j P dP
 // needs dd_i only as a factor of a row sum, so dd and b come out of ONE sweep with the five products of pass 2

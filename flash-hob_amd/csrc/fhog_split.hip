@@ -482,6 +482,13 @@ hipError_t launch_grads_most(const Params& p, int sides, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename T, int D, int MASK>
+hipError_t launch_grads_side(const Params& p, int side, int waves, hipStream_t s) {
+  return waves == 4   ? launch_grads_most<T, D, MASK, 4>(p, side, s)
+         : waves == 2 ? launch_grads_most<T, D, MASK, 2>(p, side, s)
+                      : launch_grads_most<T, D, MASK, 1>(p, side, s);
+}
+
 // Passes 3 and 4 side by side are faster than one after the other whatever the size: their workgroups fill CUs for each other where
 // one pass has too few, and the light end of a triangle goes under the other pass. Four waves on the same rows while that gives one
 // workgroup per CU, two as long as the workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. Double-backward, us,
@@ -490,10 +497,21 @@ hipError_t launch_grads_most(const Params& p, int sides, hipStream_t s) {
 //                 32 x 1024 435 -> 375 | 318 | 296, 32 x 2048 980 -> 1190 | 1034 | 950; no mask 32 x 2048 1808 -> 2186 | 1937 | 1793
 //   fp32 d = 128  (one wave at all sizes, LDS) 2 x 256 234 -> 133; causal 16 x 2048 2104 -> 1440; 32 x 2048 2383 -> 2381
 //   bf16 d = 32   2 x 256 20 -> 13 | - | -; causal 16 x 1024 99 -> 59 | 47 | 56, 32 x 1024 114 -> 119 | 90 | 96, 64 x 1024 127 -> 218 | 160 | 121
+// A side that is far shorter than the other has few workgroups with a long stream each, which nothing fills up: the two sides go
+// apart then, each with as many waves on the same rows as it needs by itself. Hessian-vector products (here and in fhog_attn_split.hip),
+// us, one launch -> apart, by how many times as many rows one side streams: bf16 d = 32 3.1 times (16 x 512 x 1600) 142 -> 147, 5 times
+// (8 x 512 x 2560) 178 -> 149, the other way round 194 -> 147, 30 times (4 x 200 x 6000) 413 -> 243; fp32 d = 64 3.1 times 370 -> 393,
+// 5 times 740 -> 609, 8 times 897 -> 874. fp32 d = 128, which has one wave at all sizes, 8 times 2260 -> 2373: not there.
 template <typename T, int D, int MASK>
 hipError_t launch_grads(const Params& p, int sides, hipStream_t s) {
-  const int64_t groups = (int64_t)((p.n_q + 127) / 128 + (p.n_k + 127) / 128) * p.batch;
+  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
   const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  if (sizeof(T) * D < 512 && lopsided(p.n_q, p.n_k, MASK != MASK_NONE ? (int64_t)p.window : (int64_t)p.n_q + p.n_k) && groups > 64) {
+    hipError_t e = hipSuccess;
+    if (sides & 1) e = launch_grads_side<T, D, MASK>(p, 1, waves_of_side(g_q, p.n_k), s);
+    if (e == hipSuccess && (sides & 2)) e = launch_grads_side<T, D, MASK>(p, 2, waves_of_side(g_k, p.n_q), s);
+    return e;
+  }
   if (groups <= 64 || (D == 32 && triangle && groups <= 128 && p.n_k >= 1024)) return launch_grads_most<T, D, MASK, 4>(p, sides, s);
   if (groups < (triangle ? (D == 32 ? 512 : 257) : 160)) return launch_grads_most<T, D, MASK, 2>(p, sides, s);
   return launch_grads_most<T, D, MASK, 1>(p, sides, s);

@@ -159,3 +159,13 @@ def test_first_backward_on_split_products(shape, dtype, d):
     for name, g, w in zip(("dq", "dk", "dv"), got, want):
         assert torch.isfinite(g.float()).all()
         assert normalised_max_error(g[sel], w) < {torch.float32: 1e-4, torch.bfloat16: 2e-2, torch.float16: 2.5e-3}[dtype], name
+
+
+# one side streams four times as many rows as the other and the two have more than 64 groups of 128 rows: each sweep runs by itself;
+# and just inside of both lines
+@pytest.mark.parametrize("shape", [(11, 40, 600, False, None), (11, 600, 40, False, None), (33, 130, 520, False, None), (33, 130, 519, False, None),
+                                   (10, 40, 600, False, None), (40, 70, 300, "bottom_right", None), (9, 1000, 100, False, None)])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 32)])
+def test_sweeps_of_lopsided_launches(shape, dtype, d):
+    test_passes_3_and_4_in_one_launch(shape, dtype, d)
+    test_first_backward_on_split_products(shape, dtype, d)
