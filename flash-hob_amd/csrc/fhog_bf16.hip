@@ -284,7 +284,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_bf16(Params 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // with a split, n_split consecutive "slices" share one (batch*head) slice and take its streamed tiles in turn
   int bh, tile, split = 0;
-  if (!decode_block((p.n_q + 32 * NW - 1) / (32 * NW), p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && NW == 4)) return;
+  if (!decode_block<MASK>((p.n_q + 32 * NW - 1) / (32 * NW), p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && NW == 4)) return;
   if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
   RowChain unused;
   q_sweep_run<F16, D, PASS, MASK, NW, SUB, false>(p, smem, bh, tile, split, unused);
@@ -298,7 +298,7 @@ template <bool F16, int D, int MASK>
 __global__ void __launch_bounds__(256, 2) q_stage1_bf16(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int bh, tile;
-  if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
   RowChain chain;
   q_sweep_run<F16, D, 1, MASK, 4, 1, true>(p, smem, bh, tile, 0, chain);   // every sweep ends on a barrier: the ring is free
   q_sweep_run<F16, D, 2, MASK, 4, 1, true>(p, smem, bh, tile, 0, chain);
@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(256, 2) dd_sweep64_bf16(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int ROWS = 256, NT = 2, TILE = TS * 2 * D, STAGE = NT * TILE, KK = D / 16;
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -614,13 +614,13 @@ __global__ void __launch_bounds__(256, 2) grads_bf16(Params p, int q_blocks, boo
   int bh, tile, split = 0, id = blockIdx.x;
   const bool pairs = MASK != MASK_NONE && !mixed;   // workgroups that join others of their own sweep on a CU
   if (first_of_two(q_blocks, mixed, MASK != MASK_NONE, id)) {
-    if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, pairs, id)) return;
+    if (!decode_block<MASK>((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, pairs, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     RowChain unused;
     q_sweep_run<F16, D, QPASS, MASK, 4, SUB, false>(p, smem, bh, tile, split, unused);
   } else {
     p.n_split = p.n_split_k, p.part = p.part_k;
-    if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, pairs && q_blocks == 0, id)) return;
+    if (!decode_block<MASK>((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, pairs && q_blocks == 0, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     k_sweep_run<F16, D, MASK, SUB>(p, smem, bh, tile, split);
   }

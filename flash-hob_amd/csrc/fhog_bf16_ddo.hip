@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_ddo(Params p
   constexpr int NT = 4, TILE = TS * 2 * D, STAGE = NT * TILE, KK = D / 16, NC = D / 32, ROWS = 32 * NW;
 
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && NW == 4)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && NW == 4)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: lets the compiler branch on scalars
   const int n = lane & 31, h = lane >> 5;

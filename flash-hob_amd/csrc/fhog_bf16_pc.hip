@@ -608,12 +608,12 @@ __global__ void __launch_bounds__(PC_THREADS) grads_pc(Params p, int q_blocks, b
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int bh, tile, split = 0, id = blockIdx.x;
   if (first_of_two(q_blocks, mixed, false, id)) {
-    if (!decode_block((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, false, id)) return;
+    if (!decode_block<MASK>((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, false, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     q_run_pc<F16, D, MASK, DQ_ONLY>(p, smem, bh, tile, split);
   } else {
     p.n_split = p.n_split_k, p.part = p.part_k;
-    if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, false, id)) return;
+    if (!decode_block<MASK>((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, false, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     k_run_pc<F16, D, MASK>(p, smem, bh, tile, split);
   }
@@ -693,7 +693,7 @@ __global__ void __launch_bounds__(PC_THREADS) attn_bwd_k_pc(AttnParams p) {
   constexpr int NC = D / 32;
 
   int bh, tile;
-  if (!decode_block((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch, false, p.tile_major_k != 0, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch, false, p.tile_major_k != 0, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool producer = wave < 4;

@@ -309,12 +309,14 @@ __device__ __forceinline__ bool in_limits(int r, int lo, int hi) {  // r: regist
 
 // XCD-aware 1-D grid. Workgroup ids go round-robin over the 8 XCDs (id % 8 = XCD), each with its own L2. Whole (batch*head) slices go
 // to one XCD each, so that all tiles of a slice stream its other side through ONE L2; the tiles of the batch % 8 slices that are left
-// are dealt out over all eight, each XCD a stretch of them or, tile-major, every eighth tile (one, two or four slices: to 8, 4 or 2 XCDs
-// each). They used to go to one XCD each when there were 5 or more in all: 5 slices left three XCDs idle, 9 gave one XCD twice the work.
+// are dealt out over all eight, each XCD a stretch of them or, tile-major and under a mask, every eighth tile (one, two or four slices: to 8, 4 or
+// 2 XCDs each). They used to go to one XCD each when there were 5 or more in all: 5 slices left three XCDs idle, 9 gave one XCD twice the work.
 // Forward | first backward | double-backward, us, so -> dealt out: bf16 d = 64 causal 6 x 4096 38 | 131 | 196 -> 29 | 107 | 167, no mask
 // 12 x 4096 89 | 240 | 635 -> 85 | 217 | 527; d = 128 no mask 9 x 4096 125 | 354 | 905 -> 125 | 352 | 760; fp32 d = 64 no mask 9 x 4096
 // 371 | 1358 | 3380 -> 360 | 1070 | 2734. With 25 slices or more the difference is small: bf16 d = 64 causal 36 x 2048 44 | 103 | 245 ->
-// 43 | 100 | 227.
+// 43 | 100 | 227. A stretch keeps an L2 to few slices, but under a mask one XCD would get the heavy end of a slice and another the light one: slices of
+// 16384 rows or more, stretches -> every eighth tile, causal: double-backward d = 128 2 x 30280 6443 -> 4087, 1 x 31258 3829 -> 2400, fp32 d = 64
+// 1 x 17018 5495 -> 3487; first backward d = 64 1 x 29336 1401 -> 765, d = 128 3 x 22609 2106 -> 1304; windows of 1 to 9 % of the rows within 2 %.
 // number of workgroups to launch for n_tiles tiles per slice
 __host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) { return (unsigned)(((int64_t)n_tiles * batch + 7) / 8 * 8); }
 // Returns false when the id falls beyond the last tile.
@@ -330,6 +332,7 @@ __host__ __forceinline__ unsigned grid_blocks(int n_tiles, int batch) { return (
 // without -> with: bf16 causal 64 x 1024, d = 32: dQ 25.8 -> 21.9, passes 3 and 4 89.5 -> 83.1; Hessian-vector product 199.4 -> 195.9,
 // fp16 48 x 1537, d = 64 347 -> 342, training step bf16 32 x 4096, d = 128 622 -> 615. With one workgroup per CU
 // (producer/consumer kernels) the ids 32.. start as CUs fall free and heaviest-first is the right order for them too.
+template <int MASK = MASK_NONE>
 __host__ __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs, int id) {
   const int xcd = id & 7, whole = batch >> 3, left = batch & 7;   // slices of this XCD alone, and those that are dealt out
   int slot = id >> 3;
@@ -353,10 +356,18 @@ __host__ __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bo
     const int s = slot / n_tiles;
     bh = xcd + 8 * s, tile = slot - s * n_tiles;
     if (s >= whole) {
-      const int from = (int)((uint32_t)(xcd * left) * (uint32_t)n_tiles >> 3), to = (int)((uint32_t)(xcd * left + left) * (uint32_t)n_tiles >> 3);
-      const int u = from + slot - whole * n_tiles;
-      if (u >= to) return false;
-      bh = u / n_tiles, tile = u - bh * n_tiles;
+      const int dealt = slot - whole * n_tiles;   // of the dealt tiles, those before this one on the XCD
+      if (MASK != MASK_NONE && (left == 1 || left == 2 || left == 4)) {
+        bh = xcd * left >> 3, tile = dealt * (8 / left) + (xcd & (8 / left - 1));
+      } else if (MASK != MASK_NONE) {
+        const int u = 8 * dealt + xcd;
+        tile = u / left, bh = u - tile * left;
+      } else {
+        const int from = (int)((uint32_t)(xcd * left) * (uint32_t)n_tiles >> 3), to = (int)((uint32_t)(xcd * left + left) * (uint32_t)n_tiles >> 3);
+        if (from + dealt >= to) return false;
+        bh = (from + dealt) / n_tiles, tile = from + dealt - bh * n_tiles;
+      }
+      if (bh >= left || tile >= n_tiles) return false;
       bh += 8 * whole;
     }
   }
@@ -364,8 +375,9 @@ __host__ __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bo
   return true;
 }
 
+template <int MASK = MASK_NONE>
 __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_first, bool tile_major, int& bh, int& tile, bool pairs = false) {
-  return decode_block(n_tiles, batch, heavy_first, tile_major, bh, tile, pairs, blockIdx.x);
+  return decode_block<MASK>(n_tiles, batch, heavy_first, tile_major, bh, tile, pairs, blockIdx.x);
 }
 
 // Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of

@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256, 2) small_stats(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 4, TILE = TS * 2 * D, STAGE = NT * TILE, NBUF = n_buffers<D, NT>;
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;   // row group of the wave, and which of its streamed tiles it takes
@@ -187,7 +187,7 @@ template <bool F16, int D, int MASK, int W>
 __device__ __forceinline__ void grads_q(const Params& p, char* smem) {
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 4, TILE = TS * 2 * D, STAGE = NT * TILE, NBUF = n_buffers<D, NT>;
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;   // row group of the wave, and which of its streamed tiles it takes
@@ -245,7 +245,7 @@ template <bool F16, int D, int MASK, int W>
 __device__ __forceinline__ void grads_k(const Params& p, char* smem, int id) {
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 3, TILE = TS * 2 * D, STAGE = grads_k_stage<D>, NBUF = n_buffers<D, 4>;
   int bh, tile;
-  if (!decode_block((p.n_k + ROWS - 1) / ROWS, p.batch, false, p.tile_major, bh, tile, false, id)) return;
+  if (!decode_block<MASK>((p.n_k + ROWS - 1) / ROWS, p.batch, false, p.tile_major, bh, tile, false, id)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;
@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(256, 2) small_fwd(AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 2, TILE = TS * 2 * D, STAGE = NT * TILE, NBUF = n_buffers<D, NT>;
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, MASK != MASK_NONE, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, MASK != MASK_NONE, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;   // row group of the wave, and which of its streamed tiles it takes
@@ -381,7 +381,7 @@ template <bool F16, int D, int MASK, int W>
 __device__ __forceinline__ void bwd_q(const AttnParams& p, char* smem) {
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 2, TILE = TS * 2 * D, STAGE = NT * TILE, NBUF = n_buffers<D, NT>;
   int bh, tile;
-  if (!decode_block((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major_q != 0, bh, tile)) return;
+  if (!decode_block<MASK>((p.n_q + ROWS - 1) / ROWS, p.batch, MASK != MASK_NONE, p.tile_major_q != 0, bh, tile)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;   // row group of the wave, and which of its streamed tiles it takes
@@ -434,7 +434,7 @@ template <bool F16, int D, int MASK, int W>
 __device__ __forceinline__ void bwd_k(const AttnParams& p, char* smem, int id) {
   constexpr int KK = D / 16, NC = D / 32, ROWS = TS * WAVES / W, NT = 3, TILE = TS * 2 * D, STAGE = bwd_k_stage<D>, NBUF = bwd_k_buffers<D>;
   int bh, tile;
-  if (!decode_block((p.n_k + ROWS - 1) / ROWS, p.batch, false, p.tile_major_k != 0, bh, tile, false, id)) return;
+  if (!decode_block<MASK>((p.n_k + ROWS - 1) / ROWS, p.batch, false, p.tile_major_k != 0, bh, tile, false, id)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave / W, ws = wave % W;

@@ -1,5 +1,6 @@
 """The order in which workgroups take the tiles of a launch (decode_block, first_of_two), compiled for the host: every tile of every slice
-is handed out exactly once, whatever the numbers of tiles and slices, and the tiles of an XCD come heaviest first where that is asked for."""
+is handed out exactly once, whatever the numbers of tiles and slices, the tiles of an XCD come heaviest first where that is asked for, and under a mask
+no XCD has more work than the others."""
 import shutil
 import subprocess
 from pathlib import Path
@@ -37,10 +38,34 @@ int main() {
 """
 
 
-@pytest.mark.skipif(not shutil.which("hipcc") and not Path("/opt/rocm/bin/hipcc").exists(), reason="needs hipcc")
-def test_every_tile_once(tmp_path):
+# the work of a tile grows with its index; slices in tile-major order and one after the other. Whole slices weigh the same on every XCD;
+# the dealt ones are taken by turns, which leaves two of the heaviest tiles between the XCDs at most
+_BALANCE = r"""
+#include <cstdio>
+#include "fhog_bf16_util.h"
+using namespace fhog::bf16k;
+int main() {
+  const int tiles[] = {8, 31, 64, 128, 143, 300};
+  for (int T : tiles) for (int B = 1; B <= 20; B++) for (int mode = 0; mode < 4; mode++) {
+    long work[8] = {}, lo = 1L << 60, hi = 0;
+    int count = 0;
+    for (unsigned i = 0; i < grid_blocks(T, B); i++) {
+      int bh, tile;
+      if (!decode_block<MASK_CAUSAL>(T, B, mode & 2, mode & 1, bh, tile, false, (int)i)) continue;
+      if (bh < 0 || bh >= B || tile < 0 || tile >= T) return printf("range: %d tiles, %d slices, mode %d, id %u\n", T, B, mode, i), 1;
+      work[i & 7] += tile + 1, count++;
+    }
+    for (long w : work) lo = w < lo ? w : lo, hi = w > hi ? w : hi;
+    if (count != T * B || hi - lo > 2 * T) return printf("%d tiles, %d slices, mode %d: %d tiles, work %ld to %ld\n", T, B, mode, count, lo, hi), 1;
+  }
+  return 0;
+}
+"""
+
+
+def _run(tmp_path, program):
     src = tmp_path / "order.hip"
-    src.write_text(_PROGRAM)
+    src.write_text(program)
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     exe = tmp_path / "order"
     r = subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{ROOT}/include", f"-I{ROOT}/flash-hob_amd/csrc", str(src), "-o", str(exe)],
@@ -48,3 +73,16 @@ def test_every_tile_once(tmp_path):
     assert r.returncode == 0, r.stderr[-2000:]
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
+
+
+_needs_hipcc = pytest.mark.skipif(not shutil.which("hipcc") and not Path("/opt/rocm/bin/hipcc").exists(), reason="needs hipcc")
+
+
+@_needs_hipcc
+def test_every_tile_once(tmp_path):
+    _run(tmp_path, _PROGRAM)
+
+
+@_needs_hipcc
+def test_xcds_have_the_same_work_under_a_mask(tmp_path):
+    _run(tmp_path, _BALANCE)
