@@ -1,0 +1,194 @@
+// Rules by which a launch is laid out: splits of the streamed side, order of the workgroups, kernels for small launches. Host code and nothing else.
+#pragma once
+#include <math.h>
+
+#include "fhog_common.h"
+
+namespace fhog {
+namespace rules {
+
+// kernel-side mask parameters: key j is visible to query i iff 0 <= i + off - j < win
+inline void mask_params(int32_t causal, int64_t window, int64_t n_q, int64_t n_k, int32_t* off, int32_t* win) {
+  *off = causal == FHOG_MASK_BOTTOM_RIGHT ? (int32_t)(n_k - n_q) : 0;
+  const int64_t reach = n_q + n_k;  // a window this long hides nothing
+  *win = (int32_t)((window == 0 || window > reach) ? reach : window);
+}
+
+
+// ---- splitting the streamed side of small launches (16-bit kernels) -------------------------------------------
+// Bytes of d | dd | b, rounded up so that what follows stays 16-byte aligned.
+inline size_t stats_bytes(const fhog_bwdbwd_args* a) { return ((size_t)3 * a->batch * a->n_q * sizeof(float) + 15) & ~(size_t)15; }
+// fp32 partial results one split of a pass writes
+inline size_t split_bytes(const fhog_bwdbwd_args* a, int pass) {
+  if (pass == FHOG_PASS_DQ_DDO) return (size_t)2 * a->batch * a->n_q * a->d * sizeof(float);
+  if (pass == FHOG_PASS_DK_DV) return (size_t)2 * a->batch * a->n_k * a->d * sizeof(float);
+  return (size_t)3 * a->batch * a->n_q * sizeof(float);
+}
+// Splits a pass would like: enough workgroups for two per CU, every split keeping at least 8 streamed tiles.
+inline int wanted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
+  if (impl != FHOG_IMPL_BF16 || pass == FHOG_PASS_D || pass > FHOG_PASS_DD_B) return 1;   // passes 6-8 never split
+  const bool kside = pass == FHOG_PASS_DK_DV;
+  const int64_t groups = ((kside ? a->n_k : a->n_q) + 127) / 128 * a->batch;
+  const int64_t streamed = ((kside ? a->n_q : a->n_k) + 31) / 32;
+  int s = 1;
+  if (!tuning().split) return s;
+  while (groups * s < 512 && s < 16 && streamed / (2 * s) >= 8) s *= 2;
+  return s;
+}
+// ... and what of that the workspace has room for
+inline int granted_split(const fhog_bwdbwd_args* a, int impl, int pass) {
+  int s = wanted_split(a, impl, pass);
+  const size_t have = a->ws_bytes > 0 ? (size_t)a->ws_bytes : 0;
+  while (s > 1 && stats_bytes(a) + (size_t)s * split_bytes(a, pass) > have) s /= 2;
+  return s;
+}
+
+// Workgroups (128 stationary rows) of a slice with a visible pair, and the tiles they visit
+struct Work {
+  int64_t live = 0, longest = 0, sum = 0;
+};
+inline Work work_of(const fhog_bwdbwd_args* a, const Params& p, bool kside) {
+  Work w;
+  const int64_t n_sta = kside ? a->n_k : a->n_q, n_str = kside ? a->n_q : a->n_k;
+  for (int64_t r0 = 0; r0 < n_sta; r0 += 128) {   // fewer than 512 workgroups on the side that would split
+    int64_t lo = 0, hi = n_str;   // streamed rows visible to [r0, r0 + 128)
+    if (p.causal) {
+      const int64_t first = kside ? r0 - p.mask_off : r0 + p.mask_off - p.window + 1;
+      const int64_t last = kside ? r0 + 127 - p.mask_off + p.window - 1 : r0 + 127 + p.mask_off;
+      lo = first > 0 ? first : 0, hi = last + 1 < n_str ? last + 1 : n_str;
+    }
+    if (lo >= hi) continue;
+    const int64_t tiles = (hi - 1) / 32 - lo / 32 + 1;
+    w.live++, w.sum += tiles, w.longest = tiles > w.longest ? tiles : w.longest;
+  }
+  return w;
+}
+
+// Splits that pass 3 or 4 runs with on its own, of `most`. At d = 128 they keep one workgroup on a CU: what matters there is rounds of 256
+// workgroups times the tiles of one, under the mask, and what the partial results cost. In steps of one tile (1.9 us): a
+// workgroup needs about 4 to start and to store, combining 2 plus its bytes at 5 TB/s (14.5 us for 66 MB, 8 for 33).
+// Where the work of the workgroups differs (causal) the longest one and the average load bound the launch.
+// bf16 16 x 1000 x 3001, window 700, us, as many splits as give 512 workgroups -> this rule: pass 3 with 4 -> 2 splits 49.2 + 14.5
+// (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
+inline int split_up_to(int most, const fhog_bwdbwd_args* a, const Params& p, int pass) {
+  if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
+  const Work w = work_of(a, p, pass == FHOG_PASS_DK_DV);
+  if (w.live == 0) return 1;
+  int best = 1;
+  double best_cost = 0;
+  for (int s = 1; s <= most; s *= 2) {
+    const double rounds = (double)((w.live * a->batch * s + 255) / 256), mean = (double)w.sum / (double)w.live;
+    const double alone = (double)w.longest / s + 4, load = rounds * (mean / s + 4);
+    double cost = alone > load ? alone : load;
+    if (s > 1) cost += 2 + (double)s * split_bytes(a, pass) / (5e6 * 1.9);
+    if (s == 1 || cost < best_cost) best = s, best_cost = cost;
+  }
+  return best;
+}
+
+inline int launch_split_of(const fhog_bwdbwd_args* a, const Params& p, int impl, int pass) {
+  return split_up_to(granted_split(a, impl, pass), a, p, pass);
+}
+
+// When the last of n_a jobs of length a and then n_b jobs of length b ends on 256 CUs, each taken by the CU that is free first
+inline double makespan(int64_t n_a, double a, int64_t n_b, double b) {
+  struct { int64_t cus; double load; } g[32] = {{256, 0}};   // CUs with the same load
+  int groups = 1;
+  double end = 0;
+  for (int side = 0; side < 2; side++) {
+    const double length = side ? b : a;
+    for (int64_t n = side ? n_b : n_a; n > 0;) {
+      int m = 0;
+      for (int i = 1; i < groups; i++)
+        if (g[i].load < g[m].load) m = i;
+      if (groups == 1 && n >= 512) {   // whole rounds
+        g[0].load += length * (double)(n / 256), n %= 256;
+      } else if (n >= g[m].cus || groups == 32) {
+        n -= g[m].cus, g[m].load += length;
+      } else {
+        g[groups++] = {n, g[m].load + length};
+        g[m].cus -= n, n = 0;
+      }
+    }
+  }
+  for (int i = 0; i < groups; i++) end = g[i].load > end ? g[i].load : end;
+  return end;
+}
+
+// Splits of the two sides where they share a launch, out of those that either would like alone and the workspace has room for. The same
+// reckoning in steps of a tile (d = 128 1.9 us, 64: 1.1), over the workgroups of both.
+inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, int* s_k) {
+  const int most_q = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DQ_DDO), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
+  *s_q = *s_k = 1;
+  const int64_t have = a->ws_bytes - (int64_t)stats_bytes(a);
+  if ((most_q == 1 && most_k == 1) || have <= 0) return;
+  const Work q = work_of(a, p, false), k = work_of(a, p, true);
+  if (q.live == 0 || k.live == 0) return;
+  const double fixed = a->d == 128 ? 4 : 2, tile_us = a->d == 128 ? 1.9 : 1.1;
+  const int64_t bytes_q = (int64_t)split_bytes(a, FHOG_PASS_DQ_DDO), bytes_k = (int64_t)split_bytes(a, FHOG_PASS_DK_DV);
+  double best = 0;
+  for (int x = 1; x <= most_q; x *= 2)
+    for (int y = 1; y <= most_k; y *= 2) {
+      const int64_t part = (x > 1 ? x * bytes_q : 0) + (y > 1 ? y * bytes_k : 0);
+      if (part > have) continue;
+      const double lq = (double)q.sum / (double)q.live / x + fixed, lk = (double)k.sum / (double)k.live / y + fixed;
+      const int64_t nq = q.live * a->batch * x, nk = k.live * a->batch * y;
+      const double longest = (double)(q.longest / x > k.longest / y ? q.longest / x : k.longest / y) + fixed;
+      double cost = makespan(nq, lq, nk, lk);   // pass 3 comes first
+      if (longest > cost) cost = longest;
+      if (part > 0) cost += (4 + (double)part / 2.5e6) / tile_us;   // a launch, and the partial results written and read
+      if ((x == 1 && y == 1) || cost < best) best = cost, *s_q = x, *s_k = y;
+    }
+}
+
+// Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all
+// of them first) balances the end of a launch; from 16384 stationary rows on a slice alone has tiles enough for that
+// and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x
+// instead of 4-10x, sweeps b, 3 and 4 0.1-3 % faster, the dd sweep with its three workgroups per CU 4 % slower).
+inline bool slice_order(const fhog_bwdbwd_args* a, const Params& p, int64_t rows) { return tuning().order < 0 && p.causal && rows >= 16384; }
+
+// ---- small launches of the 16-bit kernels (fhog_small.hip) ------------------------------------------------------
+// Waves that a launch puts on the same 32 stationary rows: 4 or 2, or 0 for the kernels with four waves on 128 rows.
+// One workgroup fits a CU: 4 waves as long as that is one round of the 256 CUs (first order, and short streams: 2 waves up to one or two
+// rounds where the other kernels would leave CUs idle). `groups` counts 128-row groups of all sides that share a launch, `tiles` the streamed
+// tiles of one. A triangle (or a window) is in favour of small workgroups, whose work evens out; the double-backward's other
+// kernels split long streams over workgroups (workspace) and win them back there.
+// us, other kernels -> 4 waves | 2 waves, square shapes, bf16:
+//   forward           d = 64: 64 x 256 9.2 -> 6.5 | 7.4; 8 x 2048 36.7 -> 19.5 | 25.2; causal 32 x 1000 23 -> 16.5 | 17.6
+//                     d = 128: 16 x 512 15.7 -> 9.5 | 13.2; 64 x 256 11.0 -> 13.5 | 10.4; 1 x 8192 163 -> 64 | 118
+//   first backward    d = 64: 8 x 256 19.0 -> 7.3 | 9.7; 32 x 256 19.4 -> 12.5 | 10.5; 16 x 1024 48 -> 42 | 37; 1 x 8192 303 -> 114 | 152
+//                     d = 128: 8 x 256 25 -> 12 | 18; causal 32 x 512 39 -> 41 | 35, no mask 38 -> 51 | 43
+//   double-backward   d = 64: 4 x 256 24.1 -> 14.7 | 18.9; 64 x 256 27.2 -> 41 | 30; causal 8 x 1024 46.6 -> 33.8 | 45; 1 x 4096 59 -> 78 | 142
+//                     d = 128: 8 x 256 33.3 -> 22.8 | 30.5; 16 x 512 49.7 -> 49.2 | 49.7; causal 3 x 1536 69 -> 62 | 101; 1 x 2048 55 -> 72 | 127
+enum class Small { forward, backward, double_backward };
+inline int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int64_t d, int32_t causal, int64_t window) {
+  if (tuning().small >= 0) return tuning().small;
+  const int64_t g_q = (n_q + 127) / 128 * batch, g_k = (n_k + 127) / 128 * batch;
+  // from 256 groups of a side on the kernels with 128 rows fill the GPU
+  if (g_q >= 256 || (what != Small::forward && g_k >= 256)) return 0;
+  const int64_t off = causal == FHOG_MASK_BOTTOM_RIGHT ? n_k - n_q : 0;
+  const bool windowed = causal != FHOG_MASK_NONE && window > 0 && window < n_k;
+  const bool uneven = causal != FHOG_MASK_NONE && (windowed || 2 * off <= n_k);
+  const int64_t streamed = what == Small::forward || n_k > n_q ? n_k : n_q;
+  const int64_t tiles = ((windowed && window + 63 < streamed ? window + 63 : streamed) + 31) / 32;
+  if (what == Small::forward) {
+    if (g_q <= 64) return 4;
+    if (g_q <= 128) return d == 64 || (uneven && tiles >= 32) ? 4 : 2;
+    if (tiles < 32) return 0;
+    return d == 64 ? (uneven ? 4 : 2) : (uneven ? 2 : 0);
+  }
+  const int64_t groups = g_q + g_k;
+  if (what == Small::backward) {
+    if (groups <= 64) return 4;
+    if (groups <= 128) return tiles <= 8 ? 2 : 4;
+    if (groups <= 256) return d == 64 || uneven ? 2 : 0;
+    return d == 64 && uneven && tiles >= 32 ? 2 : 0;
+  }
+  if (groups <= 64) return tiles <= (d == 64 ? 64 : 48) ? 4 : 0;
+  if (groups <= 128) return tiles <= 8 ? 2 : tiles <= (uneven ? (d == 64 ? 64 : groups <= 96 ? 48 : 32) : d == 64 ? 32 : 16) ? 4 : 0;
+  return groups <= 256 && d == 64 && uneven && tiles <= 32 ? 2 : 0;
+}
+inline int small_waves(Small what, const fhog_attn_args* a) { return small_waves(what, a->batch, a->n_q, a->n_k, a->d, a->causal, a->window); }
+
+}  // namespace rules
+}  // namespace fhog
