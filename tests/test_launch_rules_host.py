@@ -1,0 +1,68 @@
+"""The rules by which a launch is laid out (fhog_rules.h), compiled for the host and asked about shapes."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+pytestmark = pytest.mark.skipif(not Path(HIPCC).exists(), reason="needs hipcc")
+
+_PROGRAM = r"""
+#include <chrono>
+#include <cstdio>
+#include <cstring>
+#include "fhog_rules.h"
+namespace fhog {
+const Tuning& tuning() { static const Tuning t; return t; }
+}
+using namespace fhog;
+int main() {
+  char what[32];
+  fhog_bwdbwd_args a = {};
+  long long batch, n_q, n_k, d, window, ws;
+  int mask;
+  while (scanf("%31s %lld %lld %lld %lld %d %lld %lld", what, &batch, &n_q, &n_k, &d, &mask, &window, &ws) == 8) {
+    a.batch = batch, a.n_q = n_q, a.n_k = n_k, a.d = d, a.causal = mask, a.window = window, a.ws_bytes = ws;
+    Params p = {};
+    p.batch = (int)batch, p.n_q = (int)n_q, p.n_k = (int)n_k, p.d = (int)d, p.causal = mask != 0;
+    rules::mask_params(mask, window, n_q, n_k, &p.mask_off, &p.window);
+    if (!strcmp(what, "joint")) {
+      int x, y;
+      double best = 1e9;
+      for (int i = 0; i < 10; i++) {
+        const auto t0 = std::chrono::steady_clock::now();
+        rules::joint_splits(&a, p, &x, &y);
+        const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
+        best = us < best ? us : best;
+      }
+      printf("%d %d %.3f\n", x, y, best);
+    }
+  }
+}
+"""
+NONE, CAUSAL, BOTTOM_RIGHT = range(3)
+PLENTY = 1 << 40
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rules")
+    (folder / "rules.hip").write_text(_PROGRAM)
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O2", "-std=c++17", f"-I{ROOT}/include", f"-I{ROOT}/flash-hob_amd/csrc",
+                        str(folder / "rules.hip"), "-o", str(folder / "rules")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+    def one(*query):
+        r = subprocess.run([str(folder / "rules")], input=" ".join(map(str, query)) + "\n", capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return [float(x) for x in r.stdout.split()]
+    return one
+
+
+@pytest.mark.parametrize("mask", [NONE, BOTTOM_RIGHT])
+def test_host_time_does_not_grow_with_the_tensors(ask, mask):
+    """2^24 keys beside few queries, which would split: the rule looks at no more tiles than for 2^13 keys."""
+    short, long = (ask("joint", 1, 1024, n_k, 64, mask, 0, PLENTY)[2] for n_k in (1 << 13, 1 << 24))
+    assert long < 10 * short + 5, (short, long)
