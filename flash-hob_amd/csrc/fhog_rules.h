@@ -129,8 +129,58 @@ inline double makespan(int64_t n_a, double a, int64_t n_b, double b) {
   return end;
 }
 
+// The same with two workgroups on a CU: together they do one step of length 1 (a half each), a workgroup without company takes `alone` for it.
+// A CU takes its second workgroup when every other one has its first.
+inline double makespan_two(int64_t n_a, double a, int64_t n_b, double b, double alone) {
+  struct Cus { int64_t cus; double first, second; } g[64] = {{256, 0, 0}};   // CUs and what is left of their workgroups
+  const double kNothing = 1e-9;
+  int groups = 1;
+  double t = 0;
+  int64_t n[2] = {n_a, n_b};
+  const double length[2] = {a, b};
+  for (int side = 0; side < 2; side++)   // whole rounds: one to three are left of each side
+    if (n[side] >= 4 * 512) t += 2 * length[side] * (double)(n[side] / 512 - 3), n[side] -= (n[side] / 512 - 3) * 512;
+  for (int steps = 0; steps < 256; steps++) {
+    for (int place = 0; place < 2; place++)
+      for (int i = 0; i < groups && (n[0] > 0 || n[1] > 0); i++) {
+        if (place == 0 ? g[i].first > 0 : g[i].first <= 0 || g[i].second > 0) continue;
+        const int side = n[0] > 0 ? 0 : 1;
+        if (n[side] < g[i].cus) {
+          if (groups == 64) { n[side] = 0; continue; }
+          g[groups++] = {g[i].cus - n[side], g[i].first, g[i].second};
+          g[i].cus = n[side];
+        }
+        n[side] -= g[i].cus;
+        (place == 0 ? g[i].first : g[i].second) = length[side];
+      }
+    double next = 0;   // until the first of the workgroups ends
+    for (int i = 0; i < groups; i++) {
+      if (g[i].first <= 0) continue;
+      const double d = g[i].second > 0 ? 2 * (g[i].first < g[i].second ? g[i].first : g[i].second) : alone * g[i].first;
+      if (next == 0 || d < next) next = d;
+    }
+    if (next == 0) break;
+    t += next;
+    for (int i = 0; i < groups; i++) {
+      if (g[i].first <= 0) continue;
+      const double done = g[i].second > 0 ? next / 2 : next / alone;
+      g[i].first = g[i].first - done > kNothing ? g[i].first - done : 0;
+      if (g[i].second > 0) g[i].second = g[i].second - done > kNothing ? g[i].second - done : 0;
+      if (g[i].first == 0) g[i].first = g[i].second, g[i].second = 0;
+    }
+    for (int i = 0; i < groups; i++)   // CUs that have the same left
+      for (int k = groups - 1; k > i; k--)
+        if (fabs(g[i].first - g[k].first) < kNothing && fabs(g[i].second - g[k].second) < kNothing) g[i].cus += g[k].cus, g[k] = g[--groups];
+  }
+  return t;
+}
+
 // Splits of the two sides where they share a launch, out of those that either would like alone and the workspace has room for. The same
-// reckoning in steps of a tile (d = 128 1.9 us, 64: 1.1), over the workgroups of both.
+// reckoning in steps of a tile, over the workgroups of both. At d = 128 a CU has one workgroup and a tile takes 1.9 us; at d = 64 two, and
+// a tile takes 0.87 us in company and 1.25 times that alone: 256 workgroups there leave every CU half used. us, splits 1 | 1, 2 | 2, 4 | 4, 8 | 8:
+// fp16 d = 64 no mask 1 x 8192 369, 232, 203, 211; 1 x 16384 798, 727, 738, 750; 2 x 4096 178, 123, 115, 123; 4 x 4096 208, 203, 211, 229; 8 x 2048 110, 114,
+// 123, 142; causal 1 x 16384 683, 611, 499, 439; 2 x 8192 344, 244, 225, 245; 8 x 2048 99, 81, 85, 113. Splits of one side alone at 1 x 16384: 2 | 1 950.
+// Over 640 shapes of 1 to 64 slices with 16 to 20000 rows, against the best pair of each: 2.2 % too slow with one workgroup to a CU -> 0.9 %.
 inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, int* s_k) {
   const int most_q = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DQ_DDO), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
   *s_q = *s_k = 1;
@@ -138,7 +188,8 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, i
   if ((most_q == 1 && most_k == 1) || have <= 0) return;
   const Work q = work_of(a, p, false), k = work_of(a, p, true);
   if (q.live == 0 || k.live == 0) return;
-  const double fixed = a->d == 128 ? 4 : 2, tile_us = a->d == 128 ? 1.9 : 1.1;
+  const bool two = a->d == 64;
+  const double fixed = two ? 2 : 4, tile_us = two ? 0.87 : 1.9, alone = 1.25;
   const int64_t bytes_q = (int64_t)split_bytes(a, FHOG_PASS_DQ_DDO), bytes_k = (int64_t)split_bytes(a, FHOG_PASS_DK_DV);
   double best = 0;
   for (int x = 1; x <= most_q; x *= 2)
@@ -147,10 +198,18 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, i
       if (part > have) continue;
       const double lq = q.sum / q.live / x + fixed, lk = k.sum / k.live / y + fixed;
       const int64_t nq = llround(q.live * (double)(a->batch * x)), nk = llround(k.live * (double)(a->batch * y));
-      const double longest = (double)(q.longest / x > k.longest / y ? q.longest / x : k.longest / y) + fixed;
-      double cost = makespan(nq, lq, nk, lk);   // pass 3 comes first
+      double cost, longest;   // pass 3 comes first
+      if (two) {
+        longest = (double)((q.longest + x - 1) / x > (k.longest + y - 1) / y ? (q.longest + x - 1) / x : (k.longest + y - 1) / y) + fixed;
+        longest *= nq + nk <= 256 ? alone : 1.5;   // it comes early and has company for half of its way
+        cost = makespan_two(nq, lq, nk, lk, alone);
+      } else {
+        longest = (double)(q.longest / x > k.longest / y ? q.longest / x : k.longest / y) + fixed;
+        cost = makespan(nq, lq, nk, lk);
+      }
       if (longest > cost) cost = longest;
       if (part > 0) cost += (4 + (double)part / 2.5e6) / tile_us;   // a launch, and the partial results written and read
+      if (two && p.causal && q.groups == k.groups && x != y) cost *= 1.08;   // the sweeps do not take turns (mixed_order)
       if ((x == 1 && y == 1) || cost < best) best = cost, *s_q = x, *s_k = y;
     }
 }

@@ -66,3 +66,13 @@ def test_host_time_does_not_grow_with_the_tensors(ask, mask):
     """2^24 keys beside few queries, which would split: the rule looks at no more tiles than for 2^13 keys."""
     short, long = (ask("joint", 1, 1024, n_k, 64, mask, 0, PLENTY)[2] for n_k in (1 << 13, 1 << 24))
     assert long < 10 * short + 5, (short, long)
+
+
+@pytest.mark.parametrize("shape,splits", [((1, 16384, 16384, 64, NONE, 0), (2, 2)), ((2, 4096, 4096, 64, NONE, 0), (4, 4)), ((1, 8192, 8192, 64, NONE, 0), (4, 4)),
+                                          ((2, 8192, 8192, 64, CAUSAL, 0), (4, 4)), ((31, 5588, 980, 64, NONE, 0), (1, 2)), ((8, 2048, 2048, 64, NONE, 0), (1, 1)),
+                                          ((2, 8192, 8192, 64, CAUSAL, 500), (1, 1)), ((16, 1000, 3001, 128, BOTTOM_RIGHT, 700), (1, 1))])
+def test_splits_of_a_shared_launch(ask, shape, splits):
+    """At d = 64 two workgroups share a CU: launches of one workgroup per CU, or of few long ones beside many short ones, split further,
+    and those that have company anyway do not. Each pair was measured as the fastest, or within 2 % of it, of all that the rule chooses
+    from."""
+    assert tuple(ask("joint", *shape, PLENTY)[:2]) == splits
