@@ -141,8 +141,7 @@ int run_grads(const fhog_bwdbwd_args* a, const fhog::Params& base, int q_pass, b
     p.n_split = q_pass ? launch_split_of(a, p, FHOG_IMPL_BF16, q_pass) : 1;
     p.n_split_k = k_side ? launch_split_of(a, p, FHOG_IMPL_BF16, FHOG_PASS_DK_DV) : 1;
   }
-  if (slice_order(a, p, a->n_q)) p.tile_major = 0;
-  if (slice_order(a, p, a->n_k)) p.tile_major_k = 0;
+  grads_order(a, q_pass != 0, k_side, p);
   p.part = reinterpret_cast<float*>(reinterpret_cast<char*>(a->ws) + stats_bytes(a));
   p.part_k = p.part + (p.n_split > 1 ? p.n_split * (split_bytes(a, FHOG_PASS_DQ_DDO) / sizeof(float)) : 0);
   const hipError_t e = fhog::launch_bf16_grads(p, q_pass, k_side, s);

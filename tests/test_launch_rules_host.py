@@ -38,6 +38,11 @@ int main() {
         best = us < best ? us : best;
       }
       printf("%d %d %.3f\n", x, y, best);
+    } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
+      p.tile_major = p.tile_major_k = p.causal;
+      rules::joint_splits(&a, p, &p.n_split, &p.n_split_k);
+      rules::grads_order(&a, true, true, p);
+      printf("%d %d\n", p.tile_major, p.tile_major_k);
     }
   }
 }
@@ -76,3 +81,12 @@ def test_splits_of_a_shared_launch(ask, shape, splits):
     and those that have company anyway do not. Each pair was measured as the fastest, or within 2 % of it, of all that the rule chooses
     from."""
     assert tuple(ask("joint", *shape, PLENTY)[:2]) == splits
+
+
+@pytest.mark.parametrize("shape,order", [((1, 19472, 19472, 64, CAUSAL, 0), (1, 1)), ((2, 18809, 18809, 64, CAUSAL, 0), (1, 1)), ((32, 16384, 16384, 64, CAUSAL, 0), (0, 0)),
+                                         ((1, 30000, 30000, 64, CAUSAL, 5000), (0, 0)), ((1, 19472, 19472, 128, CAUSAL, 0), (0, 0)), ((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)),
+                                         ((4, 16383, 16383, 128, CAUSAL, 0), (1, 1)), ((1, 20000, 20000, 64, NONE, 0), (0, 0))])
+def test_order_of_a_shared_launch(ask, shape, order):
+    """Slices of 16384 rows or more go one after the other (0) instead of tile by tile together (1), each side by its own length, except at d = 64 where
+    the two sides take turns."""
+    assert tuple(ask("order", *shape, PLENTY)) == order
