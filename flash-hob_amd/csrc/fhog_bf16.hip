@@ -26,6 +26,7 @@
 // the output accumulators alone take 128 registers and the work is split over producer and consumer waves.
 
 #include "fhog_bf16_blocks.h"
+#include "fhog_rules.h"
 
 namespace fhog {
 using namespace bf16k;
@@ -613,7 +614,7 @@ __global__ void __launch_bounds__(256, 2) grads_bf16(Params p, int q_blocks, boo
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int bh, tile, split = 0, id = blockIdx.x;
   const bool pairs = MASK != MASK_NONE && !mixed;   // workgroups that join others of their own sweep on a CU
-  if (first_of_two(q_blocks, mixed, MASK != MASK_NONE, id)) {
+  if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, MASK != MASK_NONE, id)) {
     if (!decode_block<MASK>((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, pairs, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     RowChain unused;
@@ -702,7 +703,7 @@ hipError_t launch_grads64(const Params& p, bool q_side, bool k_side, hipStream_t
   const unsigned gk = k_side ? grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split_k) : 0;
   const hipError_t e = allow_dynamic_lds<grads_bf16<F16, 64, QPASS, MASK, SUB>>(q_lds > k_lds ? q_lds : k_lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((grads_bf16<F16, 64, QPASS, MASK, SUB>), dim3(gq + gk), dim3(256), q_lds > k_lds ? q_lds : k_lds, s, p, (int)gq, mixed_order(gq, gk, p.tile_major && p.tile_major_k));
+  hipLaunchKernelGGL((grads_bf16<F16, 64, QPASS, MASK, SUB>), dim3(gq + gk), dim3(256), q_lds > k_lds ? q_lds : k_lds, s, p, (int)gq, rules::mixed_order(p, gq, gk));
   return hipGetLastError();
 }
 

@@ -12,6 +12,7 @@
 // the consumer on the same SIMD can overlap; each wave fits 256 registers.
 // One barrier per 32-row step. LDS: 3-stage ring of streamed tiles + double-buffered operand tiles.
 #include "fhog_bf16_util.h"
+#include "fhog_rules.h"
 
 namespace fhog {
 using namespace bf16k;
@@ -607,7 +608,7 @@ template <bool F16, int D, int MASK, bool DQ_ONLY>
 __global__ void __launch_bounds__(PC_THREADS) grads_pc(Params p, int q_blocks, bool mixed) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int bh, tile, split = 0, id = blockIdx.x;
-  if (first_of_two(q_blocks, mixed, false, id)) {
+  if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, false, id)) {
     if (!decode_block<MASK>((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, MASK != MASK_NONE, p.tile_major, bh, tile, false, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
     q_run_pc<F16, D, MASK, DQ_ONLY>(p, smem, bh, tile, split);
@@ -843,7 +844,7 @@ hipError_t launch_grads_pc_d(const Params& p, bool q_side, bool k_side, hipStrea
   if (e != hipSuccess) return e;
   const unsigned gq = q_side ? grid_blocks((p.n_q + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split) : 0;
   const unsigned gk = k_side ? grid_blocks((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split_k) : 0;
-  hipLaunchKernelGGL((grads_pc<F16, D, MASK, DQ_ONLY>), dim3(gq + gk), dim3(PC_THREADS), smem, s, p, (int)gq, mixed_order(gq, gk, p.tile_major && p.tile_major_k));
+  hipLaunchKernelGGL((grads_pc<F16, D, MASK, DQ_ONLY>), dim3(gq + gk), dim3(PC_THREADS), smem, s, p, (int)gq, rules::mixed_order(p, gq, gk));
   return hipGetLastError();
 }
 

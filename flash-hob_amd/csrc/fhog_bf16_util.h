@@ -380,16 +380,10 @@ __device__ __forceinline__ bool decode_block(int n_tiles, int batch, bool heavy_
   return decode_block<MASK>(n_tiles, batch, heavy_first, tile_major, bh, tile, pairs, blockIdx.x);
 }
 
-// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of
-// both come first and the lightest last; one sweep after the other, the second one's heaviest start when half of the launch is over, or
-// join the first one's heaviest on their CUs. From about 1000 workgroups on a side that no longer matters, and the other order keeps fewer
-// tensors in an L2 at a time. Double-backward, us, one after the other -> in turn, bf16 causal: d = 64 16 x 2048 148 -> 124, 4 x 8192
-// 527 -> 433, 32 x 2048 213 -> 202, 64 x 2048 380 -> 387; d = 128 16 x 2048 188 -> 188, 4 x 8192 651 -> 638, 64 x 2048 675 -> 688.
-inline bool mixed_order(unsigned gq, unsigned gk, bool tile_major) { return gq == gk && tile_major && gq < 1000; }
-
-// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups: whether workgroup `id` is of the first one; id: its id there.
-// mixed (gq == gk): tile by tile in turn, heaviest first over both, instead of one sweep after the other; pairs as in decode_block.
-__host__ __device__ __forceinline__ bool first_of_two(int gq, bool mixed, bool pairs, int& id) {
+// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups (multiples of 8): whether workgroup `id` is of the first one; id: its id there.
+// mixed: tile by tile in turn, heaviest first over both, instead of one sweep after the other, and what one has more at the end; pairs as in
+// decode_block.
+__host__ __device__ __forceinline__ bool first_of_two(int gq, int gk, bool mixed, bool pairs, int& id) {
   if (!mixed) {
     const bool first = id < gq;
     if (!first) id -= gq;
@@ -397,11 +391,13 @@ __host__ __device__ __forceinline__ bool first_of_two(int gq, bool mixed, bool p
   }
   int slot = id >> 3;
   if (pairs && slot >= 32) {
-    const int last = min(64, 2 * gq / 8) - 1;
+    const int last = min(64, (gq + gk) / 8) - 1;
     if (slot <= last) slot = 32 + last - slot;
   }
-  id = (slot >> 1) * 8 + (id & 7);
-  return !(slot & 1);
+  const int both = min(gq, gk) / 8;   // turns of an XCD
+  const bool turn = slot < 2 * both, first = turn ? !(slot & 1) : gq > gk;
+  id = (turn ? slot >> 1 : slot - both) * 8 + (id & 7);
+  return first;
 }
 
 }  // namespace bf16k

@@ -214,6 +214,18 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, i
     }
 }
 
+// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of
+// both come first and the lightest last; one sweep after the other, the second one's heaviest start when half of the launch is over, or
+// join the first one's heaviest on their CUs. From about 1000 workgroups on a side that no longer matters, and the other order keeps fewer
+// tensors in an L2 at a time. Double-backward, us, one after the other -> in turn, bf16 causal: d = 64 16 x 2048 148 -> 124, 4 x 8192
+// 527 -> 433, 32 x 2048 213 -> 202, 64 x 2048 380 -> 387; d = 128 16 x 2048 188 -> 188, 4 x 8192 651 -> 638, 64 x 2048 675 -> 688.
+// At d = 64 sides of unequal length take turns too, unless a window makes their work even, and what the longer one has more (its light end) comes last. us, so:
+// bottom-right 2 x 20704 x 20814 1593 -> 1340, 1 x 18029 x 18090 638 -> 547, 2 x 7413 x 8824 345 -> 310; d = 128 16 x 1925 x 3292, window 87 91 -> 100.
+inline bool mixed_order(const Params& p, int64_t gq, int64_t gk) {
+  const int64_t most = gq > gk ? gq : gk, least = gq + gk - most;
+  return p.tile_major && p.tile_major_k && most < 1000 && (gq == gk || (p.d == 64 && most <= 2 * least && 2 * (int64_t)p.window >= p.n_k));
+}
+
 // Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all
 // of them first) balances the end of a launch; from 16384 stationary rows on a slice alone has tiles enough for that
 // and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x
@@ -223,8 +235,8 @@ inline bool slice_order(const fhog_bwdbwd_args* a, const Params& p, int64_t rows
 // window makes their work even: one sweep after the other, the second one's heavy tiles come last. Double-backward, us, slice order -> turns (two launches):
 // bf16 causal 1 x 17000 612 -> 544 (550), 1 x 35801 2358 -> 2020 (2058), 2 x 18809 1256 -> 1097 (1125); window 5000 1 x 30000 431 -> 440.
 inline void grads_order(const fhog_bwdbwd_args* a, bool q_side, bool k_side, Params& p) {
-  const int64_t tiles_q = (a->n_q + 127) / 128, tiles_k = (a->n_k + 127) / 128;
-  if (a->d == 64 && q_side && k_side && tiles_q == tiles_k && p.n_split == p.n_split_k && (tiles_q * a->batch * p.n_split + 7) / 8 * 8 < 1000 && 2 * (int64_t)p.window >= a->n_k) return;
+  const int64_t blocks_q = ((a->n_q + 127) / 128 * a->batch * p.n_split + 7) / 8 * 8, blocks_k = ((a->n_k + 127) / 128 * a->batch * p.n_split_k + 7) / 8 * 8;
+  if (a->d == 64 && q_side && k_side && 2 * (int64_t)p.window >= a->n_k && mixed_order(p, blocks_q, blocks_k)) return;
   if (slice_order(a, p, a->n_q)) p.tile_major = 0;
   if (slice_order(a, p, a->n_k)) p.tile_major_k = 0;
 }

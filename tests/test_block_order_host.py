@@ -23,7 +23,7 @@ int main() {
     int last_tile[8] = {};
     for (unsigned i = 0; i < (two ? 2 * grid : grid); i++) {
       int id = (int)i, bh, tile;
-      const int side = two && !first_of_two((int)grid, mode & 1, pairs, id);
+      const int side = two && !first_of_two((int)grid, (int)grid, mode & 1, pairs, id);
       if (!decode_block(T, B, false, major, bh, tile, pairs && !two, id)) continue;
       if (bh < 0 || bh >= B || tile < 0 || tile >= T || !seen[side].insert({bh, tile}).second) return printf("%d tiles, %d slices, mode %d, id %u\n", T, B, mode, i), 1;
       // tile by tile: nothing follows lighter tiles of the XCD's own slices
@@ -62,6 +62,36 @@ int main() {
 }
 """
 
+# two sweeps of unequal length in one launch, tile by tile in turn: every tile of both exactly once, and at turn k neither is ahead of the other
+_TURNS = r"""
+#include <cstdio>
+#include <set>
+#include <utility>
+#include "fhog_bf16_util.h"
+using namespace fhog::bf16k;
+int main() {
+  const int tiles[] = {1, 2, 5, 8, 13, 31, 64, 65, 130};
+  for (int TQ : tiles) for (int TK : tiles) for (int B = 1; B <= 12; B++) for (int pairs = 0; pairs < 2; pairs++) {
+    const int gq = grid_blocks(TQ, B), gk = grid_blocks(TK, B);
+    std::set<std::pair<int, int>> seen[2];
+    int turns[8][2] = {};
+    for (int i = 0; i < gq + gk; i++) {
+      int id = i, bh, tile;
+      const int side = !first_of_two(gq, gk, true, pairs, id), T = side ? TK : TQ;
+      if (id < 0 || id >= (side ? gk : gq)) return printf("id: %d and %d tiles, %d slices, id %d\n", TQ, TK, B, i), 1;
+      if (!pairs && (i >> 3) < 2 * (gq < gk ? gq : gk) / 8) {
+        turns[i & 7][side]++;
+        if (turns[i & 7][0] - turns[i & 7][1] < 0 || turns[i & 7][0] - turns[i & 7][1] > 1) return printf("turns: %d and %d tiles, %d slices, id %d\n", TQ, TK, B, i), 1;
+      }
+      if (!decode_block<MASK_CAUSAL>(T, B, !side, true, bh, tile, false, id)) continue;
+      if (bh < 0 || bh >= B || tile < 0 || tile >= T || !seen[side].insert({bh, tile}).second) return printf("%d and %d tiles, %d slices, id %d\n", TQ, TK, B, i), 1;
+    }
+    if ((int)seen[0].size() != TQ * B || (int)seen[1].size() != TK * B) return printf("%d and %d tiles, %d slices\n", TQ, TK, B), 1;
+  }
+  return 0;
+}
+"""
+
 
 def _run(tmp_path, program):
     src = tmp_path / "order.hip"
@@ -86,3 +116,8 @@ def test_every_tile_once(tmp_path):
 @_needs_hipcc
 def test_xcds_have_the_same_work_under_a_mask(tmp_path):
     _run(tmp_path, _BALANCE)
+
+
+@_needs_hipcc
+def test_sweeps_of_unequal_length_take_turns(tmp_path):
+    _run(tmp_path, _TURNS)

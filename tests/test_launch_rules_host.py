@@ -84,7 +84,8 @@ def test_splits_of_a_shared_launch(ask, shape, splits):
 
 
 @pytest.mark.parametrize("shape,order", [((1, 19472, 19472, 64, CAUSAL, 0), (1, 1)), ((2, 18809, 18809, 64, CAUSAL, 0), (1, 1)), ((32, 16384, 16384, 64, CAUSAL, 0), (0, 0)),
-                                         ((1, 30000, 30000, 64, CAUSAL, 5000), (0, 0)), ((1, 19472, 19472, 128, CAUSAL, 0), (0, 0)), ((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)),
+                                         ((1, 30000, 30000, 64, CAUSAL, 5000), (0, 0)), ((1, 19472, 19472, 128, CAUSAL, 0), (0, 0)), ((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 1)), ((1, 4000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)),
+                                         ((2, 9000, 17000, 64, BOTTOM_RIGHT, 500), (1, 0)), ((2, 9000, 17000, 128, BOTTOM_RIGHT, 0), (1, 0)),
                                          ((4, 16383, 16383, 128, CAUSAL, 0), (1, 1)), ((1, 20000, 20000, 64, NONE, 0), (0, 0))])
 def test_order_of_a_shared_launch(ask, shape, order):
     """Slices of 16384 rows or more go one after the other (0) instead of tile by tile together (1), each side by its own length, except at d = 64 where
