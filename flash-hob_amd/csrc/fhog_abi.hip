@@ -351,14 +351,7 @@ size_t fhog_bwdbwd_workspace_bytes(int64_t batch, int64_t n_q) {
 
 size_t fhog_bwdbwd_workspace_hint(const fhog_bwdbwd_args* args) {
   if (validate(args) != FHOG_OK) return 0;
-  const int impl = select_impl(args);
-  const fhog::Params p = to_params(args);
-  size_t extra = 0;
-  for (int pass = FHOG_PASS_DD; pass <= FHOG_PASS_DD_B; pass++) {
-    const int s = split_up_to(wanted_split(args, impl, pass), args, p, pass);
-    if (s > 1 && (size_t)s * split_bytes(args, pass) > extra) extra = (size_t)s * split_bytes(args, pass);
-  }
-  return extra ? stats_bytes(args) + extra : fhog_bwdbwd_workspace_bytes(args->batch, args->n_q);
+  return workspace_hint(args, to_params(args), select_impl(args));
 }
 
 int fhog_validate(const fhog_bwdbwd_args* args) { return validate(args); }

@@ -175,6 +175,8 @@ inline double makespan_two(int64_t n_a, double a, int64_t n_b, double b, double 
   return t;
 }
 
+constexpr int64_t kMostParts = 2 * 131072 * (int64_t)sizeof(float);   // bytes of partial results per column, at most
+
 // Splits of the two sides where they share a launch, out of those that either would like alone and the workspace has room for. The same
 // reckoning in steps of a tile, over the workgroups of both. At d = 128 a CU has one workgroup and a tile takes 1.9 us; at d = 64 two, and
 // a tile takes 0.87 us in company and 1.25 times that alone: 256 workgroups there leave every CU half used. us, splits 1 | 1, 2 | 2, 4 | 4, 8 | 8:
@@ -195,7 +197,7 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, i
   for (int x = 1; x <= most_q; x *= 2)
     for (int y = 1; y <= most_k; y *= 2) {
       const int64_t part = (x > 1 ? x * bytes_q : 0) + (y > 1 ? y * bytes_k : 0);
-      if (part > have) continue;
+      if (part > have || part > kMostParts * a->d) continue;
       const double lq = q.sum / q.live / x + fixed, lk = k.sum / k.live / y + fixed;
       const int64_t nq = llround(q.live * (double)(a->batch * x)), nk = llround(k.live * (double)(a->batch * y));
       double cost, longest;   // pass 3 comes first
@@ -239,6 +241,24 @@ inline void grads_order(const fhog_bwdbwd_args* a, bool q_side, bool k_side, Par
   if (a->d == 64 && q_side && k_side && 2 * (int64_t)p.window >= a->n_k && mixed_order(p, blocks_q, blocks_k)) return;
   if (slice_order(a, p, a->n_q)) p.tile_major = 0;
   if (slice_order(a, p, a->n_k)) p.tile_major_k = 0;
+}
+
+// Workspace with which every pass, run alone, and passes 3 and 4 in a shared launch, whose partial results are there at the same time, have the splits they would like
+inline size_t workspace_hint(const fhog_bwdbwd_args* a, const Params& p, int impl) {
+  size_t extra = 0;
+  for (int pass = FHOG_PASS_DD; pass <= FHOG_PASS_DD_B; pass++) {
+    const int s = split_up_to(wanted_split(a, impl, pass), a, p, pass);
+    if (s > 1 && (size_t)s * split_bytes(a, pass) > extra) extra = (size_t)s * split_bytes(a, pass);
+  }
+  if (impl == FHOG_IMPL_BF16) {
+    fhog_bwdbwd_args roomy = *a;
+    roomy.ws_bytes = INT64_MAX;
+    int x, y;
+    joint_splits(&roomy, p, &x, &y);
+    const size_t both = (x > 1 ? x * split_bytes(a, FHOG_PASS_DQ_DDO) : 0) + (y > 1 ? y * split_bytes(a, FHOG_PASS_DK_DV) : 0);
+    if (both > extra) extra = both;
+  }
+  return extra ? stats_bytes(a) + extra : (size_t)3 * a->batch * a->n_q * sizeof(float);
 }
 
 // ---- small launches of the 16-bit kernels (fhog_small.hip) ------------------------------------------------------

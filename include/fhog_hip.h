@@ -164,8 +164,10 @@ size_t fhog_bwdbwd_args_size(void);
    Replaces the torch allocations of D, dD, B at fhog/triton_bwdbwd.py:580-584. */
 size_t fhog_bwdbwd_workspace_bytes(int64_t batch, int64_t n_q);
 
-/* Workspace size that lets every pass of these arguments use the split it would like (>= the minimum, and equal to
-   it when no pass would split); 0 if the arguments are not valid. Host-only. No counterpart in the reference, whose
+/* Workspace size that lets every pass of these arguments, run alone (fhog_bwdbwd_pass), and passes 3 and 4 in the launch that
+   they share in fhog_bwdbwd use the splits they would like (>= the minimum, and equal to it when none would split; at most
+   2 * 131072 * d floats more); 0 if the arguments are not valid. Launches small enough for the kernels that put several waves on
+   the same rows leave what is beyond the minimum untouched. Host-only. No counterpart in the reference, whose
    kernels are always tiled over (batch*head, N / BLOCK) alone (fhog/triton_bwdbwd.py:586-646). */
 size_t fhog_bwdbwd_workspace_hint(const fhog_bwdbwd_args* args);
 

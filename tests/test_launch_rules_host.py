@@ -38,6 +38,13 @@ int main() {
         best = us < best ? us : best;
       }
       printf("%d %d %.3f\n", x, y, best);
+    } else if (!strcmp(what, "hinted")) {   // splits with the hinted workspace, and with any amount
+      int x, y, u, v;
+      a.ws_bytes = INT64_MAX;
+      rules::joint_splits(&a, p, &u, &v);
+      a.ws_bytes = (int64_t)rules::workspace_hint(&a, p, FHOG_IMPL_BF16);
+      rules::joint_splits(&a, p, &x, &y);
+      printf("%d %d %d %d\n", x, y, u, v);
     } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
       p.tile_major = p.tile_major_k = p.causal;
       rules::joint_splits(&a, p, &p.n_split, &p.n_split_k);
@@ -59,10 +66,14 @@ def ask(tmp_path_factory):
                         str(folder / "rules.hip"), "-o", str(folder / "rules")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
 
-    def one(*query):
-        r = subprocess.run([str(folder / "rules")], input=" ".join(map(str, query)) + "\n", capture_output=True, text=True, timeout=60)
+    def some(queries):
+        r = subprocess.run([str(folder / "rules")], input="".join(" ".join(map(str, q)) + "\n" for q in queries), capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, r.stderr[-2000:]
-        return [float(x) for x in r.stdout.split()]
+        return [[float(x) for x in line.split()] for line in r.stdout.splitlines()]
+
+    def one(*query):
+        return some([query])[0]
+    one.some = some
     return one
 
 
@@ -91,3 +102,15 @@ def test_order_of_a_shared_launch(ask, shape, order):
     """Slices of 16384 rows or more go one after the other (0) instead of tile by tile together (1), each side by its own length, except at d = 64 where
     the two sides take turns."""
     assert tuple(ask("order", *shape, PLENTY)) == order
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_hinted_workspace_has_room_for_both_sides(ask, d):
+    """Passes 3 and 4 in one launch hold their partial results at the same time: with the hinted workspace they split as with any amount."""
+    lengths = (300, 1000, 1024, 2000, 3000, 4096, 9000, 20000)
+    queries = [("hinted", b, n_q, n_k, d, mask, window, 0) for b in (1, 2, 3, 5, 8, 16) for n_q in lengths for n_k in lengths
+               for mask, window in ((NONE, 0), (CAUSAL, 0), (BOTTOM_RIGHT, 700)) if mask == NONE or (n_q == n_k if mask == CAUSAL else n_q <= n_k)]
+    short = [(q, got) for q, got in zip(queries, ask.some(queries)) if got[:2] != got[2:]]
+    assert not short, short[:5]
+    if d == 128:   # 38.5 steps of a tile with the room that the wider of the two passes needs, 24 so
+        assert ask("hinted", 1, 2000, 1024, 128, NONE, 0, 0)[:2] == [2, 4]
