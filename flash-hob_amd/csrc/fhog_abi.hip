@@ -135,8 +135,8 @@ fhog::Params to_params(const fhog_bwdbwd_args* a) {
 // Pass 3 or 7 (q_pass, 0: none) and pass 4 (k_side) of the 16-bit kernels, in one launch
 int run_grads(const fhog_bwdbwd_args* a, const fhog::Params& base, int q_pass, bool k_side, hipStream_t s) {
   fhog::Params p = base;
-  if (q_pass == FHOG_PASS_DQ_DDO && k_side) {
-    joint_splits(a, p, &p.n_split, &p.n_split_k);
+  if (q_pass && k_side) {
+    joint_splits(a, p, q_pass, &p.n_split, &p.n_split_k);
   } else {
     p.n_split = q_pass ? launch_split_of(a, p, FHOG_IMPL_BF16, q_pass) : 1;
     p.n_split_k = k_side ? launch_split_of(a, p, FHOG_IMPL_BF16, FHOG_PASS_DK_DV) : 1;
@@ -402,12 +402,7 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
       granted_split(args, impl, FHOG_PASS_DQ_DDO) == 1 && granted_split(args, impl, FHOG_PASS_DD) == 1)
     order = stage1, n_pass = 2;
   if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (split_products && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 3;
-  // Passes 6-8 have no split form: a launch too small to fill the GPU whose workspace lets the reference's passes split
-  // their streamed side runs the nearest schedule that can (three sweeps -> fused statistics, ddO early -> four passes).
-  // Asked of pass 3, by the splits that it runs with: under a window it may fill the GPU unsplit although the workspace has room.
-  // us, substitute -> schedule asked for, d = 128, three sweeps | ddO early: bf16 causal 2 x 16000, window 300 112 -> 92 | 141 -> 125;
-  // 32 x 1024, window 128 73.0 -> 64.5 | 91.8 -> 83.8; bottom-right 16 x 1000 x 3001, window 40 65.6 -> 59.5 | 81.2 -> 76.4.
-  const bool splits = launch_split_of(args, p, impl, FHOG_PASS_DQ_DDO) > 1;
+  const bool splits = splits_instead(args, p, impl);
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && splits) order = fused, n_pass = 3;
   if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early, n_pass = 4;
   if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three, n_pass = 3;

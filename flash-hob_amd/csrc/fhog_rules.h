@@ -183,8 +183,9 @@ constexpr int64_t kMostParts = 2 * 131072 * (int64_t)sizeof(float);   // bytes o
 // fp16 d = 64 no mask 1 x 8192 369, 232, 203, 211; 1 x 16384 798, 727, 738, 750; 2 x 4096 178, 123, 115, 123; 4 x 4096 208, 203, 211, 229; 8 x 2048 110, 114,
 // 123, 142; causal 1 x 16384 683, 611, 499, 439; 2 x 8192 344, 244, 225, 245; 8 x 2048 99, 81, 85, 113. Splits of one side alone at 1 x 16384: 2 | 1 950.
 // Over 640 shapes of 1 to 64 slices with 16 to 20000 rows, against the best pair of each: 2.2 % too slow with one workgroup to a CU -> 0.9 %.
-inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int* s_q, int* s_k) {
-  const int most_q = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DQ_DDO), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
+// q_pass: 3, or 7, which does not split.
+inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass, int* s_q, int* s_k) {
+  const int most_q = wanted_split(a, FHOG_IMPL_BF16, q_pass), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
   *s_q = *s_k = 1;
   const int64_t have = a->ws_bytes - (int64_t)stats_bytes(a);
   if ((most_q == 1 && most_k == 1) || have <= 0) return;
@@ -254,11 +255,24 @@ inline size_t workspace_hint(const fhog_bwdbwd_args* a, const Params& p, int imp
     fhog_bwdbwd_args roomy = *a;
     roomy.ws_bytes = INT64_MAX;
     int x, y;
-    joint_splits(&roomy, p, &x, &y);
+    joint_splits(&roomy, p, FHOG_PASS_DQ_DDO, &x, &y);
     const size_t both = (x > 1 ? x * split_bytes(a, FHOG_PASS_DQ_DDO) : 0) + (y > 1 ? y * split_bytes(a, FHOG_PASS_DK_DV) : 0);
     if (both > extra) extra = both;
   }
   return extra ? stats_bytes(a) + extra : (size_t)3 * a->batch * a->n_q * sizeof(float);
+}
+
+// Passes 6, 7 and 8 have no split form. Whether a launch that asks for them is too small and runs the nearest schedule whose passes split instead (three
+// sweeps -> fused statistics, ddO early -> four passes), given that the workspace lets pass 3 split: the statistics sweep has the most to gain, whose
+// workgroups are the query side's. Time of the schedule asked for over that of the substitute, 1500 shapes, d = 64 | 128, by 128-row groups of queries:
+//   no mask    64.. 1.26 | 1.18, 128.. 1.02 | 0.99, 192.. 0.96 | 0.94, 384.. 0.92 | 0.92
+//   triangle   64.. 1.73 | 1.55, 128.. 1.36 | 1.25, 192.. 1.12 | 1.08, 256.. 1.04 | 1.02, 384.. 1.01 | 0.99, 512.. 0.94 | 0.93
+//   windows of less than half the keys   64.. 0.94 | 1.04, 128.. 0.93 | 0.93, 192.. 0.85 | 0.84; of 512 keys or more, below 96 1.15 | 1.17, 96.. 1.05 | 1.01
+inline bool splits_instead(const fhog_bwdbwd_args* a, const Params& p, int impl) {
+  if (granted_split(a, impl, FHOG_PASS_DQ_DDO) == 1) return false;
+  const int64_t groups = (a->n_q + 127) / 128 * a->batch;
+  if (2 * (int64_t)p.window < a->n_k) return p.window >= 512 && groups < 112;
+  return groups < (p.causal && 2 * (int64_t)p.mask_off <= a->n_k ? 384 : 144);
 }
 
 // ---- small launches of the 16-bit kernels (fhog_small.hip) ------------------------------------------------------

@@ -101,9 +101,12 @@ extern "C" {
                                        dK2+dV2. 20 recomputed products. ddP V is formed as (P o ddS) V - dd O with the
                                        caller's 16-bit O: accurate as long as dd_i does not dominate ddS_ij - dd_i.
                                        Schedules 2 and 3 exist in the 16-bit MFMA family; the split-product family runs
-                                       schedule 1 for them. Passes 6, 7 and 8 have no split form: a launch too
-                                       small to fill the GPU, whose pass 3 would run split (ws_bytes allowing), runs the four
-                                       passes (schedule 2) or the fused statistics sweep and passes 3, 4 (schedule 3) */
+                                       schedule 1 for them. Passes 6, 7 and 8 have no split form: where the workspace lets
+                                       pass 3 split its streamed side, a launch whose query side alone has too few workgroups to
+                                       fill the GPU runs the four passes (schedule 2) or the fused statistics sweep and
+                                       passes 3, 4 (schedule 3). Launches of up to 128 groups of 128 rows (query and key side
+                                       together) that run on the kernels which put several waves on the same rows run schedule 1
+                                       there, whatever ws_bytes is: then ddO and b are those of passes 3 and 5 */
 
 /* Launch choices (the counterpart of the reference's autotune list, fhog/triton_bwdbwd.py:12-36) are fixed functions of
  * the launch size. For experiments they can be overridden through the environment variable FHOG_TUNE, a comma-separated

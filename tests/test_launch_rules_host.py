@@ -33,7 +33,7 @@ int main() {
       double best = 1e9;
       for (int i = 0; i < 10; i++) {
         const auto t0 = std::chrono::steady_clock::now();
-        rules::joint_splits(&a, p, &x, &y);
+        rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &x, &y);
         const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
         best = us < best ? us : best;
       }
@@ -41,13 +41,15 @@ int main() {
     } else if (!strcmp(what, "hinted")) {   // splits with the hinted workspace, and with any amount
       int x, y, u, v;
       a.ws_bytes = INT64_MAX;
-      rules::joint_splits(&a, p, &u, &v);
+      rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &u, &v);
       a.ws_bytes = (int64_t)rules::workspace_hint(&a, p, FHOG_IMPL_BF16);
-      rules::joint_splits(&a, p, &x, &y);
+      rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &x, &y);
       printf("%d %d %d %d\n", x, y, u, v);
+    } else if (!strcmp(what, "instead")) {
+      printf("%d\n", rules::splits_instead(&a, p, FHOG_IMPL_BF16));
     } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
       p.tile_major = p.tile_major_k = p.causal;
-      rules::joint_splits(&a, p, &p.n_split, &p.n_split_k);
+      rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &p.n_split, &p.n_split_k);
       rules::grads_order(&a, true, true, p);
       printf("%d %d\n", p.tile_major, p.tile_major_k);
     }
@@ -114,3 +116,12 @@ def test_hinted_workspace_has_room_for_both_sides(ask, d):
     assert not short, short[:5]
     if d == 128:   # 38.5 steps of a tile with the room that the wider of the two passes needs, 24 so
         assert ask("hinted", 1, 2000, 1024, 128, NONE, 0, 0)[:2] == [2, 4]
+
+
+@pytest.mark.parametrize("shape,instead", [((8, 2048, 2048, 64, NONE, 0), 1), ((24, 2048, 2048, 64, NONE, 0), 0), ((16, 2048, 2048, 128, NONE, 0), 0), ((16, 2048, 2048, 64, CAUSAL, 0), 1),
+                                           ((4, 8192, 8192, 128, CAUSAL, 0), 1), ((48, 1024, 1024, 64, CAUSAL, 0), 0), ((4, 2048, 2048, 64, CAUSAL, 100), 0),
+                                           ((6, 2048, 9000, 64, BOTTOM_RIGHT, 0), 1), ((10, 2048, 9000, 64, BOTTOM_RIGHT, 0), 0)])
+def test_schedules_without_a_split_form_are_replaced_where_that_is_faster(ask, shape, instead):
+    """By the query side's workgroups of 128 rows under the mask; never without room for partial results."""
+    assert ask("instead", *shape, PLENTY) == [instead]
+    assert ask("instead", *shape, 0) == [0]
