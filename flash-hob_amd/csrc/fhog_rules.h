@@ -267,11 +267,12 @@ inline size_t workspace_hint(const fhog_bwdbwd_args* a, const Params& p, int imp
 // workgroups are the query side's. Time of the schedule asked for over that of the substitute, 1500 shapes, d = 64 | 128, by 128-row groups of queries:
 //   no mask    64.. 1.26 | 1.18, 128.. 1.02 | 0.99, 192.. 0.96 | 0.94, 384.. 0.92 | 0.92
 //   triangle   64.. 1.73 | 1.55, 128.. 1.36 | 1.25, 192.. 1.12 | 1.08, 256.. 1.04 | 1.02, 384.. 1.01 | 0.99, 512.. 0.94 | 0.93
-//   windows of less than half the keys   64.. 0.94 | 1.04, 128.. 0.93 | 0.93, 192.. 0.85 | 0.84; of 512 keys or more, below 96 1.15 | 1.17, 96.. 1.05 | 1.01
+//   windows of less than half the keys   64.. 0.94 | 1.04, 128.. 0.93 | 0.93, 192.. 0.85 | 0.84; of 512 keys or more, below 96 1.15 | 1.17, 96.. 1.05 | 1.01;
+//   of 2048 or more, 140.. 1.2 to 1.3 on single slices of 17000 to 20000 rows
 inline bool splits_instead(const fhog_bwdbwd_args* a, const Params& p, int impl) {
   if (granted_split(a, impl, FHOG_PASS_DQ_DDO) == 1) return false;
   const int64_t groups = (a->n_q + 127) / 128 * a->batch;
-  if (2 * (int64_t)p.window < a->n_k) return p.window >= 512 && groups < 112;
+  if (2 * (int64_t)p.window < a->n_k) return groups < (p.window >= 2048 ? 192 : p.window >= 512 ? 112 : 0);
   return groups < (p.causal && 2 * (int64_t)p.mask_off <= a->n_k ? 384 : 144);
 }
 
@@ -288,6 +289,10 @@ inline bool splits_instead(const fhog_bwdbwd_args* a, const Params& p, int impl)
 //                     d = 128: 8 x 256 25 -> 12 | 18; causal 32 x 512 39 -> 41 | 35, no mask 38 -> 51 | 43
 //   double-backward   d = 64: 4 x 256 24.1 -> 14.7 | 18.9; 64 x 256 27.2 -> 41 | 30; causal 8 x 1024 46.6 -> 33.8 | 45; 1 x 4096 59 -> 78 | 142
 //                     d = 128: 8 x 256 33.3 -> 22.8 | 30.5; 16 x 512 49.7 -> 49.2 | 49.7; causal 3 x 1536 69 -> 62 | 101; 1 x 2048 55 -> 72 | 127
+// Windows of less than half the keys leave the work of the workgroups even, so only CUs left idle speak for small ones, and one or two key tiles
+// leave three or two of a forward's four waves without one. us, small workgroups -> the other kernels: forward d = 128 1 x 28 5.3 -> 3.9, 4 x 36 5.6 -> 4.8, d = 64 3 x 30
+// 4.2 -> 3.4; window 1530 d = 128 2 x 11806 x 12908 65 -> 56; first backward, window 4788 d = 64 2 x 15961 1.25 to 1, window 3261 d = 128 2 x 8150 1.12 to 1.
+// The double-backward of d = 128 with few rows on one side and more than 32 tiles for them to stream: 2 x 79 x 4228, window 1370 58 -> 48.
 enum class Small { forward, backward, double_backward };
 inline int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int64_t d, int32_t causal, int64_t window) {
   if (tuning().small >= 0) return tuning().small;
@@ -295,23 +300,25 @@ inline int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int6
   // from 256 groups of a side on the kernels with 128 rows fill the GPU
   if (g_q >= 256 || (what != Small::forward && g_k >= 256)) return 0;
   const int64_t off = causal == FHOG_MASK_BOTTOM_RIGHT ? n_k - n_q : 0;
-  const bool windowed = causal != FHOG_MASK_NONE && window > 0 && window < n_k;
+  const bool windowed = causal != FHOG_MASK_NONE && window > 0 && window < n_k, even_window = windowed && 2 * window < n_k;
   const bool uneven = causal != FHOG_MASK_NONE && (windowed || 2 * off <= n_k);
   const int64_t streamed = what == Small::forward || n_k > n_q ? n_k : n_q;
   const int64_t tiles = ((windowed && window + 63 < streamed ? window + 63 : streamed) + 31) / 32;
   if (what == Small::forward) {
+    if (n_k <= 32 || (n_k <= 64 && n_q <= (d == 64 ? 40 : 64))) return 0;
     if (g_q <= 64) return 4;
     if (g_q <= 128) return d == 64 || (uneven && tiles >= 32) ? 4 : 2;
     if (tiles < 32) return 0;
-    return d == 64 ? (uneven ? 4 : 2) : (uneven ? 2 : 0);
+    return d == 64 ? (uneven ? 4 : 2) : (uneven && !even_window ? 2 : 0);
   }
-  const int64_t groups = g_q + g_k;
+  const int64_t groups = g_q + g_k, least = g_q < g_k ? g_q : g_k;
   if (what == Small::backward) {
     if (groups <= 64) return 4;
     if (groups <= 128) return tiles <= 8 ? 2 : 4;
-    if (groups <= 256) return d == 64 || uneven ? 2 : 0;
-    return d == 64 && uneven && tiles >= 32 ? 2 : 0;
+    if (groups <= 256) return d == 64 || (uneven && !(even_window && tiles >= 32 && groups > 160 && least > 64)) ? 2 : 0;
+    return d == 64 && uneven && tiles >= 32 && !(even_window && groups > 350) ? 2 : 0;
   }
+  if (d == 128 && tiles > 32 && 4 * least < groups - least) return 0;
   if (groups <= 64) return tiles <= (d == 64 ? 64 : 48) ? 4 : 0;
   if (groups <= 128) return tiles <= 8 ? 2 : tiles <= (uneven ? (d == 64 ? 64 : groups <= 96 ? 48 : 32) : d == 64 ? 32 : 16) ? 4 : 0;
   return groups <= 256 && d == 64 && uneven && tiles <= 32 ? 2 : 0;

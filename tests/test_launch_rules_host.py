@@ -47,6 +47,10 @@ int main() {
       printf("%d %d %d %d\n", x, y, u, v);
     } else if (!strcmp(what, "instead")) {
       printf("%d\n", rules::splits_instead(&a, p, FHOG_IMPL_BF16));
+    } else if (!strcmp(what, "small")) {   // waves on the same rows: forward, first backward, double-backward
+      using rules::Small;
+      for (Small w : {Small::forward, Small::backward, Small::double_backward}) printf("%d ", rules::small_waves(w, batch, n_q, n_k, d, mask, window));
+      printf("\n");
     } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
       p.tile_major = p.tile_major_k = p.causal;
       rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &p.n_split, &p.n_split_k);
@@ -119,9 +123,19 @@ def test_hinted_workspace_has_room_for_both_sides(ask, d):
 
 
 @pytest.mark.parametrize("shape,instead", [((8, 2048, 2048, 64, NONE, 0), 1), ((24, 2048, 2048, 64, NONE, 0), 0), ((16, 2048, 2048, 128, NONE, 0), 0), ((16, 2048, 2048, 64, CAUSAL, 0), 1),
-                                           ((4, 8192, 8192, 128, CAUSAL, 0), 1), ((48, 1024, 1024, 64, CAUSAL, 0), 0), ((4, 2048, 2048, 64, CAUSAL, 100), 0),
+                                           ((4, 8192, 8192, 128, CAUSAL, 0), 1), ((48, 1024, 1024, 64, CAUSAL, 0), 0), ((4, 2048, 2048, 64, CAUSAL, 100), 0), ((1, 17845, 17845, 64, CAUSAL, 5353), 1), ((3, 4096, 4096, 128, CAUSAL, 600), 1),
                                            ((6, 2048, 9000, 64, BOTTOM_RIGHT, 0), 1), ((10, 2048, 9000, 64, BOTTOM_RIGHT, 0), 0)])
 def test_schedules_without_a_split_form_are_replaced_where_that_is_faster(ask, shape, instead):
     """By the query side's workgroups of 128 rows under the mask; never without room for partial results."""
     assert ask("instead", *shape, PLENTY) == [instead]
     assert ask("instead", *shape, 0) == [0]
+
+
+@pytest.mark.parametrize("shape,waves", [((1, 28, 28, 128, NONE, 0), (0, 4, 4)), ((85, 17, 64, 64, NONE, 0), (0, 2, 0)), ((3, 100, 64, 128, NONE, 0), (4, 4, 4)), ((3, 100, 32, 128, NONE, 0), (0, 4, 4)),
+                                         ((2, 11806, 12908, 128, BOTTOM_RIGHT, 1530), (0, 0, 0)), ((2, 11806, 12908, 128, BOTTOM_RIGHT, 7000), (2, 0, 0)),
+                                         ((2, 8150, 8150, 128, CAUSAL, 3261), (4, 0, 0)), ((1, 11600, 11600, 128, CAUSAL, 2900), (4, 0, 0)), ((1, 11600, 11600, 128, CAUSAL, 6000), (4, 2, 0)),
+                                         ((3, 368, 7676, 128, BOTTOM_RIGHT, 3000), (4, 2, 0)), ((1, 15961, 15961, 64, CAUSAL, 4788), (4, 2, 0)), ((2, 15961, 15961, 64, CAUSAL, 4788), (4, 0, 0)), ((1, 26598, 26604, 64, BOTTOM_RIGHT, 7981), (4, 0, 0)),
+                                         ((2, 79, 4228, 128, BOTTOM_RIGHT, 1370), (4, 4, 0)), ((1, 1163, 53, 128, NONE, 0), (4, 4, 0)), ((1, 60, 53, 128, NONE, 0), (0, 4, 4)), ((1, 60, 53, 64, NONE, 0), (4, 4, 4)), ((2, 1200, 1200, 128, NONE, 0), (4, 4, 4))])
+def test_small_workgroups(ask, shape, waves):
+    """Both sides of the lines that windows, few keys and lopsided shapes add to the rule."""
+    assert tuple(ask("small", *shape, 0)) == waves
