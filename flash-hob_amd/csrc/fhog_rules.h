@@ -175,6 +175,18 @@ inline double makespan_two(int64_t n_a, double a, int64_t n_b, double b, double 
   return t;
 }
 
+// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of
+// both come first and the lightest last; one sweep after the other, the second one's heaviest start when half of the launch is over, or
+// join the first one's heaviest on their CUs. From about 1000 workgroups on a side that no longer matters, and the other order keeps fewer
+// tensors in an L2 at a time. Double-backward, us, one after the other -> in turn, bf16 causal: d = 64 16 x 2048 148 -> 124, 4 x 8192
+// 527 -> 433, 32 x 2048 213 -> 202, 64 x 2048 380 -> 387; d = 128 16 x 2048 188 -> 188, 4 x 8192 651 -> 638, 64 x 2048 675 -> 688.
+// At d = 64 sides of unequal length take turns too, unless a window makes their work even, and what the longer one has more (its light end) comes last. us, so:
+// bottom-right 2 x 20704 x 20814 1593 -> 1340, 1 x 18029 x 18090 638 -> 547, 2 x 7413 x 8824 345 -> 310; d = 128 16 x 1925 x 3292, window 87 91 -> 100.
+inline bool mixed_order(const Params& p, int64_t gq, int64_t gk) {
+  const int64_t most = gq > gk ? gq : gk, least = gq + gk - most;
+  return p.tile_major && p.tile_major_k && most < 1000 && (gq == gk || (p.d == 64 && most <= 2 * least && 2 * (int64_t)p.window >= p.n_k));
+}
+
 constexpr int64_t kMostParts = 2 * 131072 * (int64_t)sizeof(float);   // bytes of partial results per column, at most
 
 // Splits of the two sides where they share a launch, out of those that either would like alone and the workspace has room for. The same
@@ -183,6 +195,8 @@ constexpr int64_t kMostParts = 2 * 131072 * (int64_t)sizeof(float);   // bytes o
 // fp16 d = 64 no mask 1 x 8192 369, 232, 203, 211; 1 x 16384 798, 727, 738, 750; 2 x 4096 178, 123, 115, 123; 4 x 4096 208, 203, 211, 229; 8 x 2048 110, 114,
 // 123, 142; causal 1 x 16384 683, 611, 499, 439; 2 x 8192 344, 244, 225, 245; 8 x 2048 99, 81, 85, 113. Splits of one side alone at 1 x 16384: 2 | 1 950.
 // Over 640 shapes of 1 to 64 slices with 16 to 20000 rows, against the best pair of each: 2.2 % too slow with one workgroup to a CU -> 0.9 %.
+// Under a mask the light end of one sweep and the heavy start of the other meet only where the two take turns: 1000 masked shapes, against the best pair of
+// each, without -> with 10 % on pairs that do not: d = 64 2.1 % -> 1.8 % too slow, d = 128 1.9 % -> 1.2 %; bottom-right 2 x 5887 x 14150 8 | 1 525, 4 | 2 412.
 // q_pass: 3, or 7, which does not split.
 inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass, int* s_q, int* s_k) {
   const int most_q = wanted_split(a, FHOG_IMPL_BF16, q_pass), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
@@ -212,21 +226,9 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass,
       }
       if (longest > cost) cost = longest;
       if (part > 0) cost += (4 + (double)part / 2.5e6) / tile_us;   // a launch, and the partial results written and read
-      if (two && p.causal && q.groups == k.groups && x != y) cost *= 1.08;   // the sweeps do not take turns (mixed_order)
+      if (p.causal && 2 * (int64_t)p.window >= a->n_k && !mixed_order(p, (q.groups * a->batch * x + 7) / 8 * 8, (k.groups * a->batch * y + 7) / 8 * 8)) cost *= 1.1;
       if ((x == 1 && y == 1) || cost < best) best = cost, *s_q = x, *s_k = y;
     }
-}
-
-// Two sweeps in one launch, Q-tiled and K-tiled, with gq and gk workgroups under a mask: taken in turn, tile by tile, the heaviest of
-// both come first and the lightest last; one sweep after the other, the second one's heaviest start when half of the launch is over, or
-// join the first one's heaviest on their CUs. From about 1000 workgroups on a side that no longer matters, and the other order keeps fewer
-// tensors in an L2 at a time. Double-backward, us, one after the other -> in turn, bf16 causal: d = 64 16 x 2048 148 -> 124, 4 x 8192
-// 527 -> 433, 32 x 2048 213 -> 202, 64 x 2048 380 -> 387; d = 128 16 x 2048 188 -> 188, 4 x 8192 651 -> 638, 64 x 2048 675 -> 688.
-// At d = 64 sides of unequal length take turns too, unless a window makes their work even, and what the longer one has more (its light end) comes last. us, so:
-// bottom-right 2 x 20704 x 20814 1593 -> 1340, 1 x 18029 x 18090 638 -> 547, 2 x 7413 x 8824 345 -> 310; d = 128 16 x 1925 x 3292, window 87 91 -> 100.
-inline bool mixed_order(const Params& p, int64_t gq, int64_t gk) {
-  const int64_t most = gq > gk ? gq : gk, least = gq + gk - most;
-  return p.tile_major && p.tile_major_k && most < 1000 && (gq == gk || (p.d == 64 && most <= 2 * least && 2 * (int64_t)p.window >= p.n_k));
 }
 
 // Workgroup order within an XCD. With a mask, tile-major (the slices of an XCD advance together, heaviest tiles of all

@@ -26,7 +26,7 @@ int main() {
   while (scanf("%31s %lld %lld %lld %lld %d %lld %lld", what, &batch, &n_q, &n_k, &d, &mask, &window, &ws) == 8) {
     a.batch = batch, a.n_q = n_q, a.n_k = n_k, a.d = d, a.causal = mask, a.window = window, a.ws_bytes = ws;
     Params p = {};
-    p.batch = (int)batch, p.n_q = (int)n_q, p.n_k = (int)n_k, p.d = (int)d, p.causal = mask != 0;
+    p.batch = (int)batch, p.n_q = (int)n_q, p.n_k = (int)n_k, p.d = (int)d, p.causal = mask != 0, p.tile_major = p.tile_major_k = p.causal, p.n_split = p.n_split_k = 1;
     rules::mask_params(mask, window, n_q, n_k, &p.mask_off, &p.window);
     if (!strcmp(what, "joint")) {
       int x, y;
@@ -52,7 +52,6 @@ int main() {
       for (Small w : {Small::forward, Small::backward, Small::double_backward}) printf("%d ", rules::small_waves(w, batch, n_q, n_k, d, mask, window));
       printf("\n");
     } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
-      p.tile_major = p.tile_major_k = p.causal;
       rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &p.n_split, &p.n_split_k);
       rules::grads_order(&a, true, true, p);
       printf("%d %d\n", p.tile_major, p.tile_major_k);
@@ -101,13 +100,18 @@ def test_splits_of_a_shared_launch(ask, shape, splits):
 
 
 @pytest.mark.parametrize("shape,order", [((1, 19472, 19472, 64, CAUSAL, 0), (1, 1)), ((2, 18809, 18809, 64, CAUSAL, 0), (1, 1)), ((32, 16384, 16384, 64, CAUSAL, 0), (0, 0)),
-                                         ((1, 30000, 30000, 64, CAUSAL, 5000), (0, 0)), ((1, 19472, 19472, 128, CAUSAL, 0), (0, 0)), ((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 1)), ((1, 4000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)),
+                                         ((1, 30000, 30000, 64, CAUSAL, 5000), (0, 0)), ((1, 19472, 19472, 128, CAUSAL, 0), (0, 0)), ((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 1)), ((8, 2000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)),
                                          ((2, 9000, 17000, 64, BOTTOM_RIGHT, 500), (1, 0)), ((2, 9000, 17000, 128, BOTTOM_RIGHT, 0), (1, 0)),
                                          ((4, 16383, 16383, 128, CAUSAL, 0), (1, 1)), ((1, 20000, 20000, 64, NONE, 0), (0, 0))])
 def test_order_of_a_shared_launch(ask, shape, order):
     """Slices of 16384 rows or more go one after the other (0) instead of tile by tile together (1), each side by its own length, except at d = 64 where
     the two sides take turns."""
     assert tuple(ask("order", *shape, PLENTY)) == order
+
+
+def test_splits_prefer_sweeps_that_take_turns(ask):
+    """Bottom-right 4 x 5012 x 9866: 4 | 1 splits would run one sweep after the other (524 us), 2 | 2 tile by tile in turn (460 us)."""
+    assert ask("joint", 4, 5012, 9866, 64, BOTTOM_RIGHT, 0, PLENTY)[:2] == [2, 2]
 
 
 @pytest.mark.parametrize("d", [64, 128])
