@@ -13,6 +13,7 @@
 // results are merged through LDS in a fixed order. dQ and dK, dV share a launch unless each fills the GPU (launch_bwd).
 #include <type_traits>
 
+#include "fhog_rules.h"
 #include "fhog_split_util.h"
 
 namespace fhog {
@@ -339,33 +340,25 @@ hipError_t launch_side(const AttnParams& p, int waves, hipStream_t s) {
 }
 
 // dQ and dK, dV side by side fill CUs for each other, as passes 3 and 4 do in fhog_split.hip, and the rule for waves on the same rows is of
-// the same kind. The price is the row sums d, which the sweep for dK, dV then takes once per key block: nothing at d = 32, 3 to 9 % on
-// fp32 tensors of d = 64 and 128, whose launches of full rounds (256 workgroups each) go one after the other. First backward, us, two
-// launches (the rule before) -> one launch with four | two | one waves on the same rows:
+// the same kind. The price is the row sums d, which the sweep for dK, dV then takes once per key block: nothing at d = 32 where the shared launch
+// leaves CUs idle, up to a fifth where it does not or the key side is the longer one; 3 to 9 % on fp32 tensors of d = 64 and 128, whose launches of full rounds (256 workgroups each) go one after the other (split_bwd_waves). First backward,
+// us, two launches (the rule before) -> one launch with four | two | one waves on the same rows:
 //   bf16 d = 32   2 x 256 11.7 -> 7.9 | 9.8 | 12; causal 16 x 1024 56 -> 28 | 34 | 38, 64 x 1024 59 -> 81 | 57 | 49; no mask 16 x 1024 53 -> 37 | 35 | 37
 //   fp32 d = 64   2 x 256 27 -> 16 | 21 | 31; causal 16 x 1024 181 -> 99 | 83 | 106, 32 x 1024 182 -> 192 | 135 | 122; no mask 48 x 1024
 //                 309 -> - | 345 | 283, 64 x 1024 338 -> - | 459 | 362
 //   fp32 d = 128  2 x 256 66 -> - | 46 | 59; causal 16 x 1024 325 -> - | 188 | 217, 64 x 1024 408 -> - | 620 | 428; no mask 64 x 1024 609 -> - | 989 | 631
 template <typename T, int D, int MASK>
 hipError_t launch_bwd(const AttnParams& p, hipStream_t s) {
-  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
-  const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
-  if (sizeof(T) * D < 512 && lopsided(p.n_q, p.n_k, MASK != MASK_NONE ? (int64_t)p.window : (int64_t)p.n_q + p.n_k) && groups > 64) {   // as in fhog_split.hip
-    const hipError_t e = launch_side<T, D, MODE_BWD_Q, MASK>(p, waves_of_side(g_q, p.n_k), s);
-    return e != hipSuccess ? e : launch_side<T, D, MODE_BWD_K, MASK>(p, waves_of_side(g_k, p.n_q), s);
+  const int waves = rules::split_bwd_waves(p, sizeof(T));
+  if (waves == 0) {
+    const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch;
+    const hipError_t e = launch_side<T, D, MODE_BWD_Q, MASK>(p, rules::waves_of_side(g_q, p.n_k), s);
+    return e != hipSuccess ? e : launch_side<T, D, MODE_BWD_K, MASK>(p, rules::waves_of_side(g_k, p.n_q), s);
   }
   if constexpr (lds_bytes<T, D, MODE_BWD_K, 4>() <= 160 * 1024) {
-    if (groups <= (triangle && p.n_k >= 1024 ? (D == 32 ? 256 : 128) : D == 32 ? 128 : 64)) return launch_bwd_ws<T, D, MASK, 4>(p, s);
+    if (waves == 4) return launch_bwd_ws<T, D, MASK, 4>(p, s);
   }
-  if (groups < (triangle ? (D == 32 ? 512 : 257) : D == 32 ? 320 : 129)) return launch_bwd_ws<T, D, MASK, 2>(p, s);
-  if constexpr (D > 32) {
-    const int64_t rounds = (groups + 255) / 256, apart = (g_q + 255) / 256 + (g_k + 255) / 256;
-    if (triangle ? groups >= (p.n_k >= 1024 ? 1024 : 512) : 12 * apart < 13 * rounds) {
-      const hipError_t e = launch_ws<T, D, MODE_BWD_Q, MASK, 1>(p, s);
-      return e != hipSuccess ? e : launch_ws<T, D, MODE_BWD_K, MASK, 1>(p, s);
-    }
-  }
-  return launch_bwd_ws<T, D, MASK, 1>(p, s);
+  return waves >= 2 ? launch_bwd_ws<T, D, MASK, 2>(p, s) : launch_bwd_ws<T, D, MASK, 1>(p, s);
 }
 
 template <typename T, int D>

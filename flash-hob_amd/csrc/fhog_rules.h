@@ -49,9 +49,10 @@ struct Work {
   double live = 0, sum = 0;
   int64_t groups = 0, longest = 0;
 };
-inline Work work_of(const fhog_bwdbwd_args* a, const Params& p, bool kside) {
+template <typename P>   // Params or AttnParams
+inline Work work_of(const P& p, bool kside) {
   Work w;
-  const int64_t n_sta = kside ? a->n_k : a->n_q, n_str = kside ? a->n_q : a->n_k;
+  const int64_t n_sta = kside ? p.n_k : p.n_q, n_str = kside ? p.n_q : p.n_k;
   w.groups = (n_sta + 127) / 128;
   const int64_t step = (w.groups + 63) / 64;
   int64_t seen = 0;
@@ -81,7 +82,7 @@ inline Work work_of(const fhog_bwdbwd_args* a, const Params& p, bool kside) {
 // (combining) -> 37.0 + 7.4, pass 4 with 2 -> 1 52.2 + 14.5 -> 56.7. The other passes and d = 64 run two workgroups on a CU.
 inline int split_up_to(int most, const fhog_bwdbwd_args* a, const Params& p, int pass) {
   if (most == 1 || a->d != 128 || (pass != FHOG_PASS_DQ_DDO && pass != FHOG_PASS_DK_DV)) return most;
-  const Work w = work_of(a, p, pass == FHOG_PASS_DK_DV);
+  const Work w = work_of(p, pass == FHOG_PASS_DK_DV);
   if (w.live == 0) return 1;
   int best = 1;
   double best_cost = 0;
@@ -203,7 +204,7 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass,
   *s_q = *s_k = 1;
   const int64_t have = a->ws_bytes - (int64_t)stats_bytes(a);
   if ((most_q == 1 && most_k == 1) || have <= 0) return;
-  const Work q = work_of(a, p, false), k = work_of(a, p, true);
+  const Work q = work_of(p, false), k = work_of(p, true);
   if (q.live == 0 || k.live == 0) return;
   const bool two = a->d == 64;
   const double fixed = two ? 2 : 4, tile_us = two ? 0.87 : 1.9, alone = 1.25;
@@ -326,6 +327,91 @@ inline int small_waves(Small what, int64_t batch, int64_t n_q, int64_t n_k, int6
   return groups <= 256 && d == 64 && uneven && tiles <= 32 ? 2 : 0;
 }
 inline int small_waves(Small what, const fhog_attn_args* a) { return small_waves(what, a->batch, a->n_q, a->n_k, a->d, a->causal, a->window); }
+
+
+// ---- split products: the query-tiled and the key-tiled sweep of a backward pass (fhog_split.hip, fhog_attn_split.hip) ----------------------
+// In one launch the two fill CUs for each other; each in a launch of its own (0 below) a side that is far shorter, whose few workgroups have a long
+// stream each, gets as many waves on the same rows as it needs by itself. waves_of_side: those, by its 128-row workgroups.
+inline int waves_of_side(int64_t groups, int64_t streamed) { return groups < 64 && streamed > 64 ? 4 : groups < 128 && streamed > 32 ? 2 : 1; }
+// Whether one side streams four times as many rows as the other
+inline bool lopsided(int64_t n_q, int64_t n_k, int64_t window) {
+  const int64_t q = n_k < window ? n_k : window, k = n_q < window ? n_q : window;   // rows that a query and a key see, at most
+  return q >= 4 * k || k >= 4 * q;
+}
+
+// The number of workgroups says what a shared launch gives where the two sides are alike. Where they are not, the two ways are reckoned up, and two
+// launches taken where they are clearly shorter. us, one launch by the number of workgroups -> apart: first backward fp32 d = 64 2 x 7490 x 2123 731 -> 383,
+// d = 128 1 x 199 x 16395 1776 -> 1235, 2 x 13595 x 68 2141 -> 1621, bf16 d = 32 1 x 7412 x 86 118 -> 88, causal 43 x 3112 291 -> 234; double-backward
+// bf16 d = 32 2 x 2417 x 9036 419 -> 303. Of 5400 shapes of 1 to 64 slices with 16 to 20000 rows 186 were more than 3 % slower than with two launches
+// and waves_of_side throughout (up to 1.5 times), 63 are (up to 1.15 times).
+// What the two ways cost, in steps of one wave's tile of the query side with one wave on 32 rows
+struct SplitCost {
+  double two, four;           // a step with two and four waves on the same rows
+  double key;                 // a step of the key side
+  double own, own_waves;      // in a shared launch, where that side takes d = rowsum(O dO) itself: with one and with more waves on the same rows
+  double alone;               // a workgroup's step without company, of those that share a CU
+  double fixed, launch;       // to start and to store; another launch
+  double heaviest;            // how long the longest workgroup has company
+  double margin;              // two launches have to be shorter than this part of the shared one
+};
+constexpr SplitCost kFirstBackward = {1.05, 1.3, 1.25, 1.25, 1.6, 1.3, 0.9, 2.5, 1.65, 0.75}, kDoubleBackward = {1.35, 1.85, 1, 1, 1, 1.07, 2, 3, 1.6, 0.9};
+
+// One launch: the query side (wq waves on the same rows; 0: not in it), then the key side
+inline double split_launch(const Work& q, const Work& k, int64_t batch, int wq, int wk, bool two_on_a_cu, const SplitCost& c) {
+  const int waves = wq > wk ? wq : wk;
+  const bool two = two_on_a_cu && waves == 1;
+  const auto length = [&](double tiles, int w, bool key) {
+    return tiles / w * (w == 4 ? c.four : w == 2 ? c.two : 1) * (key ? c.key : 1) * (key && wq ? (w == 1 ? c.own : c.own_waves) : 1) + c.fixed;
+  };
+  const int64_t nq = q.groups * batch * wq, nk = k.groups * batch * wk;
+  const double lq = wq ? length(q.sum / (double)q.groups, wq, false) : 0, lk = wk ? length(k.sum / (double)k.groups, wk, true) : 0;
+  const double hq = wq ? length((double)((q.longest + wq - 1) / wq * wq), wq, false) : 0, hk = wk ? length((double)((k.longest + wk - 1) / wk * wk), wk, true) : 0;
+  const double heaviest = (hq > hk ? hq : hk) * (!two ? 1 : nq + nk <= 256 ? c.alone : c.heaviest);
+  const double all = two ? makespan_two(nq, lq, nk, lk, c.alone) : makespan(nq, lq, nk, lk);
+  return all > heaviest ? all : heaviest;
+}
+
+template <typename P>
+inline bool apart_is_faster(const P& p, int waves, int most_waves, bool two_on_a_cu, const SplitCost& c) {
+  const Work q = work_of(p, false), k = work_of(p, true);
+  const int64_t g_q = q.groups * p.batch, g_k = k.groups * p.batch;
+  int wq = waves_of_side(g_q, p.n_k), wk = waves_of_side(g_k, p.n_q);
+  wq = wq < most_waves ? wq : most_waves, wk = wk < most_waves ? wk : most_waves;
+  return split_launch(q, k, p.batch, wq, 0, two_on_a_cu, c) + split_launch(q, k, p.batch, 0, wk, two_on_a_cu, c) + c.launch <
+         c.margin * split_launch(q, k, p.batch, waves, waves, two_on_a_cu, c);
+}
+
+// Waves on the same 32 rows for passes 3 and 4 in one launch, or 0 for two launches: four waves while that gives one workgroup per CU, two as long as the
+// workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. The figures are those of launch_grads (fhog_split.hip).
+inline int split_grads_waves(const Params& p, int bytes) {
+  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
+  const bool triangle = p.causal && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  if (bytes * p.d < 512 && groups > 64 && lopsided(p.n_q, p.n_k, p.window)) return 0;
+  const int waves = groups <= 64 || (p.d == 32 && triangle && groups <= 128 && p.n_k >= 1024) ? 4 : groups < (triangle ? (p.d == 32 ? 512 : 257) : 160) ? 2 : 1;
+  const bool counted = p.d == 32 || (bytes == 4 && p.d == 64);   // 16-bit tensors of d = 64 and 128 were not; d = 128 has one wave at all sizes
+  return counted && apart_is_faster(p, waves, 4, p.d == 32, kDoubleBackward) ? 0 : waves;
+}
+
+// ... and for the first backward, whose key side then takes the row sums d itself. The figures are those of launch_bwd (fhog_attn_split.hip).
+inline int split_bwd_waves(const AttnParams& p, int bytes) {
+  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
+  const bool triangle = p.causal && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
+  const bool fp32_128 = bytes * p.d >= 512;   // four waves do not fit the LDS
+  if (!fp32_128 && groups > 64 && lopsided(p.n_q, p.n_k, p.window)) return 0;
+  int waves = 1;
+  if (!fp32_128 && groups <= (triangle && p.n_k >= 1024 ? (p.d == 32 ? 256 : 128) : p.d == 32 ? 128 : 64)) waves = 4;
+  else if (groups < (triangle ? (p.d == 32 ? 512 : 257) : p.d == 32 ? 320 : 129)) waves = 2;
+  if (waves == 1 && p.d > 32) {
+    const int64_t rounds = (groups + 255) / 256, apart = (g_q + 255) / 256 + (g_k + 255) / 256;
+    if (triangle ? groups >= (p.n_k >= 1024 ? 1024 : 512) : 12 * apart < 13 * rounds) return 0;
+  }
+  if (bytes == 4) return apart_is_faster(p, waves, fp32_128 ? 2 : 4, p.d == 32, kFirstBackward) ? 0 : waves;
+  // 16-bit tensors of d = 32, where taking d costs the key side a fifth
+  if (p.causal) return waves == 1 && groups >= 1450 && 2 * (int64_t)p.window >= p.n_k && 2 * (int64_t)p.mask_off <= p.n_k ? 0 : waves;
+  const int64_t n_q = p.n_q, n_k = p.n_k;
+  const bool long_key_side = waves == 4 ? n_q >= 2 * n_k && n_q - n_k >= 740 : waves == 2 ? 2 * n_q >= 3 * n_k : 2 * n_q >= 5 * n_k || (groups >= 1000 && 4 * n_q >= 5 * n_k);
+  return long_key_side ? 0 : waves;
+}
 
 }  // namespace rules
 }  // namespace fhog

@@ -27,6 +27,7 @@
 //   dS = scale P u, ddP = P w, dS' = scale (P E' + ddP u)
 #include <type_traits>
 
+#include "fhog_rules.h"
 #include "fhog_split_util.h"
 
 namespace fhog {
@@ -483,10 +484,10 @@ hipError_t launch_grads_most(const Params& p, int sides, hipStream_t s) {
 }
 
 template <typename T, int D, int MASK>
-hipError_t launch_grads_side(const Params& p, int side, int waves, hipStream_t s) {
-  return waves == 4   ? launch_grads_most<T, D, MASK, 4>(p, side, s)
-         : waves == 2 ? launch_grads_most<T, D, MASK, 2>(p, side, s)
-                      : launch_grads_most<T, D, MASK, 1>(p, side, s);
+hipError_t launch_grads_side(const Params& p, int sides, int waves, hipStream_t s) {
+  return waves == 4   ? launch_grads_most<T, D, MASK, 4>(p, sides, s)
+         : waves == 2 ? launch_grads_most<T, D, MASK, 2>(p, sides, s)
+                      : launch_grads_most<T, D, MASK, 1>(p, sides, s);
 }
 
 // Passes 3 and 4 side by side are faster than one after the other whatever the size: their workgroups fill CUs for each other where
@@ -498,23 +499,19 @@ hipError_t launch_grads_side(const Params& p, int side, int waves, hipStream_t s
 //   fp32 d = 128  (one wave at all sizes, LDS) 2 x 256 234 -> 133; causal 16 x 2048 2104 -> 1440; 32 x 2048 2383 -> 2381
 //   bf16 d = 32   2 x 256 20 -> 13 | - | -; causal 16 x 1024 99 -> 59 | 47 | 56, 32 x 1024 114 -> 119 | 90 | 96, 64 x 1024 127 -> 218 | 160 | 121
 // A side that is far shorter than the other has few workgroups with a long stream each, which nothing fills up: the two sides go
-// apart then, each with as many waves on the same rows as it needs by itself. Hessian-vector products (here and in fhog_attn_split.hip),
-// us, one launch -> apart, by how many times as many rows one side streams: bf16 d = 32 3.1 times (16 x 512 x 1600) 142 -> 147, 5 times
-// (8 x 512 x 2560) 178 -> 149, the other way round 194 -> 147, 30 times (4 x 200 x 6000) 413 -> 243; fp32 d = 64 3.1 times 370 -> 393,
+// apart then (split_grads_waves), each with as many waves on the same rows as it needs by itself. Hessian-vector products (here and in
+// fhog_attn_split.hip), us, one launch -> apart, by how many times as many rows one side streams: bf16 d = 32 3.1 times (16 x 512 x 1600) 142 -> 147, 5
+// times (8 x 512 x 2560) 178 -> 149, the other way round 194 -> 147, 30 times (4 x 200 x 6000) 413 -> 243; fp32 d = 64 3.1 times 370 -> 393,
 // 5 times 740 -> 609, 8 times 897 -> 874. fp32 d = 128, which has one wave at all sizes, 8 times 2260 -> 2373: not there.
 template <typename T, int D, int MASK>
 hipError_t launch_grads(const Params& p, int sides, hipStream_t s) {
-  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch, groups = g_q + g_k;
-  const bool triangle = MASK != MASK_NONE && (p.window < p.n_k || 2 * (int64_t)p.mask_off <= p.n_k);
-  if (sizeof(T) * D < 512 && lopsided(p.n_q, p.n_k, MASK != MASK_NONE ? (int64_t)p.window : (int64_t)p.n_q + p.n_k) && groups > 64) {
-    hipError_t e = hipSuccess;
-    if (sides & 1) e = launch_grads_side<T, D, MASK>(p, 1, waves_of_side(g_q, p.n_k), s);
-    if (e == hipSuccess && (sides & 2)) e = launch_grads_side<T, D, MASK>(p, 2, waves_of_side(g_k, p.n_q), s);
-    return e;
-  }
-  if (groups <= 64 || (D == 32 && triangle && groups <= 128 && p.n_k >= 1024)) return launch_grads_most<T, D, MASK, 4>(p, sides, s);
-  if (groups < (triangle ? (D == 32 ? 512 : 257) : 160)) return launch_grads_most<T, D, MASK, 2>(p, sides, s);
-  return launch_grads_most<T, D, MASK, 1>(p, sides, s);
+  const int waves = rules::split_grads_waves(p, sizeof(T));
+  if (waves) return launch_grads_side<T, D, MASK>(p, sides, waves, s);
+  const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch;
+  hipError_t e = hipSuccess;
+  if (sides & 1) e = launch_grads_side<T, D, MASK>(p, 1, rules::waves_of_side(g_q, p.n_k), s);
+  if (e == hipSuccess && (sides & 2)) e = launch_grads_side<T, D, MASK>(p, 2, rules::waves_of_side(g_k, p.n_q), s);
+  return e;
 }
 
 template <typename T, int D>

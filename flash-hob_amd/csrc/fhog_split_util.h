@@ -250,13 +250,5 @@ __device__ __forceinline__ void store_rows(T* row, const f32x16_t (&acc)[D / 32]
     }
 }
 
-// Of two sweeps that could share a launch, query-tiled and key-tiled: whether one streams four times as many rows as the other
-inline bool lopsided(int64_t n_q, int64_t n_k, int64_t window) {
-  const int64_t q = n_k < window ? n_k : window, k = n_q < window ? n_q : window;   // rows that a query and a key see, at most
-  return q >= 4 * k || k >= 4 * q;
-}
-// Waves on the same 32 rows for a sweep that has the GPU to itself, by its 128-row workgroups
-inline int waves_of_side(int64_t groups, int64_t streamed) { return groups < 64 && streamed > 64 ? 4 : groups < 128 && streamed > 32 ? 2 : 1; }
-
 }  // namespace splitk
 }  // namespace fhog

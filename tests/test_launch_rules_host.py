@@ -47,6 +47,10 @@ int main() {
       printf("%d %d %d %d\n", x, y, u, v);
     } else if (!strcmp(what, "instead")) {
       printf("%d\n", rules::splits_instead(&a, p, FHOG_IMPL_BF16));
+    } else if (!strcmp(what, "split")) {   // split products, ws: bytes of an element; first backward and double-backward
+      AttnParams f = {};
+      f.batch = p.batch, f.n_q = p.n_q, f.n_k = p.n_k, f.d = p.d, f.causal = p.causal, f.mask_off = p.mask_off, f.window = p.window;
+      printf("%d %d\n", rules::split_bwd_waves(f, (int)ws), rules::split_grads_waves(p, (int)ws));
     } else if (!strcmp(what, "small")) {   // waves on the same rows: forward, first backward, double-backward
       using rules::Small;
       for (Small w : {Small::forward, Small::backward, Small::double_backward}) printf("%d ", rules::small_waves(w, batch, n_q, n_k, d, mask, window));
@@ -143,3 +147,13 @@ def test_schedules_without_a_split_form_are_replaced_where_that_is_faster(ask, s
 def test_small_workgroups(ask, shape, waves):
     """Both sides of the lines that windows, few keys and lopsided shapes add to the rule."""
     assert tuple(ask("small", *shape, 0)) == waves
+
+
+@pytest.mark.parametrize("bytes_,shape,waves", [
+    (4, (2, 7490, 2123, 64, NONE, 0), (0, 0)), (4, (4, 2048, 2048, 64, NONE, 0), (2, 2)), (4, (1, 199, 16395, 128, NONE, 0), (0, 2)), (4, (2, 13595, 68, 128, NONE, 0), (0, 1)),
+    (4, (32, 2048, 2048, 128, CAUSAL, 0), (0, 1)), (4, (2, 256, 256, 64, NONE, 0), (4, 4)), (2, (64, 1024, 1024, 32, CAUSAL, 0), (1, 1)), (2, (44, 2112, 2112, 32, CAUSAL, 0), (0, 1)),
+    (2, (44, 2112, 2112, 32, CAUSAL, 700), (1, 1)), (2, (1, 1799, 96, 32, NONE, 0), (0, 4)), (2, (14, 93, 17, 32, NONE, 0), (4, 4)), (2, (40, 4667, 1344, 32, NONE, 0), (0, 1)),
+    (2, (40, 2000, 2000, 32, NONE, 0), (1, 1)), (2, (2, 2417, 9036, 32, NONE, 0), (2, 0)), (2, (8, 512, 2560, 32, NONE, 0), (0, 0)), (2, (8, 512, 2560, 128, NONE, 0), (0, 0))])
+def test_sweeps_of_split_products_in_one_launch_or_apart(ask, bytes_, shape, waves):
+    """Waves on the same rows in the shared launch of first backward and double-backward, 0: two launches."""
+    assert tuple(ask("split", *shape, bytes_)) == waves
