@@ -196,8 +196,9 @@ constexpr int64_t kMostParts = 2 * 131072 * (int64_t)sizeof(float);   // bytes o
 // fp16 d = 64 no mask 1 x 8192 369, 232, 203, 211; 1 x 16384 798, 727, 738, 750; 2 x 4096 178, 123, 115, 123; 4 x 4096 208, 203, 211, 229; 8 x 2048 110, 114,
 // 123, 142; causal 1 x 16384 683, 611, 499, 439; 2 x 8192 344, 244, 225, 245; 8 x 2048 99, 81, 85, 113. Splits of one side alone at 1 x 16384: 2 | 1 950.
 // Over 640 shapes of 1 to 64 slices with 16 to 20000 rows, against the best pair of each: 2.2 % too slow with one workgroup to a CU -> 0.9 %.
-// Under a mask the light end of one sweep and the heavy start of the other meet only where the two take turns: 1000 masked shapes, against the best pair of
-// each, without -> with 10 % on pairs that do not: d = 64 2.1 % -> 1.8 % too slow, d = 128 1.9 % -> 1.2 %; bottom-right 2 x 5887 x 14150 8 | 1 525, 4 | 2 412.
+// Under a mask the light end of one sweep and the heavy start of the other meet only where both have about as many workgroups: 1000 masked shapes, against
+// the best pair of each, without -> with 10 % on pairs beyond 1.5 to 1: d = 64 2.1 % -> 1.7 % too slow, d = 128 1.9 % -> 0.8 %; bottom-right
+// d = 64 4 x 5012 x 9866 4 | 1 524, 2 | 1 471, d = 128 1 x 25434 x 25726 4 | 1 1924, 1 | 1 1645.
 // q_pass: 3, or 7, which does not split.
 inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass, int* s_q, int* s_k) {
   const int most_q = wanted_split(a, FHOG_IMPL_BF16, q_pass), most_k = wanted_split(a, FHOG_IMPL_BF16, FHOG_PASS_DK_DV);
@@ -227,7 +228,8 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass,
       }
       if (longest > cost) cost = longest;
       if (part > 0) cost += (4 + (double)part / 2.5e6) / tile_us;   // a launch, and the partial results written and read
-      if (p.causal && 2 * (int64_t)p.window >= a->n_k && !mixed_order(p, (q.groups * a->batch * x + 7) / 8 * 8, (k.groups * a->batch * y + 7) / 8 * 8)) cost *= 1.1;
+      const int64_t of_q = q.groups * x, of_k = k.groups * y;
+      if (p.causal && 2 * (int64_t)p.window >= a->n_k && (2 * of_q > 3 * of_k || 2 * of_k > 3 * of_q)) cost *= 1.1;
       if ((x == 1 && y == 1) || cost < best) best = cost, *s_q = x, *s_k = y;
     }
 }

@@ -113,9 +113,10 @@ def test_order_of_a_shared_launch(ask, shape, order):
     assert tuple(ask("order", *shape, PLENTY)) == order
 
 
-def test_splits_prefer_sweeps_that_take_turns(ask):
-    """Bottom-right 4 x 5012 x 9866: 4 | 1 splits would run one sweep after the other (524 us), 2 | 2 tile by tile in turn (460 us)."""
-    assert ask("joint", 4, 5012, 9866, 64, BOTTOM_RIGHT, 0, PLENTY)[:2] == [2, 2]
+@pytest.mark.parametrize("shape,splits", [((4, 5012, 9866, 64), (2, 1)), ((1, 25434, 25726, 128), (1, 1))])
+def test_splits_under_a_mask_give_both_sweeps_as_many_workgroups(ask, shape, splits):
+    """us: 4 | 1 splits 524 and 1924, these 471 and 1645."""
+    assert tuple(ask("joint", *shape, BOTTOM_RIGHT, 0, PLENTY)[:2]) == splits
 
 
 @pytest.mark.parametrize("d", [64, 128])
