@@ -411,7 +411,9 @@ inline int split_bwd_waves(const AttnParams& p, int bytes) {
   // 16-bit tensors of d = 32, where taking d costs the key side a fifth
   if (p.causal) return waves == 1 && groups >= 1450 && 2 * (int64_t)p.window >= p.n_k && 2 * (int64_t)p.mask_off <= p.n_k ? 0 : waves;
   const int64_t n_q = p.n_q, n_k = p.n_k;
-  const bool long_key_side = waves == 4 ? n_q >= 2 * n_k && n_q - n_k >= 740 : waves == 2 ? 2 * n_q >= 3 * n_k : 2 * n_q >= 5 * n_k || (groups >= 1000 && 4 * n_q >= 5 * n_k);
+  const bool long_key_side = waves == 4   ? n_q >= 2 * n_k && n_q - n_k >= 740
+                             : waves == 2 ? 2 * n_q >= 3 * n_k && n_q - n_k >= 250
+                                          : (2 * n_q >= 5 * n_k && n_q - n_k >= 250) || (groups >= 1000 && 4 * n_q >= 5 * n_k);
   return long_key_side ? 0 : waves;
 }
 
