@@ -158,7 +158,7 @@ int run_pass(const fhog_bwdbwd_args* a, const fhog::Params& base, int impl, int 
   if (impl == FHOG_IMPL_BF16 && pass == FHOG_PASS_DK_DV) return run_grads(a, base, 0, true, s);
   fhog::Params p = base;
   p.n_split = launch_split_of(a, p, impl, pass);
-  if (pass != FHOG_PASS_DD && slice_order(a, p, pass == FHOG_PASS_DK_DV ? a->n_k : a->n_q)) p.tile_major = 0;
+  pass_order(a, pass, p);
   p.part = reinterpret_cast<float*>(reinterpret_cast<char*>(a->ws) + stats_bytes(a));
   hipError_t e;
   if (pass == FHOG_PASS_D)

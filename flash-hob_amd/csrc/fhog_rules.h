@@ -239,7 +239,12 @@ inline void joint_splits(const fhog_bwdbwd_args* a, const Params& p, int q_pass,
 // and one slice after the other keeps the fetched bytes near the algorithmic ones (measured on N = 16384: 2.2-2.6x
 // instead of 4-10x, sweeps b, 3 and 4 0.1-3 % faster, the dd sweep with its three workgroups per CU 4 % slower).
 inline bool slice_order(const fhog_bwdbwd_args* a, const Params& p, int64_t rows) { return tuning().order < 0 && p.causal && rows >= 16384; }
-// Of passes 3 (or 7) and 4, run alone or in a shared launch. d = 64: where the two take turns tile by tile (mixed_order) they do so at any length, unless a
+// Of a statistics sweep, and of the split products' passes 3 and 4 in whatever launch: each side by its own length
+inline void pass_order(const fhog_bwdbwd_args* a, int pass, Params& p) {
+  if (pass != FHOG_PASS_DD && slice_order(a, p, a->n_q)) p.tile_major = 0;
+  if (slice_order(a, p, a->n_k)) p.tile_major_k = 0;
+}
+// Of the 16-bit kernels' passes 3 (or 7) and 4, run alone or in a shared launch. d = 64: where the two take turns tile by tile (mixed_order) they do so at any length, unless a
 // window makes their work even: one sweep after the other, the second one's heavy tiles come last. Double-backward, us, slice order -> turns (two launches):
 // bf16 causal 1 x 17000 612 -> 544 (550), 1 x 35801 2358 -> 2020 (2058), 2 x 18809 1256 -> 1097 (1125); window 5000 1 x 30000 431 -> 440.
 inline void grads_order(const fhog_bwdbwd_args* a, bool q_side, bool k_side, Params& p) {

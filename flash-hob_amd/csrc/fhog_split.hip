@@ -106,7 +106,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, p.tile_major, bh, tile, MASK != MASK_NONE && D < 64 && WS == 1, id)) return;
+  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, KSIDE ? p.tile_major_k : p.tile_major, bh, tile, MASK != MASK_NONE && D < 64 && WS == 1, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;

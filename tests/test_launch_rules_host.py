@@ -45,6 +45,9 @@ int main() {
       a.ws_bytes = (int64_t)rules::workspace_hint(&a, p, FHOG_IMPL_BF16);
       rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &x, &y);
       printf("%d %d %d %d\n", x, y, u, v);
+    } else if (!strcmp(what, "split_order")) {
+      rules::pass_order(&a, kPassGrads, p);
+      printf("%d %d\n", p.tile_major, p.tile_major_k);
     } else if (!strcmp(what, "instead")) {
       printf("%d\n", rules::splits_instead(&a, p, FHOG_IMPL_BF16));
     } else if (!strcmp(what, "split")) {   // split products, ws: bytes of an element; first backward and double-backward
@@ -158,3 +161,9 @@ def test_small_workgroups(ask, shape, waves):
 def test_sweeps_of_split_products_in_one_launch_or_apart(ask, bytes_, shape, waves):
     """Waves on the same rows in the shared launch of first backward and double-backward, 0: two launches."""
     assert tuple(ask("split", *shape, bytes_)) == waves
+
+
+@pytest.mark.parametrize("shape,order", [((2, 9000, 17000, 64, BOTTOM_RIGHT, 0), (1, 0)), ((2, 17000, 17000, 64, CAUSAL, 0), (0, 0)), ((2, 9000, 9000, 32, CAUSAL, 0), (1, 1)),
+                                         ((2, 17000, 9000, 32, NONE, 0), (0, 0))])
+def test_order_of_a_shared_launch_of_split_products(ask, shape, order):
+    assert tuple(ask("split_order", *shape, 0)) == order
