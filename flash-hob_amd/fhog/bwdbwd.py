@@ -124,6 +124,8 @@ def _build_args(Q, K, V, O, dO, ddQ, ddK, ddV, L, scale, causal, impl, outs, ws,
             raise ValueError(f"{n} has shape {tuple(t.shape)}, expected {tuple(like.shape)}")
     if K.shape[0] != Q.shape[0] or K.shape[2] != Q.shape[2]:
         raise ValueError(f"K has shape {tuple(K.shape)}, expected ({Q.shape[0]}, N_K, {Q.shape[2]})")
+    for t, like in zip(outs, (Q, K, K, Q)):     # the outputs are written by the strides of Q and K
+        assert t.shape == like.shape and t.stride() == like.stride()
     a = _lib.BwdBwdArgs()
     a.q, a.k, a.v, a.o, a.dO = Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dO.data_ptr()
     a.ddq, a.ddk, a.ddv = ddQ.data_ptr(), ddK.data_ptr(), ddV.data_ptr()
@@ -277,7 +279,9 @@ class BwdBwdPlan:
         batch, n_q, _ = q3.shape
         lse = L.reshape(batch, n_q).to(torch.float32).contiguous()
         self.keep = (q3, k3, v3, o3, do3, ddq3, ddk3, ddv3, lse)
-        self.outs = (torch.empty_like(q3), torch.empty_like(k3), torch.empty_like(v3), torch.empty_like(q3))
+        # empty_like would pack rows that are padded
+        self.outs = tuple(torch.empty_strided(t.shape, t.stride(), dtype=t.dtype, device=t.device)
+                          for t in (q3, k3, v3, q3))
         self.args = _build_args(q3, k3, v3, o3, do3, ddq3, ddk3, ddv3, lse, scale, causal, _IMPLS[impl], self.outs, None, schedule_code(schedule, fused_stats), window)
         with torch.cuda.device(Q.device):
             self.ws_all = _workspace(self.args, Q.device, split)   # d | dd | b, then partial results of split launches

@@ -751,3 +751,24 @@ def test_autograd_chain_reaches_hip_double_backward(causal):
     ref = penalty(lambda a, b, c: torch.nn.functional.scaled_dot_product_attention(a, b, c, is_causal=causal))
     for a, b in zip(ours, ref):
         assert normalised_max_error(a, b) < 1e-4
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128), (torch.float32, 32)])
+def test_plan_on_padded_rows(dtype, d, batch):
+    """A plan allocates its outputs with the strides of its inputs, which the library writes them by."""
+    from fhog import BwdBwdPlan
+    x = with_caches(make_case(batch, 200, 333, d, dtype, seed=84, grad_std=0.1), d ** -0.5, False)
+
+    def padded(t):
+        wide = torch.zeros(*t.shape[:-1], d + 16, dtype=t.dtype, device=t.device)
+        wide[..., :d] = t
+        return wide[..., :d]
+
+    names = ("Q", "K", "V", "O", "dO", "ddQ", "ddK", "ddV")
+    dense = BwdBwdPlan(*(x[n] for n in names), x["L"], d ** -0.5)
+    wide = BwdBwdPlan(*(padded(x[n]) for n in names), x["L"], d ** -0.5)
+    for t, like in zip(wide.outs, (x["Q"], x["K"], x["V"], x["Q"])):
+        assert t.shape == like.shape and t.stride() == padded(like).stride()
+    for a, b in zip(dense.run(), wide.run()):
+        assert torch.equal(a, b)
