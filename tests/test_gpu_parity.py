@@ -284,7 +284,9 @@ def test_bf16_chain_writes_row_sums_d_itself(shape, dtype, schedule):
 def test_split_streamed_side_matches_the_unsplit_launch(case, schedule):
     """Few (batch*head) slices: with the workspace of fhog_bwdbwd_workspace_hint every pass splits its
     streamed side over several workgroups (fp32 partial results, added by a second kernel). Same gate against the
-    fp64 oracle as the unsplit launch, row statistics equal up to summation order, outputs within a 16-bit rounding."""
+    fp64 oracle as the unsplit launch, row statistics equal up to summation order, outputs within a 16-bit rounding.
+    [fused_stats]: all but 130 x 4100 and causal 2048, d = 128, run the kernels for small launches, which do not split; their
+    split form is in tests/test_gpu_large_kernels.py."""
     import os
     from fhog import BwdBwdPlan, _lib
     if "split=0" in os.environ.get("FHOG_TUNE", ""):
@@ -316,7 +318,7 @@ def test_split_streamed_side_matches_the_unsplit_launch(case, schedule):
 @pytest.mark.parametrize("seed", range(12))
 def test_split_launches_on_random_shapes_against_the_fp32_family(seed):
     """Random ragged lengths, masks, head dims and row strides in the range where launches split (few slices, at least
-    16 streamed tiles): the 16-bit kernels with partial results and the split-product kernels against the oracle (fp32
+    16 streamed tiles) or run the kernels for small launches: the 16-bit kernels and the split-product kernels against the oracle (fp32
     autograd for the outputs, fp64 closed form for the row statistics), then against each other."""
     import random
     rnd = random.Random(1000 + seed)

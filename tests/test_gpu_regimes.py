@@ -102,9 +102,9 @@ for tag, (shape, causal, window) in {cases!r}.items():
     out[tag + "/three_sweep"] = [t.cpu() for t in res[:4]] + [t.cpu() for t in res[4]]
 torch.save(out, sys.argv[1])
 """
-# small, ragged and masked, d = 128: the 8-wave b and ddO sweeps, the 64-queries-per-wave dd sweep and both workgroup orders on
-# launches of a handful of workgroups (each case under the default and under the three-sweep schedule); the last shape is
-# one whose passes split their streamed side by default; d64_many: d = 64 with workgroups enough not to split (the one-launch
+# Ragged and masked, d = 128: with small=0 the 8-wave b and ddO sweeps, the 64-queries-per-wave dd sweep and both workgroup orders on launches of a
+# handful of workgroups, and "split", whose passes split their streamed side; by default the kernels for small launches, which read none of the choices,
+# run the three (each case under the default and under the three-sweep schedule). d64_many: d = 64 with workgroups enough not to split (the one-launch
 # form of sweeps 1-3 and the 64-row stage apply)
 _TUNE_CASES = {"ragged_causal": ((3, 333, 333, 128), True, None), "window": ((2, 300, 400, 128), "bottom_right", 200),
                "d64_many": ((180, 384, 300, 64), False, None), "split": ((2, 700, 700, 128), True, None)}
@@ -120,19 +120,29 @@ def _run_child(tmp_path, tune):
 
 
 def test_launch_choices_forced_through_FHOG_TUNE(tmp_path):
+    _check_launch_choices(tmp_path, "")
+
+
+def test_launch_choices_forced_without_the_small_kernels(tmp_path):
+    _check_launch_choices(tmp_path, "small=0,")
+
+
+def _check_launch_choices(tmp_path, prefix):
     """b8, dd64, order, stage64 and stage1 change which kernel, which workgroup order or how many launches run, never a bit
     of the results; split=0 changes the fp32 summation order of the launches that would split. Unknown keys are reported,
     not obeyed."""
-    base, _ = _run_child(tmp_path, "")
+    base, _ = _run_child(tmp_path, prefix.rstrip(","))
     for tune in ("b8=1,dd64=1,order=slice,stage1=1", "b8=0,dd64=0,order=tile,stage64=1"):
-        got, err = _run_child(tmp_path, tune)
+        got, err = _run_child(tmp_path, prefix + tune)
         assert "FHOG_TUNE" not in err, err
         for tag in base:
             for i, (a, b_) in enumerate(zip(got[tag], base[tag])):
                 assert torch.equal(a, b_), (tune, tag, i)
-    got, err = _run_child(tmp_path, "split=0,b9=1,order=diagonal,dd64")
+    got, err = _run_child(tmp_path, prefix + "split=0,b9=1,order=diagonal,dd64")
     assert "unknown key 'b9'" in err and "not 'diagonal'" in err and "not key=value" in err, err
-    for tag in base:          # nothing splits there (the three-sweep runs were made with the minimum workspace)
+    # What splits: "split" alone, and of the ragged and windowed launches none has 16 tiles to stream (the three-sweep runs were made with the minimum
+    # workspace)
+    for tag in base:
         if tag != "split":
             for a, b_ in zip(got[tag], base[tag]):
                 assert torch.equal(a, b_), tag

@@ -5,6 +5,9 @@ first-level products (:217-251). Here the second sweep produces ddO and takes b 
 (pinned for the exact quantities in tests/test_oracle.py::test_row_identities), and the third produces dQ2 alone. Same
 gates as the default schedule: outputs within 2e-2 of the fp64 closed form (normalised max error), row statistics
 d, dd, b read back from the workspace.
+
+Launches of up to 128 groups of 128 rows, most of those below, run the kernels for small launches whatever the schedule; the schedules' own passes
+on such shapes are in tests/test_gpu_large_kernels.py.
 """
 import ctypes
 

@@ -1,5 +1,6 @@
 """GPU tier: how many splits passes 3 and 4 run with at d = 128 (rounds of workgroups under the mask against the cost of
-combining): whatever the rule picks, results are those of the launch that does not split."""
+combining): whatever the rule picks, results are those of the launch that does not split. The picks themselves are in
+tests/test_launch_rules_host.py, launches whose picks are known in tests/test_gpu_large_kernels.py."""
 import pytest
 import torch
 
@@ -13,7 +14,7 @@ def _dev():
     return require_gpu()
 
 
-# keys without a query at the front of the K side, one split of several, uneven work of a causal mask, 2 rounds that become 1
+# keys without a query at the front of the K side (statistics sweep split), a small launch, uneven work of a causal mask, window, 1 | 8 splits, none
 @pytest.mark.parametrize("shape", [(16, 1000, 3001, "bottom_right", 700), (1, 300, 5000, "bottom_right", 64), (2, 2048, 2048, True, None),
                                    (24, 1536, 1536, True, 100), (3, 4095, 513, False, None), (40, 1025, 1024, False, None)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
