@@ -389,29 +389,29 @@ int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream) {
   // Pass sequences. The first statistics sweep writes d_i itself: no separate launch for it.
   // The schedules that take ddO out of the third sweep exist in the 16-bit family; the split-product family runs the
   // fused one for them.
-  static const int four[] = {FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
-  static const int fused[] = {FHOG_PASS_DD_B, FHOG_PASS_DQ_DDO, FHOG_PASS_DK_DV};
-  static const int ddo_early[] = {FHOG_PASS_DD, FHOG_PASS_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
-  static const int three[] = {FHOG_PASS_DD_B_DDO, FHOG_PASS_DQ, FHOG_PASS_DK_DV};
+  // The last sweep of a sequence shares its launch with pass 4, stage 1 apart, which pass 4 follows in one of its own.
+  static const int four[] = {FHOG_PASS_DD, FHOG_PASS_B, FHOG_PASS_DQ_DDO, 0};
+  static const int stage1[] = {FHOG_PASS_STAGE1, FHOG_PASS_DK_DV, 0};
+  static const int fused[] = {FHOG_PASS_DD_B, FHOG_PASS_DQ_DDO, 0};
+  static const int ddo_early[] = {FHOG_PASS_DD, FHOG_PASS_B_DDO, FHOG_PASS_DQ, 0};
+  static const int three[] = {FHOG_PASS_DD_B_DDO, FHOG_PASS_DQ, 0};
   const int* order = four;
   const bool split_products = impl != FHOG_IMPL_BF16;
-  int n_pass = 4;
   // d = 64, launch large enough to fill the GPU: the reference's own arrangement of its four passes, sweeps 1-3 in one launch
-  static const int stage1[] = {FHOG_PASS_STAGE1, FHOG_PASS_DK_DV};
   if (args->schedule == FHOG_SCHEDULE_FOUR_PASS && impl == FHOG_IMPL_BF16 && args->d == 64 && fhog::tuning().stage1 != 0 &&
       granted_split(args, impl, FHOG_PASS_DQ_DDO) == 1 && granted_split(args, impl, FHOG_PASS_DD) == 1)
-    order = stage1, n_pass = 2;
-  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (split_products && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused, n_pass = 3;
+    order = stage1;
+  if (args->schedule == FHOG_SCHEDULE_FUSED_STATS || (split_products && args->schedule != FHOG_SCHEDULE_FOUR_PASS)) order = fused;
   const bool splits = splits_instead(args, p, impl);
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && splits) order = fused, n_pass = 3;
-  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early, n_pass = 4;
-  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three, n_pass = 3;
-  for (int i = 0; i < n_pass; i++) {
-    const bool last_two = order[i] == FHOG_PASS_DQ_DDO || order[i] == FHOG_PASS_DQ;   // they share a launch
-    const int r = !last_two ? run_pass(args, p, impl, order[i], (hipStream_t)hip_stream)
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && splits) order = fused;
+  if (args->schedule == FHOG_SCHEDULE_DDO_EARLY && impl == FHOG_IMPL_BF16 && !splits) order = ddo_early;
+  if (args->schedule == FHOG_SCHEDULE_THREE_SWEEP && impl == FHOG_IMPL_BF16 && !splits) order = three;
+  for (; *order; order++) {
+    const bool last_two = *order == FHOG_PASS_DQ_DDO || *order == FHOG_PASS_DQ;
+    const int r = !last_two ? run_pass(args, p, impl, *order, (hipStream_t)hip_stream)
                   : split_products ? run_pass(args, p, impl, fhog::kPassGrads, (hipStream_t)hip_stream)
-                                   : run_grads(args, p, order[i], true, (hipStream_t)hip_stream);
-    if (r != FHOG_OK || last_two) return r;
+                                   : run_grads(args, p, *order, true, (hipStream_t)hip_stream);
+    if (r != FHOG_OK) return r;
   }
   return FHOG_OK;
 }

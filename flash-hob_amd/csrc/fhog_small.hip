@@ -35,10 +35,10 @@ __device__ __forceinline__ void stage_words(uint32_t lds, const float* src) {
 // The streamed tiles of one wave: every W-th one of [begin, end), in a ring of NBUF stages of its own.
 // issue(t, lds): requests tile t into the stage at LDS address lds, COUNT loads.
 template <int W, int NBUF, int STAGE, int COUNT, typename Issue, typename Block>
-__device__ __forceinline__ void own_tiles(int begin, int end, char* ring, bool first_ones_landed, const Issue& issue, const Block& block) {
+__device__ __forceinline__ void own_tiles(int begin, int end, char* ring, const Issue& issue, const Block& block) {
   const uint32_t lds = lds_addr(ring);
   int t = begin;
-  bool landed = first_ones_landed;
+  bool landed = true;   // first_tiles' requests: every caller has waited for them
   for (int slot = 0; t < end; t += W) {
     if (!landed) {
       // what may still travel is the tile behind this one
@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(256, 2) small_stats(Params p) {
   lane_offsets<D>(lane, aoff, troff);
   float red[5] = {};   // sum P E, and over keys of P ddS, v ddS, v and P with v = P u
   f32x16_t none[NC];
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, true, issue, [&](const char* stage, int j) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, issue, [&](const char* stage, int j) {
     const int k0 = j * TS;
     const bool masked = geo.partial(k0, q0);
     int lo = 0, hi = 0;
@@ -219,7 +219,7 @@ __device__ __forceinline__ void grads_q(const Params& p, char* smem) {
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc_dq[cb] = f32x16_t{0}, acc_ddo[cb] = f32x16_t{0};
   float none[5] = {};
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, true, issue, [&](const char* stage, int j) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, issue, [&](const char* stage, int j) {
     const int k0 = j * TS;
     const bool masked = geo.partial(k0, q0);
     int lo = 0, hi = 0;
@@ -280,7 +280,7 @@ __device__ __forceinline__ void grads_k(const Params& p, char* smem, int id) {
   f32x16_t acc_dk[NC], acc_dv[NC];
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc_dk[cb] = f32x16_t{0}, acc_dv[cb] = f32x16_t{0};
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT + 2>(t_begin + ws, t_end, ring, true, issue, [&](char* stage, int t) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT + 2>(t_begin + ws, t_end, ring, issue, [&](char* stage, int t) {
     // L, d, dd, b as they lie in memory -> L log2(e), -d, dd, -(dd d + b)
     float* const stat = reinterpret_cast<float*>(stage + NT * TILE);
     const float l = stat[n], d = stat[TS + n], dd = stat[2 * TS + n], b = stat[3 * TS + n];
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256, 2) small_fwd(AttnParams p) {
   f32x16_t acc[1][NC];
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc[0][cb] = f32x16_t{0};
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, true, issue, [&](const char* stage, int j) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, issue, [&](const char* stage, int j) {
     const int k0 = j * TS;
     const bool masked = geo.partial(k0, q0);
     int lo = 0, hi = 0;
@@ -410,7 +410,7 @@ __device__ __forceinline__ void bwd_q(const AttnParams& p, char* smem) {
   f32x16_t acc[1][NC];
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc[0][cb] = f32x16_t{0};
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, true, issue, [&](const char* stage, int j) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT>(j_begin + ws, j_end, ring, issue, [&](const char* stage, int j) {
     const int k0 = j * TS;
     const bool masked = geo.partial(k0, q0);
     int lo = 0, hi = 0;
@@ -468,7 +468,7 @@ __device__ __forceinline__ void bwd_k(const AttnParams& p, char* smem, int id) {
   f32x16_t acc[2][NC];
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc[0][cb] = f32x16_t{0}, acc[1][cb] = f32x16_t{0};
-  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT + 1>(t_begin + ws, t_end, ring, true, issue, [&](char* stage, int t) {
+  own_tiles<W, NBUF, STAGE, NT * Dma<D, 1>::IPT + 1>(t_begin + ws, t_end, ring, issue, [&](char* stage, int t) {
     float* const stat = reinterpret_cast<float*>(stage + STAT);
     bf16x8_t Ob[KK], dOb[KK];
 #pragma unroll
