@@ -119,8 +119,11 @@ extern "C" {
  *   dd64=0|1          dd sweep at d = 128 with 32 | 64 queries per wave
  *   stage64=0|1       single-role sweeps at d = 64: one | two 32-row tiles staged and consumed per barrier
  *   stage1=0|1        d = 64, four-pass schedule: sweeps 1-3 as three launches | as one launch (FHOG_PASS_STAGE1)
- * Results do not depend on any of them beyond fp32 summation order (split) - the others are bit-identical. Unknown keys
- * and values are reported on stderr and ignored. */
+ *   small=0|2|4       16-bit tensors, d = 64 and 128, first-order passes and every schedule but the reference's: the four waves of a
+ *                     workgroup on rows of their own | that many waves on the same 32 rows, whatever the size of the launch
+ * Results are bit-identical under all of them but split, which changes the order of fp32 sums, and small, which does so too and
+ * has the forward round its weights beside another running maximum (fp32 sums of the same number of bits; O may differ in its last
+ * bit). Unknown keys and values are reported on stderr and ignored. */
 typedef struct fhog_bwdbwd_args {
   /* inputs (device pointers); q, o, dO, ddq: (batch, n_q, d); k, v, ddk, ddv: (batch, n_k, d) */
   const void* q;
@@ -182,8 +185,10 @@ int fhog_validate(const fhog_bwdbwd_args* args);
    FHOG_IMPL_BF16, or a negative FHOG_E_* code. Host-only. */
 int fhog_select_impl(const fhog_bwdbwd_args* args);
 
-/* All passes in order (d, dd, b, dQ2+ddO, dK2+dV2) on `hip_stream` (a hipStream_t); with
-   schedule = FHOG_SCHEDULE_FUSED_STATS, dd and b come from one sweep (FHOG_PASS_DD_B) instead.
+/* All passes of args->schedule on `hip_stream` (a hipStream_t): d with the first statistics sweep, the other statistics, then the
+   sweep for dQ2 (and ddO, unless an earlier one wrote it) and the one for dK2, dV2 in one launch, behind each launch that was split
+   the kernel that adds its partial results. Small launches of 16-bit tensors (schedules other than FHOG_SCHEDULE_FOUR_PASS) are two
+   kernels, statistics and outputs. d, dd and b are in ws afterwards either way.
    Drop-in for the two launches + reduction of flash_bwdbwd (fhog/triton_bwdbwd.py:580-646). */
 int fhog_bwdbwd(const fhog_bwdbwd_args* args, void* hip_stream);
 
@@ -247,8 +252,8 @@ int fhog_attn_validate(const fhog_attn_args* args, int backward);
 int fhog_attn_fwd(const fhog_attn_args* args, void* hip_stream);
 
 /* dQ, dK, dV of the forward above from (q, k, v, o, dO, lse): the arithmetic of flash_backward_torch
-   (fhog/triton_flash.py:201-220) as three launches (row sums of o*dO, a Q-tiled sweep for dQ, a K-tiled
-   sweep for dK and dV), without the (batch, n_q, n_k) tensors. */
+   (fhog/triton_flash.py:201-220) as a Q-tiled sweep for dQ, which also forms the row sums of o*dO, and a K-tiled sweep for
+   dK and dV, without the (batch, n_q, n_k) tensors: two launches, or one where the call is small. */
 int fhog_attn_bwd(const fhog_attn_args* args, void* hip_stream);
 
 /* Measurement aid (no counterpart in the reference): enqueue a loop of bf16 32x32x16 MFMAs on `blocks` workgroups of 8
