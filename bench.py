@@ -8,7 +8,7 @@ metric is quoted on: bf16 causal B=2 H=16 N=4096 d=128.
 Prints ONE JSON line.  ``value`` is the whole-path algorithmic throughput
 (24*d*pairs FLOP per step: the 12 contractions of the materialised formula, recomputation
 not counted).  ``roofline`` describes the dominant kernel (pass 3, dQ'+ddO) against the dense
-bf16 MFMA peak; ``cpu_baseline`` is the torch autograd double-backward timed on this box's
+bf16 MFMA peak, launched by itself: in the timed step it shares a launch with pass 4, which would hide what either reaches; ``cpu_baseline`` is the torch autograd double-backward timed on this box's
 host cores on a few heads of the same workload.
 """
 import argparse
