@@ -282,7 +282,7 @@ class BwdBwdPlan:
         self.keep = (q3, k3, v3, o3, do3, ddq3, ddk3, ddv3, lse)
         # empty_like would pack rows that are padded
         self.outs = tuple(torch.empty_strided(t.shape, t.stride(), dtype=t.dtype, device=t.device)
-                          for t in (q3, k3, v3, q3))
+                          for t in (q3, k3, k3, q3))
         self.args = _build_args(q3, k3, v3, o3, do3, ddq3, ddk3, ddv3, lse, scale, causal, _IMPLS[impl], self.outs, None, schedule_code(schedule, fused_stats), window)
         with torch.cuda.device(Q.device):
             self.ws_all = _workspace(self.args, Q.device, split)   # d | dd | b, then partial results of split launches

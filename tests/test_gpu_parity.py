@@ -774,3 +774,13 @@ def test_plan_on_padded_rows(dtype, d, batch):
         assert t.shape == like.shape and t.stride() == padded(like).stride()
     for a, b in zip(dense.run(), wide.run()):
         assert torch.equal(a, b)
+
+
+def test_plan_on_one_slice_with_another_batch_stride():
+    """The batch stride of a single slice means nothing, and tensors that differ in it alone are one layout."""
+    from fhog import BwdBwdPlan
+    x = with_caches(make_case(1, 200, 333, 64, torch.bfloat16, seed=85, grad_std=0.1), 0.125, False)
+    y = dict(x, V=x["V"].as_strided(x["V"].shape, (2 * 333 * 64, 64, 1)), dO=x["dO"].as_strided(x["dO"].shape, (2 * 200 * 64, 64, 1)))
+    names = ("Q", "K", "V", "O", "dO", "ddQ", "ddK", "ddV", "L")
+    for a, b in zip(BwdBwdPlan(*(x[n] for n in names), 0.125).run(), BwdBwdPlan(*(y[n] for n in names), 0.125).run()):
+        assert torch.equal(a, b)
