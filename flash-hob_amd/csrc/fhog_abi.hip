@@ -287,6 +287,7 @@ const Tuning& tuning() {
       else if (!strcmp(tok, "dd64")) flag(tok, val, &r.dd64);
       else if (!strcmp(tok, "stage64")) flag(tok, val, &r.stage64);
       else if (!strcmp(tok, "stage1")) flag(tok, val, &r.stage1);
+      else if (!strcmp(tok, "few")) flag(tok, val, &r.few);
       else if (!strcmp(tok, "small")) {
         if (!strcmp(val, "0") || !strcmp(val, "2") || !strcmp(val, "4")) r.small = val[0] - '0';
         else fprintf(stderr, "libfhog_hip: FHOG_TUNE: small is '0', '2' or '4', not '%s'; ignored\n", val);

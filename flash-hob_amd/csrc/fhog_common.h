@@ -67,10 +67,11 @@ struct Params {
 //   stage64=0|1        single-role sweeps at d = 64: one | two 32-row tiles staged and consumed per barrier (default 0: measured equal within 1 %)
 //   small=0|2|4        first-order passes and the double-backward (all schedules but the reference's) on 16-bit tensors: four waves on
 //                      128 stationary rows | that many on the same 32 (fhog_small.hip; default: by the size of the launch)
+//   few=0|1            fp32 tensors, passes 3 and 4: both outputs of a side in a workgroup | one (fhog_split_few.hip; default: by the size of the launch)
 //   stage1=0|1         d = 64, reference schedule: sweeps 1-3 as three launches | as one launch whose workgroups run them one
 //                      after the other for their tile (FHOG_PASS_STAGE1)
 struct Tuning {
-  int b8 = -1, order = -1, split = 1, dd64 = -1, stage64 = 0, stage1 = 0, small = -1;
+  int b8 = -1, order = -1, split = 1, dd64 = -1, stage64 = 0, stage1 = 0, small = -1, few = -1;
 };
 const Tuning& tuning();
 
@@ -119,6 +120,7 @@ constexpr int kPassGrads = -1;   // launch_split_pass: passes 3 and 4 in one lau
 // Launchers implemented in the kernel translation units. Each returns hipGetLastError().
 hipError_t launch_rowdot(const Params& p, int dtype, hipStream_t s);                 // pass 0
 hipError_t launch_split_pass(const Params& p, int dtype, int pass, hipStream_t s);  // passes 1..5, split products
+hipError_t launch_split_few(const Params& p, int sides, hipStream_t s);              // passes 3 (sides & 1) and 4 (sides & 2) of fp32 tensors, one output to a workgroup
 hipError_t launch_bf16_pass(const Params& p, int pass, hipStream_t s);              // statistics sweeps (1, 2, 5, 6, 8) and the one-launch stage 1, 16-bit MFMA
 hipError_t launch_bf16_grads(const Params& p, int q_pass, bool k_side, hipStream_t s);   // pass 3 or 7 (0: none) beside pass 4
 hipError_t launch_grads_pc(const Params& p, int q_pass, bool k_side, hipStream_t s);     // the sweeps of that at d = 128

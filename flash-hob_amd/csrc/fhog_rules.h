@@ -388,6 +388,30 @@ inline bool apart_is_faster(const P& p, int waves, int most_waves, bool two_on_a
          c.margin * split_launch(q, k, p.batch, waves, waves, two_on_a_cu, c);
 }
 
+// Whether passes 3 and 4 of fp32 tensors run with one output to a workgroup (fhog_split_few.hip). Those workgroups are four to 32 rows of either side, with a third
+// more work in all: ahead as long as they are one round of the 256 CUs, and for two where the tiles that a wave streams are what counts, which are
+// fewer. At d = 32 a second round is level; under a triangle half of the tiles are not there. Counted are workgroups as long as
+// the longest: those of the side that streams fewer rows are shorter by its tiles. Double-backward, us, the other kernels -> these, no mask | causal:
+//   d = 32   2 x 256 22.3 -> 19.9 | 22.5 -> 20.3; 4 x 512 34.7 -> 29.7 | 35.1 -> 30.1; beyond: 8 x 512 35.3 -> 41.6 | 35.4 -> 36.8
+//   d = 64   2 x 256 44.5 -> 31.3 | 43.8 -> 31.1; 2 x 1024 138 -> 82 | 136 -> 80; 4 x 1024 138 -> 123 | 137 -> 98; 1 x 4096 506 -> 430 | 497 -> 326; beyond:
+//            8 x 1024 170 -> 233 | 134 -> 137; two rounds of short streams: 16 x 256 45.2 -> 46.2, 53 x 50 1.2 to 1
+//   d = 128  2 x 256 132 -> 73 | 136 -> 74; 2 x 1024 462 -> 241 | 472 -> 239; 16 x 256 136 -> 109 | 140 -> 92; 1 x 4096 1781 -> 1385 | 1816 -> 1094; beyond:
+//            8 x 1024 465 -> 639 | 477 -> 406
+// 600 shapes of 1 to 96 slices with 24 to 12000 rows: the 262 that this picks take 0.41 to 1.0 times as long, 46 of the others would take less than 0.9.
+// The count is that of both sides also where one is launched alone: passes 3 and 4 have the same bits apart.
+inline bool few_rows(const Params& p, int bytes) {
+  if (bytes != 4) return false;
+  if (tuning().few >= 0) return tuning().few;
+  const int64_t n_q = p.n_q, n_k = p.n_k, seen = (int64_t)p.window + 31, waves = p.d == 128 ? 2 : 4, fixed = 3;   // to start and to store, in tiles
+  const int64_t q = ((n_k < seen ? n_k : seen) + 32 * waves - 1) / (32 * waves) + fixed, k = ((n_q < seen ? n_q : seen) + 32 * waves - 1) / (32 * waves) + fixed;
+  const int64_t groups = 2 * ((n_q + 31) / 32 * q + (n_k + 31) / 32 * k) * p.batch / (q > k ? q : k);
+  const int64_t longer = n_q > n_k ? n_q : n_k;
+  if (groups > 256 && p.d != 128 && (longer < p.window ? longer : p.window) < 320) return false;
+  const bool triangle = p.causal && p.window >= p.n_k && 2 * (int64_t)p.mask_off <= p.n_k;
+  const int64_t line = p.d == 32 ? 288 : p.d == 64 ? 512 : 576;
+  return groups <= (triangle ? line + line / 4 : line);
+}
+
 // Waves on the same 32 rows for passes 3 and 4 in one launch, or 0 for two launches: four waves while that gives one workgroup per CU, two as long as the
 // workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. The figures are those of launch_grads (fhog_split.hip).
 inline int split_grads_waves(const Params& p, int bytes) {

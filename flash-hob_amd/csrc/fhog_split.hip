@@ -34,37 +34,6 @@ namespace fhog {
 using namespace splitk;
 namespace {
 
-// Stationary fp32 operands too many for their terms to stay in registers.
-template <typename T, int D>
-constexpr bool is_raw = sizeof(T) == 4 && D == 128;
-
-// Stationary operand of a lane: its row's elements 16 kk + 8 h .. + 7 of every k-step, as terms or as they lie in memory. Split
-// without ANY: where one of them is not finite, the outputs of its row are not either.
-template <typename T, int D>
-struct Resident {
-  static constexpr int KK = D / 16, NF = Terms<T>::NF;
-  typename std::conditional<is_raw<T, D>, Chunk<T>, bf16x8_t[NF]>::type r[KK];
-  __device__ __forceinline__ void load(const T* row, int h) {
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++) {
-      const Chunk<T> c = load_chunk<T>(row + 16 * kk + 8 * h);
-      if constexpr (is_raw<T, D>) r[kk] = c;
-      else chunk_terms<T, true, false>(c, r[kk]);
-    }
-  }
-  __device__ __forceinline__ void terms(int kk, bf16x8_t (&out)[NF]) const {
-    if constexpr (is_raw<T, D>) {
-      Chunk<T> c = r[kk];
-      // splitting is to happen here, tile after tile: hoisted out of the sweep, the terms would be spilled
-      asm volatile("" : "+v"(c.v[0]), "+v"(c.v[1]));
-      chunk_terms<T, true, false>(c, out);
-    } else {
-#pragma unroll
-      for (int q = 0; q < NF; q++) out[q] = r[kk][q];
-    }
-  }
-};
-
 // Stages of the ring: two where they fit (a wave split stages WS tiles at a time instead).
 template <typename T, int D, int WS>
 constexpr int n_buffers(int stage) { return WS == 1 && !is_raw<T, D> && 2 * stage <= 160 * 1024 ? 2 : 1; }
@@ -505,6 +474,7 @@ hipError_t launch_grads_side(const Params& p, int sides, int waves, hipStream_t 
 // 5 times 740 -> 609, 8 times 897 -> 874. fp32 d = 128, which has one wave at all sizes, 8 times 2260 -> 2373: not there.
 template <typename T, int D, int MASK>
 hipError_t launch_grads(const Params& p, int sides, hipStream_t s) {
+  if (rules::few_rows(p, sizeof(T))) return launch_split_few(p, sides, s);
   const int waves = rules::split_grads_waves(p, sizeof(T));
   if (waves) return launch_grads_side<T, D, MASK>(p, sides, waves, s);
   const int64_t g_q = (int64_t)(p.n_q + 127) / 128 * p.batch, g_k = (int64_t)(p.n_k + 127) / 128 * p.batch;

@@ -7,6 +7,8 @@
 // The S-shaped operands of the second-level products (P, dS, dS', ddP) are fp32 numbers whatever the tensors are, and three
 // terms for every tensor type: two carry 16 bits, which shows in sums that cancel.
 #pragma once
+#include <type_traits>
+
 #include "fhog_bf16_util.h"
 
 namespace fhog {
@@ -130,6 +132,37 @@ __device__ __forceinline__ void load_resident_terms(bf16x8_t (&dst)[D / 16][Term
   for (int kk = 0; kk < D / 16; kk++)
     chunk_terms<T, true, true>(load_chunk<T>(base + (int64_t)row * ld + 16 * kk + 8 * h), dst[kk]);
 }
+
+// Stationary fp32 operands too many for their terms to stay in registers.
+template <typename T, int D>
+constexpr bool is_raw = sizeof(T) == 4 && D == 128;
+
+// Stationary operand of a lane: its row's elements 16 kk + 8 h .. + 7 of every k-step, as terms or as they lie in memory. Split
+// without ANY: where one of them is not finite, the outputs of its row are not either.
+template <typename T, int D>
+struct Resident {
+  static constexpr int KK = D / 16, NF = Terms<T>::NF;
+  typename std::conditional<is_raw<T, D>, Chunk<T>, bf16x8_t[NF]>::type r[KK];
+  __device__ __forceinline__ void load(const T* row, int h) {
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+      const Chunk<T> c = load_chunk<T>(row + 16 * kk + 8 * h);
+      if constexpr (is_raw<T, D>) r[kk] = c;
+      else chunk_terms<T, true, false>(c, r[kk]);
+    }
+  }
+  __device__ __forceinline__ void terms(int kk, bf16x8_t (&out)[NF]) const {
+    if constexpr (is_raw<T, D>) {
+      Chunk<T> c = r[kk];
+      // splitting is to happen here, tile after tile: hoisted out of the sweep, the terms would be spilled
+      asm volatile("" : "+v"(c.v[0]), "+v"(c.v[1]));
+      chunk_terms<T, true, false>(c, out);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NF; q++) out[q] = r[kk][q];
+    }
+  }
+};
 
 // acc += a b for operands in NF terms each; the small terms first
 template <typename T>

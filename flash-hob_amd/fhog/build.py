@@ -17,7 +17,7 @@ PKG_DIR = Path(__file__).resolve().parent            # .../flash-hob_amd/fhog
 CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libfhog_hip.so"
-SOURCES = ["fhog_abi.hip", "fhog_rowdot.hip", "fhog_split.hip", "fhog_bf16.hip", "fhog_bf16_pc.hip", "fhog_bf16_ddo.hip", "fhog_small.hip", "fhog_attn.hip", "fhog_attn_split.hip", "fhog_probe.hip"]
+SOURCES = ["fhog_abi.hip", "fhog_rowdot.hip", "fhog_split.hip", "fhog_split_few.hip", "fhog_bf16.hip", "fhog_bf16_pc.hip", "fhog_bf16_ddo.hip", "fhog_small.hip", "fhog_attn.hip", "fhog_attn_split.hip", "fhog_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

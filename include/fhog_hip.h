@@ -121,7 +121,8 @@ extern "C" {
  *   stage1=0|1        d = 64, four-pass schedule: sweeps 1-3 as three launches | as one launch (FHOG_PASS_STAGE1)
  *   small=0|2|4       16-bit tensors, d = 64 and 128, first-order passes and every schedule but the reference's: the four waves of a
  *                     workgroup on rows of their own | that many waves on the same 32 rows, whatever the size of the launch
- * Results are bit-identical under all of them but split, which changes the order of fp32 sums, and small, which does so too and
+ *   few=0|1           fp32 tensors, passes 3 and 4: both outputs of a side in one workgroup | in workgroups of their own
+ * Results are bit-identical under all of them but split and few, which change the order of fp32 sums, and small, which does so too and
  * has the forward round its weights beside another running maximum (fp32 sums of the same number of bits; O may differ in its last
  * bit). Unknown keys and values are reported on stderr and ignored. */
 typedef struct fhog_bwdbwd_args {
