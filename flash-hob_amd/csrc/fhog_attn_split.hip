@@ -8,7 +8,7 @@
 // LDS in 32-row tiles that are split once per workgroup. A lane owns ONE stationary row: in the forward the running maximum,
 // the running sum and the rescaling factor of a query are per-lane scalars. Two terms per fp32 operand less than the
 // double-backward needs leave room for the terms of d = 128 (one wave per SIMD); only dK, dV on fp32 tensors there does not quite
-// fit and keeps 44 VGPRs of a lane in scratch memory under a mask, 76 with two waves on the same rows.
+// fit and keeps 43 to 118 VGPRs of a lane in scratch memory under a mask or with two waves on the same rows.
 // Small launches (WS = 2 or 4) put WS waves on the same 32 rows: each takes every WS-th streamed tile, and the partial
 // results are merged through LDS in a fixed order. dQ and dK, dV share a launch unless each fills the GPU (launch_bwd).
 #include <type_traits>
@@ -22,18 +22,35 @@ namespace {
 
 constexpr int MODE_FWD = 0, MODE_BWD_Q = 1, MODE_BWD_K = 2;
 
+// Workgroups on a CU that the registers are to leave room for. At d = 64 two keep a SIMD busy where one waits (for LDS operands, the
+// splitting, a barrier): everything fits 256 registers. us, one -> two, fp32 causal 32 x 2048 | no mask 64 x 2048: forward 146 -> 128 |
+// 410 -> 368, dQ 193 -> 158 | 528 -> 495, dK, dV 238 -> 209 | 783 -> 648. At d = 128 so does the forward (TWO), without the second stage of
+// the ring and with the query's numbers instead of their terms; worth it in launches with work for two on every CU (launch_fwd).
+template <typename T, int D, int WS, bool TWO>
+constexpr int min_workgroups = WS > 1 || (sizeof(T) * D > 256 && !TWO) ? 1 : 2;
+
+// Stages of the ring. With a wave split the WS tiles of a step take the room of the second one.
+template <int WS, bool TWO>
+constexpr int n_buffers = WS == 1 && !TWO ? 2 : 1;
+
 // OWN_D: dK, dV without the sweep for dQ before it
-template <typename T, int D, int MODE, int MASK, int WS, bool OWN_D>
+template <typename T, int D, int MODE, int MASK, int WS, bool OWN_D, bool TWO = false>
 __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id) {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
+  // split_pair: two waves of fp32 tensors on a SIMD run faster without the dot products (dK, dV causal 32 x 2048, d = 64 231 -> 217 us), the VALU-bound ones of
+  // 16-bit tensors with them (bf16 causal 64 x 1024, d = 32 86.5 against 89.3 us for both first-order passes)
+  constexpr bool DOT = sizeof(T) == 2;
   constexpr int NR = MODE == MODE_FWD ? 1 : 2;             // stationary tensors: Q | Q, dO | K, V
   constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
-  using Stage = Stager<T, D, 2, true, 0>;                     // streamed tensors: K, V | Q, dO
+  using Stage = Stager<T, D, 2, true, 0, DOT>;                     // streamed tensors: K, V | Q, dO
   constexpr int TENSOR = Stage::PLANES * Stage::TILE;
   constexpr int STAT = KSIDE ? 2 * TS * 4 : 0;             // L log2(e), -d of the 32 staged queries
   constexpr int STAGE = Stage::BYTES + STAT;
-  constexpr int NBUF = WS == 1 ? 2 : 1;                    // with a wave split the WS tiles of a step take the room of the second buffer
+  constexpr int NBUF = n_buffers<WS, TWO>;
   constexpr int nw = 4 / WS, ROWS = 32 * nw;
+  constexpr bool RAW = TWO;
+  // the next tile is split and written to LDS behind the MFMAs of this one: forward of fp32, d = 64, no mask 64 x 2048 383 -> 371 us
+  constexpr bool INTERLEAVED = MODE == MODE_FWD && sizeof(T) == 4 && D == 64 && WS == 1;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -41,7 +58,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, MASK != MASK_NONE && sizeof(T) * D < 256 && WS == 1, id)) return;
+  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, MASK != MASK_NONE && min_workgroups<T, D, WS, TWO> == 2, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
@@ -95,7 +112,13 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   if (t_begin < t_end) fetch(t_begin);
 
   bf16x8_t res[NR][KK][NF];
-  load_resident_terms<T, D>(res[0], KSIDE ? (const T*)p.k + koff : (const T*)p.q + qoff, sta_ld, rr, h);
+  Chunk<T> raw[KK];                // RAW: the fp32 numbers of a query, split again for every tile
+  if constexpr (RAW) {
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) raw[kk] = load_chunk<T>((const T*)p.q + qoff + (int64_t)rr * sta_ld + 16 * kk + 8 * h);
+  } else {
+    load_resident_terms<T, D>(res[0], KSIDE ? (const T*)p.k + koff : (const T*)p.q + qoff, sta_ld, rr, h);
+  }
   if constexpr (MODE != MODE_FWD)
     load_resident_terms<T, D>(res[NR - 1], KSIDE ? (const T*)p.v + koff : (const T*)p.dO + qoff, sta_ld, rr, h);
   const int64_t row = srow + rr;   // Q-tiled kernels
@@ -127,7 +150,27 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
 #pragma unroll
   for (int cb = 0; cb < NC; cb++) acc0[cb] = f32x16_t{0}, acc1[cb] = f32x16_t{0};
 
-  const auto block = [&](const char* stage, int s0) {
+  // INTERLEAVED: the first level of a tile; LDS operands are read behind the MFMAs of the k-step before, and behind(slot, slots) is what
+  // else is to be done behind MFMA `slot`. The fences hold the order.
+  const auto first_level = [&](const char* stage, f32x16_t& s, auto behind) {
+    constexpr TermPairs<NF, NF> kPairs{};
+    constexpr int P = kPairs.n;
+    bf16x8_t a[2][NF];
+    read_terms<T, Stage::TILE>(stage, aoff[0], a[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        s = mfma<false>(a[kk & 1][kPairs.a[i]], res[0][kk][kPairs.b[i]], s);
+        if (i == 0 && kk + 1 < KK) read_terms<T, Stage::TILE>(stage, aoff[kk + 1], a[(kk + 1) & 1]);
+        behind(P * kk + i, P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    asm volatile("" : "+v"(s));   // holds the products in front of the branches that follow: the compiler sinks them to the use of their sum
+  };
+
+  const auto block = [&](const char* stage, int s0, auto behind) {
     const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
     f32x16_t s = {0}, dp = {0};
     if constexpr (MODE == MODE_BWD_Q) {   // u = dP - d comes straight from an accumulator that starts at -d
@@ -141,15 +184,27 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
         for (int i = 0; i < 4; i++) dp[4 * g + i] = md4[i];
       }
     }
+    if constexpr (INTERLEAVED) {
+      first_level(stage, s, behind);
+    } else {
 #pragma unroll
-    for (int kk = 0; kk < KK; kk++) {
-      bf16x8_t a[NF];
-      read_terms<T, Stage::TILE>(stage, aoff[kk], a);
-      s = mma1<T>(s, a, res[0][kk]);                          // K Q^T | Q K^T
-      if constexpr (MODE != MODE_FWD) {
-        bf16x8_t g[NF];
-        read_terms<T, Stage::TILE>(stage + TENSOR, aoff[kk], g);
-        dp = mma1<T>(dp, g, res[NR - 1][kk]);                 // V dO^T | dO V^T
+      for (int kk = 0; kk < KK; kk++) {
+        bf16x8_t a[NF];
+        read_terms<T, Stage::TILE>(stage, aoff[kk], a);
+        if constexpr (RAW) {
+          bf16x8_t q[NF];
+          // splitting is to happen here, tile after tile: hoisted out of the sweep, the terms would be spilled
+          asm volatile("" : "+v"(raw[kk].v[0]), "+v"(raw[kk].v[1]));
+          chunk_terms<T, true, true, DOT>(raw[kk], q);
+          s = mma1<T>(s, a, q);
+        } else {
+          s = mma1<T>(s, a, res[0][kk]);                        // K Q^T | Q K^T
+        }
+        if constexpr (MODE != MODE_FWD) {
+          bf16x8_t g[NF];
+          read_terms<T, Stage::TILE>(stage + TENSOR, aoff[kk], g);
+          dp = mma1<T>(dp, g, res[NR - 1][kk]);                 // V dO^T | dO V^T
+        }
       }
     }
     const bool masked = geo.partial(s0, rw);   // wave-uniform: the block holds hidden pairs (mask edge or tensor end)
@@ -186,7 +241,13 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
           for (int r = 0; r < 16; r++) acc0[cb][r] *= alpha;
       }
       m = m_new;
-      second_level<T, D>(acc0, stage + TENSOR, troff, pv);    // O += P V
+      if constexpr (INTERLEAVED) {
+        SecondLevel<T, D> second{troff[0][0], troff[0][1]};
+        second.start(stage + TENSOR, pv);
+        second.template run<false>(acc0, stage + TENSOR, pv, stage, pv, [](int) {});   // O += P V
+      } else {
+        second_level<T, D, false, DOT>(acc0, stage + TENSOR, troff, pv);
+      }
     } else {
 #pragma unroll
       for (int g = 0; g < 4; g++) {
@@ -202,19 +263,35 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
       }
 #pragma unroll
       for (int r = 0; r < 16; r++) dp[r] *= pv[r];            // dS = P (dP - d) (scale applied to the accumulators at the end)
-      second_level<T, D>(acc0, stage, troff, dp);             // dQ += dS K | dK += dS^T Q
-      if constexpr (KSIDE) second_level<T, D>(acc1, stage + TENSOR, troff, pv);   // dV += P^T dO
+      second_level<T, D, false, DOT>(acc0, stage, troff, dp);             // dQ += dS K | dK += dS^T Q
+      if constexpr (KSIDE) second_level<T, D, false, DOT>(acc1, stage + TENSOR, troff, pv);   // dV += P^T dO
     }
   };
 
   if (t_begin < t_end) publish(0);
+  if (INTERLEAVED && t_begin < t_end) fetch(t_begin + 1);
   __syncthreads();
   for (int t = t_begin; t < t_end; t += WS) {
     const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
+    if constexpr (INTERLEAVED) {
+      // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
+      char* const next = smem + (buf ^ 1) * STAGE;
+      const int s0 = t * TS, row0 = min(s0 + 2 * TS, n_str - 1);
+      if (!geo.dead(s0, rw)) {
+        block(smem + buf * STAGE, s0, [&](int slot, int slots) {
+          st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
+        });
+      } else {
+        publish(buf ^ 1);
+        fetch(t + 2);
+      }
+      __syncthreads();
+      continue;
+    }
     const bool more = t + WS < t_end;
     if (more) fetch(t + WS);
     const int s0 = (t + ws) * TS;
-    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0);
+    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0, [](int, int) {});
     if (NBUF == 1) __syncthreads();   // the tiles are no longer read
     if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
     __syncthreads();
@@ -271,27 +348,24 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   }
 }
 
-template <typename T, int D, int WS>
-constexpr int min_workgroups = sizeof(T) * D >= 256 || WS > 1 ? 1 : 2;
-
-template <typename T, int D, int MODE, int MASK, int WS>
-__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS>)) attn_split(AttnParams p) {
+template <typename T, int D, int MODE, int MASK, int WS, bool TWO>
+__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, TWO>)) attn_split(AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  attn_run<T, D, MODE, MASK, WS, false>(p, smem, blockIdx.x);
+  attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x);
 }
 
 // dQ (workgroups [0, q_blocks)) and dK, dV (the others) in one launch
 template <typename T, int D, int MASK, int WS>
-__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS>)) attn_split_bwd(AttnParams p, int q_blocks) {
+__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, false>)) attn_split_bwd(AttnParams p, int q_blocks) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   if ((int)blockIdx.x < q_blocks) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, blockIdx.x);
   else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, (int)blockIdx.x - q_blocks);
 }
 
-template <typename T, int D, int MODE, int WS>
+template <typename T, int D, int MODE, int WS, bool TWO = false>
 constexpr int lds_bytes() {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
-  constexpr int stages = (WS == 1 ? 2 : WS) * (Stager<T, D, 2, true, 0>::BYTES + (KSIDE ? 2 * TS * 4 : 0));
+  constexpr int stages = n_buffers<WS, TWO> * WS * (Stager<T, D, 2, true, 0>::BYTES + (KSIDE ? 2 * TS * 4 : 0));
   constexpr int xch = WS > 1 ? (4 / WS) * (WS - 1) * ((KSIDE ? 2 : 1) * D / 32 * 16 + 2) * 64 * 4 : 0;
   return stages > xch ? stages : xch;
 }
@@ -299,13 +373,13 @@ constexpr int lds_bytes() {
 template <int WS>
 unsigned blocks(int rows, int batch) { return grid_blocks((rows + 128 / WS - 1) / (128 / WS), batch); }
 
-template <typename T, int D, int MODE, int MASK, int WS>
+template <typename T, int D, int MODE, int MASK, int WS, bool TWO = false>
 hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
-  constexpr int smem = lds_bytes<T, D, MODE, WS>();
+  constexpr int smem = lds_bytes<T, D, MODE, WS, TWO>();
   static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
-  const hipError_t e = allow_dynamic_lds<attn_split<T, D, MODE, MASK, WS>>(smem);
+  const hipError_t e = allow_dynamic_lds<attn_split<T, D, MODE, MASK, WS, TWO>>(smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((attn_split<T, D, MODE, MASK, WS>), dim3(blocks<WS>(MODE == MODE_BWD_K ? p.n_k : p.n_q, p.batch)), dim3(256), smem, s, p);
+  hipLaunchKernelGGL((attn_split<T, D, MODE, MASK, WS, TWO>), dim3(blocks<WS>(MODE == MODE_BWD_K ? p.n_k : p.n_q, p.batch)), dim3(256), smem, s, p);
   return hipGetLastError();
 }
 
@@ -328,6 +402,12 @@ hipError_t launch_fwd(const AttnParams& p, hipStream_t s) {
     if (groups < 64 && p.n_k > 2 * TS) return launch_ws<T, D, MODE_FWD, MASK, 4>(p, s);
   }
   if (groups < 128 && p.n_k > TS) return launch_ws<T, D, MODE_FWD, MASK, 2>(p, s);
+  // fp32, d = 128: two workgroups on a CU once there are more than one for each, under a mask more than two (a heavy and a light tile
+  // that share a CU leave the heavy one alone for most of its time). us, one -> two, at so many workgroups: no mask 422 -> 364 (320), 436
+  // -> 420 (512), 857 -> 816 (1024), but 234 -> 258 (256); causal 324 -> 290 (640), 466 -> 435 (1024), but 235 -> 260 (512).
+  if constexpr (is_raw<T, D>) {
+    if (groups > (MASK == MASK_NONE ? 256 : 512)) return launch_ws<T, D, MODE_FWD, MASK, 1, true>(p, s);
+  }
   return launch_ws<T, D, MODE_FWD, MASK, 1>(p, s);
 }
 

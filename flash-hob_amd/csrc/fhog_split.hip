@@ -13,13 +13,19 @@
 //
 // What bounds it: fp32 tensors the matrix pipe (216 MFMAs of 32 cycles per 32 x 32 block in pass 3 at d = 64, against 288 of
 // 64 cycles as v_mfma_f32_32x32x2_f32), 16-bit tensors at d = 32 the VALU (34 MFMAs beside some 400
-// VALU instructions, half of them the split of P, dS, dS' and ddP). Some do not quite fit the register file and keep VGPRs of a
-// lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 54 to 60, in pass 4 at d = 64 with
-// four waves on the same rows 18 to 21, at d = 32 under a mask in pass 3 6 and without one in pass 4 15; 16-bit tensors at d = 128 up to 89.
+// VALU instructions, half of them the split of P, dS, dS' and ddP). A wave of fp32 tensors is alone on its SIMD (d >= 64), so whatever it does
+// between two MFMAs the pipe waits for: LDS operands are read and numbers split behind the MFMAs of the step before (AHEAD, SecondLevel). Cycles of a
+// step of pass 5 at d = 64 without a mask: 120 MFMAs 3936; all products 4260; with the next tile split and written behind them 5370, elementwise
+// arithmetic 810, barrier 360 (splitting by itself: 1140 and 370 of requests more). Double-backward, us, without -> so: fp32 causal
+// 32 x 2048 d = 128 pass 5 629 -> 561, passes 3 and 4 2021 -> 1978; d = 64 941 -> 920; no mask 40 x 1024, d = 64 704 -> 677; two workgroups of pass 5 on a
+// CU (d = 64, numbers split again for every tile): 226 -> 319.
+// Some do not quite fit the register file and keep VGPRs of a
+// lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 62 to 72, at d = 64 with four waves on the same
+// rows 43 to 52, with one at d = 32 8; 16-bit tensors at d = 128 up to 53.
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 121     fp32 causal 64 x 1024, d = 32: 672 -> 279
-//   fp32 causal 32 x 2048, d = 64: 2101 -> 950    fp32 64 x 2048, d = 64: 7521 -> 3590
-//   fp32 causal 32 x 2048, d = 128: 3833 -> 2381
+//   fp32 causal 32 x 2048, d = 64: 2101 -> 915    fp32 64 x 2048, d = 64: 7521 -> 3490
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2300
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
@@ -66,8 +72,12 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   constexpr bool LAST_IN_LDS = RAW && !STATS;
   constexpr int NREG = LAST_IN_LDS ? NR - 1 : NR;
   constexpr bool DIRECT = is_direct<PASS, WS>;
+  // A wave is alone on its SIMD: what it waits for is put behind its own MFMAs. At d = 128 the first level of passes 3 and 4 has no registers for that.
+  constexpr bool AHEAD2 = sizeof(T) == 4 && D >= 64 && !DIRECT && PASS != 1, AHEAD = AHEAD2 && !LAST_IN_LDS;
   constexpr int NBUF = n_buffers<T, D, WS>(STAGE);
   constexpr int nw = 4 / WS, ROWS = 32 * nw;
+
+  constexpr bool INTERLEAVED = AHEAD && STATS && WS == 1 && NBUF == 2;   // the next tile is split and written to LDS behind the MFMAs of this one
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -95,21 +105,23 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   const int64_t srow = (int64_t)bh * p.n_q;
   Stage st[WS];
   float stat_reg[WS] = {}, stat_d[WS] = {}, stat_dd[WS] = {};
-  // pass 4: thread t < 128 carries statistic t / 32 of staged query t % 32
-  const float* stat_src = p.lse;
-  if ((tid >> 5) == 1) stat_src = p.ws_d;
-  if ((tid >> 5) == 2) stat_src = p.ws_dd;
-  if ((tid >> 5) == 3) stat_src = p.ws_b;
+  // pass 4: threads t and t + 128 carry statistic t / 32 of staged query t % 32
+  const int which = (tid >> 5) & 3;
+  const float* const stat_src = which == 0 ? p.lse : which == 1 ? p.ws_d : which == 2 ? p.ws_dd : p.ws_b;
+  const auto fetch_stat = [&](int g, int row0) {
+    const int64_t q = srow + min(row0 + (tid & 31), p.n_q - 1);
+    stat_reg[g] = stat_src[q], stat_d[g] = p.ws_d[q], stat_dd[g] = p.ws_dd[q];
+  };
+  const auto publish_stat = [&](int g, char* stage) {
+    reinterpret_cast<float*>(stage + Stage::BYTES)[tid & 127] =
+        which == 0 ? stat_reg[g] * kLog2e : which == 1 ? -stat_reg[g] : which == 2 ? stat_reg[g] : -__builtin_fmaf(stat_dd[g], stat_d[g], stat_reg[g]);
+  };
   const auto fetch = [&](int t) {
 #pragma unroll
     for (int g = 0; g < WS; g++) {
       const int row0 = (t + g) * TS;
       st[g].fetch(src, str_ld, min(row0, n_str - 1), n_str, tid);   // a tile past the end is never computed on
-      if (KSIDE && tid < 4 * TS) {
-        const int64_t q = srow + min(row0 + (tid & 31), p.n_q - 1);
-        stat_reg[g] = stat_src[q];
-        if (tid >= 3 * TS) stat_d[g] = p.ws_d[q], stat_dd[g] = p.ws_dd[q];
-      }
+      if (KSIDE) fetch_stat(g, row0);
     }
   };
   const auto publish = [&](int buf) {
@@ -117,11 +129,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
     for (int g = 0; g < WS; g++) {
       char* stage = smem + (buf * WS + g) * STAGE;
       st[g].publish(stage, tid);
-      if (KSIDE && tid < 4 * TS) {
-        const int k = tid / TS;
-        reinterpret_cast<float*>(stage + Stage::BYTES)[tid] =
-            k == 0 ? stat_reg[g] * kLog2e : k == 1 ? -stat_reg[g] : k == 2 ? stat_reg[g] : -__builtin_fmaf(stat_dd[g], stat_d[g], stat_reg[g]);
-      }
+      if (KSIDE) publish_stat(g, stage);
     }
   };
   if (!DIRECT && t_begin < t_end) fetch(t_begin);
@@ -164,6 +172,8 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   const float kc = __builtin_fmaf(dd, dsum, b);
   const float c_scale_log2 = p.scale * kLog2e;
 
+  // AHEAD: the other offsets follow from these by an exclusive or; kept in registers, they would be spilled
+  int aoff0 = tile_off<D>(n, h), tr0 = tr_lane_off_acc<D>(0, 0, lane), tr1 = tr_lane_off_acc<D>(0, 1, lane);
   int aoff[KK], troff[NC][2];
 #pragma unroll
   for (int kk = 0; kk < KK; kk++) aoff[kk] = tile_off<D>(n, 2 * kk + h);
@@ -182,8 +192,83 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
     for (int x = 0; x < NT; x++) ahead[kk & 1][x] = load_chunk<T>(src[x] + off);
   };
 
+  // AHEAD: the first level of one tile for a lone wave on its SIMD. What a group of MFMAs takes from LDS is read, and the terms that it
+  // takes of a stationary row are split (RAW), behind the MFMAs of the group before; the fences hold that order. Two chains
+  // of products take turns where a group has two.
+  const auto first_level = [&](const char* stage, int s0, f32x16_t& s, f32x16_t& dds, f32x16_t& dp, f32x16_t& e, auto behind) {
+    constexpr TermPairs<NF, NF> kPairs{};
+    bf16x8_t a[NT][NF];
+    Splitting<NF> terms[NR];   // RAW
+    Chunk<T> last_chunk;
+    const auto read = [&](int x, int kk) { read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff0 ^ (32 * kk), a[x]); };
+    // what is due behind MFMA `slot` of `slots` of the terms of k-step kk of stationary tensor y
+    const auto split = [&](int y, int kk, int slot, int slots) {
+      if constexpr (RAW) {
+        const Chunk<T>& c = LAST_IN_LDS && y == NR - 1 ? last_chunk : res[y < NREG ? y : 0].r[kk];
+        terms[y].at(slot, slots, [&](int i, float& lo, float& hi) {
+          lo = chunk_elem(c, 2 * i), hi = chunk_elem(c, 2 * i + 1);
+          asm("" : "+v"(lo), "+v"(hi) : "s"(s0));   // here, tile after tile: hoisted out of the sweep, the terms would be spilled
+        });
+      }
+    };
+    const auto sta_term = [&](int y, int kk, int q) {
+      if constexpr (RAW) return terms[y].term(q);
+      else return res[y].r[kk][q];
+    };
+    constexpr int P = kPairs.n;
+    read(0, 0), read(1, 0);
+    split(0, 0, 0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        s = mfma<false>(a[0][kPairs.a[i]], sta_term(0, kk, kPairs.b[i]), s);         // K Q^T | Q K^T
+        if (LAST_IN_LDS && i == 0) {
+          last_chunk.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]);
+          last_chunk.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
+        }
+        split(1, kk, 2 * i, 2 * P);
+        if (KSIDE) split(2, kk, 2 * i, 2 * P);
+        behind(5 * P * kk + 2 * i, 5 * P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+        dds = mfma<false>(a[1][kPairs.a[i]], sta_term(0, kk, kPairs.b[i]), dds);     // ddK Q^T | ddQ K^T
+        if (i == 0) read(2, kk);
+        if (!KSIDE && i == 1) read(NT - 1, kk);
+        split(1, kk, 2 * i + 1, 2 * P);
+        if (KSIDE) split(2, kk, 2 * i + 1, 2 * P);
+        behind(5 * P * kk + 2 * i + 1, 5 * P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        dds = mfma<false>(a[0][kPairs.a[i]], sta_term(1, kk, kPairs.b[i]), dds);     // + K ddQ^T | Q ddK^T
+        split(NR - 1, kk, i, P);
+        behind(5 * P * kk + 2 * P + i, 5 * P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        dp = mfma<false>(a[2][kPairs.a[i]], sta_term(2, kk, kPairs.b[i]), dp);       // V dO^T | dO V^T
+        if (kk + 1 < KK) {
+          if (i == 0) read(0, kk + 1), read(1, kk + 1);
+          split(0, kk + 1, 2 * i, 2 * P);
+        }
+        behind(5 * P * kk + 3 * P + 2 * i, 5 * P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+        e = mfma<false>(a[NT - 1][kPairs.a[i]], sta_term(NR - 1, kk, kPairs.b[i]), e);   // ddV dO^T | dO ddV^T
+        if (kk + 1 < KK) split(0, kk + 1, 2 * i + 1, 2 * P);
+        behind(5 * P * kk + 3 * P + 2 * i + 1, 5 * P * KK);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // holds the products in front of the branches that follow: the compiler sinks a chain of MFMAs to the block that uses its sum
+    asm volatile("" : "+v"(s), "+v"(dds), "+v"(dp), "+v"(e));
+  };
+
   // prefetch: what requests the next tile; called where the registers it lands in are free
-  const auto block = [&](const char* stage, int s0, auto prefetch) {
+  // behind(slot, slots): what is to be done behind MFMA `slot` of the first level (AHEAD)
+  const auto block = [&](const char* stage, int s0, auto prefetch, auto behind) {
     const float* stat = reinterpret_cast<const float*>(stage + Stage::BYTES);
     f32x16_t s = {0}, dds = {0}, dp = {0}, e = {0};
     // u = dP - d and E' = E - (dd d + b) come straight from accumulators that start at the row constants
@@ -202,41 +287,47 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
         if (PASS != 5) e[r] = -kc;
       }
     }
+    if constexpr (AHEAD2) asm volatile("" : "+v"(tr0), "+v"(tr1));
+    if constexpr (AHEAD) {
+      asm volatile("" : "+v"(aoff0));
+      first_level(stage, s0, s, dds, dp, e, behind);
+    } else {
 #pragma unroll
-    for (int kk = 0; kk < KK; kk++) {
-      bf16x8_t r0[NF], r1[NF], r2[NF], r3[NF], a[NF];
-      res[0].terms(kk, r0), res[1].terms(kk, r1);
-      const auto last_terms = [&](bf16x8_t (&out)[NF]) {
-        if constexpr (LAST_IN_LDS) {
-          Chunk<T> c;
-          c.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]), c.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
-          chunk_terms<T, true, false>(c, out);
-        } else {
-          res[NREG - 1].terms(kk, out);
+      for (int kk = 0; kk < KK; kk++) {
+        bf16x8_t r0[NF], r1[NF], r2[NF], r3[NF], a[NF];
+        res[0].terms(kk, r0), res[1].terms(kk, r1);
+        const auto last_terms = [&](bf16x8_t (&out)[NF]) {
+          if constexpr (LAST_IN_LDS) {
+            Chunk<T> c;
+            c.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]), c.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
+            chunk_terms<T, true, false>(c, out);
+          } else {
+            res[NREG - 1].terms(kk, out);
+          }
+        };
+        if constexpr (KSIDE) res[2].terms(kk, r2), last_terms(r3);
+        else if constexpr (PASS != 1) last_terms(r2);
+        const auto streamed = [&](int x) {
+          if constexpr (DIRECT) chunk_terms<T, true, false>(ahead[kk & 1][x], a);
+          else read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a);
+        };
+        streamed(0);
+        s = mma1<T>(s, a, r0);                                  // K Q^T | Q K^T
+        dds = mma1<T>(dds, a, r1);                              // K ddQ^T | Q ddK^T
+        if constexpr (PASS != 1) {
+          streamed(2);
+          dp = mma1<T>(dp, a, r2);                              // V dO^T | dO V^T
+          if constexpr (KSIDE) e = mma1<T>(e, a, r3);           // dO ddV^T
         }
-      };
-      if constexpr (KSIDE) res[2].terms(kk, r2), last_terms(r3);
-      else if constexpr (PASS != 1) last_terms(r2);
-      const auto streamed = [&](int x) {
-        if constexpr (DIRECT) chunk_terms<T, true, false>(ahead[kk & 1][x], a);
-        else read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff[kk], a);
-      };
-      streamed(0);
-      s = mma1<T>(s, a, r0);                                  // K Q^T | Q K^T
-      dds = mma1<T>(dds, a, r1);                              // K ddQ^T | Q ddK^T
-      if constexpr (PASS != 1) {
-        streamed(2);
-        dp = mma1<T>(dp, a, r2);                              // V dO^T | dO V^T
-        if constexpr (KSIDE) e = mma1<T>(e, a, r3);           // dO ddV^T
+        streamed(1);
+        dds = mma1<T>(dds, a, r0);                              // + ddK Q^T | ddQ K^T
+        if constexpr (PASS != 1 && !KSIDE) {
+          streamed(NT - 1);
+          e = mma1<T>(e, a, r2);                                // ddV dO^T
+        }
+        if constexpr (DIRECT) load_step(s0 / TS + (kk + 2 < KK ? 0 : WS), (kk + 2) % KK);   // past the last tile: its last row again
+        if constexpr (RAW || DIRECT) __builtin_amdgcn_sched_barrier(0);
       }
-      streamed(1);
-      dds = mma1<T>(dds, a, r0);                              // + ddK Q^T | ddQ K^T
-      if constexpr (PASS != 1 && !KSIDE) {
-        streamed(NT - 1);
-        e = mma1<T>(e, a, r2);                                // ddV dO^T
-      }
-      if constexpr (DIRECT) load_step(s0 / TS + (kk + 2 < KK ? 0 : WS), (kk + 2) % KK);   // past the last tile: its last row again
-      if constexpr (RAW || DIRECT) __builtin_amdgcn_sched_barrier(0);
     }
     f32x16_t pv;
 #pragma unroll
@@ -274,6 +365,32 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
         red[3] += v;
         red[4] += pv[r];
       }
+    } else if constexpr (AHEAD2) {
+      f32x4_t dd4[4];
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        if constexpr (KSIDE) dd4[g] = *reinterpret_cast<const f32x4_t*>(stat + 2 * TS + 8 * g + 4 * h);
+      }
+      const auto elementwise = [&](int r) {
+        if (r < 0 || r >= 16) return;
+        dds[r] = pv[r] * __builtin_fmaf(dds[r], p.scale, KSIDE ? -dd4[r / 4][r % 4] : -dd);   // ddP = P w
+        if (!KSIDE) s[r] = pv[r] * dp[r];                                                      // dS = P u (scale applied to the accumulators at the end)
+        e[r] = __builtin_fmaf(pv[r], e[r], dds[r] * dp[r]);                                    // dS' = P E' + ddP u
+      };
+      SecondLevel<T, D> second{tr0, tr1};
+      if constexpr (!KSIDE) {
+        second.start(stage + (NT - 1) * TENSOR, pv);
+        second.template run<true>(acc1, stage + (NT - 1) * TENSOR, pv, stage + TENSOR, s, elementwise);         // ddO += P ddV
+        second.template run<true>(acc0, stage + TENSOR, s, stage + 2 * TENSOR, dds, [](int) {});                // dQ2 += dS ddK
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = pv[r] * dp[r];
+        second.start(stage + TENSOR, s);
+        second.template run<true>(acc0, stage + TENSOR, s, stage + 2 * TENSOR, dds, elementwise);               // dK2 += dS^T ddQ
+      }
+      second.template run<true>(acc1, stage + 2 * TENSOR, dds, stage, e, [](int) {});                           // ddO += ddP V | dV2 += ddP^T dO
+      prefetch();
+      second.template run<false>(acc0, stage, e, stage, e, [](int) {});                                         // dQ2 += dS' K | dK2 += dS'^T Q
     } else {
 #pragma unroll
       for (int g = 0; g < 4; g++) {
@@ -299,32 +416,50 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   if constexpr (DIRECT) {
     // the range of 32 rows holds no tile that is dead to the wave
     if (t_begin + ws < t_end) load_step(t_begin + ws, 0), load_step(t_begin + ws, 1);
-    for (int t = t_begin + ws; t < t_end; t += WS) block(smem, t * TS, [] {});
+    for (int t = t_begin + ws; t < t_end; t += WS) block(smem, t * TS, [] {}, [](int, int) {});
   }
   if (!DIRECT && t_begin < t_end) publish(0);
+  if (INTERLEAVED && t_begin < t_end) fetch(t_begin + 1);
   if (!DIRECT) __syncthreads();
   for (int t = t_begin; !DIRECT && t < t_end; t += WS) {
     const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
-    const bool more = t + WS < t_end;
-    const auto next = [&]() {
-      if (more) fetch(t + WS);
-    };
-    if (!LATE) next();
     const int s0 = (t + ws) * TS;
-    if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, rw))) {
-      block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
-        if (LATE) {
-          __builtin_amdgcn_sched_barrier(0);
-          next();
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      });
-    } else if (LATE) {
-      next();
+    if constexpr (INTERLEAVED) {
+      // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
+      char* const next = smem + (buf ^ 1) * STAGE;
+      const int row0 = min(s0 + 2 * TS, n_str - 1);
+      if (!geo.dead(s0, rw)) {
+        block(smem + buf * STAGE, s0, [] {}, [&](int slot, int slots) {
+          st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
+          if (KSIDE && slot == 1) publish_stat(0, next);
+          if (KSIDE && slot == 2) fetch_stat(0, row0);
+        });
+      } else {
+        publish(buf ^ 1);
+        fetch(t + 2);
+      }
+      __syncthreads();
+    } else {
+      const bool more = t + WS < t_end;
+      const auto next = [&]() {
+        if (more) fetch(t + WS);
+      };
+      if (!LATE) next();
+      if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, rw))) {
+        block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
+          if (LATE) {
+            __builtin_amdgcn_sched_barrier(0);
+            next();
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }, [](int, int) {});
+      } else if (LATE) {
+        next();
+      }
+      if (NBUF == 1) __syncthreads();   // the tiles are no longer read
+      if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
+      __syncthreads();
     }
-    if (NBUF == 1) __syncthreads();   // the tiles are no longer read
-    if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
-    __syncthreads();
   }
 
   if constexpr (WS > 1) {
