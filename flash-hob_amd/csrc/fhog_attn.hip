@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16(AttnParams p) {
     const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-    if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
+    if (MASK == MASK_NONE || !geo.dead(k0, geo.first_row(qw, p.n_q))) {  // else every key of the tile is hidden from this wave
       const char* stage = smem + u * STAGE;
       fwd_block<F16, D>(stage, aoff, troff, Qb, masked, lo, hi, c_scale_log2, m, l, acc);
     }
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
     const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-    if (!geo.dead(k0, qw)) {
+    if ((MASK == MASK_NONE && D == 64) || !geo.dead(k0, geo.first_row(qw, p.n_q))) {
       const char* stage = smem + u * STAGE;
       bwd_q_block<F16, D>(stage, aoff, troff, Qb, dOb, masked, lo, hi, c_scale_log2, l_log2, dsum, acc);
     }
@@ -268,7 +268,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_k_bf16(AttnParams p) {
       dma.template issue_all<2>(dst, TILE, src, adv, wave, p.n_q - (j + 1) * TS);
     }
     const int qb = j * TS;
-    if (!geo.dead(qb, kw)) {  // else no query of the tile sees a key of this wave
+    if (!geo.dead(qb, geo.first_row(kw, p.n_k))) {  // else no query of the tile sees a key of this wave
       const char* stage = smem + st * STAGE;
       bwd_k_block<F16, D>(geo, stage, aoff, troff, Kb, Vb, qb, kw, kj, h, c_scale_log2, acc);
     }

@@ -277,7 +277,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
       // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
       char* const next = smem + (buf ^ 1) * STAGE;
       const int s0 = t * TS, row0 = min(s0 + 2 * TS, n_str - 1);
-      if (!geo.dead(s0, rw)) {
+      if (!geo.dead(s0, geo.first_row(rw, n_sta))) {
         block(smem + buf * STAGE, s0, [&](int slot, int slots) {
           st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
         });
@@ -291,7 +291,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
     const bool more = t + WS < t_end;
     if (more) fetch(t + WS);
     const int s0 = (t + ws) * TS;
-    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, rw)) block(smem + (buf * WS + ws) * STAGE, s0, [](int, int) {});
+    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, geo.first_row(rw, n_sta))) block(smem + (buf * WS + ws) * STAGE, s0, [](int, int) {});
     if (NBUF == 1) __syncthreads();   // the tiles are no longer read
     if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
     __syncthreads();

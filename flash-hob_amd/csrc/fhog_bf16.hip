@@ -201,7 +201,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
       const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
       int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
       if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-      if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
+      if (!geo.dead(k0, geo.first_row(qw, p.n_q))) {  // else every key of the tile is hidden from this wave
         const char* stage = smem + (GRP + u) * STAGE;
         q_block<F16, D, PASS>(stage, aoff, troff, Qb, ddQb, dOb, masked, lo, hi, c_scale_log2, l_log2, p.scale, dsum, dd, kc, red, red_dd, red_vdds,
                               red_pu, red_p, acc_dq, acc_ddo);
@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(256, 2) dd_sweep64_bf16(Params p) {
     int lo[2] = {0, 0}, hi[2] = {0, 0};   // key k0 + 8g + 4h + e is visible to the lane's query of block rb iff lo <= 8g + e <= hi
 #pragma unroll
     for (int rb = 0; rb < 2; rb++) {
-      act[rb] = !geo.dead(k0, qw + 32 * rb);
+      act[rb] = !geo.dead(k0, geo.first_row(qw + 32 * rb, p.n_q));
       masked[rb] = act[rb] && geo.partial(k0, qw + 32 * rb);
       if (masked[rb]) keep_branch(), geo.limits(k0, qi[rb], h, lo[rb], hi[rb]);
     }
@@ -560,7 +560,7 @@ __device__ __forceinline__ void k_sweep_run(const Params& p, char* smem, int bh,
       const int j = jj + u;
       if (SUB > 1 && j >= t_end) continue;
       const int qb = j * TS;
-      if (!geo.dead(qb, kw)) {  // else no query of the tile sees a key of this wave
+      if (!geo.dead(qb, geo.first_row(kw, p.n_k))) {  // else no query of the tile sees a key of this wave
         const char* stage = smem + (grp + u) * STAGE;
         k_block<F16, D>(geo, stage, aoff, troff, Kb, ddKb, Vb, ddVb, qb, kw, kj, h, c_scale_log2, p.scale, acc_dk, acc_dv);
       }

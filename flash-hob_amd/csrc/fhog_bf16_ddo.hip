@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) q_sweep_ddo(Params p
     const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-    if (!geo.dead(k0, qw)) {  // else every key of the tile is hidden from this wave
+    if (!geo.dead(k0, geo.first_row(qw, p.n_q))) {  // else every key of the tile is hidden from this wave
       const char* stage = smem + decltype(slot)::value * STAGE;
       // first level, a stream of 2 KK k-steps with the LDS operands fetched PF steps ahead (stage order K, ddK, V, ddV):
       //   K  : S += K Q^T, ddS += K ddQ^T

@@ -180,8 +180,8 @@ __device__ __forceinline__ void consume_q(const Params& p, char* smem, const Str
       dma.template issue_all<4>(dst, SM::TILE, src, adv, wq, p.n_k - (j + 1) * TS);
     }
     // block j-1: query block qb of the pair took part iff the tile held a key visible to it
-    const bool act0 = j > j_begin && !geo.dead((j - 1) * TS, qw0);
-    const bool act1 = j > j_begin && !geo.dead((j - 1) * TS, qw0 + 32);
+    const bool act0 = j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0, p.n_q));
+    const bool act1 = j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0 + 32, p.n_q));
     const bool act = act0 || act1;
     const char* stage = smem + sc * SM::STAGE;
     const char* sop = sop_pair + ((j - 1) & 1) * SM::SOP_BUF;
@@ -291,7 +291,7 @@ __device__ __forceinline__ void consume_dq(const Params& p, char* smem, const St
       const uint32_t dst = ring_lds + sn * SM::STAGE;
       dma.template issue_all<4>(dst, SM::TILE, src, (int64_t)(j + 1) * TS * p.stride_kn, wq, p.n_k - (j + 1) * TS);
     }
-    if (j > j_begin && !geo.dead((j - 1) * TS, qw0)) {   // block j-1 took part
+    if (j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0, p.n_q))) {   // block j-1 took part
       const char* stage = smem + sc * SM::STAGE;
       const char* sop = sop_wave + ((j - 1) & 1) * SM::SOP_BUF;
       bf16x8_t bop[2][2][2];   // [buffer][column block of the pair][ddK | K]
@@ -370,7 +370,7 @@ __device__ __forceinline__ void q_run_pc(const Params& p, char* smem, int bh, in
     int sp = 0;  // ring slot of tile j
     for (int j = j_begin; j <= j_end; j++) {
       const int k0 = j * TS;
-      if (j < j_end && !geo.dead(k0, qw)) {
+      if (j < j_end && !geo.dead(k0, geo.first_row(qw, p.n_q))) {
         const char* stage = smem + sp * SM::STAGE;
         char* sop = sop_base + (j & 1) * SM::SOP_BUF;
         const bool masked = geo.partial(k0, qw);
@@ -435,7 +435,7 @@ __device__ __forceinline__ void k_run_pc(const Params& p, char* smem, int bh, in
     int sp = 0;  // ring slot of tile j (slot 0 holds tile t_begin)
     for (int j = t_begin; j <= t_end; j++) {
       const int qb = j * TS;
-      if (j < t_end && !geo.dead(qb, kw)) {
+      if (j < t_end && !geo.dead(qb, geo.first_row(kw, p.n_k))) {
         const char* stage = smem + sp * SM::STAGE;
         char* sop = sop_base + (j & 1) * SM::SOP_BUF;
         const bool masked = geo.partial(qb, kw);
@@ -512,8 +512,8 @@ __device__ __forceinline__ void k_run_pc(const Params& p, char* smem, int bh, in
         dma.template issue_all<3>(dst, SM::TILE, src, adv, wq, p.n_q - (j + 1) * TS);
       }
       // block j-1: key block kb of the pair took part iff the tile held a query that sees one of its keys
-      const bool act0 = j > t_begin && !geo.dead((j - 1) * TS, kw2);
-      const bool act1 = j > t_begin && !geo.dead((j - 1) * TS, kw2 + 32);
+      const bool act0 = j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw2, p.n_k));
+      const bool act1 = j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw2 + 32, p.n_k));
       if (act0 || act1) {
         const char* stage = smem + sc * SM::STAGE;
         const char* sop = sop_pair + ((j - 1) & 1) * SM::SOP_BUF;
@@ -718,7 +718,7 @@ __global__ void __launch_bounds__(PC_THREADS) attn_bwd_k_pc(AttnParams p) {
     int sp = 0;  // ring slot of tile j (slot 0 holds tile t_begin)
     for (int j = t_begin; j <= t_end; j++) {
       const int qb = j * TS;
-      if (j < t_end && !geo.dead(qb, kw)) {
+      if (j < t_end && !geo.dead(qb, geo.first_row(kw, p.n_k))) {
         const char* stage = smem + sp * SM::STAGE;
         char* sop = sop_base + (j & 1) * SM::SOP_BUF;
         const bool masked = geo.partial(qb, kw);
@@ -779,7 +779,7 @@ __global__ void __launch_bounds__(PC_THREADS) attn_bwd_k_pc(AttnParams p) {
         load_stat((j + 1) * TS);
         dma.template issue_all<2>(dst, SM::TILE, src, adv, wq, p.n_q - (j + 1) * TS);
       }
-      if (j > t_begin && !geo.dead((j - 1) * TS, kw)) {
+      if (j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw, p.n_k))) {
         const char* stage = smem + sc * SM::STAGE;
         const char* sop = sop_base + ((j - 1) & 1) * SM::SOP_BUF;
         bf16x8_t a_op[2][2];   // [k-step][dS | P]

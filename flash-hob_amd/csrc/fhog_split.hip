@@ -428,7 +428,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
       // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
       char* const next = smem + (buf ^ 1) * STAGE;
       const int row0 = min(s0 + 2 * TS, n_str - 1);
-      if (!geo.dead(s0, rw)) {
+      if (!geo.dead(s0, geo.first_row(rw, n_sta))) {
         block(smem + buf * STAGE, s0, [] {}, [&](int slot, int slots) {
           st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
           if (KSIDE && slot == 1) publish_stat(0, next);
@@ -445,7 +445,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
         if (more) fetch(t + WS);
       };
       if (!LATE) next();
-      if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, rw))) {
+      if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, geo.first_row(rw, n_sta)))) {
         block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
           if (LATE) {
             __builtin_amdgcn_sched_barrier(0);

@@ -1,9 +1,10 @@
-"""GPU tier: fp32 tensors in launches that fill the GPU, where a workgroup's four waves have 32 rows each: the next tile is split behind the
-MFMAs of this one (statistics sweeps and forward at d = 64), two workgroups share a CU (first order at d = 64, forward at d = 128)."""
+"""GPU tier: launches that fill the GPU, where a workgroup's four waves have 32 rows each. fp32 tensors: the next tile is split behind the
+MFMAs of this one (statistics sweeps and forward at d = 64), two workgroups share a CU (first order at d = 64, forward at d = 128). All: waves
+whose rows lie past the end of their tensor compute nothing."""
 import pytest
 import torch
 
-from gpu_util import NAMES, errors, make_case, reference_fp64_cpu, require_gpu, run_fhog, with_caches
+from gpu_util import NAMES, TOL, errors, make_case, reference_fp64_cpu, require_gpu, run_fhog, with_caches
 
 pytestmark = pytest.mark.gpu
 
@@ -37,13 +38,14 @@ def _first_order_fp64(x, scale, causal, window):
     return (o.detach(), *torch.autograd.grad(o, (q, k, v), x["dO"].double().cpu()[sel]))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("form", FORMS, ids=str)
-def test_first_order_and_double_backward(form, d):
-    """Gate of fp32 tensors, 1e-4 of the largest number. One key: dS is rounding of d, and so are dQ, dK, dQ2 and dK2."""
+def test_first_order_and_double_backward(form, d, dtype):
+    """The gate of the type. One key: dS is rounding of d, and so are dQ, dK, dQ2 and dK2."""
     import fhog
     batch, n_q, n_k, causal, window = form
-    x = make_case(batch, n_q, n_k, d, torch.float32, seed=n_q + n_k)
+    x = make_case(batch, n_q, n_k, d, dtype, seed=n_q + n_k)
     scale, sel = d ** -0.5, _slices(batch)
     leaves = [x[n].clone().requires_grad_(True) for n in ("Q", "K", "V")]
     out = fhog.attention(*(t[None] for t in leaves), causal, window)[0]
@@ -51,11 +53,11 @@ def test_first_order_and_double_backward(form, d):
     for name, g, r in zip(("o", "dq", "dk", "dv"), got, _first_order_fp64(x, scale, causal, window)):
         assert torch.isfinite(g).all(), name
         if n_k > 1 or name in ("o", "dv"):
-            assert (g.double().cpu()[sel] - r).abs().max() <= 1e-4 * r.abs().max(), name
+            assert (g.double().cpu()[sel] - r).abs().max() <= TOL[dtype] * r.abs().max(), name
     c = with_caches(x, scale, causal, window)
     outs = run_fhog(c, scale, causal, window=window)
     ref = reference_fp64_cpu({n: t for n, t in x.items()}, scale, causal, window, heads=sel)
     for name, e in errors([t.cpu()[sel] for t in outs], [torch.from_numpy(ref[n]) for n in NAMES]).items():
         if n_k > 1 or name in ("dv2", "ddo"):
-            assert e <= 1e-4, (name, e)
+            assert e <= TOL[dtype], (name, e)
     assert all(torch.isfinite(t).all() for t in outs)
