@@ -21,7 +21,7 @@
 // CU (d = 64, numbers split again for every tile): 226 -> 319.
 // Some do not quite fit the register file and keep VGPRs of a
 // lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 62 to 72, at d = 64 with four waves on the same
-// rows 43 to 52, with one at d = 32 8; 16-bit tensors at d = 128 up to 53.
+// rows 43 to 46, with one at d = 32 6 to 8; 16-bit tensors at d = 128 up to 53.
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 121     fp32 causal 64 x 1024, d = 32: 672 -> 279
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 915    fp32 64 x 2048, d = 64: 7521 -> 3490
