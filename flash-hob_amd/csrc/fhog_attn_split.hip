@@ -33,9 +33,9 @@ constexpr int min_workgroups = WS > 1 || (sizeof(T) * D > 256 && !TWO) ? 1 : 2;
 template <int WS, bool TWO>
 constexpr int n_buffers = WS == 1 && !TWO ? 2 : 1;
 
-// OWN_D: dK, dV without the sweep for dQ before it
+// OWN_D: dK, dV without the sweep for dQ before it; pairs: as decode_block takes it
 template <typename T, int D, int MODE, int MASK, int WS, bool OWN_D, bool TWO = false>
-__device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id) {
+__device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id, bool pairs) {
   constexpr bool KSIDE = MODE == MODE_BWD_K;
   // split_pair: two waves of fp32 tensors on a SIMD run faster without the dot products (dK, dV causal 32 x 2048, d = 64 231 -> 217 us), the VALU-bound ones of
   // 16-bit tensors with them (bf16 causal 64 x 1024, d = 32 86.5 against 89.3 us for both first-order passes)
@@ -58,7 +58,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, MASK != MASK_NONE && min_workgroups<T, D, WS, TWO> == 2, id)) return;
+  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, MASK != MASK_NONE, bh, tile, pairs, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
@@ -351,15 +351,17 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
 template <typename T, int D, int MODE, int MASK, int WS, bool TWO>
 __global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, TWO>)) attn_split(AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x);
+  attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x, MASK != MASK_NONE && min_workgroups<T, D, WS, TWO> == 2);
 }
 
-// dQ (workgroups [0, q_blocks)) and dK, dV (the others) in one launch
+// dQ (workgroups [0, q_blocks)) and dK, dV (the others; mixed: tile by tile in turn) in one launch
 template <typename T, int D, int MASK, int WS>
-__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, false>)) attn_split_bwd(AttnParams p, int q_blocks) {
+__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, false>)) attn_split_bwd(AttnParams p, int q_blocks, bool mixed) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  if ((int)blockIdx.x < q_blocks) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, blockIdx.x);
-  else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, (int)blockIdx.x - q_blocks);
+  constexpr bool joins = MASK != MASK_NONE && min_workgroups<T, D, WS, false> == 2;   // workgroups of a masked launch that share a CU
+  int id = blockIdx.x;
+  if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, joins, id)) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, id, joins && !mixed);
+  else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, id, joins && !mixed);
 }
 
 template <typename T, int D, int MODE, int WS, bool TWO = false>
@@ -390,7 +392,7 @@ hipError_t launch_bwd_ws(const AttnParams& p, hipStream_t s) {
   const hipError_t e = allow_dynamic_lds<attn_split_bwd<T, D, MASK, WS>>(smem);
   if (e != hipSuccess) return e;
   const unsigned gq = blocks<WS>(p.n_q, p.batch), gk = blocks<WS>(p.n_k, p.batch);
-  hipLaunchKernelGGL((attn_split_bwd<T, D, MASK, WS>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq);
+  hipLaunchKernelGGL((attn_split_bwd<T, D, MASK, WS>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq, WS == 1 && rules::split_in_turn(p, gq, gk));
   return hipGetLastError();
 }
 

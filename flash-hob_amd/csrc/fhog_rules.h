@@ -412,6 +412,17 @@ inline bool few_rows(const Params& p, int bytes) {
   return groups <= (triangle ? line + line / 4 : line);
 }
 
+// Both sweeps of a launch of split products at d = 32, gq and gk workgroups of one wave to 32 rows, in turn as in mixed_order: the second one's heavy tiles
+// otherwise start when half of the launch is over. Equal sides of fewer than 1000 workgroups under a mask that leaves their work uneven. us, one after
+// the other -> in turn: double-backward bf16 causal 32 x 1024 104 -> 80, 64 x 1024 137 -> 128, 8 x 4096 440 -> 324, 2 x 17000 1522 -> 1166, window 1200
+// 32 x 2000 190 -> 179, fp32 32 x 2048 516 -> 502; training step bf16 64 x 1024 79 -> 75, 8 x 4096 327 -> 281. Not there: 1024 workgroups 225 -> 224,
+// 3072 1559 -> 1611; bottom-right 32 x 1000 x 1500 127 -> 131; window 500 32 x 1000 x 3000 82 -> 84; four waves on the same rows fp32 16 x 1024 98 -> 106;
+// fp32 d = 64 48 x 1537 889 -> 919, d = 128 32 x 2048 2206 -> 2247, where a CU has one workgroup.
+template <typename P>
+bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
+  return p.d == 32 && p.causal && gq == gk && gq < 1000 && 2 * (int64_t)p.window >= p.n_k;
+}
+
 // Waves on the same 32 rows for passes 3 and 4 in one launch, or 0 for two launches: four waves while that gives one workgroup per CU, two as long as the
 // workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. The figures are those of launch_grads (fhog_split.hip).
 inline int split_grads_waves(const Params& p, int bytes) {

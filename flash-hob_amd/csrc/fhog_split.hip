@@ -53,8 +53,9 @@ template <int PASS, int WS>
 constexpr bool is_direct = WS == 4 && (PASS == 1 || PASS == 2 || PASS == 5);
 
 // PASS 1: d, dd; 2: b; 3: dQ2, ddO; 4: dK2, dV2 (K-tiled); 5: d, dd, b.
+// pairs: as decode_block takes it
 template <typename T, int D, int PASS, int MASK, int WS>
-__device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
+__device__ __forceinline__ void split_run(const Params& p, char* smem, int id, bool pairs) {
   constexpr bool KSIDE = PASS == 4, STATS = PASS == 1 || PASS == 2 || PASS == 5;
   constexpr int NT = PASS == 1 ? 2 : (KSIDE ? 3 : 4);      // streamed tensors: K, ddK, V, ddV | Q, ddQ, dO
   constexpr int NR = PASS == 1 ? 2 : (KSIDE ? 4 : 3);      // stationary tensors: Q, ddQ, dO | K, ddK, V, ddV
@@ -85,7 +86,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
   const int n = lane & 31, h = lane >> 5;
   const int n_sta = KSIDE ? p.n_k : p.n_q, n_str = KSIDE ? p.n_q : p.n_k;
   int bh, tile;
-  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, KSIDE ? p.tile_major_k : p.tile_major, bh, tile, MASK != MASK_NONE && D < 64 && WS == 1, id)) return;
+  if (!decode_block<MASK>((n_sta + ROWS - 1) / ROWS, p.batch, !KSIDE && MASK != MASK_NONE, KSIDE ? p.tile_major_k : p.tile_major, bh, tile, pairs, id)) return;
   const int64_t qoff = (int64_t)bh * p.stride_qb, koff = (int64_t)bh * p.stride_kb;
   const int64_t sta_ld = KSIDE ? p.stride_kn : p.stride_qn, str_ld = KSIDE ? p.stride_qn : p.stride_kn;
   const int r0 = tile * ROWS, rw = r0 + 32 * group, ri = rw + n;
@@ -511,18 +512,23 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id) {
 template <int D, int WS>
 constexpr int min_workgroups = D >= 64 || WS > 1 ? 1 : 2;
 
+// workgroups of a masked launch that share a CU
+template <int D, int MASK, int WS>
+constexpr bool joins = MASK != MASK_NONE && D < 64 && WS == 1;
+
 template <typename T, int D, int PASS, int MASK, int WS>
 __global__ void __launch_bounds__(256, (min_workgroups<D, WS>)) split_sweep(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  split_run<T, D, PASS, MASK, WS>(p, smem, blockIdx.x);
+  split_run<T, D, PASS, MASK, WS>(p, smem, blockIdx.x, joins<D, MASK, WS>);
 }
 
-// Passes 3 (workgroups [0, q_blocks)) and 4 (the others) in one launch: given the row statistics neither needs the other.
+// Passes 3 (workgroups [0, q_blocks)) and 4 (the others; mixed: tile by tile in turn) in one launch: given the row statistics neither needs the other.
 template <typename T, int D, int MASK, int WS3, int WS4>
-__global__ void __launch_bounds__(256, (min_workgroups<D, (WS3 > WS4 ? WS3 : WS4)>)) split_grads(Params p, int q_blocks) {
+__global__ void __launch_bounds__(256, (min_workgroups<D, (WS3 > WS4 ? WS3 : WS4)>)) split_grads(Params p, int q_blocks, bool mixed) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  if ((int)blockIdx.x < q_blocks) split_run<T, D, 3, MASK, WS3>(p, smem, blockIdx.x);
-  else split_run<T, D, 4, MASK, WS4>(p, smem, (int)blockIdx.x - q_blocks);
+  int id = blockIdx.x;
+  if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, joins<D, MASK, WS3>, id)) split_run<T, D, 3, MASK, WS3>(p, smem, id, joins<D, MASK, WS3> && !mixed);
+  else split_run<T, D, 4, MASK, WS4>(p, smem, id, joins<D, MASK, WS4> && !mixed);
 }
 
 template <typename T, int D, int PASS, int WS>
@@ -583,7 +589,7 @@ hipError_t launch_grads_most(const Params& p, int sides, hipStream_t s) {
   const hipError_t e = allow_dynamic_lds<split_grads<T, D, MASK, ws3, ws4>>(smem);
   if (e != hipSuccess) return e;
   const unsigned gq = sides & 1 ? blocks<ws3>(p.n_q, p.batch) : 0, gk = sides & 2 ? blocks<ws4>(p.n_k, p.batch) : 0;
-  hipLaunchKernelGGL((split_grads<T, D, MASK, ws3, ws4>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq);
+  hipLaunchKernelGGL((split_grads<T, D, MASK, ws3, ws4>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq, ws3 == 1 && ws4 == 1 && rules::split_in_turn(p, gq, gk));
   return hipGetLastError();
 }
 
