@@ -25,9 +25,10 @@ constexpr int MODE_FWD = 0, MODE_BWD_Q = 1, MODE_BWD_K = 2;
 // Workgroups on a CU that the registers are to leave room for. At d = 64 two keep a SIMD busy where one waits (for LDS operands, the
 // splitting, a barrier): everything fits 256 registers. us, one -> two, fp32 causal 32 x 2048 | no mask 64 x 2048: forward 146 -> 128 |
 // 410 -> 368, dQ 193 -> 158 | 528 -> 495, dK, dV 238 -> 209 | 783 -> 648. At d = 128 so does the forward (TWO), without the second stage of
-// the ring and with the query's numbers instead of their terms; worth it in launches with work for two on every CU (launch_fwd).
+// the ring and with the query's numbers instead of their terms; worth it in launches with work for two on every CU (launch_fwd). At d = 32 also with
+// waves on the same rows: first backward of fp32 causal 16 x 1024, four of them, 53 us with two workgroups and 66 with one.
 template <typename T, int D, int WS, bool TWO>
-constexpr int min_workgroups = WS > 1 || (sizeof(T) * D > 256 && !TWO) ? 1 : 2;
+constexpr int min_workgroups = (WS > 1 && D > 32) || (sizeof(T) * D > 256 && !TWO) ? 1 : 2;
 
 // Stages of the ring. With a wave split the WS tiles of a step take the room of the second one.
 template <int WS, bool TWO>
@@ -39,7 +40,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   constexpr bool KSIDE = MODE == MODE_BWD_K;
   // split_pair: two waves of fp32 tensors on a SIMD run faster without the dot products (dK, dV causal 32 x 2048, d = 64 231 -> 217 us), the VALU-bound ones of
   // 16-bit tensors with them (bf16 causal 64 x 1024, d = 32 86.5 against 89.3 us for both first-order passes)
-  constexpr bool DOT = sizeof(T) == 2;
+  constexpr bool DOT = sizeof(T) == 2 || D == 32;
   constexpr int NR = MODE == MODE_FWD ? 1 : 2;             // stationary tensors: Q | Q, dO | K, V
   constexpr int KK = D / 16, NC = D / 32, NF = Terms<T>::NF;
   using Stage = Stager<T, D, 2, true, 0, DOT>;                     // streamed tensors: K, V | Q, dO
@@ -351,14 +352,14 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
 template <typename T, int D, int MODE, int MASK, int WS, bool TWO>
 __global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, TWO>)) attn_split(AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x, MASK != MASK_NONE && min_workgroups<T, D, WS, TWO> == 2);
+  attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x, MASK != MASK_NONE && WS == 1 && min_workgroups<T, D, WS, TWO> == 2);
 }
 
 // dQ (workgroups [0, q_blocks)) and dK, dV (the others; mixed: tile by tile in turn) in one launch
 template <typename T, int D, int MASK, int WS>
 __global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, false>)) attn_split_bwd(AttnParams p, int q_blocks, bool mixed) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr bool joins = MASK != MASK_NONE && min_workgroups<T, D, WS, false> == 2;   // workgroups of a masked launch that share a CU
+  constexpr bool joins = MASK != MASK_NONE && WS == 1 && min_workgroups<T, D, WS, false> == 2;   // workgroups of a masked launch that share a CU
   int id = blockIdx.x;
   if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, joins, id)) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, id, joins && !mixed);
   else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, id, joins && !mixed);
