@@ -440,7 +440,8 @@ __global__ void __launch_bounds__(256, 2) dd_sweep64_bf16(Params p) {
     const char* stage = smem + (j & 1) * STAGE;
     if (act[0] && act[1]) dd_block64<F16, D, true, true>(stage, aoff, Qb, ddQb, c_scale_log2, l_log2, masked, lo, hi, red);
     else if (act[1]) dd_block64<F16, D, false, true>(stage, aoff, Qb, ddQb, c_scale_log2, l_log2, masked, lo, hi, red);
-    else if (MASK == MASK_BAND && act[0]) dd_block64<F16, D, true, false>(stage, aoff, Qb, ddQb, c_scale_log2, l_log2, masked, lo, hi, red);
+    // block 1 lies past the end of the tensor (under any mask), or the tile before its window
+    else if (act[0]) dd_block64<F16, D, true, false>(stage, aoff, Qb, ddQb, c_scale_log2, l_log2, masked, lo, hi, red);
     dma_wait();
     __syncthreads();
   }

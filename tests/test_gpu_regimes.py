@@ -98,15 +98,19 @@ for tag, (shape, causal, window) in {cases!r}.items():
     x = with_caches(make_case(batch, n_q, n_k, d, torch.bfloat16, seed=45, grad_std=0.1), d ** -0.5, causal, window)
     res = run_fhog(x, d ** -0.5, causal, window=window, return_stats=True)
     out[tag] = [t.cpu() for t in res[:4]] + [t.cpu() for t in res[4]]
-    res = run_fhog(x, d ** -0.5, causal, window=window, return_stats=True, schedule="three_sweep", split=False)
-    out[tag + "/three_sweep"] = [t.cpu() for t in res[:4]] + [t.cpu() for t in res[4]]
+    for schedule in ("three_sweep", "four_pass"):
+        res = run_fhog(x, d ** -0.5, causal, window=window, return_stats=True, schedule=schedule, split=False)
+        out[tag + "/" + schedule] = [t.cpu() for t in res[:4]] + [t.cpu() for t in res[4]]
 torch.save(out, sys.argv[1])
 """
 # Ragged and masked, d = 128: with small=0 the 8-wave b and ddO sweeps, the 64-queries-per-wave dd sweep and both workgroup orders on launches of a
 # handful of workgroups, and "split", whose passes split their streamed side; by default the kernels for small launches, which read none of the choices,
-# run the three (each case under the default and under the three-sweep schedule). d64_many: d = 64 with workgroups enough not to split (the one-launch
-# form of sweeps 1-3 and the 64-row stage apply)
+# run the default schedule and the three-sweep one. Each case also under the four-pass schedule, the one with a dd sweep of its own. tail_*: that
+# many queries in the last 64 (of them the dd sweep's wave has two blocks of 32, whose second may be empty). d64_many: d = 64 with workgroups
+# enough not to split (the one-launch form of sweeps 1-3 and the 64-row stage apply)
 _TUNE_CASES = {"ragged_causal": ((3, 333, 333, 128), True, None), "window": ((2, 300, 400, 128), "bottom_right", 200),
+               "tail_1": ((2, 257, 200, 128), False, None), "tail_19": ((3, 275, 275, 128), True, None), "tail_32": ((2, 288, 200, 128), False, None),
+               "tail_33": ((2, 289, 289, 128), True, None), "tail_44": ((2, 300, 200, 128), False, None),
                "d64_many": ((180, 384, 300, 64), False, None), "split": ((2, 700, 700, 128), True, None)}
 
 
@@ -127,11 +131,24 @@ def test_launch_choices_forced_without_the_small_kernels(tmp_path):
     _check_launch_choices(tmp_path, "small=0,")
 
 
+def _check_against_fp64(tag, got, heads=(0, -1)):
+    """Row statistics and outputs of some slices at the gates of this file."""
+    (batch, n_q, n_k, d), causal, window = _TUNE_CASES[tag.split("/")[0]]
+    x = make_case(batch, n_q, n_k, d, torch.bfloat16, seed=45, grad_std=0.1, device="cpu")
+    sel = list(heads)
+    ref = reference_fp64_cpu(x, d ** -0.5, causal, window, heads=sel)
+    for i, name in enumerate(("dq2", "dk2", "dv2", "ddo", "d", "dd", "b")):
+        e = normalised_max_error(got[i][sel].float(), ref[name])
+        assert e < (2e-2 if i < 4 else 1e-2), (tag, name, e)
+
+
 def _check_launch_choices(tmp_path, prefix):
     """b8, dd64, order, stage64 and stage1 change which kernel, which workgroup order or how many launches run, never a bit
     of the results; split=0 changes the fp32 summation order of the launches that would split. Unknown keys are reported,
     not obeyed."""
     base, _ = _run_child(tmp_path, prefix.rstrip(","))
+    for tag in base:
+        _check_against_fp64(tag, base[tag])
     for tune in ("b8=1,dd64=1,order=slice,stage1=1", "b8=0,dd64=0,order=tile,stage64=1"):
         got, err = _run_child(tmp_path, prefix + tune)
         assert "FHOG_TUNE" not in err, err
@@ -148,3 +165,15 @@ def _check_launch_choices(tmp_path, prefix):
                 assert torch.equal(a, b_), tag
     for i, (a, b_) in enumerate(zip(got["split"], base["split"])):
         assert normalised_max_error(a, b_.float()) < (1e-5 if i >= 4 else 8e-3), i   # row statistics in fp32, outputs rounded to bf16
+
+
+@pytest.mark.parametrize("shape,causal", [((2050, 20, 40), False), ((1030, 275, 275), True), ((1030, 289, 40), False)])
+def test_dd_sweep_of_large_launches(shape, causal):
+    """From 2048 workgroups of 256 rows on a wave of the dd sweep has 64 queries in two blocks of 32: a last wave whose second block is past the end."""
+    x = with_caches(make_case(*shape, 128, torch.bfloat16, seed=47, grad_std=0.1), 128 ** -0.5, causal)
+    heads = [0, 1, shape[0] // 2, shape[0] - 1]
+    *outs, stats = run_fhog(x, 128 ** -0.5, causal, return_stats=True, schedule="four_pass", split=False)
+    ref = reference_fp64_cpu({n: t for n, t in x.items() if n not in ("O", "L")}, 128 ** -0.5, causal, heads=heads)
+    for name, t in zip((*NAMES, "d", "dd", "b"), (*outs, *stats)):
+        e = normalised_max_error(t[heads].float(), ref[name])
+        assert e < (2e-2 if name in NAMES else 1e-2), (name, e)
