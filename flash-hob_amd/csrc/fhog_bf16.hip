@@ -25,6 +25,8 @@
 // streamed rows), the A operands are transposing reads of the staged tiles in the same row order. At d = 128
 // the output accumulators alone take 128 registers and the work is split over producer and consumer waves.
 
+#include <type_traits>
+
 #include "fhog_bf16_blocks.h"
 #include "fhog_rules.h"
 
@@ -187,8 +189,8 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
   dma_wait();
   __syncthreads();
 
-  // one group of SUB tiles, in the first or the second half of the ring
-  const auto group = [&](auto half_of_ring, int jj) {
+  // one group of SUB tiles, in the first or the second half of the ring; rows (without a mask): some of the wave's queries exist, else it only stages
+  const auto group = [&](auto half_of_ring, auto rows, int jj) {
     constexpr int GRP = decltype(half_of_ring)::value * SUB;
 #pragma unroll
     for (int u = 0; u < SUB; u++)
@@ -201,7 +203,7 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
       const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
       int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
       if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-      if (!geo.dead(k0, geo.first_row(qw, p.n_q))) {  // else every key of the tile is hidden from this wave
+      if (MASK == MASK_NONE ? decltype(rows)::value : !geo.dead(k0, geo.first_row(qw, p.n_q))) {  // else every key of the tile is hidden from this wave
         const char* stage = smem + (GRP + u) * STAGE;
         q_block<F16, D, PASS>(stage, aoff, troff, Qb, ddQb, dOb, masked, lo, hi, c_scale_log2, l_log2, p.scale, dsum, dd, kc, red, red_dd, red_vdds,
                               red_pu, red_p, acc_dq, acc_ddo);
@@ -212,9 +214,13 @@ __device__ __forceinline__ void q_sweep_run(const Params& p, char* smem, int bh,
     dma_wait();
     __syncthreads();
   };
-  int jj = j_begin;
-  for (; jj + SUB < j_end; jj += 2 * SUB) group(Slot<0>{}, jj), group(Slot<1>{}, jj + SUB);
-  if (jj < j_end) group(Slot<0>{}, jj);
+  const auto sweep = [&](auto rows) {
+    int jj = j_begin;
+    for (; jj + SUB < j_end; jj += 2 * SUB) group(Slot<0>{}, rows, jj), group(Slot<1>{}, rows, jj + SUB);
+    if (jj < j_end) group(Slot<0>{}, rows, jj);
+  };
+  if (MASK == MASK_NONE && qw >= p.n_q) sweep(std::false_type{});
+  else sweep(std::true_type{});
   if (WITH_DDO && p.n_split > 1) {   // fp32 partial rows [split][dQ2 | ddO][batch * n_q][D]
     if (qi >= p.n_q) return;
     const int64_t rows = (int64_t)p.batch * p.n_q;
@@ -548,7 +554,7 @@ __device__ __forceinline__ void k_sweep_run(const Params& p, char* smem, int bh,
   dma_wait();
   __syncthreads();
 
-  const auto group = [&](auto half_of_ring, int jj) {
+  const auto group = [&](auto half_of_ring, auto rows, int jj) {   // rows: as in q_sweep_run
     constexpr int grp = decltype(half_of_ring)::value * SUB;   // first ring slot of this group; the other group starts at grp ^ SUB
 #pragma unroll
     for (int u = 0; u < SUB; u++)
@@ -561,7 +567,7 @@ __device__ __forceinline__ void k_sweep_run(const Params& p, char* smem, int bh,
       const int j = jj + u;
       if (SUB > 1 && j >= t_end) continue;
       const int qb = j * TS;
-      if (!geo.dead(qb, geo.first_row(kw, p.n_k))) {  // else no query of the tile sees a key of this wave
+      if (MASK == MASK_NONE ? decltype(rows)::value : !geo.dead(qb, geo.first_row(kw, p.n_k))) {  // else no query of the tile sees a key of this wave
         const char* stage = smem + (grp + u) * STAGE;
         k_block<F16, D>(geo, stage, aoff, troff, Kb, ddKb, Vb, ddVb, qb, kw, kj, h, c_scale_log2, p.scale, acc_dk, acc_dv);
       }
@@ -575,9 +581,13 @@ __device__ __forceinline__ void k_sweep_run(const Params& p, char* smem, int bh,
     dma_wait();
     __syncthreads();
   };
-  int jj = t_begin;
-  for (; jj + SUB < t_end; jj += 2 * SUB) group(Slot<0>{}, jj), group(Slot<1>{}, jj + SUB);
-  if (jj < t_end) group(Slot<0>{}, jj);
+  const auto sweep = [&](auto rows) {
+    int jj = t_begin;
+    for (; jj + SUB < t_end; jj += 2 * SUB) group(Slot<0>{}, rows, jj), group(Slot<1>{}, rows, jj + SUB);
+    if (jj < t_end) group(Slot<0>{}, rows, jj);
+  };
+  if (MASK == MASK_NONE && kw >= p.n_k) sweep(std::false_type{});
+  else sweep(std::true_type{});
   if (kj >= p.n_k) return;
   if (p.n_split > 1) {   // fp32 partial rows [split][dK2 | dV2][batch * n_k][D]
     const int64_t rows = (int64_t)p.batch * p.n_k;
