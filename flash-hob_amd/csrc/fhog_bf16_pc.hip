@@ -181,7 +181,10 @@ __device__ __forceinline__ void consume_q(const Params& p, char* smem, const Str
     }
     // block j-1: query block qb of the pair took part iff the tile held a key visible to it
     const bool act0 = j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0, p.n_q));
-    const bool act1 = j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0 + 32, p.n_q));
+    // Without a mask block 1 goes along with block 0, past the end of the tensor too (as below under a plain causal one): its operand tiles are not
+    // written then, and what is made of them stays in rows that are not stored. Branches around its MFMAs, here and in pass 4, cost every length: double-backward,
+    // us, with | without: 4 x 4096 313.0 | 308.8, fp16 1 x 8192 340.6 | 335.8, 64 x 2048 1194.6 | 1190.4; 128 x 400 147.2 | 147.4.
+    const bool act1 = MASK == MASK_NONE ? act0 : j > j_begin && !geo.dead((j - 1) * TS, geo.first_row(qw0 + 32, p.n_q));
     const bool act = act0 || act1;
     const char* stage = smem + sc * SM::STAGE;
     const char* sop = sop_pair + ((j - 1) & 1) * SM::SOP_BUF;
@@ -218,7 +221,7 @@ __device__ __forceinline__ void consume_q(const Params& p, char* smem, const Str
 #pragma unroll
           for (int cl = 0; cl < 2; cl++) {
             if (act0) acc[0][2 * cp + cl] = mfma<F16>(a_op[t][0][pr], bop[c][cl][pr], acc[0][2 * cp + cl]);
-            // with a plain causal mask (or none) a tile that block 0 takes part in is also one for block 1
+            // with a plain causal mask a tile that block 0 takes part in is also one for block 1, unless that is past the end of the tensor
             if (MASK != MASK_BAND || act1) acc[1][2 * cp + cl] = mfma<F16>(a_op[t][1][pr], bop[c][cl][pr], acc[1][2 * cp + cl]);
           }
         __builtin_amdgcn_sched_barrier(0);
@@ -404,7 +407,8 @@ __device__ __forceinline__ int sop_tr_lane_off(int s, int lane) {
   return r * 64 + (((2 * b + (cg & 1)) ^ sop_swz(r)) << 4) + 8 * (cg >> 1);
 }
 
-template <bool F16, int D, int MASK>
+// DQ_ONLY: beside the sweep for dQ2 alone
+template <bool F16, int D, int MASK, bool DQ_ONLY>
 __device__ __forceinline__ void k_run_pc(const Params& p, char* smem, int bh, int tile, int split) {
   using SM = PCSmem<D, true>;
   constexpr int NC = D / 32;
@@ -513,7 +517,8 @@ __device__ __forceinline__ void k_run_pc(const Params& p, char* smem, int bh, in
       }
       // block j-1: key block kb of the pair took part iff the tile held a query that sees one of its keys
       const bool act0 = j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw2, p.n_k));
-      const bool act1 = j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw2 + 32, p.n_k));
+      // Without a mask as in consume_q; but beside the sweep for dQ2 alone the branch is the faster form (64 x 2048 1139 -> 1125)
+      const bool act1 = MASK == MASK_NONE && !DQ_ONLY ? act0 : j > t_begin && !geo.dead((j - 1) * TS, geo.first_row(kw2 + 32, p.n_k));
       if (act0 || act1) {
         const char* stage = smem + sc * SM::STAGE;
         const char* sop = sop_pair + ((j - 1) & 1) * SM::SOP_BUF;
@@ -616,7 +621,7 @@ __global__ void __launch_bounds__(PC_THREADS) grads_pc(Params p, int q_blocks, b
     p.n_split = p.n_split_k, p.part = p.part_k;
     if (!decode_block<MASK>((p.n_k + WG_ROWS - 1) / WG_ROWS, p.batch * p.n_split, false, p.tile_major_k, bh, tile, false, id)) return;
     if (p.n_split > 1) split = bh % p.n_split, bh /= p.n_split;
-    k_run_pc<F16, D, MASK>(p, smem, bh, tile, split);
+    k_run_pc<F16, D, MASK, DQ_ONLY>(p, smem, bh, tile, split);
   }
 }
 
