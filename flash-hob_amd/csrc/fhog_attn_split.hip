@@ -247,7 +247,7 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
         second.start(stage + TENSOR, pv);
         second.template run<false>(acc0, stage + TENSOR, pv, stage, pv, [](int) {});   // O += P V
       } else {
-        second_level<T, D, false, DOT>(acc0, stage + TENSOR, troff, pv);
+        second_level<T, D, DOT>(acc0, stage + TENSOR, troff, pv);
       }
     } else {
 #pragma unroll
@@ -264,8 +264,8 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
       }
 #pragma unroll
       for (int r = 0; r < 16; r++) dp[r] *= pv[r];            // dS = P (dP - d) (scale applied to the accumulators at the end)
-      second_level<T, D, false, DOT>(acc0, stage, troff, dp);             // dQ += dS K | dK += dS^T Q
-      if constexpr (KSIDE) second_level<T, D, false, DOT>(acc1, stage + TENSOR, troff, pv);   // dV += P^T dO
+      second_level<T, D, DOT>(acc0, stage, troff, dp);             // dQ += dS K | dK += dS^T Q
+      if constexpr (KSIDE) second_level<T, D, DOT>(acc1, stage + TENSOR, troff, pv);   // dV += P^T dO
     }
   };
 

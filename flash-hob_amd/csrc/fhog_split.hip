@@ -67,8 +67,8 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
   constexpr int STAT = KSIDE ? 4 * TS * 4 : 0;             // L log2(e), -d, dd, -(dd d + b) of the 32 staged queries
   constexpr int STAGE = Stage::BYTES + STAT;
   // fp32, d = 128: the terms of three or four stationary tensors are 288 or 384 registers, so the wave keeps the fp32 numbers
-  // (the last tensor of passes 3 and 4, dO or ddV, in LDS) and splits them again for every tile, one k-step at a time behind the MFMAs of
-  // the one before: 28 VALU instructions per tensor and k-step beside 30 MFMAs.
+  // (the last tensor of passes 3 and 4, dO or ddV, in LDS) and splits them again for every tile, one k-step at a time, in the statistics sweeps behind the
+  // MFMAs of the one before: 28 VALU instructions per tensor and k-step beside 30 MFMAs.
   constexpr bool RAW = is_raw<T, D>;
   constexpr bool LAST_IN_LDS = RAW && !STATS;
   constexpr int NREG = LAST_IN_LDS ? NR - 1 : NR;
@@ -106,23 +106,19 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
   const int64_t srow = (int64_t)bh * p.n_q;
   Stage st[WS];
   float stat_reg[WS] = {}, stat_d[WS] = {}, stat_dd[WS] = {};
-  // pass 4: threads t and t + 128 carry statistic t / 32 of staged query t % 32
+  // pass 4: threads t and t + 128 carry statistic t / 32 of staged query t % 32. All of them without a branch, or 128 that load what they need, us: fp32
+  // causal 64 x 1024, d = 32 271 | 276; no mask bf16 d = 32 2 x 256 11.9 | 13.4, 8 x 512 18.0 | 20.0, 16 x 4096 705 | 702; others within 0.5 %.
   const int which = (tid >> 5) & 3;
   const float* const stat_src = which == 0 ? p.lse : which == 1 ? p.ws_d : which == 2 ? p.ws_dd : p.ws_b;
-  const auto fetch_stat = [&](int g, int row0) {
-    const int64_t q = srow + min(row0 + (tid & 31), p.n_q - 1);
-    stat_reg[g] = stat_src[q], stat_d[g] = p.ws_d[q], stat_dd[g] = p.ws_dd[q];
-  };
-  const auto publish_stat = [&](int g, char* stage) {
-    reinterpret_cast<float*>(stage + Stage::BYTES)[tid & 127] =
-        which == 0 ? stat_reg[g] * kLog2e : which == 1 ? -stat_reg[g] : which == 2 ? stat_reg[g] : -__builtin_fmaf(stat_dd[g], stat_d[g], stat_reg[g]);
-  };
   const auto fetch = [&](int t) {
 #pragma unroll
     for (int g = 0; g < WS; g++) {
       const int row0 = (t + g) * TS;
       st[g].fetch(src, str_ld, min(row0, n_str - 1), n_str, tid);   // a tile past the end is never computed on
-      if (KSIDE) fetch_stat(g, row0);
+      if constexpr (KSIDE) {
+        const int64_t q = srow + min(row0 + (tid & 31), p.n_q - 1);
+        stat_reg[g] = stat_src[q], stat_d[g] = p.ws_d[q], stat_dd[g] = p.ws_dd[q];
+      }
     }
   };
   const auto publish = [&](int buf) {
@@ -130,7 +126,10 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
     for (int g = 0; g < WS; g++) {
       char* stage = smem + (buf * WS + g) * STAGE;
       st[g].publish(stage, tid);
-      if (KSIDE) publish_stat(g, stage);
+      if constexpr (KSIDE) {
+        reinterpret_cast<float*>(stage + Stage::BYTES)[tid & 127] =
+            which == 0 ? stat_reg[g] * kLog2e : which == 1 ? -stat_reg[g] : which == 2 ? stat_reg[g] : -__builtin_fmaf(stat_dd[g], stat_d[g], stat_reg[g]);
+      }
     }
   };
   if (!DIRECT && t_begin < t_end) fetch(t_begin);
@@ -200,12 +199,11 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
     constexpr TermPairs<NF, NF> kPairs{};
     bf16x8_t a[NT][NF];
     Splitting<NF> terms[NR];   // RAW
-    Chunk<T> last_chunk;
     const auto read = [&](int x, int kk) { read_terms<T, Stage::TILE>(stage + x * TENSOR, aoff0 ^ (32 * kk), a[x]); };
     // what is due behind MFMA `slot` of `slots` of the terms of k-step kk of stationary tensor y
     const auto split = [&](int y, int kk, int slot, int slots) {
       if constexpr (RAW) {
-        const Chunk<T>& c = LAST_IN_LDS && y == NR - 1 ? last_chunk : res[y < NREG ? y : 0].r[kk];
+        const Chunk<T>& c = res[y].r[kk];
         terms[y].at(slot, slots, [&](int i, float& lo, float& hi) {
           lo = chunk_elem(c, 2 * i), hi = chunk_elem(c, 2 * i + 1);
           asm("" : "+v"(lo), "+v"(hi) : "s"(s0));   // here, tile after tile: hoisted out of the sweep, the terms would be spilled
@@ -225,19 +223,13 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
 #pragma unroll
       for (int i = 0; i < P; i++) {
         s = mfma<false>(a[0][kPairs.a[i]], sta_term(0, kk, kPairs.b[i]), s);         // K Q^T | Q K^T
-        if (LAST_IN_LDS && i == 0) {
-          last_chunk.v[0] = __builtin_bit_cast(u32x4_t, last[(2 * kk) * 64]);
-          last_chunk.v[sizeof(T) / 2 - 1] = __builtin_bit_cast(u32x4_t, last[(2 * kk + 1) * 64]);
-        }
         split(1, kk, 2 * i, 2 * P);
-        if (KSIDE) split(2, kk, 2 * i, 2 * P);
         behind(5 * P * kk + 2 * i, 5 * P * KK);
         __builtin_amdgcn_sched_barrier(0);
         dds = mfma<false>(a[1][kPairs.a[i]], sta_term(0, kk, kPairs.b[i]), dds);     // ddK Q^T | ddQ K^T
         if (i == 0) read(2, kk);
         if (!KSIDE && i == 1) read(NT - 1, kk);
         split(1, kk, 2 * i + 1, 2 * P);
-        if (KSIDE) split(2, kk, 2 * i + 1, 2 * P);
         behind(5 * P * kk + 2 * i + 1, 5 * P * KK);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -405,11 +397,10 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
           e[r] = __builtin_fmaf(pv[r], e[r], dds[r] * dp[r]);           // dS' = P E' + ddP u
         }
       }
-      if constexpr (!KSIDE) second_level<T, D, RAW>(acc1, stage + (NT - 1) * TENSOR, troff, pv);   // ddO += P ddV
-      second_level<T, D, RAW>(acc0, stage + 1 * TENSOR, troff, s);           // dQ2 += dS ddK | dK2 += dS^T ddQ
-      second_level<T, D, RAW>(acc1, stage + 2 * TENSOR, troff, dds);         // ddO += ddP V | dV2 += ddP^T dO
-      prefetch();
-      second_level<T, D, RAW>(acc0, stage, troff, e);                        // dQ2 += dS' K | dK2 += dS'^T Q
+      if constexpr (!KSIDE) second_level<T, D>(acc1, stage + (NT - 1) * TENSOR, troff, pv);   // ddO += P ddV
+      second_level<T, D>(acc0, stage + 1 * TENSOR, troff, s);           // dQ2 += dS ddK | dK2 += dS^T ddQ
+      second_level<T, D>(acc1, stage + 2 * TENSOR, troff, dds);         // ddO += ddP V | dV2 += ddP^T dO
+      second_level<T, D>(acc0, stage, troff, e);                        // dQ2 += dS' K | dK2 += dS'^T Q
     }
   };
 
@@ -432,8 +423,6 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
       if (!geo.dead(s0, geo.first_row(rw, n_sta))) {
         block(smem + buf * STAGE, s0, [] {}, [&](int slot, int slots) {
           st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
-          if (KSIDE && slot == 1) publish_stat(0, next);
-          if (KSIDE && slot == 2) fetch_stat(0, row0);
         });
       } else {
         publish(buf ^ 1);

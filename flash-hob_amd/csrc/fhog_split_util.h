@@ -323,7 +323,7 @@ __device__ __forceinline__ void read_terms_tr(const char* tensor, int o0, int o1
 }
 
 // acc += X^T W for a staged tensor X (32 rows) and an S-shaped tile W whose registers run over those rows
-template <typename T, int D, bool FENCED = false, bool DOT = true>
+template <typename T, int D, bool DOT = true>
 __device__ __forceinline__ void second_level(f32x16_t (&acc)[D / 32], const char* tensor, const int (&troff)[D / 32][2], const f32x16_t& w) {
 #pragma unroll
   for (int t = 0; t < 2; t++) {
@@ -334,7 +334,6 @@ __device__ __forceinline__ void second_level(f32x16_t (&acc)[D / 32], const char
       bf16x8_t a[Terms<T>::N2];
       read_terms_tr<T, D>(tensor, troff[cb][0], troff[cb][1], t, a);
       acc[cb] = mma2<T>(acc[cb], a, op);
-      if constexpr (FENCED) __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
