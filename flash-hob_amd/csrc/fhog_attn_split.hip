@@ -272,31 +272,41 @@ __device__ __forceinline__ void attn_run(const AttnParams& p, char* smem, int id
   if (t_begin < t_end) publish(0);
   if (INTERLEAVED && t_begin < t_end) fetch(t_begin + 1);
   __syncthreads();
-  for (int t = t_begin; t < t_end; t += WS) {
-    const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
-    if constexpr (INTERLEAVED) {
-      // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
-      char* const next = smem + (buf ^ 1) * STAGE;
-      const int s0 = t * TS, row0 = min(s0 + 2 * TS, n_str - 1);
-      if (!geo.dead(s0, geo.first_row(rw, n_sta))) {
-        block(smem + buf * STAGE, s0, [&](int slot, int slots) {
-          st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
-        });
-      } else {
-        publish(buf ^ 1);
-        fetch(t + 2);
+  // Without a mask only waves whose rows all lie past the end of the tensor see nothing. fp32, d = 128: a test for them in the loop has the compiler spill
+  // what a wave keeps (dK, dV 42 VGPRs), so they have a loop of their own; with two waves on the same rows they compute on copies of the last row. First-order
+  // passes, us, no test | the test | two loops: 32 x 1024 430 | 459 | 425, 64 x 2048 3280 | 3554 | 3213, 2000 | 900 rows 432 | 501 | 423, 128 x 300 249 |
+  // 264 | 233; two waves 16 x 300 84.3 | 85.2 | 86.3, 4 x 1024 228 | 231 | 229. At d = 32 the test is the faster (bf16 16 x 4096 412 | 420).
+  constexpr bool NO_TEST = MASK == MASK_NONE && is_raw<T, D>;
+  const auto sweep = [&](auto has_rows) {
+    const auto works = [&](int s0) { return NO_TEST ? decltype(has_rows)::value : !geo.dead(s0, geo.first_row(rw, n_sta)); };
+    for (int t = t_begin; t < t_end; t += WS) {
+      const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
+      if constexpr (INTERLEAVED) {
+        // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
+        char* const next = smem + (buf ^ 1) * STAGE;
+        const int s0 = t * TS, row0 = min(s0 + 2 * TS, n_str - 1);
+        if (works(s0)) {
+          block(smem + buf * STAGE, s0, [&](int slot, int slots) {
+            st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
+          });
+        } else {
+          publish(buf ^ 1);
+          fetch(t + 2);
+        }
+        __syncthreads();
+        continue;
       }
+      const bool more = t + WS < t_end;
+      if (more) fetch(t + WS);
+      const int s0 = (t + ws) * TS;
+      if ((WS == 1 || t + ws < t_end) && works(s0)) block(smem + (buf * WS + ws) * STAGE, s0, [](int, int) {});
+      if (NBUF == 1) __syncthreads();   // the tiles are no longer read
+      if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
       __syncthreads();
-      continue;
     }
-    const bool more = t + WS < t_end;
-    if (more) fetch(t + WS);
-    const int s0 = (t + ws) * TS;
-    if ((WS == 1 || t + ws < t_end) && !geo.dead(s0, geo.first_row(rw, n_sta))) block(smem + (buf * WS + ws) * STAGE, s0, [](int, int) {});
-    if (NBUF == 1) __syncthreads();   // the tiles are no longer read
-    if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
-    __syncthreads();
-  }
+  };
+  if (NO_TEST && WS == 1 && rw >= n_sta) sweep(std::false_type{});
+  else sweep(std::true_type{});
 
   if constexpr (WS > 1) {
     // the WS waves of a row group merge their partial results in the order of ws; the wave with ws == 0 holds the outcome
