@@ -413,44 +413,53 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
   if (!DIRECT && t_begin < t_end) publish(0);
   if (INTERLEAVED && t_begin < t_end) fetch(t_begin + 1);
   if (!DIRECT) __syncthreads();
-  for (int t = t_begin; !DIRECT && t < t_end; t += WS) {
-    const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
-    const int s0 = (t + ws) * TS;
-    if constexpr (INTERLEAVED) {
-      // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
-      char* const next = smem + (buf ^ 1) * STAGE;
-      const int row0 = min(s0 + 2 * TS, n_str - 1);
-      if (!geo.dead(s0, geo.first_row(rw, n_sta))) {
-        block(smem + buf * STAGE, s0, [] {}, [&](int slot, int slots) {
-          st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
-        });
+  // Without a mask only waves whose rows all lie past the end of the tensor see nothing. At d = 32 they have a loop of their own, for the test in the loop
+  // costs every length: double-backward, us, neither | the test | two loops: bf16 16 x 4096 701 | 710 | 697, 64 x 1024 183 | 185 | 183, fp32 16 x 1000 159 |
+  // 163 | 160, 16 x 4096 1835 | 1836 | 1822, 128 x 300 124 | 119 | 118. At d = 64 the test is the faster (fp32 16 x 2048 878 | 888).
+  constexpr bool NO_TEST = MASK == MASK_NONE && D == 32;
+  const auto sweep = [&](auto has_rows) {
+    const auto works = [&](int s0) { return NO_TEST ? decltype(has_rows)::value : !geo.dead(s0, geo.first_row(rw, n_sta)); };
+    for (int t = t_begin; !DIRECT && t < t_end; t += WS) {
+      const int buf = NBUF == 2 ? (t - t_begin) & 1 : 0;
+      const int s0 = (t + ws) * TS;
+      if constexpr (INTERLEAVED) {
+        // The rows of the tile after this one came in during the step before; behind the last tile they are copies of the last row.
+        char* const next = smem + (buf ^ 1) * STAGE;
+        const int row0 = min(s0 + 2 * TS, n_str - 1);
+        if (works(s0)) {
+          block(smem + buf * STAGE, s0, [] {}, [&](int slot, int slots) {
+            st[0].publish_at(next, tid, slot, slots, [&](int i) { st[0].fetch_chunk(i, src, str_ld, row0, n_str, tid); });
+          });
+        } else {
+          publish(buf ^ 1);
+          fetch(t + 2);
+        }
+        __syncthreads();
       } else {
-        publish(buf ^ 1);
-        fetch(t + 2);
+        const bool more = t + WS < t_end;
+        const auto next = [&]() {
+          if (more) fetch(t + WS);
+        };
+        if (!LATE) next();
+        if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || works(s0))) {
+          block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
+            if (LATE) {
+              __builtin_amdgcn_sched_barrier(0);
+              next();
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }, [](int, int) {});
+        } else if (LATE) {
+          next();
+        }
+        if (NBUF == 1) __syncthreads();   // the tiles are no longer read
+        if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
+        __syncthreads();
       }
-      __syncthreads();
-    } else {
-      const bool more = t + WS < t_end;
-      const auto next = [&]() {
-        if (more) fetch(t + WS);
-      };
-      if (!LATE) next();
-      if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || !geo.dead(s0, geo.first_row(rw, n_sta)))) {
-        block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
-          if (LATE) {
-            __builtin_amdgcn_sched_barrier(0);
-            next();
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }, [](int, int) {});
-      } else if (LATE) {
-        next();
-      }
-      if (NBUF == 1) __syncthreads();   // the tiles are no longer read
-      if (more) publish(NBUF == 2 ? buf ^ 1 : 0);
-      __syncthreads();
     }
-  }
+  };
+  if (NO_TEST && rw >= n_sta) sweep(std::false_type{});
+  else sweep(std::true_type{});
 
   if constexpr (WS > 1) {
     // the WS waves of a row group add their partial results in the order of ws; the wave with ws == 0 holds the sum

@@ -39,7 +39,7 @@ def _first_order_fp64(x, scale, causal, window):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("form", FORMS, ids=str)
 def test_first_order_and_double_backward(form, d, dtype):
     """The gate of the type. One key: dS is rounding of d, and so are dQ, dK, dQ2 and dK2."""
