@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_bf16(AttnParams p) {
     const bool masked = geo.partial(k0, qw);  // wave-uniform: the block holds hidden keys (mask edge or tensor end)
     int lo = 0, hi = 0;                       // key k0 + 8g + 4h + e is visible iff lo <= 8g + e <= hi
     if (masked) keep_branch(), geo.limits(k0, qi, h, lo, hi);
-    if ((MASK == MASK_NONE && D == 64) || !geo.dead(k0, geo.first_row(qw, p.n_q))) {
+    if (MASK == MASK_NONE || !geo.dead(k0, geo.first_row(qw, p.n_q))) {
       const char* stage = smem + u * STAGE;
       bwd_q_block<F16, D>(stage, aoff, troff, Qb, dOb, masked, lo, hi, c_scale_log2, l_log2, dsum, acc);
     }

@@ -247,7 +247,7 @@ struct StreamKeys {
   // so: fp16 48 x 1537, d = 64, three sweeps, Hessian-vector product 364 -> 350; double-backward bf16 128 x 400 no mask d = 64 87 -> 83, d = 128
   // 164 -> 151; training step 48 x 1537 no mask, d = 128 329 -> 317; under a mask lengths without such waves within 0.5 %. Without
   // one the test is all that the loops have of it, and its branch costs the scheduling around the blocks: the forward (32 x 2048 d = 64 55.1 -> 59.1, d = 128
-  // 83.9 -> 87.4) and the sweep for dQ at d = 64 (58.8 -> 59.9) do without, and the sweeps of fhog_bf16.hip have a loop of their own for such waves (double-backward
+  // 83.9 -> 87.4) and the sweep for dQ (d = 64 58.8 -> 59.9; training step d = 128 4 x 6144 409 -> 412, 16 x 256 | 8192 288 -> 292) do without, and the sweeps of fhog_bf16.hip have a loop of their own for such waves (double-backward
   // d = 64, no mask, neither | the test | two loops: fp16 1 x 8192 208.3 | 210.7 | 208.9, 4 x 4096 201.6 | 204.3 | 202.3, bf16 2 x 16384 1342 | 1353 | 1344,
   // 128 x 400 88.2 | 82.4 | 83.0).
   __device__ __forceinline__ static int first_row(int r0, int n) { return r0 < n ? r0 : -(1 << 29); }
