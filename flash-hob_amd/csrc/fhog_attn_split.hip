@@ -415,11 +415,8 @@ hipError_t launch_fwd(const AttnParams& p, hipStream_t s) {
     if (groups < 64 && p.n_k > 2 * TS) return launch_ws<T, D, MODE_FWD, MASK, 4>(p, s);
   }
   if (groups < 128 && p.n_k > TS) return launch_ws<T, D, MODE_FWD, MASK, 2>(p, s);
-  // fp32, d = 128: two workgroups on a CU once there are more than one for each, under a mask more than two (a heavy and a light tile
-  // that share a CU leave the heavy one alone for most of its time). us, one -> two, at so many workgroups: no mask 422 -> 364 (320), 436
-  // -> 420 (512), 857 -> 816 (1024), but 234 -> 258 (256); causal 324 -> 290 (640), 466 -> 435 (1024), but 235 -> 260 (512).
   if constexpr (is_raw<T, D>) {
-    if (groups > (MASK == MASK_NONE ? 256 : 512)) return launch_ws<T, D, MODE_FWD, MASK, 1, true>(p, s);
+    if (rules::two_forwards_on_a_cu(groups, MASK != MASK_NONE)) return launch_ws<T, D, MODE_FWD, MASK, 1, true>(p, s);
   }
   return launch_ws<T, D, MODE_FWD, MASK, 1>(p, s);
 }

@@ -423,6 +423,11 @@ bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
   return p.d == 32 && p.causal && gq == gk && gq < 1000 && 2 * (int64_t)p.window >= p.n_k;
 }
 
+// Forward of fp32 tensors, d = 128: two workgroups on a CU once there are more than one for each, under a mask more than two (a heavy and a light tile
+// that share a CU leave the heavy one alone for most of its time). us, one -> two, at so many workgroups: no mask 422 -> 364 (320), 436
+// -> 420 (512), 857 -> 816 (1024), but 234 -> 258 (256); causal 324 -> 290 (640), 466 -> 435 (1024), but 235 -> 260 (512).
+inline bool two_forwards_on_a_cu(int64_t groups, bool masked) { return groups > (masked ? 512 : 256); }
+
 // Waves on the same 32 rows for passes 3 and 4 in one launch, or 0 for two launches: four waves while that gives one workgroup per CU, two as long as the
 // workgroups of 128 rows leave CUs idle (a triangle: or end unevenly), else one. The figures are those of launch_grads (fhog_split.hip).
 inline int split_grads_waves(const Params& p, int bytes) {

@@ -38,3 +38,23 @@ def test_batched_launch_equals_its_slices(slices, tiles, d, causal):
         for a, b in zip(got, other):
             assert torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1])
     assert all(torch.isfinite(t.float()).all() for t in got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_two_sweeps_in_turn_equal_one_after_the_other(dtype):
+    """Split products at d = 32: 512 workgroups of 128 rows a side take turns with those of the other side, 1040 do not. The first backward of 16-bit tensors
+    has two launches by then, whose dK, dV take the row sums d from the sweep for dQ instead of adding them up in another order: fp32 ones only."""
+    import fhog
+    slices, copies, n, scale = 64, 130, 1019, 32 ** -0.5
+    x = make_case(slices, n, n, 32, dtype, seed=73, grad_std=0.1)
+
+    def outputs(x):
+        o, L = fhog.attention_forward(x["Q"], x["K"], x["V"], scale, True, use_hip=True)
+        first = fhog.attention_backward(x["Q"], x["K"], x["V"], o, x["dO"], L, scale, True, use_hip=True) if dtype == torch.float32 else ()
+        return (*first, *run_fhog(dict(x, O=o, L=L), scale, True))
+
+    got = outputs(x)
+    assert all(torch.isfinite(t.float()).all() for t in got)
+    for s in (0, slices // 2, slices - 1):
+        other = outputs({name: t[s:s + 1].expand(copies, -1, -1).contiguous() for name, t in x.items()})
+        assert all(torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1]) for a, b in zip(got, other))

@@ -58,6 +58,11 @@ int main() {
       using rules::Small;
       for (Small w : {Small::forward, Small::backward, Small::double_backward}) printf("%d ", rules::small_waves(w, batch, n_q, n_k, d, mask, window));
       printf("\n");
+    } else if (!strcmp(what, "few")) {   // passes 3 and 4 with one output to a workgroup, ws: bytes of an element
+      printf("%d\n", rules::few_rows(p, (int)ws));
+    } else if (!strcmp(what, "in_turn")) {   // both sweeps of split products tile by tile; two workgroups of the forward on a CU
+      const int64_t gq = (n_q + 127) / 128 * batch, gk = (n_k + 127) / 128 * batch;
+      printf("%d %d\n", rules::split_in_turn(p, gq, gk), rules::two_forwards_on_a_cu(gq, p.causal));
     } else if (!strcmp(what, "order")) {   // of passes 3 and 4 in one launch
       rules::joint_splits(&a, p, FHOG_PASS_DQ_DDO, &p.n_split, &p.n_split_k);
       rules::grads_order(&a, true, true, p);
@@ -167,3 +172,20 @@ def test_sweeps_of_split_products_in_one_launch_or_apart(ask, bytes_, shape, wav
                                          ((2, 17000, 9000, 32, NONE, 0), (0, 0))])
 def test_order_of_a_shared_launch_of_split_products(ask, shape, order):
     assert tuple(ask("split_order", *shape, 0)) == order
+
+
+@pytest.mark.parametrize("shape,few", [((8, 256, 256, 32, NONE, 0), 1), ((12, 256, 256, 32, NONE, 0), 0), ((8, 512, 512, 32, CAUSAL, 0), 0), ((8, 512, 512, 64, NONE, 0), 1), ((8, 1024, 1024, 64, NONE, 0), 0),
+                                       ((16, 256, 256, 64, NONE, 0), 0), ((4, 1024, 1024, 64, CAUSAL, 0), 1), ((8, 1024, 1024, 64, CAUSAL, 0), 0), ((4, 955, 955, 128, NONE, 0), 1), ((5, 955, 955, 128, NONE, 0), 0),
+                                       ((5, 955, 955, 128, CAUSAL, 0), 1), ((5, 955, 955, 128, CAUSAL, 500), 0), ((16, 256, 256, 128, NONE, 0), 1), ((32, 256, 256, 128, NONE, 0), 0), ((8, 48, 2858, 128, NONE, 0), 1)])
+def test_small_launches_of_fp32_tensors(ask, shape, few):
+    """One output to a workgroup in passes 3 and 4, on both sides of the lines; never for 16-bit tensors."""
+    assert ask("few", *shape, 4) == [few]
+    assert ask("few", *shape, 2) == [0]
+
+
+@pytest.mark.parametrize("shape,picks", [((64, 1024, 1024, 32, CAUSAL, 0), (1, 0)), ((124, 1024, 1024, 32, CAUSAL, 0), (1, 1)), ((125, 1024, 1024, 32, CAUSAL, 0), (0, 1)), ((64, 1024, 1024, 32, NONE, 0), (0, 1)),
+                                         ((64, 1000, 1200, 32, BOTTOM_RIGHT, 0), (0, 0)), ((32, 2000, 2000, 32, CAUSAL, 1000), (1, 0)), ((32, 2000, 2000, 32, CAUSAL, 999), (0, 0)),
+                                         ((32, 1024, 1024, 64, CAUSAL, 0), (0, 0)), ((32, 1024, 1024, 128, NONE, 0), (0, 0)), ((33, 1024, 1024, 128, NONE, 0), (0, 1)), ((65, 1024, 1024, 128, CAUSAL, 0), (0, 1))])
+def test_company_in_launches_of_split_products(ask, shape, picks):
+    """Whether the two sweeps take turns (d = 32), and whether two workgroups of the forward share a CU (fp32, d = 128)."""
+    assert tuple(ask("in_turn", *shape, 0)) == picks
