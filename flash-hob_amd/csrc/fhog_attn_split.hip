@@ -365,11 +365,11 @@ __global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, TWO>)) attn_spl
   attn_run<T, D, MODE, MASK, WS, false, TWO>(p, smem, blockIdx.x, MASK != MASK_NONE && WS == 1 && min_workgroups<T, D, WS, TWO> == 2);
 }
 
-// dQ (workgroups [0, q_blocks)) and dK, dV (the others; mixed: tile by tile in turn) in one launch
-template <typename T, int D, int MASK, int WS>
-__global__ void __launch_bounds__(256, (min_workgroups<T, D, WS, false>)) attn_split_bwd(AttnParams p, int q_blocks, bool mixed) {
+// dQ (workgroups [0, q_blocks)) and dK, dV (the others; mixed: tile by tile in turn) in one launch; ON_CU: workgroups on a CU
+template <typename T, int D, int MASK, int WS, int ON_CU>
+__global__ void __launch_bounds__(256, ON_CU) attn_split_bwd(AttnParams p, int q_blocks, bool mixed) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr bool joins = MASK != MASK_NONE && WS == 1 && min_workgroups<T, D, WS, false> == 2;   // workgroups of a masked launch that share a CU
+  constexpr bool joins = MASK != MASK_NONE && WS == 1 && ON_CU == 2;   // workgroups of a masked launch that share a CU
   int id = blockIdx.x;
   if (first_of_two(q_blocks, (int)gridDim.x - q_blocks, mixed, joins, id)) attn_run<T, D, MODE_BWD_Q, MASK, WS, false>(p, smem, id, joins && !mixed);
   else attn_run<T, D, MODE_BWD_K, MASK, WS, true>(p, smem, id, joins && !mixed);
@@ -396,14 +396,14 @@ hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <typename T, int D, int MASK, int WS>
-hipError_t launch_bwd_ws(const AttnParams& p, hipStream_t s) {
+template <typename T, int D, int MASK, int WS, int ON_CU = min_workgroups<T, D, WS, false>>
+hipError_t launch_bwd_ws(const AttnParams& p, hipStream_t s, bool mixed = false) {
   constexpr int lq = lds_bytes<T, D, MODE_BWD_Q, WS>(), lk = lds_bytes<T, D, MODE_BWD_K, WS>(), smem = lq > lk ? lq : lk;
   static_assert(smem <= 160 * 1024, "stages and exchange buffer have to fit the LDS");
-  const hipError_t e = allow_dynamic_lds<attn_split_bwd<T, D, MASK, WS>>(smem);
+  const hipError_t e = allow_dynamic_lds<attn_split_bwd<T, D, MASK, WS, ON_CU>>(smem);
   if (e != hipSuccess) return e;
   const unsigned gq = blocks<WS>(p.n_q, p.batch), gk = blocks<WS>(p.n_k, p.batch);
-  hipLaunchKernelGGL((attn_split_bwd<T, D, MASK, WS>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq, WS == 1 && rules::split_in_turn(p, gq, gk));
+  hipLaunchKernelGGL((attn_split_bwd<T, D, MASK, WS, ON_CU>), dim3(gq + gk), dim3(256), smem, s, p, (int)gq, mixed);
   return hipGetLastError();
 }
 
@@ -448,7 +448,12 @@ hipError_t launch_bwd(const AttnParams& p, hipStream_t s) {
   if constexpr (lds_bytes<T, D, MODE_BWD_K, 4>() <= 160 * 1024) {
     if (waves == 4) return launch_bwd_ws<T, D, MASK, 4>(p, s);
   }
-  return waves >= 2 ? launch_bwd_ws<T, D, MASK, 2>(p, s) : launch_bwd_ws<T, D, MASK, 1>(p, s);
+  if (waves >= 2) return launch_bwd_ws<T, D, MASK, 2>(p, s);
+  if constexpr (sizeof(T) == 4 && D == 64 && MASK != MASK_NONE) {
+    const rules::Company company = rules::bwd_company(p);
+    return company == rules::Company::none ? launch_bwd_ws<T, D, MASK, 1, 1>(p, s) : launch_bwd_ws<T, D, MASK, 1>(p, s, company == rules::Company::in_turn);
+  }
+  return launch_bwd_ws<T, D, MASK, 1>(p, s, rules::split_in_turn(p, blocks<1>(p.n_q, p.batch), blocks<1>(p.n_k, p.batch)));
 }
 
 template <typename T, int D>

@@ -423,6 +423,25 @@ bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
   return p.d == 32 && p.causal && gq == gk && gq < 1000 && 2 * (int64_t)p.window >= p.n_k;
 }
 
+// First backward of fp32 tensors, both sweeps in one launch with one wave to 32 rows, d = 64 under a mask: whether two workgroups share a CU, and then whether
+// the sweeps take turns. One after the other the heaviest workgroups of both meet on the same CUs. With fewer than two workgroups for every CU a heavy
+// one that is joined by another takes nearly as long as both, while other CUs have one: there each has a CU to itself. Short and even ones
+// are better off in company at any number. Counted are workgroups that see a row. Training step, us, a CU to each | two, one sweep after the other | two, in turn:
+//   causal        10 x 2048 309 | 321 | 325; 17 x 1024 161 | 170 | 171; 30 x 1024 176 | 204 | 179; 3 x 10000 1453 | 1777 | 1594; but 50 x 500 97.7 | 94.3 | 97.4;
+//                 from 480 workgroups on 40 x 700 128 | 138 | 121; 8 x 4096 649 | 747 | 640; 12 x 4096 826 | 773 | 730; 31 x 2048 496 | 453 | 438
+//   window        500, 5 x 4096 157 | 135 | 135; after other keys with up to 128 workgroups of queries 600, 16 x 1000 x 1700 127 | 143 | 143; 800, 14 x 1000 x 2200 142 | 172 | -;
+//                 with more of them 500, 18 x 900 x 1300 142 | 120 | -; 700, 12 x 1500 x 2500 191 | 172 | -; from 480 on 600, 40 x 1100 x 1800 279 | 256 | 231
+//   bottom-right  22 x 1000 x 1300 206 | 212 | 191; 20 x 700 x 1400 193 | 167 | 164; 10 x 3000 x 3500 553 | 599 | 523
+enum class Company { none, two, in_turn };
+inline Company bwd_company(const AttnParams& p) {
+  const Work q = work_of(p, false), k = work_of(p, true);
+  const double groups = (q.live + k.live) * (double)p.batch;
+  if (groups >= 480) return groups < 1024 ? Company::in_turn : Company::two;
+  const int64_t longest = q.longest < k.longest ? q.longest : k.longest;   // the longest workgroup of either side, in tiles
+  if (p.mask_off > 0 && p.window < p.n_k) return q.live * (double)p.batch <= 128 && longest >= 16 ? Company::none : Company::two;
+  return longest >= 19 && 4 * (int64_t)p.mask_off <= p.n_k && 2 * (int64_t)p.window >= p.n_k ? Company::none : Company::two;
+}
+
 // Forward of fp32 tensors, d = 128: two workgroups on a CU once there are more than one for each, under a mask more than two (a heavy and a light tile
 // that share a CU leave the heavy one alone for most of its time). us, one -> two, at so many workgroups: no mask 422 -> 364 (320), 436
 // -> 420 (512), 857 -> 816 (1024), but 234 -> 258 (256); causal 324 -> 290 (640), 466 -> 435 (1024), but 235 -> 260 (512).

@@ -3,7 +3,7 @@ workgroup of an XCD: every tile of every slice is computed, exactly as in a laun
 import pytest
 import torch
 
-from gpu_util import make_case, require_gpu, run_fhog
+from gpu_util import TOL, make_case, require_gpu, run_fhog
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +58,28 @@ def test_two_sweeps_in_turn_equal_one_after_the_other(dtype):
     for s in (0, slices // 2, slices - 1):
         other = outputs({name: t[s:s + 1].expand(copies, -1, -1).contiguous() for name, t in x.items()})
         assert all(torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1]) for a, b in zip(got, other))
+
+
+# fp32 tensors: launches whose workgroups have a CU to themselves, share it with another or take turns by sweep, each against copies
+# of a slice in a launch of another of these kinds, with the two sweeps in one launch in both
+@pytest.mark.parametrize("slices,copies,n_q,n_k,d,causal,window", [(24, 40, 1100, 1100, 64, True, None), (16, 30, 1000, 1700, 64, "bottom_right", 600),
+                                                                   (18, 40, 900, 1300, 64, "bottom_right", 500)])
+def test_company_does_not_change_the_first_backward(slices, copies, n_q, n_k, d, causal, window):
+    import fhog
+    scale = d ** -0.5
+    x = make_case(slices, n_q, n_k, d, torch.float32, seed=75)
+
+    def outputs(x):
+        o, L = fhog.attention_forward(x["Q"], x["K"], x["V"], scale, causal, window=window, use_hip=True)
+        return fhog.attention_backward(x["Q"], x["K"], x["V"], o, x["dO"], L, scale, causal, window=window, use_hip=True)
+
+    got = outputs(x)
+    for s in (0, slices // 2, slices - 1):
+        other = outputs({name: t[s:s + 1].expand(copies, -1, -1).contiguous() for name, t in x.items()})
+        assert all(torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1]) for a, b in zip(got, other))
+    q, k, v = (x[name][-1].double().cpu().requires_grad_(True) for name in ("Q", "K", "V"))
+    i, j = torch.arange(n_q)[:, None] + (n_k - n_q if causal == "bottom_right" else 0), torch.arange(n_k)[None, :]
+    hidden = ((j > i) | (i - j >= (window or n_k))) if causal else torch.zeros(n_q, n_k, dtype=torch.bool)
+    o = torch.softmax((q @ k.T * scale).masked_fill(hidden, float("-inf")), -1) @ v
+    for a, r in zip(got, torch.autograd.grad(o, (q, k, v), x["dO"][-1].double().cpu())):
+        assert (a[-1].double().cpu() - r).abs().max() <= TOL[torch.float32] * r.abs().max()

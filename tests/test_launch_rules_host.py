@@ -54,6 +54,10 @@ int main() {
       AttnParams f = {};
       f.batch = p.batch, f.n_q = p.n_q, f.n_k = p.n_k, f.d = p.d, f.causal = p.causal, f.mask_off = p.mask_off, f.window = p.window;
       printf("%d %d\n", rules::split_bwd_waves(f, (int)ws), rules::split_grads_waves(p, (int)ws));
+    } else if (!strcmp(what, "company")) {   // workgroups of the first backward on a CU, and whether its sweeps take turns
+      AttnParams f = {};
+      f.batch = p.batch, f.n_q = p.n_q, f.n_k = p.n_k, f.d = p.d, f.causal = p.causal, f.mask_off = p.mask_off, f.window = p.window;
+      printf("%d\n", (int)rules::bwd_company(f));
     } else if (!strcmp(what, "small")) {   // waves on the same rows: forward, first backward, double-backward
       using rules::Small;
       for (Small w : {Small::forward, Small::backward, Small::double_backward}) printf("%d ", rules::small_waves(w, batch, n_q, n_k, d, mask, window));
@@ -189,3 +193,15 @@ def test_small_launches_of_fp32_tensors(ask, shape, few):
 def test_company_in_launches_of_split_products(ask, shape, picks):
     """Whether the two sweeps take turns (d = 32), and whether two workgroups of the forward share a CU (fp32, d = 128)."""
     assert tuple(ask("in_turn", *shape, 0)) == picks
+
+
+ALONE, TWO, IN_TURN = range(3)
+
+
+@pytest.mark.parametrize("shape,pick", [((29, 1024, 1024, 64, CAUSAL, 0), ALONE), ((30, 1024, 1024, 64, CAUSAL, 0), IN_TURN), ((63, 1024, 1024, 64, CAUSAL, 0), IN_TURN), ((64, 1024, 1024, 64, CAUSAL, 0), TWO),
+                                        ((40, 600, 600, 64, CAUSAL, 0), ALONE), ((50, 500, 500, 64, CAUSAL, 0), TWO), ((20, 1024, 1024, 64, CAUSAL, 512), ALONE), ((20, 1024, 1024, 64, CAUSAL, 511), TWO),
+                                        ((22, 1000, 1300, 64, BOTTOM_RIGHT, 0), ALONE), ((20, 700, 1400, 64, BOTTOM_RIGHT, 0), TWO), ((16, 1000, 1700, 64, BOTTOM_RIGHT, 600), ALONE),
+                                        ((17, 1000, 1700, 64, BOTTOM_RIGHT, 600), TWO), ((16, 1000, 1700, 64, BOTTOM_RIGHT, 300), TWO), ((40, 1100, 1800, 64, BOTTOM_RIGHT, 600), IN_TURN)])
+def test_company_of_the_first_backward(ask, shape, pick):
+    """fp32 tensors, one launch for both sweeps with one wave to 32 rows."""
+    assert ask("company", *shape, 0) == [pick]
