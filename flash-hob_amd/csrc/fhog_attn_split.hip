@@ -453,6 +453,9 @@ hipError_t launch_bwd(const AttnParams& p, hipStream_t s) {
     const rules::Company company = rules::bwd_company(p);
     return company == rules::Company::none ? launch_bwd_ws<T, D, MASK, 1, 1>(p, s) : launch_bwd_ws<T, D, MASK, 1>(p, s, company == rules::Company::in_turn);
   }
+  if constexpr (sizeof(T) == 4 && D == 32 && MASK == MASK_NONE) {
+    if (rules::bwd_company(p) == rules::Company::three) return launch_bwd_ws<T, D, MASK, 1, 3>(p, s);
+  }
   return launch_bwd_ws<T, D, MASK, 1>(p, s, rules::split_in_turn(p, blocks<1>(p.n_q, p.batch), blocks<1>(p.n_k, p.batch)));
 }
 

@@ -423,7 +423,7 @@ bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
   return p.d == 32 && p.causal && gq == gk && gq < 1000 && 2 * (int64_t)p.window >= p.n_k;
 }
 
-// First backward of fp32 tensors, both sweeps in one launch with one wave to 32 rows, d = 64 under a mask: whether two workgroups share a CU, and then whether
+// First backward of fp32 tensors, both sweeps in one launch with one wave to 32 rows. d = 64 under a mask: whether two workgroups share a CU, and then whether
 // the sweeps take turns. One after the other the heaviest workgroups of both meet on the same CUs. With fewer than two workgroups for every CU a heavy
 // one that is joined by another takes nearly as long as both, while other CUs have one: there each has a CU to itself. Short and even ones
 // are better off in company at any number. Counted are workgroups that see a row. Training step, us, a CU to each | two, one sweep after the other | two, in turn:
@@ -432,8 +432,15 @@ bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
 //   window        500, 5 x 4096 157 | 135 | 135; after other keys with up to 128 workgroups of queries 600, 16 x 1000 x 1700 127 | 143 | 143; 800, 14 x 1000 x 2200 142 | 172 | -;
 //                 with more of them 500, 18 x 900 x 1300 142 | 120 | -; 700, 12 x 1500 x 2500 191 | 172 | -; from 480 on 600, 40 x 1100 x 1800 279 | 256 | 231
 //   bottom-right  22 x 1000 x 1300 206 | 212 | 191; 20 x 700 x 1400 193 | 167 | 164; 10 x 3000 x 3500 553 | 599 | 523
-enum class Company { none, two, in_turn };
+// d = 32 without a mask: three workgroups on a CU (168 registers) where that saves a part of a round; two, which are 2 to 4 % ahead in whole rounds, elsewhere.
+// Two | three: 60 x 500 x 900 130 | 114, 12 x 3000 519 | 499, 24 x 2048 377 | 372, 80 x 1024 293 | 290; but 32 x 1024 127 | 128, 100 x 512 114 | 119, 30 x 1537 314 | 326.
+enum class Company { none, two, in_turn, three };
 inline Company bwd_company(const AttnParams& p) {
+  if (p.d == 32) {
+    const int64_t all = ((int64_t)(p.n_q + 127) / 128 + (p.n_k + 127) / 128) * p.batch;
+    return !p.causal && ((all > 512 && all <= 768) || all > 1024) ? Company::three : Company::two;
+  }
+  if (!p.causal) return Company::two;
   const Work q = work_of(p, false), k = work_of(p, true);
   const double groups = (q.live + k.live) * (double)p.batch;
   if (groups >= 480) return groups < 1024 ? Company::in_turn : Company::two;

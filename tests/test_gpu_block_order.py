@@ -60,10 +60,10 @@ def test_two_sweeps_in_turn_equal_one_after_the_other(dtype):
         assert all(torch.equal(a[s], b[0]) and torch.equal(a[s], b[-1]) for a, b in zip(got, other))
 
 
-# fp32 tensors: launches whose workgroups have a CU to themselves, share it with another or take turns by sweep, each against copies
+# fp32 tensors: launches whose workgroups have a CU to themselves, share it with another, take turns by sweep or share it with two more, each against copies
 # of a slice in a launch of another of these kinds, with the two sweeps in one launch in both
 @pytest.mark.parametrize("slices,copies,n_q,n_k,d,causal,window", [(24, 40, 1100, 1100, 64, True, None), (16, 30, 1000, 1700, 64, "bottom_right", 600),
-                                                                   (18, 40, 900, 1300, 64, "bottom_right", 500)])
+                                                                   (18, 40, 900, 1300, 64, "bottom_right", 500), (30, 45, 1019, 1000, 32, False, None)])
 def test_company_does_not_change_the_first_backward(slices, copies, n_q, n_k, d, causal, window):
     import fhog
     scale = d ** -0.5

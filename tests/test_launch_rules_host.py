@@ -195,13 +195,15 @@ def test_company_in_launches_of_split_products(ask, shape, picks):
     assert tuple(ask("in_turn", *shape, 0)) == picks
 
 
-ALONE, TWO, IN_TURN = range(3)
+ALONE, TWO, IN_TURN, THREE = range(4)
 
 
 @pytest.mark.parametrize("shape,pick", [((29, 1024, 1024, 64, CAUSAL, 0), ALONE), ((30, 1024, 1024, 64, CAUSAL, 0), IN_TURN), ((63, 1024, 1024, 64, CAUSAL, 0), IN_TURN), ((64, 1024, 1024, 64, CAUSAL, 0), TWO),
                                         ((40, 600, 600, 64, CAUSAL, 0), ALONE), ((50, 500, 500, 64, CAUSAL, 0), TWO), ((20, 1024, 1024, 64, CAUSAL, 512), ALONE), ((20, 1024, 1024, 64, CAUSAL, 511), TWO),
                                         ((22, 1000, 1300, 64, BOTTOM_RIGHT, 0), ALONE), ((20, 700, 1400, 64, BOTTOM_RIGHT, 0), TWO), ((16, 1000, 1700, 64, BOTTOM_RIGHT, 600), ALONE),
-                                        ((17, 1000, 1700, 64, BOTTOM_RIGHT, 600), TWO), ((16, 1000, 1700, 64, BOTTOM_RIGHT, 300), TWO), ((40, 1100, 1800, 64, BOTTOM_RIGHT, 600), IN_TURN)])
+                                        ((17, 1000, 1700, 64, BOTTOM_RIGHT, 600), TWO), ((16, 1000, 1700, 64, BOTTOM_RIGHT, 300), TWO), ((40, 1100, 1800, 64, BOTTOM_RIGHT, 600), IN_TURN), ((64, 1024, 1024, 64, NONE, 0), TWO),
+                                        ((32, 1024, 1024, 32, NONE, 0), TWO), ((33, 1024, 1024, 32, NONE, 0), THREE), ((48, 1024, 1024, 32, NONE, 0), THREE), ((49, 1024, 1024, 32, NONE, 0), TWO),
+                                        ((65, 1024, 1024, 32, NONE, 0), THREE), ((33, 1024, 1024, 32, CAUSAL, 0), TWO)])
 def test_company_of_the_first_backward(ask, shape, pick):
     """fp32 tensors, one launch for both sweeps with one wave to 32 rows."""
     assert ask("company", *shape, 0) == [pick]
