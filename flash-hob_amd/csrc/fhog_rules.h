@@ -413,14 +413,15 @@ inline bool few_rows(const Params& p, int bytes) {
 }
 
 // Both sweeps of a launch of split products at d = 32, gq and gk workgroups of one wave to 32 rows, in turn as in mixed_order: the second one's heavy tiles
-// otherwise start when half of the launch is over. Equal sides of fewer than 1000 workgroups under a mask that leaves their work uneven. us, one after
+// otherwise start when half of the launch is over. Equal sides of fewer than 800 workgroups under a mask that leaves their work uneven. us, one after
 // the other -> in turn: double-backward bf16 causal 32 x 1024 104 -> 80, 64 x 1024 137 -> 128, 8 x 4096 440 -> 324, 2 x 17000 1522 -> 1166, window 1200
-// 32 x 2000 190 -> 179, fp32 32 x 2048 516 -> 502; training step bf16 64 x 1024 79 -> 75, 8 x 4096 327 -> 281. Not there: 1024 workgroups 225 -> 224,
-// 3072 1559 -> 1611; bottom-right 32 x 1000 x 1500 127 -> 131; window 500 32 x 1000 x 3000 82 -> 84; four waves on the same rows fp32 16 x 1024 98 -> 106;
-// fp32 d = 64 48 x 1537 889 -> 919, d = 128 32 x 2048 2206 -> 2247, where a CU has one workgroup.
+// 32 x 2000 190 -> 179, fp32 32 x 2048 516 -> 502; training step bf16 64 x 1024 79 -> 75, 8 x 4096 327 -> 281. Not there: 960 workgroups 120 x 900 174 -> 178,
+// 1024 225 -> 224, 3072 1559 -> 1611; bottom-right 32 x 1000 x 1500 127 -> 131; window 550 40 x 1000 73 -> 76, 500 32 x 1000 x 3000 82 -> 84; four waves on the
+// same rows fp32 16 x 1024 98 -> 106; fp32 d = 64 48 x 1537 889 -> 919, d = 128 32 x 2048 2206 -> 2247, where a CU has one workgroup. Two tiles of rows leave little
+// to even out, three or four only launches that end soon: bf16 150 x 256 31 -> 36, 200 x 300 53 -> 57, fp32 198 x 402 189 -> 199; but 87 x 384 42 -> 37, 150 x 450 76 -> 72.
 template <typename P>
 bool split_in_turn(const P& p, int64_t gq, int64_t gk) {
-  return p.d == 32 && p.causal && gq == gk && gq < 1000 && 2 * (int64_t)p.window >= p.n_k;
+  return p.d == 32 && p.causal && gq == gk && gq < (p.n_k >= 450 ? 800 : p.n_k > 256 ? 320 : 0) && 5 * (int64_t)p.window >= 3 * (int64_t)p.n_k;
 }
 
 // First backward of fp32 tensors, both sweeps in one launch with one wave to 32 rows. d = 64 under a mask: whether two workgroups share a CU, and then whether

@@ -187,8 +187,9 @@ def test_small_launches_of_fp32_tensors(ask, shape, few):
     assert ask("few", *shape, 2) == [0]
 
 
-@pytest.mark.parametrize("shape,picks", [((64, 1024, 1024, 32, CAUSAL, 0), (1, 0)), ((124, 1024, 1024, 32, CAUSAL, 0), (1, 1)), ((125, 1024, 1024, 32, CAUSAL, 0), (0, 1)), ((64, 1024, 1024, 32, NONE, 0), (0, 1)),
-                                         ((64, 1000, 1200, 32, BOTTOM_RIGHT, 0), (0, 0)), ((32, 2000, 2000, 32, CAUSAL, 1000), (1, 0)), ((32, 2000, 2000, 32, CAUSAL, 999), (0, 0)),
+@pytest.mark.parametrize("shape,picks", [((64, 1024, 1024, 32, CAUSAL, 0), (1, 0)), ((99, 1024, 1024, 32, CAUSAL, 0), (1, 1)), ((100, 1024, 1024, 32, CAUSAL, 0), (0, 1)), ((64, 1024, 1024, 32, NONE, 0), (0, 1)),
+                                         ((64, 1000, 1200, 32, BOTTOM_RIGHT, 0), (0, 0)), ((32, 2000, 2000, 32, CAUSAL, 1200), (1, 0)), ((32, 2000, 2000, 32, CAUSAL, 1199), (0, 0)),
+                                         ((150, 450, 450, 32, CAUSAL, 0), (1, 1)), ((150, 449, 449, 32, CAUSAL, 0), (0, 1)), ((106, 384, 384, 32, CAUSAL, 0), (1, 0)), ((107, 384, 384, 32, CAUSAL, 0), (0, 0)), ((150, 256, 256, 32, CAUSAL, 0), (0, 0)),
                                          ((32, 1024, 1024, 64, CAUSAL, 0), (0, 0)), ((32, 1024, 1024, 128, NONE, 0), (0, 0)), ((33, 1024, 1024, 128, NONE, 0), (0, 1)), ((65, 1024, 1024, 128, CAUSAL, 0), (0, 1))])
 def test_company_in_launches_of_split_products(ask, shape, picks):
     """Whether the two sweeps take turns (d = 32), and whether two workgroups of the forward share a CU (fp32, d = 128)."""
