@@ -19,13 +19,13 @@
 // arithmetic 810, barrier 360 (splitting by itself: 1140 and 370 of requests more). Double-backward, us, without -> so: fp32 causal
 // 32 x 2048 d = 128 pass 5 629 -> 561, passes 3 and 4 2021 -> 1978; d = 64 941 -> 920; no mask 40 x 1024, d = 64 704 -> 677; two workgroups of pass 5 on a
 // CU (d = 64, numbers split again for every tile): 226 -> 319.
-// Some do not quite fit the register file and keep VGPRs of a
-// lane in scratch memory through the sweep: fp32 tensors in passes 3 and 4 at d = 128 62 to 72, at d = 64 with four waves on the same
-// rows 43 to 46, with one at d = 32 6 to 8; 16-bit tensors at d = 128 up to 53.
+// Some do not quite fit the register file and keep bytes of a lane in scratch memory (spilled VGPRs as the compiler counts them, one that is spilled twice
+// as two): fp32 tensors in passes 3 and 4 at d = 128 312 without a mask and 264 with one (110, 103), at d = 64 in the launch with two waves on the
+// same rows beside four 160 and 208 (45, 51), with one wave at d = 32 24 and 40 (6, 11); 16-bit tensors at d = 128 up to 212 (52).
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
 //   bf16 causal 64 x 1024, d = 32: 734 -> 121     fp32 causal 64 x 1024, d = 32: 672 -> 279
 //   fp32 causal 32 x 2048, d = 64: 2101 -> 915    fp32 64 x 2048, d = 64: 7521 -> 3490
-//   fp32 causal 32 x 2048, d = 128: 3833 -> 2300
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2165
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
@@ -415,7 +415,9 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
   if (!DIRECT) __syncthreads();
   // Without a mask only waves whose rows all lie past the end of the tensor see nothing. At d = 32 they have a loop of their own, for the test in the loop
   // costs every length: double-backward, us, neither | the test | two loops: bf16 16 x 4096 701 | 710 | 697, 64 x 1024 183 | 185 | 183, fp32 16 x 1000 159 |
-  // 163 | 160, 16 x 4096 1835 | 1836 | 1822, 128 x 300 124 | 119 | 118. At d = 64 the test is the faster (fp32 16 x 2048 878 | 888).
+  // 163 | 160, 16 x 4096 1835 | 1836 | 1822, 128 x 300 124 | 119 | 118. At d = 64 the test is the faster (fp32 16 x 2048 878 | 888), and in passes 3 and 4
+  // of fp32 tensors at d = 128, which spill less with its branch, whichever mask. Double-backward, us, every tile computed | the test: no mask 32 x 2048 4131 |
+  // 3986, 40 x 300 199 | 193, 2000 | 900 rows 1524 | 1459; causal 32 x 2048 2262 | 2156, 48 x 1537 2244 | 2130; window 700 16 x 1000 x 3000 569 | 541.
   constexpr bool NO_TEST = MASK == MASK_NONE && D == 32;
   const auto sweep = [&](auto has_rows) {
     const auto works = [&](int s0) { return NO_TEST ? decltype(has_rows)::value : !geo.dead(s0, geo.first_row(rw, n_sta)); };
@@ -441,7 +443,7 @@ __device__ __forceinline__ void split_run(const Params& p, char* smem, int id, b
           if (more) fetch(t + WS);
         };
         if (!LATE) next();
-        if ((WS == 1 || t + ws < t_end) && ((RAW && !STATS) || works(s0))) {
+        if ((WS == 1 || t + ws < t_end) && works(s0)) {
           block(smem + (buf * WS + ws) * STAGE, s0, [&]() {
             if (LATE) {
               __builtin_amdgcn_sched_barrier(0);
