@@ -8,7 +8,7 @@
 // LDS in 32-row tiles that are split once per workgroup. A lane owns ONE stationary row: in the forward the running maximum,
 // the running sum and the rescaling factor of a query are per-lane scalars. Two terms per fp32 operand less than the
 // double-backward needs leave room for the terms of d = 128 (one wave per SIMD); only dK, dV on fp32 tensors there does not quite
-// fit and keeps 43 to 118 VGPRs of a lane in scratch memory under a mask or with two waves on the same rows.
+// fit and keeps 42 to 118 VGPRs of a lane in scratch memory under a mask or with two waves on the same rows.
 // Small launches (WS = 2 or 4) put WS waves on the same 32 rows: each takes every WS-th streamed tile, and the partial
 // results are merged through LDS in a fixed order. dQ and dK, dV share a launch unless each fills the GPU (launch_bwd).
 #include <type_traits>
@@ -23,7 +23,7 @@ namespace {
 constexpr int MODE_FWD = 0, MODE_BWD_Q = 1, MODE_BWD_K = 2;
 
 // Workgroups on a CU that the registers are to leave room for. At d = 64 two keep a SIMD busy where one waits (for LDS operands, the
-// splitting, a barrier): everything fits 256 registers. us, one -> two, fp32 causal 32 x 2048 | no mask 64 x 2048: forward 146 -> 128 |
+// splitting, a barrier): 256 registers each, short of 2 (no mask) and 8 where dQ and dK, dV share a launch. us, one -> two, fp32 causal 32 x 2048 | no mask 64 x 2048: forward 146 -> 128 |
 // 410 -> 368, dQ 193 -> 158 | 528 -> 495, dK, dV 238 -> 209 | 783 -> 648. At d = 128 so does the forward (TWO), without the second stage of
 // the ring and with the query's numbers instead of their terms; worth it in launches with work for two on every CU (launch_fwd). At d = 32 also with
 // waves on the same rows: first backward of fp32 causal 16 x 1024, four of them, 53 us with two workgroups and 66 with one.

@@ -395,9 +395,10 @@ inline bool apart_is_faster(const P& p, int waves, int most_waves, bool two_on_a
 //   d = 32   2 x 256 22.3 -> 19.9 | 22.5 -> 20.3; 4 x 512 34.7 -> 29.7 | 35.1 -> 30.1; beyond: 8 x 512 35.3 -> 41.6 | 35.4 -> 36.8
 //   d = 64   2 x 256 44.5 -> 31.3 | 43.8 -> 31.1; 2 x 1024 138 -> 82 | 136 -> 80; 4 x 1024 138 -> 123 | 137 -> 98; 1 x 4096 506 -> 430 | 497 -> 326; beyond:
 //            8 x 1024 170 -> 233 | 134 -> 137; two rounds of short streams: 16 x 256 45.2 -> 46.2, 53 x 50 1.2 to 1
-//   d = 128  2 x 256 132 -> 73 | 136 -> 74; 2 x 1024 462 -> 241 | 472 -> 239; 16 x 256 136 -> 109 | 140 -> 92; 1 x 4096 1781 -> 1385 | 1816 -> 1094; beyond:
-//            8 x 1024 465 -> 639 | 477 -> 406
-// 600 shapes of 1 to 96 slices with 24 to 12000 rows: the 262 that this picks take 0.41 to 1.0 times as long, 46 of the others would take less than 0.9.
+//   d = 128  14 x 256 128 -> 107 | 126 -> 91; 4 x 1024 432 -> 362 | 429 -> 292; 2 x 2048 837 -> 702 | 836 -> 555; 1 x 4096 1647 -> 1380 | 1644 -> 1087; beyond:
+//            7 x 1024 435 -> 609 | 433 -> 384; 27 x 256 131 -> 179 | 131 -> 130; 2 x 4096 1658 -> 2481 | 1649 -> 1502
+// 274 shapes around the lines, of 1 to 56 slices with 32 to 4096 rows: the 131 that this picks take 0.51 to 1.02 times as long, 12 of the others would take
+// less than 0.9, most of them triangles with up to a fifth more workgroups than the line.
 // The count is that of both sides also where one is launched alone: passes 3 and 4 have the same bits apart.
 inline bool few_rows(const Params& p, int bytes) {
   if (bytes != 4) return false;

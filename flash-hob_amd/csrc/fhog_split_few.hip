@@ -8,7 +8,8 @@
 //
 // A wave takes every W-th streamed tile by itself. Its rows come straight into registers, two k-steps ahead, which is how the first level reads them; split
 // into terms, those of the tensors that the second level contracts with are left in LDS of the wave's own for the transposing reads. So
-// the sweep has no barrier; the partial results of the W waves are added through LDS in their order.
+// the sweep has no barrier; the partial results of the W waves are added through LDS in their order. At d = 128 a lane keeps 36 VGPRs (132 bytes) in
+// scratch memory.
 #include <type_traits>
 
 #include "fhog_rules.h"
