@@ -23,9 +23,9 @@
 // as two): fp32 tensors in passes 3 and 4 at d = 128 312 without a mask and 264 with one (110, 103), at d = 64 in the launch with two waves on the
 // same rows beside four 160 and 208 (45, 51), with one wave at d = 32 24 and 40 (6, 11); 16-bit tensors at d = 128 up to 212 (52).
 // Whole chain, us, against kernels on v_mfma_f32_32x32x2_f32 with the same tiling (same card):
-//   bf16 causal 64 x 1024, d = 32: 734 -> 121     fp32 causal 64 x 1024, d = 32: 672 -> 279
-//   fp32 causal 32 x 2048, d = 64: 2101 -> 915    fp32 64 x 2048, d = 64: 7521 -> 3490
-//   fp32 causal 32 x 2048, d = 128: 3833 -> 2165
+//   bf16 causal 64 x 1024, d = 32: 734 -> 122     fp32 causal 64 x 1024, d = 32: 672 -> 272
+//   fp32 causal 32 x 2048, d = 64: 2101 -> 919    fp32 64 x 2048, d = 64: 7521 -> 3453
+//   fp32 causal 32 x 2048, d = 128: 3833 -> 2190
 // and no result is less accurate: against fp64, fp32 outputs are off by 3e-7 to 1.2e-6 (2-norm) either way.
 //
 // Math per tile pair (fhog/triton_bwdbwd.py:194-202, 229-243, 266-288, 485-507), with u = dP - d, w = ddS - dd:
